@@ -5,19 +5,32 @@
 //
 //   key(x)  = the 32-bit pattern of x mapped monotonically to an unsigned integer (-0 = +0;
 //             NaN maps to 0, below every number, so a NaN is chosen only when nothing else is left)
-//   T       = the k-th largest key, found by a radix select: four passes over the row, most
-//             significant byte first, each a 256-bin histogram of the keys that share the prefix
-//             found so far, and a scan from the top bin for the bin that holds the k-th key
+//   T       = the k-th largest key
 //   chosen  = keys > T, plus the first (k - #greater) keys == T in index order
 //
-// One workgroup of 1024 lanes per request. Rows of up to 32768 scores are held in registers: lane
-// t owns the consecutive entries [t*P, (t+1)*P) (P = 4, 8, 16 or 32), read once with all loads in
-// flight; the histograms are LDS atomics into 8 interleaved copies of the 256 bins (scores share
-// few exponents, so a single copy would serialise on two or three bins); the output needs one
-// workgroup-wide exclusive scan of the lanes' counts, after which every lane writes its chosen
-// entries in order. Longer rows are read five times from memory (four histograms, one output
-// pass walking the row 1024 entries per round with a prefix count per round). Either way the
-// output order does not depend on timing.
+// One workgroup of 1024 lanes per request: nothing outside the outputs can be written, so the CUs of the chip cannot
+// share a row. What bounds it is the vector ALU of that one CU (64 lanes a clock: one instruction per entry of a row
+// of 65536 is 0.43 us) and the chain of barriers, so an entry is touched by as few instructions as possible:
+//
+//   pivot    an eighth of the row (spread evenly) goes into a histogram of 4096 key ranges; the rank in it that leaves
+//            1.5 times the wanted entries plus four standard deviations of an independent sample gives a lower bound
+//   collect  entries >= pivot, compared as floats, are appended to a list in LDS (about 3700 for k = 2048)
+//   select   the list's keys are counted by their distance from the pivot, 2^13 keys to a bin; the few keys in the
+//            bin of the k-th largest are sorted out bit by bit. Chosen entries become bits of a bitmap of the row,
+//            whose words are placed in the output by a workgroup-wide scan
+//
+// If the list turns out shorter than k or longer than it may be (rows of few distinct values, a sample that
+// misled), and for rows of up to 8192 entries or k above 3072, the whole row is searched instead: a radix select with
+// digits of 11, 11 and 10 bits, most significant first, which stops as soon as all keys of a digit's bin are wanted.
+//
+// Rows of up to 65536 scores are held in registers, in words of 64 consecutive entries (a load instruction fetches
+// 256 consecutive bytes; with 16-byte pieces of 64 different lines, as each lane owning consecutive entries asks for,
+// the row came through L1 eight times). Longer rows are read again by each step. The output never depends on timing.
+//
+// Measured (us; one row unless stated, k = 2048; radix select over four 8-bit digits before): n = 16384 10.2 -> 8.1,
+// 32768 19.3 -> 9.4, 64 rows of it 20.2 -> 10.9; 24 rows of 33024 62.9 -> 12.0; n = 65536 115 -> 13.4; 131072
+// 220 -> 20.3. Constant rows, which the whole-row search takes: n = 16384 13.9 -> 16.6, 32768 26 -> 21, 65536 266 -> 32.
+//
 // Entries beyond a request's valid length (lengths[b], optional) are not candidates; if fewer
 // than k candidates exist the remaining outputs are -1, which the attention treats as padding.
 #include <hip/hip_runtime.h>
@@ -30,12 +43,22 @@ namespace {
 constexpr int SELECT_THREADS = 1024;
 constexpr int SELECT_WAVES = SELECT_THREADS / 64;
 
+template <int N>
+struct IntConstant {
+    static constexpr int value = N;
+};
+
 __device__ __forceinline__ uint32_t score_key(float x) {
     if (x != x) return 0u;
     x += 0.f;  // -0 -> +0
     const uint32_t u = __float_as_uint(x);
     // monotone in the float order; the smallest number (-inf) maps to 0x007fffff, above NaN's 0
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// the score with the smallest key that is at least `key` (key above that of -inf)
+__device__ __forceinline__ float key_score(uint32_t key) {
+    return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
 
 // Inclusive prefix sum over the lanes of a wavefront: running sums inside each row of 16 lanes on DPP row
@@ -55,256 +78,454 @@ __device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
     return v + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
+// Sum of the entries of `sums` before entry `wave` (uniform). The 16 entries are scanned by the lanes of a row.
+__device__ __forceinline__ int sum_before(const int* sums, int wave, int lane) {
+    static_assert(SELECT_WAVES == 16, "one row of 16 lanes");
+    int v = sums[lane & 15];
+#define ROW_SHR_ADD(n) v += __builtin_amdgcn_update_dpp(0, v, 0x110 + (n), 0xf, 0xf, false);
+    ROW_SHR_ADD(1)
+    ROW_SHR_ADD(2)
+    ROW_SHR_ADD(4)
+    ROW_SHR_ADD(8)
+#undef ROW_SHR_ADD
+    const int before = __builtin_amdgcn_readlane(v, wave == 0 ? 0 : wave - 1);
+    return wave == 0 ? 0 : before;
+}
+
+constexpr int DIGIT_BINS = 2048;    // the digits of a key are 11, 11 and 10 bits
+constexpr int SAMPLE_BITS = 12;     // of the histogram of the sample
+constexpr int MAX_CANDIDATES = 6144;
+constexpr int MAX_FILTER_WANT = 3072;   // (1.5 times it and the margin of the sample stay below MAX_CANDIDATES)
+constexpr int MAX_FILTER_ROW = 262144;  // entries the two bitmaps of the filter can be made for
+
+// Of a word of 32 or 64 flags keep the `take` lowest that are set (take < number set)
+template <typename Word>
+__device__ __forceinline__ Word lowest_set(Word w, int take) {
+    int low = 0;  // the most bits of the word that hold at most `take` flags
+#pragma unroll
+    for (int step = 4 * sizeof(Word); step >= 1; step >>= 1)
+        if (__popcll(w & (((Word)1 << (low + step)) - 1)) <= take) low += step;
+    return w & (((Word)1 << low) - 1);
+}
+
+// P words of 64 entries per wavefront; the row is taken in chunks of CHUNK = 1024 * P entries. RESIDENT: one chunk
+// holds the whole row and stays in registers; else the row is read again by every step.
+template <int P, bool RESIDENT>
 __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     const float* __restrict__ scores, const int* __restrict__ lengths, int* __restrict__ idx_out,
     int n, int k) {
-    __shared__ int s_hist[256];
-    __shared__ uint32_t s_prefix;   // key bits fixed so far
-    __shared__ int s_remaining;     // how many more keys are wanted from the bins below the prefix
-    __shared__ int s_wave_gt[2][SELECT_WAVES];
-    __shared__ int s_wave_eq[2][SELECT_WAVES];
+    constexpr int CHUNK = SELECT_THREADS * P;
+    constexpr int GROUP = P < 8 ? P : 8;  // words handled under one test of the row's end
+    constexpr bool FILTER = P >= 16;
+    constexpr int HIST_COPIES = FILTER ? 2 : 4;  // of the first digit's histogram
+    __shared__ __attribute__((aligned(16))) int s_hist[DIGIT_BINS * HIST_COPIES];  // [bin][copy]
+    __shared__ int s_wave_sum[2][SELECT_WAVES];
+    __shared__ int s_bin, s_above, s_in_bin, s_count, s_near_count;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = blockIdx.x;
     const float* row = scores + (size_t)b * n;
     int valid = lengths != nullptr ? lengths[b] : n;
     valid = valid < 0 ? 0 : (valid > n ? n : valid);
     const int want = k < valid ? k : valid;  // entries that will be chosen
+    int* dst = idx_out + (size_t)b * k;
+    for (int j = want + tid; j < k; j += SELECT_THREADS) dst[j] = -1;
+    if (want == 0) return;
 
-    if (tid == 0) {
-        s_prefix = 0u;
-        s_remaining = want;
-    }
-    // radix select of the want-th largest key, most significant byte first
-    for (int pass = 0; pass < 4 && want > 0; ++pass) {
-        const int shift = 24 - 8 * pass;
-        if (tid < 256) s_hist[tid] = 0;
-        __syncthreads();
-        const uint32_t prefix = s_prefix;
-        const uint32_t prefix_mask = pass == 0 ? 0u : 0xffffffffu << (shift + 8);
-        for (int base = 0; base < valid; base += SELECT_THREADS) {
-            const int i = base + tid;
-            uint32_t bin = 0u;
-            bool active = false;
-            if (i < valid) {
-                const uint32_t key = score_key(row[i]);
-                active = (key & prefix_mask) == prefix;
-                bin = (key >> shift) & 255u;
-            }
-            if (active) atomicAdd(&s_hist[bin], 1);
-        }
-        __syncthreads();
-        if (wave == 0) {
-            // lane l owns bins 255-4l .. 252-4l (descending); suffix counts from the top bin
-            int c[4];
-            int mine = 0;
+    // Word j of this wavefront in chunk c: entries first + 64*j .. first + 64*j + 63, one per lane, with
+    // first = c*CHUNK + wave*64*P. `left` entries of the wavefront's span exist (uniform); lanes past the end hold NaN.
+    const int span = wave * 64 * P;
+    auto load_chunk = [&](float (&val)[P], int first, int left) {
+        const float* src = row + first;
+        if (left >= 64 * P) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                c[j] = s_hist[255 - 4 * lane - j];
-                mine += c[j];
-            }
-            int above = mine;  // inclusive scan over lanes (lane 0 = top bins)
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int v = __shfl_up(above, d);
-                if (lane >= d) above += v;
-            }
-            above -= mine;  // keys in bins above this lane's four
-            const int remaining = s_remaining;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                // the bin where the running count reaches `remaining` holds the wanted key
-                if (above < remaining && above + c[j] >= remaining) {
-                    s_prefix = prefix | ((uint32_t)(255 - 4 * lane - j) << shift);
-                    s_remaining = remaining - above;
-                }
-                above += c[j];
-            }
-        }
-        __syncthreads();
-    }
-    const uint32_t threshold = s_prefix;  // the want-th largest key
-    const int need_eq = s_remaining;      // how many keys equal to it are chosen (>= 1 if want > 0)
-
-    // output pass in index order
-    int run_gt = 0, run_eq = 0;
-    const unsigned long long below = (1ull << lane) - 1ull;
-    int round = 0;
-    for (int base = 0; base < valid && want > 0; base += SELECT_THREADS, ++round) {
-        const int i = base + tid;
-        bool gt = false, eq = false;
-        if (i < valid) {
-            const uint32_t key = score_key(row[i]);
-            gt = key > threshold;
-            eq = key == threshold;
-        }
-        const unsigned long long m_gt = __ballot(gt);
-        const unsigned long long m_eq = __ballot(eq);
-        const int buf = round & 1;
-        if (lane == 0) {
-            s_wave_gt[buf][wave] = __popcll(m_gt);
-            s_wave_eq[buf][wave] = __popcll(m_eq);
-        }
-        __syncthreads();  // (one barrier per round: the two buffers alternate)
-        int gt_before = run_gt + __popcll(m_gt & below);
-        int eq_before = run_eq + __popcll(m_eq & below);
-        int tot_gt = 0, tot_eq = 0;
-#pragma unroll
-        for (int w = 0; w < SELECT_WAVES; ++w) {
-            const int g = s_wave_gt[buf][w];
-            const int e = s_wave_eq[buf][w];
-            if (w < wave) {
-                gt_before += g;
-                eq_before += e;
-            }
-            tot_gt += g;
-            tot_eq += e;
-        }
-        if (gt || (eq && eq_before < need_eq)) {
-            const int pos = gt_before + (eq_before < need_eq ? eq_before : need_eq);
-            idx_out[(size_t)b * k + pos] = i;
-        }
-        run_gt += tot_gt;
-        run_eq += tot_eq;
-    }
-    for (int j = want + tid; j < k; j += SELECT_THREADS) idx_out[(size_t)b * k + j] = -1;
-}
-
-constexpr int HIST_COPIES = 8;
-
-// P entries per lane, row in registers (n <= 1024 * P)
-template <int P>
-__global__ __launch_bounds__(SELECT_THREADS) void topk_select_regs_kernel(
-    const float* __restrict__ scores, const int* __restrict__ lengths, int* __restrict__ idx_out,
-    int n, int k) {
-    __shared__ int s_hist[256 * HIST_COPIES];  // [bin][copy]: the copies of a bin sit in different banks
-    __shared__ uint32_t s_prefix;
-    __shared__ int s_remaining;
-    __shared__ int s_wave_gt[SELECT_WAVES];
-    __shared__ int s_wave_eq[SELECT_WAVES];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int b = blockIdx.x;
-    const float* row = scores + (size_t)b * n;
-    int valid = lengths != nullptr ? lengths[b] : n;
-    valid = valid < 0 ? 0 : (valid > n ? n : valid);
-    const int want = k < valid ? k : valid;
-    const int first = tid * P;
-
-    // Keys of this lane's entries; entries that are no candidates are marked in `live`.
-    uint32_t key[P];
-    uint32_t live = 0u;
-    if (first + P <= n && (reinterpret_cast<uintptr_t>(row + first) & 15u) == 0) {
-        typedef float floatx4 __attribute__((ext_vector_type(4)));
-        floatx4 v[P / 4];
-#pragma unroll
-        for (int j = 0; j < P / 4; ++j) v[j] = reinterpret_cast<const floatx4*>(row + first)[j];
-#pragma unroll
-        for (int j = 0; j < P; ++j) key[j] = score_key(v[j / 4][j % 4]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < P; ++j) key[j] = first + j < n ? score_key(row[first + j]) : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < P; ++j) live |= (first + j < valid ? 1u : 0u) << j;
-    // Entries that are no candidates get the smallest key: the passes below then need no test of `live`
-    // (such an entry lands in the lowest bin of every digit, below the `want` largest live keys, or among
-    // the ties of key 0, of which the emission takes live ones only).
-#pragma unroll
-    for (int j = 0; j < P; ++j) key[j] = ((live >> j) & 1u) ? key[j] : 0u;
-
-    if (tid == 0) {
-        s_prefix = 0u;
-        s_remaining = want;
-    }
-    const int copy = lane & (HIST_COPIES - 1);
-    for (int pass = 0; pass < 4 && want > 0; ++pass) {
-        const int shift = 24 - 8 * pass;
-        for (int i = tid; i < 256 * HIST_COPIES; i += SELECT_THREADS) s_hist[i] = 0;
-        __syncthreads();
-        const uint32_t prefix = s_prefix;
-        const uint32_t prefix_mask = pass == 0 ? 0u : 0xffffffffu << (shift + 8);
-        if (pass == 0) {
-#pragma unroll
-            for (int j = 0; j < P; ++j) atomicAdd(&s_hist[(key[j] >> 24) * HIST_COPIES + copy], 1);
+            for (int j = 0; j < P; ++j) val[j] = src[64 * j + lane];
         } else {
 #pragma unroll
-            for (int j = 0; j < P; ++j) {
-                if ((key[j] & prefix_mask) == prefix)
-                    atomicAdd(&s_hist[((key[j] >> shift) & 255u) * HIST_COPIES + copy], 1);
-            }
-        }
-        __syncthreads();
-        if (wave == 0) {
-            int c[4];
-            int mine = 0;
+            for (int g = 0; g < P; g += GROUP) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int bin = 255 - 4 * lane - j;
-                c[j] = 0;
+                for (int j = g; j < g + GROUP; ++j) val[j] = __builtin_nanf("");
+                if (64 * g < left) {
 #pragma unroll
-                for (int h = 0; h < HIST_COPIES; ++h) c[j] += s_hist[bin * HIST_COPIES + h];
-                mine += c[j];
-            }
-            int above = wave_inclusive_sum(mine, lane) - mine;
-            const int remaining = s_remaining;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (above < remaining && above + c[j] >= remaining) {
-                    s_prefix = prefix | ((uint32_t)(255 - 4 * lane - j) << shift);
-                    s_remaining = remaining - above;
+                    for (int j = g; j < g + GROUP; ++j) {
+                        const int i = 64 * j + lane;
+                        const float v = src[i < left ? i : 0];
+                        val[j] = i < left ? v : __builtin_nanf("");
+                    }
                 }
-                above += c[j];
             }
         }
-        __syncthreads();
-    }
-    const uint32_t threshold = s_prefix;
-    const int need_eq = s_remaining;
-
-    if (want > 0) {
-        int n_gt = 0, n_eq = 0;
+    };
+    // f(g) for the groups of words g .. g + GROUP - 1 of the span that hold entries of the row
+    auto for_groups = [&](int left, auto f) {
 #pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const bool on = (live >> j) & 1u;
-            n_gt += (on && key[j] > threshold) ? 1 : 0;
-            n_eq += (on && key[j] == threshold) ? 1 : 0;
+        for (int g = 0; g < P; g += GROUP)
+            if (64 * g < left) f(g);
+    };
+    auto clear_hist = [&](int words) {
+        for (int i = tid; i < words / 4; i += SELECT_THREADS) reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
+    };
+    // In the histogram of 2^BITS bins x COPIES: the bin in which the rank-th largest key lies (counting from the top
+    // bin down), the keys in bins above it and in it; bin = -1 if there are fewer than `rank` keys.
+    auto find_bin = [&](auto bits_tag, auto copies_tag, int rank, int& bin, int& above_bin, int& in_bin) {
+        constexpr int BINS = 1 << decltype(bits_tag)::value;
+        constexpr int COPIES = decltype(copies_tag)::value;
+        constexpr int PER = BINS / SELECT_THREADS;  // bins of a lane
+        if (tid == 0) s_bin = -1;
+        __syncthreads();  // the counts are complete
+        int c[PER];
+        int mine = 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            c[j] = 0;
+#pragma unroll
+            for (int h = 0; h < COPIES; ++h) c[j] += s_hist[(BINS - 1 - (PER * tid + j)) * COPIES + h];
+            mine += c[j];
         }
-        // exclusive scan of (n_gt, n_eq) over the 1024 lanes, in lane order = index order
-        // (both counts fit 16 bits: one scan of the packed pair)
-        const int packed_before = wave_inclusive_sum(n_gt | (n_eq << 16), lane);
-        int gt_before = packed_before & 0xffff, eq_before = packed_before >> 16;
-        if (lane == 63) {
-            s_wave_gt[wave] = gt_before;
-            s_wave_eq[wave] = eq_before;
-        }
-        gt_before -= n_gt;
-        eq_before -= n_eq;
+        const int upto = wave_inclusive_sum(mine, lane);
+        if (lane == 63) s_wave_sum[0][wave] = upto;
         __syncthreads();
+        int above = upto - mine + sum_before(s_wave_sum[0], wave, lane);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (above < rank && above + c[j] >= rank) {  // one bin of the workgroup
+                s_bin = BINS - 1 - (PER * tid + j);
+                s_above = above;
+                s_in_bin = c[j];
+            }
+            above += c[j];
+        }
+        __syncthreads();
+        bin = s_bin, above_bin = s_above, in_bin = s_in_bin;
+    };
+    // The want-th largest key (`threshold`) and how many of the keys equal to it are chosen, most significant digit
+    // first; if all keys of a digit's bin are wanted the digits below do not matter and the threshold is the bin's
+    // lowest key. count(shift_tag, bits_tag, copies_tag, threshold) adds the keys that share the digits found so far
+    // to the histogram.
+    auto radix_select = [&](auto copies_tag, auto count, uint32_t& threshold, int& need_eq) {
+        threshold = 0u;
+        int remaining = want;
+        auto digit = [&](auto shift_tag, auto bits_tag, auto copies) {
+            clear_hist((1 << decltype(bits_tag)::value) * decltype(copies)::value);
+            __syncthreads();
+            count(shift_tag, bits_tag, copies, threshold);
+            int bin, above, in_bin;
+            find_bin(bits_tag, copies, remaining, bin, above, in_bin);
+            threshold |= (uint32_t)bin << decltype(shift_tag)::value;
+            remaining -= above;
+            return in_bin == remaining;
+        };
+        bool done = digit(IntConstant<21>{}, IntConstant<11>{}, copies_tag);
+        if (!done) done = digit(IntConstant<10>{}, IntConstant<11>{}, IntConstant<1>{});
+        if (!done) done = digit(IntConstant<0>{}, IntConstant<10>{}, IntConstant<1>{});
+        need_eq = done ? valid : remaining;
+    };
+
+    float val[P];
+    if (RESIDENT) load_chunk(val, span, valid - span);
+
+    if constexpr (FILTER) {
+        constexpr int BITMAP = (RESIDENT ? CHUNK : MAX_FILTER_ROW) / 32;
+        __shared__ uint2 s_list[MAX_CANDIDATES];  // (score bits, index), in no particular order
+        __shared__ uint32_t s_gt[BITMAP], s_eq[BITMAP];
+        if (want <= MAX_FILTER_WANT && want < valid && (RESIDENT || valid <= MAX_FILTER_ROW)) {
+            // An eighth of the row, spread evenly: lane l takes word g + l % 8 of every group of words.
+            clear_hist(1 << SAMPLE_BITS);
+            if (tid == 0) s_count = s_near_count = 0;
+            const int words = (valid + 31) / 32;
+            for (int i = tid; i < words; i += SELECT_THREADS) s_gt[i] = s_eq[i] = 0u;
+            __syncthreads();
+            for (int c0 = 0; c0 < valid; c0 += CHUNK) {
+                const int left = valid - c0 - span;
+                if constexpr (RESIDENT) {
+                    for_groups(left, [&](int g) {
+                        float v = val[g];
+#pragma unroll
+                        for (int j = 1; j < 8; ++j) {
+                            v = (lane & 7) == j ? val[g + j] : v;
+                            asm("" : "+v"(v));  // (a chain of selects, not an array in memory with an index)
+                        }
+                        if (v == v) atomicAdd(&s_hist[score_key(v) >> (32 - SAMPLE_BITS)], 1);
+                    });
+                    break;
+                } else {
+                    float v[P / 8];
+#pragma unroll
+                    for (int g = 0; g < P; g += 8) {
+                        const int i = 64 * (g + (lane & 7)) + lane;
+                        v[g / 8] = i < left ? row[c0 + span + i] : __builtin_nanf("");
+                    }
+#pragma unroll
+                    for (int g = 0; g < P / 8; ++g)
+                        if (v[g] == v[g]) atomicAdd(&s_hist[score_key(v[g]) >> (32 - SAMPLE_BITS)], 1);
+                }
+            }
+            // The pivot: the rank in the sample that leaves half as many entries again as are wanted, plus four
+            // standard deviations of an independent sample and a few.
+            const float expect = 0.125f * (float)want;
+            const int rank = (int)(1.5f * expect + 4.f * __builtin_sqrtf(expect)) + 16;
+            int bin, above, in_bin;
+            find_bin(IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, rank, bin, above, in_bin);
+            const uint32_t pivot_key = (uint32_t)bin << (32 - SAMPLE_BITS);
+            if (bin > 0 && pivot_key > 0x007fffffu) {  // (a number: NaN and -inf are below it)
+                const float pivot = key_score(pivot_key);
+                // (a lane appends its own entries one after the other: what a word costs is VALU time, of which one CU
+                // has 64 lanes a clock)
+                auto collect = [&](const float (&v)[P], int first, int left) {
+                    int mine = 0;
+                    for_groups(left, [&](int g) {
+#pragma unroll
+                        for (int j = g; j < g + GROUP; ++j) mine += v[j] >= pivot ? 1 : 0;
+                    });
+                    const int upto = wave_inclusive_sum(mine, lane);
+                    const int total = __builtin_amdgcn_readlane(upto, 63);
+                    if (total == 0) return;
+                    int at = 0;
+                    if (lane == 0) at = atomicAdd(&s_count, total);
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    if (at + total > MAX_CANDIDATES) return;  // (the count says that the list is not complete)
+                    uint2* to = s_list + at + upto - mine;
+                    const uint32_t index = (uint32_t)(first + lane);
+                    for_groups(left, [&](int g) {
+#pragma unroll
+                        for (int j = g; j < g + GROUP; ++j) {
+                            if (v[j] >= pivot) {
+                                *to = make_uint2(__float_as_uint(v[j]), index + 64u * j);
+                                ++to;
+                            }
+                        }
+                    });
+                };
+                if constexpr (RESIDENT) {
+                    collect(val, span, valid - span);
+                } else {
+                    float next[P];
+                    load_chunk(val, span, valid - span);
+                    for (int c0 = 0; c0 < valid; c0 += CHUNK) {
+                        const int c1 = c0 + CHUNK;
+                        if (c1 < valid) load_chunk(next, c1 + span, valid - c1 - span);
+                        collect(val, c0 + span, valid - c0 - span);
+#pragma unroll
+                        for (int j = 0; j < P; ++j) val[j] = next[j];
+                    }
+                }
+                __syncthreads();
+                const int count = s_count;
+                if (count >= want && count <= MAX_CANDIDATES) {
+                    constexpr int PER = MAX_CANDIDATES / SELECT_THREADS;
+                    uint32_t lkey[PER], lidx[PER];
+#pragma unroll
+                    for (int r = 0; r < PER; ++r) {
+                        lkey[r] = lidx[r] = 0u;  // (key 0 is below every candidate's)
+                        const int i = tid + r * SELECT_THREADS;
+                        if (i < count) {
+                            const uint2 e = s_list[i];
+                            lkey[r] = score_key(__uint_as_float(e.x));
+                            lidx[r] = e.y;
+                        }
+                    }
+                    // The threshold among the candidates. Keys are counted by their distance from the pivot, 2^13 keys to
+                    // a bin (1/1024 of an octave): few share a bin, and those of the threshold's bin, if at most 64, are
+                    // sorted out bit by bit by one wavefront. A threshold four octaves above the pivot lands in
+                    // the last bin with everything beyond it: then digit by digit.
+                    constexpr int NEAR_BITS = 13;
+                    auto near_bin = [&](uint32_t x) {
+                        const uint32_t d = (x - pivot_key) >> NEAR_BITS;
+                        return d < (1u << SAMPLE_BITS) ? d : (1u << SAMPLE_BITS) - 1u;
+                    };
+                    uint32_t threshold = 0u;
+                    int need_eq = valid;
+                    clear_hist(1 << SAMPLE_BITS);
+                    __syncthreads();
+#pragma unroll
+                    for (int r = 0; r < PER; ++r)
+                        if (lkey[r] != 0u) atomicAdd(&s_hist[near_bin(lkey[r])], 1);
+                    int tbin, tabove, tin;
+                    find_bin(IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, want, tbin, tabove, tin);
+                    if (tin == want - tabove) {
+                        threshold = pivot_key + ((uint32_t)tbin << NEAR_BITS);
+                    } else if (tin <= 64 && tbin < (1 << SAMPLE_BITS) - 1) {
+#pragma unroll
+                        for (int r = 0; r < PER; ++r)
+                            if (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin)
+                                s_hist[atomicAdd(&s_near_count, 1)] = (int)(lkey[r] - pivot_key);
+                        __syncthreads();
+                        if (wave == 0) {
+                            const uint32_t x = lane < tin ? (uint32_t)s_hist[lane] : 0u;
+                            unsigned long long alive = tin == 64 ? ~0ull : (1ull << tin) - 1ull;
+                            int remaining = want - tabove;
+                            uint32_t t = (uint32_t)tbin << NEAR_BITS;
+#pragma unroll
+                            for (int bit = NEAR_BITS - 1; bit >= 0; --bit) {
+                                const unsigned long long ones = alive & __ballot((x >> bit) & 1u);
+                                const int n_ones = __popcll(ones);
+                                if (n_ones >= remaining) {
+                                    alive = ones;
+                                    t |= 1u << bit;
+                                } else {
+                                    alive &= ~ones;
+                                    remaining -= n_ones;
+                                }
+                            }
+                            if (lane == 0) s_bin = (int)(pivot_key + t), s_above = remaining;
+                        }
+                        __syncthreads();
+                        threshold = (uint32_t)s_bin;
+                        need_eq = s_above;
+                    } else {
+                        radix_select(IntConstant<1>{}, [&](auto shift_tag, auto bits_tag, auto, uint32_t prefix) {
+                            constexpr int shift = decltype(shift_tag)::value, bits = decltype(bits_tag)::value;
+#pragma unroll
+                            for (int r = 0; r < PER; ++r) {
+                                if (lkey[r] != 0u && (shift + bits == 32 || ((lkey[r] ^ prefix) >> ((shift + bits) & 31)) == 0u))
+                                    atomicAdd(&s_hist[(lkey[r] >> shift) & ((1u << bits) - 1u)], 1);
+                            }
+                        }, threshold, need_eq);
+                    }
+#pragma unroll
+                    for (int r = 0; r < PER; ++r) {
+                        const uint32_t flag = 1u << (lidx[r] & 31);
+                        if (lkey[r] > threshold) atomicOr(&s_gt[lidx[r] >> 5], flag);
+                        if (lkey[r] == threshold) atomicOr(&s_eq[lidx[r] >> 5], flag);
+                    }
+                    __syncthreads();
+                    // the words of a lane are consecutive; their places come from a workgroup-wide scan
+                    const int per = (words + SELECT_THREADS - 1) / SELECT_THREADS;
+                    const int w0 = tid * per, w1 = w0 + per < words ? w0 + per : words;
+                    int n_gt = 0, n_eq = 0;
+                    for (int w = w0; w < w1; ++w) n_gt += __popc(s_gt[w]), n_eq += __popc(s_eq[w]);
+                    // (at most MAX_CANDIDATES of either: one scan of the packed pair)
+                    const int upto = wave_inclusive_sum(n_gt | (n_eq << 16), lane);
+                    if (lane == 63) s_wave_sum[0][wave] = upto;
+                    __syncthreads();
+                    const int before = upto - (n_gt | (n_eq << 16)) + sum_before(s_wave_sum[0], wave, lane);
+                    int gt_at = before & 0xffff, eq_at = before >> 16;
+                    for (int w = w0; w < w1; ++w) {
+                        uint32_t word = s_gt[w], ties = s_eq[w];
+                        int at = gt_at + (eq_at < need_eq ? eq_at : need_eq);
+                        gt_at += __popc(word);
+                        const int n_ties = __popc(ties), take = need_eq > eq_at ? need_eq - eq_at : 0;
+                        eq_at += n_ties;
+                        if (take < n_ties) ties = lowest_set(ties, take);
+                        for (word |= ties; word != 0u; word &= word - 1u) dst[at++] = 32 * w + __builtin_ctz(word);
+                    }
+                    return;
+                }
+            }
+            __syncthreads();  // the shared words are used again below
+        }
+    }
+
+    // The whole row, digit by digit
+    uint32_t key[P];
+    auto make_keys = [&]() {
+#pragma unroll
+        for (int j = 0; j < P; ++j) key[j] = score_key(val[j]);
+    };
+    // (entries past the end hold the smallest key: they land in the lowest bin of every digit and can only be among
+    // the ties of key 0, from which the emission takes entries of the row alone)
+    if (RESIDENT) make_keys();
+    uint32_t threshold = 0u;
+    int need_eq = valid;
+    if (want < valid) {
+        radix_select(IntConstant<HIST_COPIES>{}, [&](auto shift_tag, auto bits_tag, auto copies_tag, uint32_t prefix) {
+            constexpr int shift = decltype(shift_tag)::value, bits = decltype(bits_tag)::value;
+            constexpr int COPIES = decltype(copies_tag)::value;
+            const int copy = lane & (COPIES - 1);
+            auto in_prefix = [&](uint32_t x) { return shift + bits == 32 || ((x ^ prefix) >> ((shift + bits) & 31)) == 0u; };
+            for (int c0 = 0; c0 < valid; c0 += CHUNK) {
+                const int left = valid - c0 - span;
+                if constexpr (!RESIDENT) {
+                    load_chunk(val, c0 + span, left);
+                    make_keys();
+                }
+                for_groups(left, [&](int g) {
+                    // a group of one value (rows that are masked, say) is one addition
+                    uint32_t differ = 0u;
+#pragma unroll
+                    for (int j = g + 1; j < g + GROUP; ++j) differ |= key[j] ^ key[g];
+                    const uint32_t key0 = __builtin_amdgcn_readfirstlane(key[g]);
+                    differ |= key[g] ^ key0;
+                    if (__ballot(differ == 0u) == ~0ull) {
+                        if (lane == 0 && in_prefix(key0))
+                            atomicAdd(&s_hist[((key0 >> shift) & ((1u << bits) - 1u)) * COPIES], 64 * GROUP);
+                        return;
+                    }
+#pragma unroll
+                    for (int j = g; j < g + GROUP; ++j) {
+                        if (in_prefix(key[j]))
+                            atomicAdd(&s_hist[((key[j] >> shift) & ((1u << bits) - 1u)) * COPIES + copy], 1);
+                    }
+                });
+                if (RESIDENT) break;
+            }
+        }, threshold, need_eq);
+    }
+
+    // Emission. Lane j of a wavefront holds word j of the span as two masks (keys above / equal to the threshold);
+    // a scan of their counts gives every word its place in the output.
+    int gt_before = 0, eq_before = 0;  // in earlier chunks
+    for (int c0 = 0; c0 < valid; c0 += CHUNK) {
+        const int left = valid - c0 - span;
+        if constexpr (!RESIDENT) {
+            load_chunk(val, c0 + span, left);
+            make_keys();
+        }
+        uint32_t gt_lo = 0u, gt_hi = 0u, eq_lo = 0u, eq_hi = 0u;
+        for_groups(left, [&](int g) {
+#pragma unroll
+            for (int j = g; j < g + GROUP; ++j) {
+                const unsigned long long gt = __ballot(key[j] > threshold);
+                const unsigned long long eq = __ballot(key[j] == threshold);
+                gt_lo = lane == j ? (uint32_t)gt : gt_lo;
+                gt_hi = lane == j ? (uint32_t)(gt >> 32) : gt_hi;
+                eq_lo = lane == j ? (uint32_t)eq : eq_lo;
+                eq_hi = lane == j ? (uint32_t)(eq >> 32) : eq_hi;
+            }
+        });
+        unsigned long long word = ((unsigned long long)gt_hi << 32) | gt_lo;
+        unsigned long long ties = ((unsigned long long)eq_hi << 32) | eq_lo;
+        const int in_word = left - 64 * lane;  // entries of the row in this lane's word
+        ties &= in_word >= 64 ? ~0ull : in_word <= 0 ? 0ull : (1ull << in_word) - 1ull;
+        const int n_gt = __popcll(word), n_eq = __popcll(ties);
+        const int gt_upto = wave_inclusive_sum(n_gt, lane), eq_upto = wave_inclusive_sum(n_eq, lane);
+        if (c0 > 0) __syncthreads();  // the sums of the chunk before have been read
+        if (lane == 63) {
+            s_wave_sum[0][wave] = gt_upto;
+            s_wave_sum[1][wave] = eq_upto;
+        }
+        __syncthreads();
+        int gt_at = gt_before + gt_upto - n_gt, eq_at = eq_before + eq_upto - n_eq;
 #pragma unroll
         for (int w = 0; w < SELECT_WAVES; ++w) {
-            if (w < wave) {
-                gt_before += s_wave_gt[w];
-                eq_before += s_wave_eq[w];
-            }
+            const int g = s_wave_sum[0][w], e = s_wave_sum[1][w];
+            gt_at += w < wave ? g : 0;
+            eq_at += w < wave ? e : 0;
+            gt_before += g;
+            eq_before += e;
         }
-        int* dst = idx_out + (size_t)b * k;
+        // the ties of this word that are still wanted: its lowest ones
+        const int take = need_eq > eq_at ? need_eq - eq_at : 0;
+        if (take < n_eq) ties = lowest_set(ties, take);
+        word |= ties;
+        int at = gt_at + (eq_at < need_eq ? eq_at : need_eq);
+        if constexpr (P <= 8) {
+            // few words with many entries each: every lane writes its own entry of each word
 #pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const bool on = (live >> j) & 1u;
-            const bool gt = on && key[j] > threshold;
-            const bool eq = on && key[j] == threshold;
-            if (gt || (eq && eq_before < need_eq))
-                dst[gt_before + (eq_before < need_eq ? eq_before : need_eq)] = first + j;
-            gt_before += gt ? 1 : 0;
-            eq_before += eq ? 1 : 0;
+            for (int j = 0; j < P; ++j) {
+                const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)word, j);
+                const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(word >> 32), j);
+                const int place = __builtin_amdgcn_readlane(at, j) + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+                if (((((unsigned long long)hi << 32) | lo) >> lane) & 1ull) dst[place] = c0 + span + 64 * j + lane;
+            }
+        } else {
+            const int first = c0 + span + 64 * lane;
+            for (; word != 0ull; word &= word - 1ull) dst[at++] = first + __builtin_ctzll(word);
         }
+        if (RESIDENT) break;
     }
-    for (int j = want + tid; j < k; j += SELECT_THREADS) idx_out[(size_t)b * k + j] = -1;
 }
 
 }  // namespace
@@ -325,15 +546,20 @@ extern "C" void topk_select_launcher(int* idx_out, const float* scores, const in
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
+#define TOPK_LAUNCH(P, RESIDENT) \
+    topk_select_kernel<P, RESIDENT><<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k)
     if (n <= 4 * SELECT_THREADS) {
-        topk_select_regs_kernel<4><<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k);
+        TOPK_LAUNCH(4, true);
     } else if (n <= 8 * SELECT_THREADS) {
-        topk_select_regs_kernel<8><<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k);
+        TOPK_LAUNCH(8, true);
     } else if (n <= 16 * SELECT_THREADS) {
-        topk_select_regs_kernel<16><<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k);
+        TOPK_LAUNCH(16, true);
     } else if (n <= 32 * SELECT_THREADS) {
-        topk_select_regs_kernel<32><<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k);
+        TOPK_LAUNCH(32, true);
+    } else if (n <= 64 * SELECT_THREADS) {
+        TOPK_LAUNCH(64, true);
     } else {
-        topk_select_kernel<<<batch, SELECT_THREADS, 0, stream>>>(scores, lengths, idx_out, n, k);
+        TOPK_LAUNCH(32, false);
     }
+#undef TOPK_LAUNCH
 }

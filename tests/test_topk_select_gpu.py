@@ -50,6 +50,33 @@ def test_denormals_and_close_values(capi, dev):
         assert torch.equal(run_kernel(capi, dev, scores, k), mla.topk_select(scores, k))
 
 
+def _rows(kind, n, gen):
+    x = torch.randn(4, n, generator=gen)
+    if kind == 'clustered':      # the large scores are neighbours: a sample of the row misjudges their number
+        x[:, n // 3:n // 3 + 3000] += 6
+    elif kind == 'distinct':     # few values: the threshold is shared by many entries
+        x = (x * 8).round() / 8
+    elif kind == 'wide':         # forty octaves, the threshold far above the sampled pivot or below zero
+        x = torch.exp2(x * 10) * torch.where(torch.rand(4, n, generator=gen) < 0.01, 1.0, -1.0)
+    elif kind == 'special':
+        x[0, ::3] = float('nan')
+        x[1, torch.rand(n, generator=gen) < 0.95] = float('-inf')
+        x[2, ::2] = float('inf')
+        x[3] = torch.where(x[3] > 1.5, x[3], torch.zeros(()))
+    return x
+
+
+@pytest.mark.parametrize('n', [8192, 8193, 16385, 32768, 32769, 65536, 65537, 98305, 262144, 262145])
+@pytest.mark.parametrize('kind', ['normal', 'clustered', 'distinct', 'wide', 'special'])
+def test_long_rows(capi, dev, n, kind):
+    # edges of the row classes (in registers, read again, filtered or not), k at the limits of the candidate list
+    gen = torch.Generator().manual_seed(n)
+    scores = _rows(kind, n, gen)
+    lengths = torch.tensor([n, n - 1, n // 2 + 7, 5000], dtype=torch.int32)
+    for k, ln in ((2048, None), (2048, lengths), (1, None), (3072, lengths), (3073, None)):
+        assert torch.equal(run_kernel(capi, dev, scores, k, ln), mla.topk_select(scores, k, ln)), (k, ln is not None)
+
+
 def test_selected_indices_feed_the_attention(capi, dev):
     # selection -> sparse-MLA decode; shorter requests leave -1 entries, which the attention skips
     gen = torch.Generator().manual_seed(43)
