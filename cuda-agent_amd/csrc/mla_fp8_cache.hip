@@ -12,10 +12,10 @@
 //
 // Decode has two forms with the same result, bit for bit what sparse_mla_decode_launcher gives on the
 // dequantised cache (code * scale in fp32, rounded to nearest-even bf16).
-//   * Head counts that are multiples of 128: the 8-wavefront kernel of sparse_mla.hip gathers the 656-byte
+//   * The 8-wavefront kernel of sparse_mla.hip gathers the 656-byte
 //     rows itself and converts every key tile in LDS (its FP8 instantiation); the selected rows cross HBM once
 //     and nothing else is written.
-//   * Otherwise, or with 5000 added to config, two steps: the kernel below gathers the selected rows of every
+//   * For caches of 4 GB and more per addressed block, config >= 1000, or with 5000 added to config, two steps: the kernel below gathers the selected rows of every
 //     request and dequantises them into a compact per-request block [batch, topk, 576] in the workspace, with
 //     an index list 0..topk-1 beside it (-1 where the caller's entry was padding); the decode kernels of
 //     sparse_mla.hip then run on that block unchanged. The compact block is written and read back.
@@ -220,7 +220,7 @@ void launch_decode_fp8(void* out, const void* q, const void* kv_fp8, const int* 
         return;
     }
     // config 5000 + n: the two-step form (gather + dequantise into the workspace, then the bf16 kernels) with
-    // config n; otherwise the 128-head kernel dequantises its tiles itself where the shape allows
+    // config n; otherwise the 8-wavefront kernel dequantises its tiles itself where the shape allows
     const bool two_step = config >= 5000;
     if (two_step) config -= 5000;
     const size_t base_bytes = align16(sparse_mla_decode_workspace_bytes(batch, n_heads, topk, config));

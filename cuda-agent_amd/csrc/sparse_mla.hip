@@ -29,8 +29,8 @@
 //
 // Two split kernels share this data path. sparse_mla_split_kernel<NW> is the form described
 // above (one wavefront per 32 heads; used for 32 and 64 heads and for caches of 4 GB and more
-// per request). sparse_mla_split8_kernel, further down, is the default for multiples of 128
-// heads: two wavefronts per 32 heads that split Q by d and the accumulator by dv.
+// per request). sparse_mla_split8_kernel, further down, is the default: two wavefronts per 32 heads
+// that split Q by d and the accumulator by dv.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -460,6 +460,10 @@ __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
 // ---------------------------------------------------------------------------------------------
 // 128 heads per workgroup, 8 wavefronts (two per SIMD).
 //
+// With 32 or 64 heads the same 8 wavefronts run, the ones without heads gathering only (then the gather is not in
+// the chain of a wavefront that also multiplies): the kernel above, one wavefront per 32 heads fetching 36 loads per
+// tile itself, took 60 us for 16 requests of 32 heads and 2048 rows, this one 23; 48 requests 239 -> 36, 64 heads 244 -> 48.
+//
 // The per-head-group state of the kernel above (Q: 144 registers, O^T: 256) fills a SIMD's
 // whole register file with one wavefront, so nothing can overlap: MFMA, softmax arithmetic, LDS
 // reads and the issue of the gather loads simply add up. Here each head group is a PAIR of
@@ -651,7 +655,8 @@ template <bool FP8>
 __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     const __bf16* __restrict__ q, const __bf16* __restrict__ kv, const int* __restrict__ idx,
     _Float16* __restrict__ o_part, float* __restrict__ lse_part, float* __restrict__ scale_part,
-    int n_heads, int n_kv_rows, int topk, int rows_per_split, float scale_log2, KvAddressing kva) {
+    int n_heads, int n_kv_rows, int topk, int rows_per_split, float scale_log2, KvAddressing kva,
+    void* __restrict__ out, int out_dtype) {
     typedef const __attribute__((address_space(3))) uintx4* lds_x4;
     typedef shortx4 __attribute__((address_space(3)))* lds_s4;
     __shared__ uint4 tiles[3 * TILE_CHUNKS];  // ring of three resident tiles
@@ -684,6 +689,8 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
         b = (linear & 7) + 8 * (j / n_splits);
     }
     const int head0 = blockIdx.z * 128 + hg * 32;
+    // with 32 or 64 heads the wavefronts of the missing head groups take part in the gather and the barriers only
+    const bool live = head0 < n_heads;
     const int half = lane >> 5;
 
     const int row_begin = split * rows_per_split;
@@ -708,7 +715,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     // loading the operand layout directly needs); the operand layout is made below through LDS.
     uintx4 qraw[HALF_K_STEPS];
     {
-        const char* qsrc = reinterpret_cast<const char*>(q + ((size_t)b * n_heads + head0) * D_QK) +
+        const char* qsrc = reinterpret_cast<const char*>(q + ((size_t)b * n_heads + (live ? head0 : 0)) * D_QK) +
                            (size_t)(lane >> 2) * ROW_BYTES + 64 * dh + 16 * (lane & 3);
 #pragma unroll
         for (int l = 0; l < HALF_K_STEPS; ++l) {
@@ -868,6 +875,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
                 }
             }
             PHASE_MARK(2);  // gather issue
+            if (live) {
             uintx4 kbuf[3];  // K operands are read two MFMAs ahead
             auto k_read = [&](int l) { kbuf[l % 3] = *(lds_x4)(base + qk_l[l & 1] + (l >> 1) * 128); };
             k_read(0);
@@ -882,6 +890,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
                 my_xchg[qd * 64 + lane] = floatx4{s[4 * qd], s[4 * qd + 1], s[4 * qd + 2], s[4 * qd + 3]};
+            }
             }
             __builtin_amdgcn_sched_barrier(0);  // (the scores leave their registers before the conversion needs them)
             if constexpr (FP8) {
@@ -900,7 +909,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
             }
             PHASE_MARK(3);  // QK^T
         }
-        if (!(active && (mine & 1) == 1)) continue;
+        if (!(active && live && (mine & 1) == 1)) continue;
 
         // full scores = partial of d-slices 0 + partial of d-slices 1, in that order in both
         // partners, so that they compute bit-identical probabilities
@@ -1001,6 +1010,60 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     const float l_total = st.l + __shfl_xor(st.l, 32);
     const float inv_l = l_total > 0.f ? 1.f / l_total : 0.f;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
+    constexpr int STAGE_STRIDE = 64 + 4;
+    float* stage = reinterpret_cast<float*>(tiles + (wave >> 2) * TILE_CHUNKS) + (wave & 3) * (32 * STAGE_STRIDE);
+    typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+    // O^T half times `scale`, row r of the 32 heads and columns 64*ps + 4*(lane%16) .. +3 of the half to store(r, ps, v)
+    auto write_rows = [&](float scale, auto store) {
+#pragma unroll
+        for (int ps = 0; ps < 4; ++ps) {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const floatx16 a = acc[2 * ps + tt];
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {
+                    floatx4 v = {a[4 * qd] * scale, a[4 * qd + 1] * scale, a[4 * qd + 2] * scale, a[4 * qd + 3] * scale};
+                    *reinterpret_cast<floatx4*>(stage + (lane & 31) * STAGE_STRIDE + 32 * tt + 8 * qd + 4 * half) = v;
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int r = 4 * it + (lane >> 4);
+                store(r, ps, *reinterpret_cast<const floatx4*>(stage + r * STAGE_STRIDE + 4 * (lane & 15)));
+            }
+        }
+    };
+    if (n_splits == 1) {
+        // the only split of its request: this is the output (there is no merge)
+        __syncthreads();  // every wavefront is done with the tiles
+        if (!live) return;
+        const size_t o0 = part0 * D_V + 256 * dh + 4 * (lane & 15);
+        if (out_dtype == 0) {
+            write_rows(inv_l, [&](int r, int ps, floatx4 v) {
+                const bf16x4 x = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+                *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(out) + o0 + (size_t)r * D_V + 64 * ps) = x;
+            });
+        } else {
+            write_rows(inv_l, [&](int r, int ps, floatx4 v) {
+                *reinterpret_cast<floatx4*>(static_cast<float*>(out) + o0 + (size_t)r * D_V + 64 * ps) = v;
+            });
+        }
+        PHASE_TIMING_END(wave, lane);
+        return;
+    }
+    if (scale_part == nullptr) {  // fp32 partials (fewer than 128 heads: they are small)
+        __syncthreads();
+        if (!live) return;
+        if (dh == 0 && half == 0) {
+            lse_part[part0 + lane] = l_total > 0.f ? st.m + __builtin_amdgcn_logf(l_total) : -INFINITY;
+        }
+        float* o_rows = reinterpret_cast<float*>(o_part) + part0 * D_V + 256 * dh + 4 * (lane & 15);
+        write_rows(inv_l, [&](int r, int ps, floatx4 v) {
+            *reinterpret_cast<floatx4*>(o_rows + (size_t)r * D_V + 64 * ps) = v;
+        });
+        PHASE_TIMING_END(wave, lane);
+        return;
+    }
     float amax = 0.f;
 #pragma unroll
     for (int t = 0; t < 8; ++t)
@@ -1008,51 +1071,34 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
         for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[t][i]));
     amax = fmaxf(amax, __shfl_xor(amax, 32));
     if (half == 0) s_head_max[wave][lane] = amax;
+    __syncthreads();
+    if (!live) return;
     if (dh == 0 && half == 0) {
         lse_part[part0 + lane] = l_total > 0.f ? st.m + __builtin_amdgcn_logf(l_total) : -INFINITY;
     }
-    __syncthreads();
     // exponent field of the bound + 1: 2^e > |O| for every element of the head (1 if the head is 0)
     const float bound = fmaxf(s_head_max[wave][lane & 31], s_head_max[wave ^ 1][lane & 31]) * inv_l;
     uint32_t e_bits = ((__float_as_uint(bound) >> 23) & 255u) + 1u;
     e_bits = bound > 0.f ? (e_bits > 253u ? 253u : e_bits) : 127u;
     const float inv_scale = __uint_as_float((254u - e_bits) << 23) * inv_l;
     if (dh == 0 && half == 0) scale_part[part0 + lane] = __uint_as_float(e_bits << 23);
-    constexpr int STAGE_STRIDE = 64 + 4;
-    float* stage = reinterpret_cast<float*>(tiles + (wave >> 2) * TILE_CHUNKS) + (wave & 3) * (32 * STAGE_STRIDE);
-    _Float16* o_rows = o_part + part0 * D_V + 256 * dh;
-    typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-    for (int ps = 0; ps < 4; ++ps) {
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const floatx16 a = acc[2 * ps + tt];
-#pragma unroll
-            for (int qd = 0; qd < 4; ++qd) {
-                floatx4 v = {a[4 * qd] * inv_scale, a[4 * qd + 1] * inv_scale, a[4 * qd + 2] * inv_scale,
-                             a[4 * qd + 3] * inv_scale};
-                *reinterpret_cast<floatx4*>(stage + (lane & 31) * STAGE_STRIDE + 32 * tt + 8 * qd +
-                                            4 * half) = v;
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int r = 4 * it + (lane >> 4);
-            const floatx4 v = *reinterpret_cast<const floatx4*>(stage + r * STAGE_STRIDE + 4 * (lane & 15));
-            const halfx4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
-            *reinterpret_cast<halfx4*>(o_rows + (size_t)r * D_V + 64 * ps + 4 * (lane & 15)) = h;
-        }
-    }
+    _Float16* o_rows = o_part + part0 * D_V + 256 * dh + 4 * (lane & 15);
+    write_rows(inv_scale, [&](int r, int ps, floatx4 v) {
+        const halfx4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+        *reinterpret_cast<halfx4*>(o_rows + (size_t)r * D_V + 64 * ps) = h;
+    });
     PHASE_MARK(10);  // epilogue
     PHASE_TIMING_END(wave, lane);
 }
 
-// out[b, h, :] = sum_s w_s o_part[b, s, h, :],  w_s = exp2(lse_s - max) / sum. One wavefront per
-// (b, h), 8 output columns per lane, 4 heads per workgroup (grid x = n_heads / 4, y = request): the
-// rows of all splits are requested before the first is used. PART is the type the split kernel
-// stored: float, or fp16 of O / scale with the per-head scale in scale_part.
-// BATCH = splits whose rows a lane requests at once.
-template <typename OUT, typename PART, int BATCH>
+// out[b, h, :] = sum_s w_s o_part[b, s, h, :],  w_s = exp2(lse_s - max) / sum. NW wavefronts per (b, h), 8 output
+// columns per lane, 4 / NW heads per workgroup (grid x = n_heads * NW / 4, y = request); wavefront i of a head takes
+// the splits i, i + NW, ... of every 64, BATCH of them requested at once, the first before anything else. PART is the
+// type the split kernel stored: float, or fp16 of O / scale with the per-head scale in scale_part.
+// The kernel is a chain of memory latencies: with one request and 64 splits on one wavefront per head, 8 rows at a
+// time and the log-sum-exps one after the other, it took 37 us, three times the split kernel before it; lane s now
+// fetches the log-sum-exp of split s, and above 8 splits four wavefronts share a head (3.9 us).
+template <typename OUT, typename PART, int NW, int BATCH>
 __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __restrict__ o_part,
                                                                const float* __restrict__ lse_part,
                                                                const float* __restrict__ scale_part,
@@ -1061,6 +1107,7 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
     typedef PART partx8 __attribute__((ext_vector_type(8)));
     typedef float floatx8 __attribute__((ext_vector_type(8)));
     const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int hg = blockIdx.x;
     int b = blockIdx.y;
     // request b on XCD b % 8, where the split kernel wrote its partials (see there)
@@ -1070,44 +1117,61 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
         hg = j % (int)gridDim.x;
         b = (linear & 7) + 8 * (j / (int)gridDim.x);
     }
-    const int h = hg * 4 + (threadIdx.x >> 6);
+    const int h = hg * (4 / NW) + wave / NW;
+    const int part = wave % NW;
     const size_t base = (size_t)b * n_splits * n_heads + h;
     floatx8 o = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float wsum = 0.f;
     partx8 rows[BATCH];
     auto load_rows = [&](int s0) {
 #pragma unroll
         for (int j = 0; j < BATCH; ++j) {
             // (splits past the end repeat the last one; their weight is 0)
-            const int s = s0 + j < n_splits ? s0 + j : n_splits - 1;
+            const int s = s0 + NW * j < n_splits ? s0 + NW * j : n_splits - 1;
             rows[j] = __builtin_nontemporal_load(
                 reinterpret_cast<const partx8*>(o_part + (base + (size_t)s * n_heads) * D_V) + lane);
         }
     };
-    // the first rows are requested before anything depends on the log-sum-exps
-    load_rows(0);
+    load_rows(part);
     float mx = -INFINITY;
-    for (int s = 0; s < n_splits; ++s) mx = fmaxf(mx, lse_part[base + (size_t)s * n_heads]);
-    for (int s0 = 0; s0 < n_splits; s0 += BATCH) {
-        if (s0 > 0) load_rows(s0);
-        float w[BATCH], sc[BATCH];
+    for (int s = lane; s < n_splits; s += 64) mx = fmaxf(mx, lse_part[base + (size_t)s * n_heads]);
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-            const int s = s0 + j < n_splits ? s0 + j : n_splits - 1;
-            const size_t row = base + (size_t)s * n_heads;
-            // (mx = -inf: every split is empty, all weights 0)
-            w[j] = s0 + j < n_splits && mx > -INFINITY ? __builtin_amdgcn_exp2f(lse_part[row] - mx) : 0.f;
-            sc[j] = 1.f;
-            if constexpr (sizeof(PART) == 2) sc[j] = scale_part[row];
+    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    float wsum = 0.f;
+    for (int c0 = 0; c0 < n_splits; c0 += 64) {
+        // weight of split c0 + lane (mx = -inf: every split is empty, all weights 0)
+        float w = 0.f, ws = 0.f;
+        if (c0 + lane < n_splits && mx > -INFINITY) {
+            const size_t row = base + (size_t)(c0 + lane) * n_heads;
+            w = __builtin_amdgcn_exp2f(lse_part[row] - mx);
+            ws = w;
+            if constexpr (sizeof(PART) == 2) ws = w * scale_part[row];  // (a power of two)
         }
+        wsum += w;
+        for (int s0 = c0 + part; s0 < n_splits && s0 < c0 + 64; s0 += NW * BATCH) {
+            if (s0 != part) load_rows(s0);
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-            if (w[j] > 0.f) {  // (a split without rows has weight 0 and is not looked at)
-                const float ws = w[j] * sc[j];  // sc is a power of two
+            for (int j = 0; j < BATCH; ++j) {
+                const int at = s0 - c0 + NW * j;
+                const float wj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ws), at & 63));
+                if (at < 64 && wj > 0.f) {  // (a split without rows has weight 0 and is not looked at)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) o[i] += (float)rows[j][i] * ws;
-                wsum += w[j];
+                    for (int i = 0; i < 8; ++i) o[i] += (float)rows[j][i] * wj;
+                }
             }
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) wsum += __shfl_xor(wsum, off);
+    if constexpr (NW > 1) {
+        __shared__ floatx4 s_o[4][2][64];
+        s_o[wave][0][lane] = floatx4{o[0], o[1], o[2], o[3]};
+        s_o[wave][1][lane] = floatx4{o[4], o[5], o[6], o[7]};
+        __syncthreads();
+        if (part != 0) return;
+#pragma unroll
+        for (int i = 1; i < NW; ++i) {
+            const floatx4 lo = s_o[wave + i][0][lane], hi = s_o[wave + i][1][lane];
+            o += floatx8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         }
     }
     if (wsum > 0.f) o *= 1.f / wsum;
@@ -1122,11 +1186,23 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
     }
 }
 
-int pick_splits(int batch, int head_groups, int topk, int config) {
+// Microseconds of a launch of `wgs` workgroups of `tiles` tiles each, one workgroup per CU at a time, as measured for
+// 128 heads: a workgroup starts and ends in 8 us on an empty chip and 15 on a full one (they compete for memory),
+// and takes 2.35 us per tile up to about 140 busy CUs, then more (memory again, and the clock), 3 on 256.
+float split_kernel_us(int wgs, int tiles) {
+    auto round_us = [&](int n) {
+        const float crowd = n > 140 ? (n - 140) / 116.f : 0.f;
+        return 8.f + 0.029f * n + (2.35f + 0.65f * crowd * crowd) * tiles;
+    };
+    return (wgs / 256) * round_us(256) + (wgs % 256 ? round_us(wgs % 256) : 0.f);
+}
+
+// The most splits a launch may use, which sizes the workspace: config if it asks for a number, else as many as put a
+// workgroup on each of the 256 CUs.
+int max_splits(int batch, int head_groups, int topk, int config) {
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     int splits = config > 0 ? config : 0;
     if (splits == 0) {
-        // fill the 256 CUs once (one resident workgroup per CU)
         const int wgs = batch * head_groups;
         splits = (256 + wgs - 1) / wgs;
     }
@@ -1137,18 +1213,44 @@ int pick_splits(int batch, int head_groups, int topk, int config) {
     return splits;
 }
 
+// The splits of a launch: config if it asks for a number, else the one with the least time for the split kernel and
+// the merge (5 us and 16 ns per partial of 128 heads; none for a single split). The maximum above puts a few
+// workgroups into a second round whenever the number of requests is not a divisor of 256: with it 24 requests of 2048
+// rows took 57 us, now 37; 48: 86, 58; 96: 136, 103; 150: 198, 164; 200: 211, 180; 4 requests (many partials): 28, 24.
+int pick_splits(int batch, int head_groups, int topk, int config) {
+    const int most = max_splits(batch, head_groups, topk, config);
+    if (config > 0) return most;
+    const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
+    const int wgs = batch * head_groups;
+    int best = most;
+    float best_us = 0.f;
+    for (int per = MAX_SPLIT_ROWS / TILE_ROWS < tiles ? MAX_SPLIT_ROWS / TILE_ROWS : tiles; per >= 1; --per) {
+        const int splits = (tiles + per - 1) / per;  // of `per` tiles each
+        if (splits > most) break;
+        const float us = split_kernel_us(wgs * splits, per) + (splits > 1 ? 5.f + 0.016f * wgs * splits : 0.f);
+        if (best_us == 0.f || us < best_us) best_us = us, best = splits;
+    }
+    return best;
+}
+
 }  // namespace
 
+namespace {
+
+int head_groups_of(int n_heads) { return n_heads <= 128 ? 1 : n_heads / 128; }
+
+}  // namespace
+
+// config 1000 + n: n splits on the kernel with one wavefront per 32 heads
 extern "C" int sparse_mla_decode_num_splits(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
-    if (config >= 1000) config -= 1000;  // 1000 + n: n splits on the one-wavefront-per-head-group kernel
-    const int head_groups = n_heads <= 128 ? 1 : n_heads / 128;
-    return pick_splits(batch, head_groups, topk, config);
+    return pick_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config);
 }
 
 // bytes of scratch sparse_mla_decode_launcher needs for these sizes
 extern "C" size_t sparse_mla_decode_workspace_bytes(int batch, int n_heads, int topk, int config) {
-    const int splits = sparse_mla_decode_num_splits(batch, n_heads, topk, config);
+    if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
+    const int splits = max_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config);
     // partial outputs (sized for fp32), log-sum-exp and scale of every (request, split, head)
     return (size_t)batch * splits * n_heads * (D_V + 2) * sizeof(float);
 }
@@ -1157,7 +1259,7 @@ namespace {
 
 // shared by the two launchers: n_kv_rows is the number of rows of the block a request's keys
 // resolve into (the request's own cache, or the whole pool)
-// fp8_cache: kv is in the 656-byte e4m3 form, which only the 128-head kernel reads (the caller has checked
+// fp8_cache: kv is in the 656-byte e4m3 form, which only the 8-wavefront kernel reads (the caller has checked
 // the shape with fp8_cache_fused_ok)
 void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx, void* workspace,
                        size_t workspace_bytes, int batch, int n_heads, int n_kv_rows, int topk,
@@ -1181,14 +1283,13 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
         caa::set_status(CAA_WORKSPACE_TOO_SMALL);
         return;
     }
-    // config >= 1000: the one-wavefront-per-SIMD kernel for 128 heads (config - 1000 is then the
-    // split count)
+    // config >= 1000: the kernel with one wavefront per 32 heads (config - 1000 is then the split count)
     // The 8-wavefront kernel addresses a request's cache block with 32-bit byte offsets.
-    const bool four_wave_kernel =
+    const bool one_wave_per_group =
         config >= 1000 ||
         (unsigned long long)n_kv_rows * (fp8_cache ? FP8_ROW_BYTES : ROW_BYTES) >= 0xffffffffull;
     if (config >= 1000) config -= 1000;
-    const int head_groups = n_heads <= 128 ? 1 : n_heads / 128;
+    const int head_groups = head_groups_of(n_heads);
     const int splits = pick_splits(batch, head_groups, topk, config);
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int rows_per_split = ((tiles + splits - 1) / splits) * TILE_ROWS;
@@ -1199,43 +1300,43 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     const __bf16* qb = static_cast<const __bf16*>(q);
     const __bf16* kvb = static_cast<const __bf16*>(kv);
     const dim3 grid(splits, batch, head_groups);
-    const dim3 merge_grid(n_heads / 4, batch);
     bool half_parts = false;
-    if (n_heads == 32) {
+    if (one_wave_per_group && n_heads == 32) {
         sparse_mla_split_kernel<1><<<grid, 64, 0, stream>>>(qb, kvb, idx, o_part, lse_part, n_heads,
                                                             n_kv_rows, topk, rows_per_split,
                                                             scale_log2, kva);
-    } else if (n_heads == 64) {
+    } else if (one_wave_per_group && n_heads == 64) {
         sparse_mla_split_kernel<2><<<grid, 128, 0, stream>>>(qb, kvb, idx, o_part, lse_part, n_heads,
                                                              n_kv_rows, topk, rows_per_split,
                                                              scale_log2, kva);
-    } else if (four_wave_kernel) {
+    } else if (one_wave_per_group) {
         sparse_mla_split_kernel<4><<<grid, 256, 0, stream>>>(qb, kvb, idx, o_part, lse_part, n_heads,
                                                              n_kv_rows, topk, rows_per_split,
                                                              scale_log2, kva);
     } else {
-        half_parts = true;  // this kernel stores its partials as scaled fp16
+        half_parts = n_heads >= 128;  // this kernel then stores its partials as scaled fp16
+        if (!half_parts) scale_part = nullptr;
         if (fp8_cache) {
             sparse_mla_split8_kernel<true><<<grid, 512, 0, stream>>>(
                 qb, kvb, idx, reinterpret_cast<_Float16*>(o_part), lse_part, scale_part, n_heads, n_kv_rows,
-                topk, rows_per_split, scale_log2, kva);
+                topk, rows_per_split, scale_log2, kva, out, out_dtype);
         } else {
             sparse_mla_split8_kernel<false><<<grid, 512, 0, stream>>>(
                 qb, kvb, idx, reinterpret_cast<_Float16*>(o_part), lse_part, scale_part, n_heads, n_kv_rows,
-                topk, rows_per_split, scale_log2, kva);
+                topk, rows_per_split, scale_log2, kva, out, out_dtype);
         }
     }
-    // rows requested at once per lane: as many as there are splits, up to 8
-#define MLA_MERGE(OUT_T, PART_T, PARTS, SCALES)                                                   \
-    if (splits <= 2)                                                                              \
-        sparse_mla_merge_kernel<OUT_T, PART_T, 2><<<merge_grid, 256, 0, stream>>>(                \
-            PARTS, lse_part, SCALES, static_cast<OUT_T*>(out), n_heads, splits);                  \
-    else if (splits <= 4)                                                                         \
-        sparse_mla_merge_kernel<OUT_T, PART_T, 4><<<merge_grid, 256, 0, stream>>>(                \
-            PARTS, lse_part, SCALES, static_cast<OUT_T*>(out), n_heads, splits);                  \
-    else                                                                                          \
-        sparse_mla_merge_kernel<OUT_T, PART_T, 8><<<merge_grid, 256, 0, stream>>>(                \
-            PARTS, lse_part, SCALES, static_cast<OUT_T*>(out), n_heads, splits);
+    if (!one_wave_per_group && splits == 1) return;  // (written by the split kernel)
+    // wavefronts per head, and rows requested at once per lane
+#define MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, NW, BATCH)                                      \
+    sparse_mla_merge_kernel<OUT_T, PART_T, NW, BATCH><<<dim3(n_heads * NW / 4, batch), 256, 0, stream>>>( \
+        PARTS, lse_part, SCALES, static_cast<OUT_T*>(out), n_heads, splits)
+#define MLA_MERGE(OUT_T, PART_T, PARTS, SCALES)                                       \
+    if (splits <= 2) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 2);              \
+    else if (splits <= 4) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 4);         \
+    else if (splits <= 8) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 8);         \
+    else if (splits <= 32) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 4, 8);        \
+    else MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 4, 16);
     if (half_parts) {
         const _Float16* parts = reinterpret_cast<const _Float16*>(o_part);
         if (out_dtype == 0) {
@@ -1249,6 +1350,7 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
         MLA_MERGE(float, float, o_part, nullptr)
     }
 #undef MLA_MERGE
+#undef MLA_MERGE_FORM
 }
 
 }  // namespace
@@ -1369,8 +1471,7 @@ extern "C" void sparse_mla_decode_static_launcher(void* out, const void* q, cons
 // Decode over a cache in the 656-byte e4m3 form with the dequantisation inside the 128-head kernel (see
 // gather_quarter_fp8 / dequant_quarter). Internal to the library: mla_fp8_cache.hip calls it from
 // sparse_mla_decode_fp8_launcher and its paged form; it is not part of the public header. Returns 1 if the launch was made (or rejected with a status), 0 if
-// this shape has to take the two-step form of sparse_mla_decode_fp8_launcher: head counts other than
-// multiples of 128, config >= 1000, caches of 4 GB and more per addressed block.
+// this shape has to take the two-step form of sparse_mla_decode_fp8_launcher: config >= 1000, caches of 4 GB and more per addressed block.
 // block_table / table_stride / page_shift / batch_rows: the addressing of the cache, as in KvAddressing.
 extern "C" int sparse_mla_decode_fp8_fused(void* out, const void* q, const void* kv_fp8, const int* idx,
                                            void* workspace, size_t workspace_bytes, int batch, int n_heads,
@@ -1378,7 +1479,7 @@ extern "C" int sparse_mla_decode_fp8_fused(void* out, const void* q, const void*
                                            int out_dtype, int config, const int* block_table,
                                            int table_stride, int page_shift, int batch_rows,
                                            hipStream_t stream) {
-    if (n_heads <= 0 || n_heads % 128 != 0 || config >= 1000 || n_kv_rows <= 0 ||
+    if (n_heads <= 0 || (n_heads % 128 != 0 && n_heads != 32 && n_heads != 64) || config >= 1000 || n_kv_rows <= 0 ||
         (unsigned long long)n_kv_rows * FP8_ROW_BYTES >= 0xffffffffull)
         return 0;
     const KvAddressing kva{block_table, table_stride, page_shift, batch_rows};

@@ -60,6 +60,33 @@ def test_matches_oracle(capi, dev, shape, config):
     check(capi, q, kv, idx, config, oracle_on_gpu(q, kv, idx))
 
 
+@pytest.mark.parametrize('heads', [32, 64, 128, 256])
+@pytest.mark.parametrize('splits', [1, 3, 8, 9, 32, 33, 65, 128])
+def test_split_counts(capi, dev, heads, splits):
+    # one split (no merge), and the edges of the merge kernel's forms: up to 8, 32, 64 and more splits
+    gen = torch.Generator().manual_seed(heads + splits)
+    topk = 4090 if splits > 2 else 2048
+    q, kv, idx = (t.to(dev) for t in mla.mla_make_inputs(2, heads, 4500, topk, generator=gen))
+    idx[1, topk // 3:topk - 5] = -1          # splits without rows
+    check(capi, q, kv, idx, splits, oracle_on_gpu(q, kv, idx))
+
+
+@pytest.mark.parametrize('shape', [(3, 32, 700, 300), (5, 64, 900, 129), (1, 64, 2100, 2048)])
+def test_few_heads_over_the_fp8_cache(capi, dev, shape):
+    # the kernel that dequantises its tiles against the bf16 decode of the dequantised cache, bit for bit
+    B, H, N, topk = shape
+    gen = torch.Generator().manual_seed(B + topk)
+    q, kv, idx = (t.to(dev) for t in mla.mla_make_inputs(B, H, N, topk, generator=gen))
+    cache = torch.empty(B, N, capi.LATENT_ROW_BYTES, dtype=torch.uint8, device=dev)
+    capi.mla_latent_quant_launch(cache, kv)
+    rows = mla.latent_dequantize(cache.cpu()).to(dev)
+    out = torch.empty(B, H, 512, dtype=torch.float32, device=dev)
+    ws = torch.empty(capi.sparse_mla_fp8_workspace_bytes(B, H, topk), dtype=torch.uint8, device=dev)
+    capi.sparse_mla_decode_fp8_launch(out, q, cache, idx, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, run_kernel(capi, q, rows, idx, 0, torch.float32))
+
+
 def test_against_cpu_oracle_small(capi, dev):
     gen = torch.Generator().manual_seed(77)
     q, kv, idx = mla.mla_make_inputs(2, 128, 500, 200, generator=gen)
