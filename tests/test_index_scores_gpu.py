@@ -267,3 +267,43 @@ def test_fp8_rejects_unsupported_shapes(capi, dev):
     qc, kc, ks, w = make_fp8(1, 48, 64, 1)
     with pytest.raises(capi.LaunchRejected):
         run_fp8(capi, dev, qc, kc, ks, w)
+
+
+@pytest.mark.parametrize('fp8', [False, True])
+@pytest.mark.parametrize('shape', [(1, 64, 64), (2, 4096, 16), (3, 3008, 32), (9, 16384, 64), (17, 16384, 128), (34, 16384, 64)])
+def test_paged_equals_contiguous(capi, dev, shape, fp8):
+    # every number of tiles per wavefront, pages below and above a tile, requests that end inside a tile, at its
+    # edge and before the first, unmapped pages: bit for bit the scores of the contiguous cache, -inf elsewhere
+    B, N, page = shape
+    gen = torch.Generator(device=dev).manual_seed(N + page)
+    q = torch.randn(B, 64, 128, device=dev, generator=gen)
+    k = torch.randn(B, N, 128, device=dev, generator=gen)
+    w = torch.randn(B, 64, device=dev, generator=gen)
+    ks = torch.rand(B, N, device=dev, generator=gen) + 0.5
+    lengths = torch.randint(0, N + 1, (B,), device=dev, generator=gen, dtype=torch.int32)
+    lengths[0] = N - 1
+    if B > 2:
+        lengths[1], lengths[2] = 0, 32 * (N // 64)
+    table = torch.randperm(B * N // page, device=dev, generator=gen).int().view(B, N // page)
+    flat, got = torch.empty(B, N, device=dev), torch.empty(B, N, device=dev)
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    q, k = q.to(dt), k.to(dt)
+    pool = torch.empty_like(k).view(B * N // page, page, 128)
+    pool.view(torch.uint8)[table.long()] = k.view(B, N // page, page, 128).view(torch.uint8)
+    scale_pool = torch.empty_like(ks).view(-1, page)
+    scale_pool[table.long()] = ks.view(B, N // page, page)
+    unmapped = torch.rand(B, N // page, device=dev, generator=gen) < 0.05
+    table[unmapped] = -1
+    if fp8:
+        capi.mla_index_scores_fp8_launch(flat, q, k, ks, w, lengths)
+        capi.mla_index_scores_fp8_paged_launch(got, q, pool, scale_pool, table, w, lengths)
+    else:
+        capi.mla_index_scores_launch(flat, q, k, w, lengths)
+        capi.mla_index_scores_paged_launch(got, q, pool, table, w, lengths)
+    if fp8:
+        check_fp8(flat[:1].cpu(), q[:1].view(torch.uint8).cpu(), k[:1].view(torch.uint8).cpu(), ks[:1].cpu(),
+                  w[:1].cpu(), lengths[:1].cpu())
+    else:
+        check(flat[:1].cpu(), q[:1].cpu(), k[:1].cpu(), w[:1].cpu(), lengths[:1].cpu())
+    flat.view(B, N // page, page)[unmapped] = float('-inf')
+    assert torch.equal(got, flat)
