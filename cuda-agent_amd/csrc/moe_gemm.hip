@@ -74,6 +74,50 @@ __device__ __forceinline__ floatx4 block_dot_bf16(const Bf16Block& a, const Bf16
     return part;
 }
 
+// The expert of grid row `y`. With fewer pairs than experts the grid has one row per pair instead of one per expert,
+// and row y takes the y-th expert that has pairs (-1: there are no more): a workgroup of these kernels needs most of a
+// CU's LDS, so that the empty workgroups of 248 idle experts went through the CUs one at a time before and between
+// the working ones (gate/up of two tokens of the 256-expert layer 106 -> 77 us, of four 171 -> 144). last_first: the last expert is the heaviest (a
+// shared expert that every token uses): its workgroups are dispatched first, so that its several passes do not become
+// the launch's tail.
+constexpr int MAX_LISTED_EXPERTS = 512;
+
+__device__ __forceinline__ int grid_expert(const int* __restrict__ expert_offsets, int n_experts, int y, int rows,
+                                           bool last_first, int lane) {
+    const bool all = rows >= n_experts;
+    if (last_first) {
+        if (y == 0) return n_experts - 1;
+        --y, --n_experts;
+    }
+    if (all) return y;
+    // lane l looks at experts l*per .. l*per + per - 1
+    constexpr int MOST = MAX_LISTED_EXPERTS / 64;
+    const int per = (n_experts + 63) / 64;
+    const int first = lane * per;
+    int off[MOST + 1];
+#pragma unroll
+    for (int i = 0; i <= MOST; ++i) off[i] = expert_offsets[first + i < n_experts ? first + i : n_experts];
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) mine += i < per && off[i + 1] > off[i] ? 1 : 0;
+    int upto = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(upto, d);
+        if (lane >= d) upto += v;
+    }
+    int left = y - (upto - mine), e = -1;
+#pragma unroll
+    for (int i = 0; i < MOST; ++i) {
+        if (i < per && off[i + 1] > off[i]) {
+            if (left == 0) e = first + i;
+            --left;
+        }
+    }
+    const unsigned long long owner = __ballot(e >= 0);
+    return owner ? __builtin_amdgcn_readlane(e, __builtin_ctzll(owner)) : -1;
+}
+
 // Epilogue of the streaming gate/up kernels: h = silu(gate) * up, e4m3 with one scale per pair over the
 // workgroup's 128 columns. acc[nt][t]: tiles 0, 1 gate, 2, 3 up; a lane holds rows 4g..4g+3 of each 16-row
 // tile for pair column `col`.
@@ -132,13 +176,12 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_kernel(
     const float* __restrict__ a_s, const int* __restrict__ sorted_pairs,
     const int* __restrict__ expert_offsets, uint8_t* __restrict__ h_q, float* __restrict__ h_s,
     float* __restrict__ y, int K, int n_rows, int inter, int top_k, bool pow2,
-    bool last_first) {
+    bool last_first, int n_experts) {
     constexpr int TILES = GATE_UP ? 4 : 2;
     __shared__ float s_amax[4][NT * 16];
 
-    // last_first: the last expert is the heaviest (a shared expert that every token uses): its
-    // workgroups are dispatched first, so that its several passes do not become the launch's tail
-    const int e = last_first ? (blockIdx.y == 0 ? (int)gridDim.y - 1 : (int)blockIdx.y - 1) : (int)blockIdx.y;
+    const int e = grid_expert(expert_offsets, n_experts, blockIdx.y, gridDim.y, last_first, threadIdx.x & 63);
+    if (e < 0) return;
     const int rb = blockIdx.x;  // 128-row block of the output dimension
     const int begin = expert_offsets[e];
     const int end = expert_offsets[e + 1];
@@ -322,7 +365,7 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     const float* __restrict__ a_s, const int* __restrict__ sorted_pairs,
     const int* __restrict__ expert_offsets, uint8_t* __restrict__ h_q, float* __restrict__ h_s,
     float* __restrict__ y, int K, int n_rows, int inter, int top_k, bool pow2,
-    bool last_first) {
+    bool last_first, int n_experts) {
     constexpr int TILES = 4;
     constexpr int DEPTH = 3;
     constexpr int TILE_BYTES = 16 * GROUP;                       // 2 KB
@@ -333,9 +376,8 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     __shared__ float s_bscale[MAX_KB][NT * 16];
     __shared__ float s_amax[4][NT * 16];
 
-    // last_first: the last expert is the heaviest (a shared expert that every token uses): its
-    // workgroups are dispatched first, so that its several passes do not become the launch's tail
-    const int e = last_first ? (blockIdx.y == 0 ? (int)gridDim.y - 1 : (int)blockIdx.y - 1) : (int)blockIdx.y;
+    const int e = grid_expert(expert_offsets, n_experts, blockIdx.y, gridDim.y, last_first, threadIdx.x & 63);
+    if (e < 0) return;
     const int rb = blockIdx.x;  // block of 256 output rows (GATE_UP: 128 gate + 128 up)
     const int begin = expert_offsets[e];
     const int end = expert_offsets[e + 1];
@@ -506,6 +548,12 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     }
 }
 
+// rows of the grid: see grid_expert
+int grid_rows(int tokens, int top_k, int n_experts) {
+    const long pairs = (long)tokens * top_k;
+    return n_experts <= MAX_LISTED_EXPERTS && pairs < n_experts ? (int)pairs : n_experts;
+}
+
 bool check_common(int hidden, int inter, int n_experts) {
     return hidden > 0 && inter > 0 && n_experts > 0 && hidden % GROUP == 0 && inter % GROUP == 0 &&
            n_experts <= 65535;
@@ -536,7 +584,7 @@ extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, con
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
-    const dim3 grid(inter / GROUP, n_experts);
+    const dim3 grid(inter / GROUP, grid_rows(tokens, top_k, n_experts));
     auto* hq = static_cast<uint8_t*>(h_q);
     const auto* xq = static_cast<const uint8_t*>(x_q);
     const auto* wq = static_cast<const uint8_t*>(w13_q);
@@ -553,7 +601,7 @@ extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, con
 #define MOE_GATE_UP_LAUNCH(KERNEL, NT_, EXACT_)                                                           \
     KERNEL<true, NT_, EXACT_><<<grid, 256, 0, stream>>>(wq, w13_s, xq, x_s, sorted_pairs, expert_offsets, \
                                                        hq, h_s, nullptr, hidden, 2 * inter, inter, top_k, \
-                                                       pow2, last_first)
+                                                       pow2, last_first, n_experts)
 #define MOE_GATE_UP_CASE(NT_)                                                           \
     if (lds_path && exact) MOE_GATE_UP_LAUNCH(moe_stream_gemm_lds_kernel, NT_, true);   \
     else if (lds_path) MOE_GATE_UP_LAUNCH(moe_stream_gemm_lds_kernel, NT_, false);      \
@@ -588,7 +636,8 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
-    const dim3 grid(hidden / GROUP, n_experts);
+    const int rows = grid_rows(tokens, top_k, n_experts);
+    const dim3 grid(hidden / GROUP, rows);
     const auto* hq = static_cast<const uint8_t*>(h_q);
     const auto* wq = static_cast<const uint8_t*>(w2_q);
     const bool last_first = (config & CONFIG_LAST_EXPERT_FIRST) != 0;
@@ -600,34 +649,34 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
         nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
     }
     const bool lds_path = config < 8 && hidden % 256 == 0 && inter / GROUP <= 64;
-    const dim3 grid256(hidden / 256, n_experts);
+    const dim3 grid256(hidden / 256, rows);
     switch (nt) {
         case 1:
             if (lds_path) {
                 moe_stream_gemm_lds_kernel<false, 1><<<grid256, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first);
+                    inter, top_k, false, last_first, n_experts);
             } else {
                 moe_stream_gemm_kernel<false, 1><<<grid, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first);
+                    inter, top_k, false, last_first, n_experts);
             }
             break;
         case 2:
             if (lds_path) {
                 moe_stream_gemm_lds_kernel<false, 2><<<grid256, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first);
+                    inter, top_k, false, last_first, n_experts);
             } else {
                 moe_stream_gemm_kernel<false, 2><<<grid, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first);
+                    inter, top_k, false, last_first, n_experts);
             }
             break;
         default:
             moe_stream_gemm_kernel<false, 4><<<grid, 256, 0, stream>>>(
                 wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden, inter,
-                top_k, false, last_first);
+                top_k, false, last_first, n_experts);
             break;
     }
 }

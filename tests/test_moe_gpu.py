@@ -260,6 +260,13 @@ def test_layer_ragged_expert_load(capi, dev):
     check_layer(capi, dev, T=1, H=128, I=128, E=8, k=8, seed=44)
 
 
+@pytest.mark.parametrize('shape', [(1, 9, 8), (1, 8, 8), (2, 16, 8), (2, 17, 8), (3, 200, 5), (5, 512, 3)])
+def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
+    # one grid row per pair instead of per expert: pairs one below, equal to and above the number of experts
+    T, E, k = shape
+    check_layer(capi, dev, T=T, H=256, I=128, E=E, k=k, seed=600 + E)
+
+
 def test_layer_passes_reference_harness_bound(capi, dev):
     out, ref = check_layer(capi, dev, T=32, H=512, I=2048, E=16, k=8, seed=45)
     torch.testing.assert_close(out, ref.bfloat16(), atol=1e-2, rtol=1e-2)   # outputs are O(0.2)

@@ -93,7 +93,9 @@ def run_fused(capi, dts, top_k, config=0, dtype=torch.float32):
 
 @pytest.mark.parametrize('config', [16, 4, 0])
 @pytest.mark.parametrize('shape', [(64, 512, 256, 16, 4), (300, 256, 128, 8, 2), (1, 256, 128, 4, 1),
-                                   (1100, 512, 256, 5, 2), (33, 768, 384, 40, 8), (128, 512, 256, 256, 7)])
+                                   (1100, 512, 256, 5, 2), (33, 768, 384, 40, 8), (128, 512, 256, 256, 7),
+                                   # pairs below, equal to and above the number of stored experts
+                                   (2, 256, 128, 18, 8), (2, 256, 128, 17, 8), (2, 256, 128, 16, 8), (3, 256, 128, 300, 4)])
 def test_shared_expert_inside_the_routed_launch(capi, dev, shape, config):
     T, H, I, E, k = shape
     x, logits, w, sw, dts = make_case(dev, T, H, I, I, E, 4000 + T)
