@@ -260,11 +260,13 @@ def test_layer_ragged_expert_load(capi, dev):
     check_layer(capi, dev, T=1, H=128, I=128, E=8, k=8, seed=44)
 
 
-@pytest.mark.parametrize('shape', [(1, 9, 8), (1, 8, 8), (2, 16, 8), (2, 17, 8), (3, 200, 5), (5, 512, 3)])
+@pytest.mark.parametrize('shape', [(1, 9, 8), (1, 8, 8), (2, 16, 8), (2, 17, 8), (3, 200, 5), (5, 300, 3)])
 def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
     # one grid row per pair instead of per expert: pairs one below, equal to and above the number of experts
+    # (inter 2048: check_layer allows 2e-4 of the codes to be undecided ones, which must be more than one code:
+    # 12 to 50 per million are expected)
     T, E, k = shape
-    check_layer(capi, dev, T=T, H=256, I=128, E=E, k=k, seed=600 + E)
+    check_layer(capi, dev, T=T, H=256, I=2048, E=E, k=k, seed=600 + E)
 
 
 def test_layer_passes_reference_harness_bound(capi, dev):
