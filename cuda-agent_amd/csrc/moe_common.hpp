@@ -121,6 +121,38 @@ __device__ __forceinline__ float group_scale(float amax, bool pow2) {
 }
 #endif
 
+#ifdef __HIPCC__
+// Activation quantisation of one 128-wide group by 16 lanes, 8 values (16 bytes in, 8 codes out) each; `sub` is the
+// lane's number among them. The division is IEEE fp32 so that the codes are bit-identical to a CPU evaluation of the
+// same formula; v_cvt_pk_fp8_f32 rounds to nearest even but does not saturate (465 -> NaN), hence the clamp.
+__device__ __forceinline__ void quantise_group16(const void* __restrict__ x, uint8_t* __restrict__ q,
+                                                 float* __restrict__ scales, long group, int sub, bool pow2) {
+    typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+    typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+    const uintx4 raw = reinterpret_cast<const uintx4*>(x)[group * (GROUP / 8) + sub];
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = __uint_as_float(raw[j] << 16);
+        v[2 * j + 1] = __uint_as_float(raw[j] & 0xffff0000u);
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    const float scale = group_scale(amax, pow2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);
+    int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+    lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
+    int hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
+    hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
+    *reinterpret_cast<uintx2*>(q + group * GROUP + 8 * sub) = uintx2{(unsigned)lo, (unsigned)hi};
+    if (sub == 0) scales[group] = scale;
+}
+#endif
+
 // Device scratch of one forward pass, carved from the caller's workspace.
 struct Workspace {
     int* ids;             // [T*k]  expert of every (token, slot) pair, slots by descending logit

@@ -16,6 +16,9 @@ extern "C" void moe_route_sort_launcher(int* ids, float* weights, int* sorted_pa
                                         hipStream_t stream);
 extern "C" void moe_quant_bf16_launcher(void* q, float* scales, const void* x, int rows, int cols,
                                         int config, hipStream_t stream);
+extern "C" int moe_front_small(int* ids, float* weights, int* sorted_pairs, int* pair_pos, int* expert_offsets,
+                               void* x_q, float* x_s, const float* logits, const void* x, int tokens, int hidden,
+                               int n_experts, int top_k, int config, hipStream_t stream);
 extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, const float* x_s,
                                      const void* w13_q, const float* w13_s, const int* sorted_pairs,
                                      const int* expert_offsets, int tokens, int hidden, int inter,
@@ -213,6 +216,17 @@ GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int
     return plan;
 }
 
+// routing (shared_slot: CONFIG_SHARED_SLOT or 0), sort and activation quantiser
+void run_front(const moe::Workspace& w, const void* x, const float* logits, int tokens, int hidden, int n_experts,
+               int top_k, int shared_slot, int ue8m0, hipStream_t stream) {
+    if (moe_front_small(w.ids, w.weights, w.sorted_pairs, w.pair_pos, w.expert_offsets, w.x_q, w.x_s, logits, x, tokens,
+                        hidden, n_experts, top_k, shared_slot | ue8m0, stream))
+        return;
+    moe_route_sort_launcher(w.ids, w.weights, w.sorted_pairs, w.pair_pos, w.expert_offsets, w.chunk_hist, logits,
+                            tokens, n_experts, top_k, shared_slot, stream);
+    moe_quant_bf16_launcher(w.x_q, w.x_s, x, tokens, hidden, ue8m0, stream);
+}
+
 // gate/up and down GEMMs of the experts over the quantised activations and the sort in `w`; result
 // in w.y. Many pairs per expert: LDS-tiled GEMMs (256 x 256 tiles). Few: the weight-streaming form.
 void run_expert_gemms(const moe::Workspace& w, const GemmPlan& plan, const void* w13_q, const float* w13_s,
@@ -285,9 +299,7 @@ extern "C" void moe_fp8_launcher(void* out, const void* x, const float* logits, 
         caa::set_status(CAA_WORKSPACE_TOO_SMALL);
         return;
     }
-    moe_route_sort_launcher(w.ids, w.weights, w.sorted_pairs, w.pair_pos, w.expert_offsets, w.chunk_hist,
-                            logits, tokens, n_experts, top_k, 0, stream);
-    moe_quant_bf16_launcher(w.x_q, w.x_s, x, tokens, hidden, config & CONFIG_UE8M0, stream);
+    run_front(w, x, logits, tokens, hidden, n_experts, top_k, 0, config & CONFIG_UE8M0, stream);
     run_expert_gemms(w, plan, w13_q, w13_s, w2_q, w2_s, tokens, hidden, inter, n_experts, top_k, config, stream);
     launch_combine(out, w.y, plan.tiled ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,
                    top_k, out_dtype, stream);
@@ -336,9 +348,7 @@ extern "C" void moe_fp8_shared_launcher(void* out, const void* x, const float* l
         caa::set_status(CAA_WORKSPACE_TOO_SMALL);
         return;
     }
-    moe_route_sort_launcher(w.ids, w.weights, w.sorted_pairs, w.pair_pos, w.expert_offsets, w.chunk_hist,
-                            logits, tokens, n_experts, top_k, 0, stream);
-    moe_quant_bf16_launcher(w.x_q, w.x_s, x, tokens, hidden, config & CONFIG_UE8M0, stream);
+    run_front(w, x, logits, tokens, hidden, n_experts, top_k, 0, config & CONFIG_UE8M0, stream);
     run_expert_gemms(w, plan, w13_q, w13_s, w2_q, w2_s, tokens, hidden, inter, n_experts, top_k, config, stream);
     sh.x_q = w.x_q;
     sh.x_s = w.x_s;
@@ -380,9 +390,7 @@ extern "C" void moe_fp8_fused_shared_launcher(void* out, const void* x, const fl
         caa::set_status(CAA_WORKSPACE_TOO_SMALL);
         return;
     }
-    moe_route_sort_launcher(w.ids, w.weights, w.sorted_pairs, w.pair_pos, w.expert_offsets, w.chunk_hist,
-                            logits, tokens, n_experts, top_k, CONFIG_SHARED_SLOT, stream);
-    moe_quant_bf16_launcher(w.x_q, w.x_s, x, tokens, hidden, config & CONFIG_UE8M0, stream);
+    run_front(w, x, logits, tokens, hidden, n_experts, top_k, CONFIG_SHARED_SLOT, config & CONFIG_UE8M0, stream);
     run_expert_gemms(w, plan, w13_q, w13_s, w2_q, w2_s, tokens, hidden, inter, n_experts + 1, top_k + 1,
                      (config & ~CONFIG_LAST_EXPERT_FIRST) | CONFIG_LAST_EXPERT_FIRST, stream);
     launch_combine(out, w.y, plan.tiled ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,

@@ -39,35 +39,8 @@ __global__ __launch_bounds__(256) void moe_quant_bf16_vec_kernel(const __hip_bfl
                                                                  uint8_t* __restrict__ q,
                                                                  float* __restrict__ scales,
                                                                  long n_groups, bool pow2) {
-    typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-    typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
-    const int sub = threadIdx.x & 15;
     const long g = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
-    if (g >= n_groups) return;
-    const uintx4 raw = *reinterpret_cast<const uintx4*>(x + g * GROUP + 8 * sub);
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        v[2 * j] = __uint_as_float(raw[j] << 16);
-        v[2 * j + 1] = __uint_as_float(raw[j] & 0xffff0000u);
-    }
-    float amax = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    const float scale = group_scale(amax, pow2);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);
-    uintx2 packed;
-    int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
-    int hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
-    packed[0] = (unsigned)lo;
-    packed[1] = (unsigned)hi;
-    *reinterpret_cast<uintx2*>(q + g * GROUP + 8 * sub) = packed;
-    if (sub == 0) scales[g] = scale;
+    if (g < n_groups) quantise_group16(x, q, scales, g, threadIdx.x & 15, pow2);
 }
 
 }  // namespace

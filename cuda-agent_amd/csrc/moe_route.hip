@@ -62,6 +62,38 @@ __device__ __forceinline__ unsigned long long wave_max_key(unsigned long long ke
     return ((unsigned long long)hi_max << 32) | lo_max;
 }
 
+// The top_k experts of a token by one wavefront: lane k < top_k gets the k-th choice and its normalised weight.
+template <int PER_LANE>
+__device__ __forceinline__ void route_token(const float* __restrict__ row, int n_experts, int top_k, int lane,
+                                            int& my_id, float& my_weight) {
+    unsigned long long key[PER_LANE];
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) {
+        const int e = j * 64 + lane;
+        key[j] = e < n_experts ? rank_key(row[e], e) : 0ull;
+    }
+    float my_score = 0.f, total = 0.f;
+    my_id = 0;
+    for (int k = 0; k < top_k; ++k) {
+        unsigned long long best = 0ull;
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j) best = key[j] > best ? key[j] : best;
+        best = wave_max_key(best);
+        const int id = 0x7fffffff - (int)(unsigned)(best & 0xffffffffull);
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j) {
+            if (j * 64 + lane == id) key[j] = 0ull;  // taken
+        }
+        const float score = 1.f / (1.f + expf(-key_logit(best)));
+        total += score;
+        if (lane == k) {
+            my_score = score;
+            my_id = id;
+        }
+    }
+    my_weight = my_score / total;
+}
+
 template <int PER_LANE>
 __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits,
                                                         int* __restrict__ ids,
@@ -73,36 +105,12 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= tokens) return;
-    unsigned long long key[PER_LANE];
-#pragma unroll
-    for (int j = 0; j < PER_LANE; ++j) {
-        const int e = j * 64 + lane;
-        key[j] = e < n_experts ? rank_key(logits[(size_t)t * n_experts + e], e) : 0ull;
-    }
-    float my_score = 0.f;  // lane k keeps the k-th choice
-    int my_id = 0;
-    float total = 0.f;
-    for (int k = 0; k < top_k; ++k) {
-        unsigned long long best = 0ull;
-#pragma unroll
-        for (int j = 0; j < PER_LANE; ++j) best = key[j] > best ? key[j] : best;
-        best = wave_max_key(best);
-        const int id = 0x7fffffff - (int)(unsigned)(best & 0xffffffffull);
-#pragma unroll
-        for (int j = 0; j < PER_LANE; ++j) {
-            if (j * 64 + lane == id) key[j] = 0ull;  // taken
-        }
-        const float logit = key_logit(best);
-        const float score = 1.f / (1.f + expf(-logit));
-        total += score;
-        if (lane == k) {
-            my_score = score;
-            my_id = id;
-        }
-    }
+    int my_id;
+    float my_weight;
+    route_token<PER_LANE>(logits + (size_t)t * n_experts, n_experts, top_k, lane, my_id, my_weight);
     if (lane < top_k) {
         ids[(size_t)t * slots + lane] = my_id;
-        weights[(size_t)t * slots + lane] = my_score / total;
+        weights[(size_t)t * slots + lane] = my_weight;
     } else if (lane == top_k && shared) {
         ids[(size_t)t * slots + lane] = n_experts;
         weights[(size_t)t * slots + lane] = 1.f;
@@ -395,34 +403,12 @@ __global__ __launch_bounds__(1024) void moe_route_sort_small_kernel(
     for (int e = threadIdx.x; e <= sorted_experts; e += 1024) s_count[e] = 0;
     for (int i = threadIdx.x; i < 16 * (512 + 1); i += 1024) (&s_wave_count[0][0])[i] = 0;
     for (int t = wave; t < tokens; t += 16) {
-        unsigned long long key[PER_LANE];
-#pragma unroll
-        for (int j = 0; j < PER_LANE; ++j) {
-            const int e = j * 64 + lane;
-            key[j] = e < n_experts ? rank_key(logits[(size_t)t * n_experts + e], e) : 0ull;
-        }
-        float my_score = 0.f, total = 0.f;
-        int my_id = 0;
-        for (int k = 0; k < top_k; ++k) {
-            unsigned long long best = 0ull;
-#pragma unroll
-            for (int j = 0; j < PER_LANE; ++j) best = key[j] > best ? key[j] : best;
-            best = wave_max_key(best);
-            const int id = 0x7fffffff - (int)(unsigned)(best & 0xffffffffull);
-#pragma unroll
-            for (int j = 0; j < PER_LANE; ++j) {
-                if (j * 64 + lane == id) key[j] = 0ull;
-            }
-            const float score = 1.f / (1.f + expf(-key_logit(best)));
-            total += score;
-            if (lane == k) {
-                my_score = score;
-                my_id = id;
-            }
-        }
+        int my_id;
+        float my_weight;
+        route_token<PER_LANE>(logits + (size_t)t * n_experts, n_experts, top_k, lane, my_id, my_weight);
         if (lane < top_k) {
             ids[(size_t)t * slots + lane] = my_id;
-            weights[(size_t)t * slots + lane] = my_score / total;
+            weights[(size_t)t * slots + lane] = my_weight;
             s_ids[t * slots + lane] = my_id;
         } else if (lane == top_k && shared) {
             ids[(size_t)t * slots + lane] = n_experts;
@@ -505,7 +491,85 @@ __global__ __launch_bounds__(1024) void moe_sort_small_kernel(const int* __restr
     }
 }
 
+// Everything in front of the GEMMs for a few tokens in one launch: workgroup 0 routes (one wavefront per token at a
+// time) and sorts, the others quantise the activations, 64 groups each. As three launches (routing, the sort, the
+// quantiser) this took 15 us of the 85 one token needs; at 16 tokens the wavefronts of one CU still take one token
+// each. The sort of at most MAX_FRONT_PAIRS pairs counts, for every pair, the pairs in front of it in sorted order.
+constexpr int MAX_FRONT_TOKENS = 16;
+constexpr int MAX_FRONT_PAIRS = 256;
+
+template <int PER_LANE>
+__global__ __launch_bounds__(1024) void moe_front_small_kernel(
+    const float* __restrict__ logits, const void* __restrict__ x, int* __restrict__ ids, float* __restrict__ weights,
+    int* __restrict__ sorted_pairs, int* __restrict__ pair_pos, int* __restrict__ expert_offsets,
+    uint8_t* __restrict__ x_q, float* __restrict__ x_s, int tokens, int n_experts, int top_k, int shared,
+    long n_groups, bool pow2) {
+    if (blockIdx.x > 0) {
+        const long g = (long)(blockIdx.x - 1) * 64 + (threadIdx.x >> 4);
+        if (g < n_groups) quantise_group16(x, x_q, x_s, g, threadIdx.x & 15, pow2);
+        return;
+    }
+    __shared__ int4 s_ids[MAX_FRONT_PAIRS / 4];
+    int* flat = reinterpret_cast<int*>(s_ids);
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int slots = top_k + shared;  // see moe_route_kernel
+    const int pairs = tokens * slots;
+    // (entries past the last pair belong to no expert and stand behind all others)
+    if (threadIdx.x < MAX_FRONT_PAIRS && (int)threadIdx.x >= pairs) flat[threadIdx.x] = 0x7fffffff;
+    for (int t = wave; t < tokens; t += 16) {
+        int my_id;
+        float my_weight;
+        route_token<PER_LANE>(logits + (size_t)t * n_experts, n_experts, top_k, lane, my_id, my_weight);
+        if (lane == top_k) my_id = n_experts, my_weight = 1.f;
+        if (lane < slots) {
+            ids[t * slots + lane] = my_id;
+            weights[t * slots + lane] = my_weight;
+            flat[t * slots + lane] = my_id;
+        }
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i > n_experts + shared && i >= pairs) return;
+    const int mine = i < pairs ? flat[i] : -1;
+    int pos = 0, before = 0;  // of pair i; pairs of the experts before expert i
+    for (int p = 0; p < pairs; p += 4) {
+        const int4 v = s_ids[p / 4];
+        const int e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pos += e[j] < mine || (e[j] == mine && p + j < i) ? 1 : 0;
+            before += e[j] < i ? 1 : 0;
+        }
+    }
+    if (i < pairs) {
+        sorted_pairs[pos] = i;
+        pair_pos[i] = pos;
+    }
+    if (i <= n_experts + shared) expert_offsets[i] = before;
+}
+
 }  // namespace
+
+// Routing, sort and quantiser of a small batch in one launch. Internal to the library: moe_layer.hip calls it after
+// its own checks. Returns 0, without launching, for batches it is not made for; config: CONFIG_SHARED_SLOT,
+// CONFIG_UE8M0.
+extern "C" int moe_front_small(int* ids, float* weights, int* sorted_pairs, int* pair_pos, int* expert_offsets,
+                               void* x_q, float* x_s, const float* logits, const void* x, int tokens, int hidden,
+                               int n_experts, int top_k, int config, hipStream_t stream) {
+    const int shared = (config & CONFIG_SHARED_SLOT) ? 1 : 0;
+    if (tokens > MAX_FRONT_TOKENS || tokens * (top_k + shared) > MAX_FRONT_PAIRS || top_k + shared > 64 ||
+        n_experts > 512 || hidden % GROUP != 0 || (reinterpret_cast<uintptr_t>(x) & 15u) ||
+        (reinterpret_cast<uintptr_t>(x_q) & 7u))
+        return 0;
+    const long n_groups = (long)tokens * (hidden / GROUP);
+    const bool pow2 = (config & CONFIG_UE8M0) != 0;
+    const dim3 grid((unsigned)(1 + (n_groups + 63) / 64));
+    const auto kernel = n_experts <= 256 ? moe_front_small_kernel<4> : moe_front_small_kernel<8>;
+    kernel<<<grid, 1024, 0, stream>>>(logits, x, ids, weights, sorted_pairs, pair_pos, expert_offsets,
+                                      static_cast<uint8_t*>(x_q), x_s, tokens, n_experts, top_k, shared, n_groups, pow2);
+    return 1;
+}
 
 // Routing followed by the sort. Small batches (tokens*top_k <= 1024): the routing kernel, then the
 // single-workgroup sort (config 2: one kernel that does both in one workgroup); otherwise
