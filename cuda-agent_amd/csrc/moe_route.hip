@@ -155,25 +155,31 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
-    // lane g: value of group g
-    float value = -INFINITY;
-    if (lane < n_group) {
-        float first = -INFINITY, second = -INFINITY;
-        for (int i = 0; i < group_size; ++i) {
-            const float c = s_choice[lane * group_size + i];
-            if (c > first) {
-                second = first;
-                first = c;
-            } else if (c > second) {
-                second = c;
-            }
+    // Value of every group: `share` lanes (a power of two, 64 / share >= n_group) take every share-th expert of one
+    // group each and merge their two largest; lane g * share then holds group g's.
+    int share = 1;
+    while (2 * share * n_group <= 64) share *= 2;
+    float first = -INFINITY, second = -INFINITY;
+    if (lane < share * n_group) {
+        const float* mine = s_choice + (lane / share) * group_size;
+        for (int i = lane & (share - 1); i < group_size; i += share) {
+            const float c = mine[i];
+            second = fmaxf(second, fminf(first, c));
+            first = fmaxf(first, c);
         }
-        value = group_size > 1 ? first + second : first;
     }
+    for (int d = 1; d < share; d <<= 1) {
+        const float f = __shfl_xor(first, d), g = __shfl_xor(second, d);
+        second = fmaxf(fmaxf(second, g), fminf(first, f));
+        first = fmaxf(first, f);
+    }
+    const float held = group_size > 1 ? first + second : first;
+    float value = __shfl(held, (lane * share) & 63);  // lane g: value of group g
+    if (lane >= n_group) value = -INFINITY;
     // rank of group `lane` among the groups; the topk_group best stay
     int better = 0;
     for (int g = 0; g < n_group; ++g) {
-        const float other = __shfl(value, g);
+        const float other = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(value), g));
         better += (other > value || (other == value && g < lane)) ? 1 : 0;
     }
     const unsigned long long stay_mask = __ballot(lane < n_group && better < topk_group);
@@ -185,9 +191,7 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(
         const bool stays = e < n_experts && ((stay_mask >> (e / group_size)) & 1ull);
         key[j] = stays ? rank_key(choice[j], e) : 0ull;
     }
-    float my_score = 0.f;  // lane k keeps the k-th choice
-    int my_id = 0;
-    float total = 0.f;
+    int my_id = 0;  // lane k keeps the k-th choice
     for (int k = 0; k < top_k; ++k) {
         unsigned long long best = 0ull;
 #pragma unroll
@@ -198,13 +202,11 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(
         for (int j = 0; j < PER_LANE; ++j) {
             if (j * 64 + lane == id) key[j] = 0ull;  // taken
         }
-        const float score = s_score[id];
-        total += score;
-        if (lane == k) {
-            my_score = score;
-            my_id = id;
-        }
+        if (lane == k) my_id = id;
     }
+    const float my_score = lane < top_k ? s_score[my_id] : 0.f;
+    float total = 0.f;  // in the order of the choices
+    for (int k = 0; k < top_k; ++k) total += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_score), k));
     if (lane < top_k) {
         ids[(size_t)t * top_k + lane] = my_id;
         const float w = normalise ? my_score / (total + 1e-20f) : my_score;
