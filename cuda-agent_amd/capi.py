@@ -565,7 +565,7 @@ def moe_workspace_bytes(tokens, hidden, inter, n_experts, top_k=8):
 
 def moe_workspace_views(workspace, tokens, hidden, inter, n_experts, top_k=8):
     """Typed views of the intermediate buffers inside a workspace tensor (uint8, 1-D). ``y`` is laid out as
-    fp32 rows; when the layer ran the LDS-tiled GEMMs (``moe_fp8_uses_tiled_gemms`` returns 1) it holds fp16 rows
+    fp32 rows; when the layer stores it the other way (``moe_fp8_uses_tiled_gemms`` returns 1) it holds fp16 rows
     with the scales in ``y_scale`` instead and must be read through ``moe_expert_outputs``."""
     offs = (c_size_t * len(MOE_WORKSPACE_FIELDS))()
     n = library().moe_fp8_workspace_layout(offs, len(MOE_WORKSPACE_FIELDS), tokens, hidden, inter, n_experts, top_k)
@@ -593,7 +593,7 @@ def moe_workspace_views(workspace, tokens, hidden, inter, n_experts, top_k=8):
 
 def moe_expert_outputs(views, tokens, hidden, inter, n_experts, top_k=8, config=0):
     """The expert outputs y [tokens*top_k, hidden] of a finished layer as fp32, whichever way the layer stored
-    them: fp32 rows (weight-streaming GEMMs) or fp16 rows with power-of-two scales (LDS-tiled GEMMs)."""
+    them: fp32 rows, or fp16 rows with power-of-two scales (LDS-tiled GEMMs, more than 32 pairs per expert)."""
     tiled = library().moe_fp8_uses_tiled_gemms(tokens, hidden, inter, n_experts, top_k, config)
     _require(tiled >= 0, 'moe_expert_outputs: unsupported shape')
     if not tiled:

@@ -55,6 +55,9 @@ constexpr int CONFIG_SIGNIF_SHIFT = 12;
 constexpr int CONFIG_SIGNIF_MASK = 15 << CONFIG_SIGNIF_SHIFT;
 constexpr int CONFIG_REQUANT_BITS = CONFIG_EXACT_REQUANT | CONFIG_APPROX_REQUANT | CONFIG_BAND_MASK | CONFIG_SIGNIF_MASK;
 
+// config value of the layer (with the bits above): the narrow tiles whatever the number of pairs per expert
+constexpr int CONFIG_NARROW_TILES = 1 << 16;
+
 // marks of one element of h
 constexpr uint32_t MARK_NEAR = 1;       // the scaled value may round to either of two codes
 constexpr uint32_t MARK_CANDIDATE = 2;  // the element may be the largest magnitude of its group

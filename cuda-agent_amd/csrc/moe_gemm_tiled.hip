@@ -24,22 +24,11 @@
 // rows, each wavefront holding 32 of either, so SiLU(gate)*up and the e4m3 requantisation of
 // the 128-column group happen in the epilogue without leaving the workgroup.
 #include "launch_status.hpp"
-#include "moe_common.hpp"
+#include "moe_tile.hpp"
 
 namespace {
 
 using namespace moe;
-
-typedef int intx8 __attribute__((ext_vector_type(8)));
-typedef int intx4 __attribute__((ext_vector_type(4)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
-typedef const __attribute__((address_space(3))) uint8_t* lds_bytes;
-typedef const __attribute__((address_space(3))) intx4* lds_x4;
 
 constexpr int TILE_PAIRS = 256;
 constexpr int TILE_ROWS = 256;
@@ -47,37 +36,12 @@ constexpr int STAGE_A = TILE_ROWS * GROUP;    // 32 KB
 constexpr int STAGE_B = TILE_PAIRS * GROUP;   // 32 KB
 constexpr int STAGE_S = TILE_PAIRS * 4;       // 1 KB of scales
 constexpr int STAGE_BYTES = STAGE_A + STAGE_B + STAGE_S;
-constexpr int SUPER_ROWS = 4;   // row tiles and pair tiles of the block of workgroups that
-constexpr int SUPER_PAIRS = 8;  // share one XCD's L2
-
-inline int tiled_grid(int row_tiles, int max_pair_tiles) {
-    const int supers = ((row_tiles + SUPER_ROWS - 1) / SUPER_ROWS) * ((max_pair_tiles + SUPER_PAIRS - 1) / SUPER_PAIRS);
-    return ((supers + 7) / 8) * 8 * SUPER_ROWS * SUPER_PAIRS;
-}
-
-template <int N>
-struct IntConstant {
-    static constexpr int value = N;
-};
-
-__device__ __forceinline__ intx8 join(intx4 lo, intx4 hi) {
-    return intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-}
 
 // x / (1 + exp(-x)) on the hardware's exp2 and reciprocal (a few units in the last place of the exact value:
 // far inside what the e4m3 matrix core leaves of the pre-activation; the library routines for exp and the IEEE
 // division were a tenth of a full tile's time in the gate/up epilogue)
 __device__ __forceinline__ float silu(float x) {
     return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
-}
-
-// 8 e4m3 codes (two dwords) -> 8 bf16, exactly (every e4m3 value is a bf16 value)
-__device__ __forceinline__ bf16x8 e4m3x8_to_bf16(int lo, int hi) {
-    const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-    const bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-    const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-    const bf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-    return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
 // sum over 16 e4m3 pairs of a * b, in fp32 (the products are exact, the sum is rounded 15 times)
@@ -103,35 +67,16 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-__device__ __forceinline__ void wait_all_loads() {
-    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0)
-    asm volatile("" ::: "memory");
-}
-
-// 64 lanes x 16 bytes, global -> LDS (lds_base + lane*16); asm so that the compiler does not
-// make every later LDS read wait for it: completion is awaited once per block, before the barrier.
-__device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ void dma16_ptr(const void* lane_ptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(lane_ptr), "s"(lds_base)
-                 : "memory", "m0");
-}
-
-// The order in which the experts' pair tiles are numbered, and with it dispatched. Experts with two or more
-// 256-pair tiles (the heavily loaded ones, whose tiles are bound by the matrix cores) are spread evenly among the
+// The order in which the experts' tiles of `tile_pairs` pairs are numbered, and with it dispatched. Experts with two or
+// more tiles (the heavily loaded ones, whose tiles are bound by the matrix cores) are spread evenly among the
 // others (one tile each, bound by the stream of their weights) instead of standing wherever their numbers put them:
 // slot s of the order holds expert slot_expert[s], and tile_start[s] = number of tiles of the slots before s
 // (tile_start[E] = total). Measured on the prefill workload: 2.4 % of the layer's time between the heavily loaded
 // experts evenly spread and all in a row.
 // tile_table: tile_start [n_experts + 1], then slot_expert [n_experts].
 __global__ __launch_bounds__(1024) void moe_tile_start_kernel(const int* __restrict__ expert_offsets,
-                                                              int* __restrict__ tile_table, int n_experts) {
+                                                              int* __restrict__ tile_table, int n_experts,
+                                                              int tile_pairs) {
     __shared__ int s_scan[1024];
     __shared__ int s_list[2][1024];  // experts with several tiles, and the others, each in ascending order
     __shared__ int s_slot_expert[1024];
@@ -149,7 +94,7 @@ __global__ __launch_bounds__(1024) void moe_tile_start_kernel(const int* __restr
         }
         return v;
     };
-    const int mine = t < n_experts ? (expert_offsets[t + 1] - expert_offsets[t] + TILE_PAIRS - 1) / TILE_PAIRS : 0;
+    const int mine = t < n_experts ? (expert_offsets[t + 1] - expert_offsets[t] + tile_pairs - 1) / tile_pairs : 0;
     const bool loaded = mine >= 2;
     const int loaded_upto = scan(loaded ? 1 : 0);  // experts with several tiles among 0..t
     const int n_loaded = s_scan[n_experts - 1];
@@ -165,7 +110,7 @@ __global__ __launch_bounds__(1024) void moe_tile_start_kernel(const int* __restr
     if (t < n_experts) s_slot_expert[t] = j >= 0 ? s_list[0][j] : s_list[1][free_upto - 1];
     __syncthreads();
     const int tiles_here = t < n_experts ? (expert_offsets[s_slot_expert[t] + 1] - expert_offsets[s_slot_expert[t]] +
-                                            TILE_PAIRS - 1) / TILE_PAIRS
+                                            tile_pairs - 1) / tile_pairs
                                          : 0;
     const int upto = scan(tiles_here);
     if (t < n_experts) {
@@ -236,26 +181,9 @@ __global__ __launch_bounds__(512) void moe_tiled_gemm_kernel(
     float err_coef, float v_min) {
     __shared__ __attribute__((aligned(16))) uint8_t s_stage[2 * STAGE_BYTES];
 
-    // Workgroup -> (row tile, pair tile). Consecutive workgroup ids go round-robin to the 8 XCDs,
-    // each with its own L2, so the 32 workgroups that run together on one XCD are given a
-    // 4 x 8 block of (row tile, pair tile): they share 4 weight tiles and 8 activation tiles
-    // through that L2 instead of pulling 18 different ones.
-    const int total_tiles = tile_start[n_experts];
-    const int row_tiles = GATE_UP ? inter / GROUP : n_rows / TILE_ROWS;
-    const int row_blocks4 = (row_tiles + SUPER_ROWS - 1) / SUPER_ROWS;
-    const int linear = blockIdx.x;
-    const int super = ((linear >> 3) / (SUPER_ROWS * SUPER_PAIRS)) * 8 + (linear & 7);
-    const int within = (linear >> 3) % (SUPER_ROWS * SUPER_PAIRS);
-    const int rb = (super % row_blocks4) * SUPER_ROWS + within % SUPER_ROWS;
-    const int pt = (super / row_blocks4) * SUPER_PAIRS + within / SUPER_ROWS;
-    if (rb >= row_tiles || pt >= total_tiles) return;
-    int lo = 0, hi = n_experts;  // largest slot with tile_start[slot] <= pt
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (tile_start[mid] <= pt) lo = mid; else hi = mid;
-    }
-    const int e = tile_start[n_experts + 1 + lo];  // the expert in that slot of the dispatch order
-    const int begin = expert_offsets[e] + (pt - tile_start[lo]) * TILE_PAIRS;
+    int rb, e, in_expert;
+    if (!find_tile(tile_start, n_experts, GATE_UP ? inter / GROUP : n_rows / TILE_ROWS, rb, e, in_expert)) return;
+    const int begin = expert_offsets[e] + in_expert * TILE_PAIRS;
     int cnt = expert_offsets[e + 1] - begin;
     cnt = cnt > TILE_PAIRS ? TILE_PAIRS : cnt;
 
@@ -900,20 +828,22 @@ __global__ __launch_bounds__(512) void moe_tiled_gemm_kernel(
 
 }  // namespace
 
+extern "C" int moe_tiled_tile_pairs() { return TILE_PAIRS; }
+
 // Scratch the tiled path needs beyond the layer's common workspace:
-//   tile_start [2*n_experts+1] ints (moe_tile_start_kernel); xs_t [hidden/128][stride] and hs_t [inter/128][stride] floats
-//   with stride = pairs rounded up to 256, plus 256.
+//   tile_start [2*n_experts+1] ints (moe_tile_start_kernel, for tiles of tile_pairs pairs); xs_t [hidden/128][stride] and
+//   hs_t [inter/128][stride] floats with stride = pairs rounded up to 256, plus 256.
 extern "C" void moe_tiled_prepare_launcher(int* tile_start, float* xs_t, const float* x_s,
                                            const int* sorted_pairs, const int* expert_offsets,
                                            int tokens, int hidden, int n_experts, int top_k,
-                                           int scale_stride, hipStream_t stream) {
+                                           int scale_stride, int tile_pairs, hipStream_t stream) {
     if (tokens <= 0) return;
     if (n_experts <= 0 || n_experts > 1024 || hidden <= 0 || hidden % GROUP != 0 || top_k <= 0) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);  // (the tile scan is one workgroup of 1024 lanes)
         return;
     }
     const int pairs = tokens * top_k;
-    moe_tile_start_kernel<<<1, 1024, 0, stream>>>(expert_offsets, tile_start, n_experts);
+    moe_tile_start_kernel<<<1, 1024, 0, stream>>>(expert_offsets, tile_start, n_experts, tile_pairs);
     moe_gather_scales_kernel<<<(pairs + 255) / 256, 256, 0, stream>>>(x_s, sorted_pairs, xs_t, pairs,
                                                                     scale_stride, hidden / GROUP, top_k);
 }

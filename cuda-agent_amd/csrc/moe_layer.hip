@@ -30,7 +30,7 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
 extern "C" void moe_tiled_prepare_launcher(int* tile_start, float* xs_t, const float* x_s,
                                            const int* sorted_pairs, const int* expert_offsets,
                                            int tokens, int hidden, int n_experts, int top_k,
-                                           int scale_stride, hipStream_t stream);
+                                           int scale_stride, int tile_pairs, hipStream_t stream);
 extern "C" void moe_gate_up_tiled_launcher(void* h_q, float* h_s, float* hs_t, const void* x_q,
                                            const float* xs_t, const void* w13_q, const float* w13_s,
                                            const int* sorted_pairs, const int* expert_offsets,
@@ -42,6 +42,18 @@ extern "C" void moe_down_tiled_launcher(void* y, float* y_scale, const void* h_q
                                         const int* tile_start, int tokens, int hidden, int inter,
                                         int n_experts, int top_k, int scale_stride, int ue8m0,
                                         hipStream_t stream);
+
+extern "C" int moe_narrow_tile_pairs();
+extern "C" int moe_tiled_tile_pairs();
+extern "C" void moe_gate_up_narrow_launcher(void* h_q, float* h_s, float* hs_t, const void* x_q, const float* xs_t,
+                                            const void* w13_q, const float* w13_s, const int* sorted_pairs,
+                                            const int* expert_offsets, const int* tile_start, int tokens, int hidden,
+                                            int inter, int n_experts, int top_k, int scale_stride, int ue8m0,
+                                            hipStream_t stream);
+extern "C" void moe_down_narrow_launcher(float* y, float* y_scale, const void* h_q, const float* hs_t, const void* w2_q,
+                                         const float* w2_s, const int* expert_offsets, const int* tile_start, int tokens,
+                                         int hidden, int inter, int n_experts, int top_k, int scale_stride,
+                                         hipStream_t stream);
 
 namespace {
 
@@ -196,23 +208,42 @@ extern "C" int moe_fp8_workspace_layout(size_t* offsets, int n_offsets, int toke
 
 namespace {
 
-// How the expert GEMMs of one group of experts run: LDS-tiled or weight-streaming form. Resolved, and checked
-// against what the chosen kernels support, before the first launch of a layer, so that a shape one stage rejects
-// launches nothing at all.
+// How the expert GEMMs of one group of experts run: weight-streaming, on narrow or on 256-pair LDS tiles. Resolved, and
+// checked against what the chosen kernels support, before the first launch of a layer, so that a shape one stage
+// rejects launches nothing at all.
 struct GemmPlan {
+    enum Form { STREAMING, NARROW, TILED };
     bool ok;
-    bool tiled;
+    Form form;
+    bool y_half;  // y leaves as fp16 with power-of-two scales (always from 256-pair tiles, never from the streaming form)
 };
 
-GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int top_k, int config) {
+bool aligned16(const void* a, const void* b) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
+}
+
+// aligned: both weight tensors start on 16 bytes
+GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int top_k, int config, bool aligned) {
     const int form = config & ~(CONFIG_UE8M0 | CONFIG_LAST_EXPERT_FIRST | CONFIG_REQUANT_BITS);
     // (the tiled kernels address activations with 32-bit byte offsets and scan the tiles of at most 1024 experts)
     const bool tiled_ok = hidden % 256 == 0 && n_experts <= 1024 &&
                           (unsigned long long)tokens * hidden < (1ull << 32) &&
                           (unsigned long long)tokens * top_k * inter < (1ull << 32);
+    const long pairs = (long)tokens * top_k;
     GemmPlan plan{};
-    plan.tiled = form == 16 || (form == 0 && (long)tokens * top_k > 32L * n_experts && tiled_ok);
-    plan.ok = !plan.tiled || tiled_ok;
+    plan.y_half = form == 16 || ((form == 0 || form == CONFIG_NARROW_TILES) && pairs > 32L * n_experts && tiled_ok);
+    plan.form = plan.y_half ? GemmPlan::TILED : GemmPlan::STREAMING;
+    // Narrow tiles from 10 pairs per expert (256 experts of 7168 x 2048, 8 pairs: 1.73 ms streaming, 1.77 narrow; 12:
+    // 1.84, 1.79; 16: 2.36, 1.82; 31: 2.61, 1.92) to where an expert's second tile, and with it its weights through L2
+    // once more, costs what a 256-pair tile loses while it starts and ends. That is the share of a tile's K blocks:
+    // 7168 x 2048 (56 blocks) 47 pairs 2.34 ms tiled, 2.00 narrow; 53: 2.36, 2.09; 64: 2.41, 2.54; 4096 x 1536 (32)
+    // 94: 0.428, 0.385; 106: 0.436, 0.414; 128: 0.462 both; 2048 x 768 (16) 128: 0.350, 0.318; 192: 0.399, 0.413.
+    // (They have the exact requantisation only.)
+    const bool narrow = !(config & CONFIG_APPROX_REQUANT) && aligned && pairs > 10L * n_experts &&
+                        pairs <= 128L * n_experts && pairs * (hidden / GROUP) <= 3000L * n_experts;
+    if (tiled_ok && (form == CONFIG_NARROW_TILES || (form == 0 && narrow)))
+        plan.form = GemmPlan::NARROW;
+    plan.ok = tiled_ok || (plan.form == GemmPlan::STREAMING && form != CONFIG_NARROW_TILES);
     return plan;
 }
 
@@ -228,7 +259,7 @@ void run_front(const moe::Workspace& w, const void* x, const float* logits, int 
 }
 
 // gate/up and down GEMMs of the experts over the quantised activations and the sort in `w`; result
-// in w.y. Many pairs per expert: LDS-tiled GEMMs (256 x 256 tiles). Few: the weight-streaming form.
+// in w.y.
 void run_expert_gemms(const moe::Workspace& w, const GemmPlan& plan, const void* w13_q, const float* w13_s,
                       const void* w2_q, const float* w2_s, int tokens, int hidden, int inter,
                       int n_experts, int top_k, int config, hipStream_t stream) {
@@ -238,9 +269,17 @@ void run_expert_gemms(const moe::Workspace& w, const GemmPlan& plan, const void*
     if (!(requant & CONFIG_SIGNIF_MASK)) requant |= default_requant_significance(inter, top_k) << CONFIG_SIGNIF_SHIFT;
     const int approx = config & CONFIG_APPROX_REQUANT;
     config &= ~(CONFIG_UE8M0 | CONFIG_LAST_EXPERT_FIRST | CONFIG_REQUANT_BITS);
-    if (plan.tiled) {
+    if (plan.form != GemmPlan::STREAMING) {
+        const int tile_pairs = plan.form == GemmPlan::NARROW ? moe_narrow_tile_pairs() : moe_tiled_tile_pairs();
         moe_tiled_prepare_launcher(w.tile_start, w.xs_t, w.x_s, w.sorted_pairs, w.expert_offsets, tokens,
-                                   hidden, n_experts, top_k, w.scale_stride, stream);
+                                   hidden, n_experts, top_k, w.scale_stride, tile_pairs, stream);
+    }
+    if (plan.form == GemmPlan::NARROW) {
+        moe_gate_up_narrow_launcher(w.h_q, w.h_s, w.hs_t, w.x_q, w.xs_t, w13_q, w13_s, w.sorted_pairs, w.expert_offsets,
+                                    w.tile_start, tokens, hidden, inter, n_experts, top_k, w.scale_stride, ue8m0, stream);
+        moe_down_narrow_launcher(w.y, plan.y_half ? w.y_scale : nullptr, w.h_q, w.hs_t, w2_q, w2_s, w.expert_offsets,
+                                 w.tile_start, tokens, hidden, inter, n_experts, top_k, w.scale_stride, stream);
+    } else if (plan.form == GemmPlan::TILED) {
         moe_gate_up_tiled_launcher(w.h_q, w.h_s, w.hs_t, w.x_q, w.xs_t, w13_q, w13_s, w.sorted_pairs,
                                    w.expert_offsets, w.tile_start, tokens, hidden, inter, n_experts, top_k,
                                    w.scale_stride, ue8m0, requant, stream);
@@ -262,19 +301,20 @@ bool layer_shape_ok(int hidden, int inter, int n_experts, int top_k, int tokens,
 
 }  // namespace
 
-// 1 if moe_fp8_launcher runs these sizes and this config on the LDS-tiled GEMMs, 0 if on the weight-streaming
-// ones (for checkers: the form decides how the workspace's y buffer is laid out), -1 for an unsupported shape.
+// 1 if moe_fp8_launcher leaves the workspace's y buffer for these sizes and this config in the fp16 form (LDS-tiled
+// GEMMs for more than 32 pairs per expert), 0 if in fp32 rows (for checkers), -1 for an unsupported shape.
 extern "C" int moe_fp8_uses_tiled_gemms(int tokens, int hidden, int inter, int n_experts, int top_k, int config) {
     if (tokens <= 0 || !layer_shape_ok(hidden, inter, n_experts, top_k, tokens, 0)) return -1;
-    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config);
-    return plan.ok ? (plan.tiled ? 1 : 0) : -1;
+    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config, true);
+    return plan.ok ? (plan.y_half ? 1 : 0) : -1;
 }
 
 // The whole layer. out [tokens, hidden] bf16 (out_dtype 0) or fp32 (out_dtype 1).
-// config: 0 = choose by the average number of pairs per expert (above 32: LDS-tiled GEMMs, else
-// weight streaming); 16 forces the tiled GEMMs; 1, 2, 4 (+8) force streaming, see moe_gate_up_launcher.
+// config: 0 = choose by the average number of pairs per expert (weight streaming, narrow tiles, 256-pair tiles: see
+// plan_expert_gemms); 16 forces the 256-pair tiles, 65536 (CONFIG_NARROW_TILES) the narrow ones; 1, 2, 4 (+8) force
+// streaming, see moe_gate_up_launcher.
 // +256: with the tiled GEMMs, the exact requantisation pass (CONFIG_EXACT_REQUANT in moe_common.hpp; the
-// streaming gate/up GEMM is exact by itself); +512: the streaming gate/up GEMM on the e4m3 matrix core.
+// streaming and the narrow-tile gate/up GEMMs are exact by themselves); +512: the streaming gate/up GEMM on the e4m3 matrix core.
 // +32: all block scales are powers of two (UE8M0). The caller's weight scales must be; x and h are
 // then quantised with the smallest power-of-two scale >= amax/448, and the tiled GEMMs let the MFMA
 // apply the scales (no per-block multiply-add on the VALU).
@@ -284,7 +324,7 @@ extern "C" void moe_fp8_launcher(void* out, const void* x, const float* logits, 
                                  int inter, int n_experts, int top_k, int out_dtype, int config,
                                  hipStream_t stream) {
     if (tokens <= 0) return;
-    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config);
+    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config, aligned16(w13_q, w2_q));
     if (!layer_shape_ok(hidden, inter, n_experts, top_k, tokens, out_dtype) || !plan.ok) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);
         return;
@@ -301,7 +341,7 @@ extern "C" void moe_fp8_launcher(void* out, const void* x, const float* logits, 
     }
     run_front(w, x, logits, tokens, hidden, n_experts, top_k, 0, config & CONFIG_UE8M0, stream);
     run_expert_gemms(w, plan, w13_q, w13_s, w2_q, w2_s, tokens, hidden, inter, n_experts, top_k, config, stream);
-    launch_combine(out, w.y, plan.tiled ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,
+    launch_combine(out, w.y, plan.y_half ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,
                    top_k, out_dtype, stream);
 }
 
@@ -329,8 +369,9 @@ extern "C" void moe_fp8_shared_launcher(void* out, const void* x, const float* l
                                         int shared_inter, int n_experts, int top_k, int out_dtype,
                                         int config, hipStream_t stream) {
     if (tokens <= 0) return;
-    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config);
-    const GemmPlan shared_plan = plan_expert_gemms(tokens, hidden, shared_inter > 0 ? shared_inter : 1, 1, 1, config);
+    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts, top_k, config, aligned16(w13_q, w2_q));
+    const GemmPlan shared_plan = plan_expert_gemms(tokens, hidden, shared_inter > 0 ? shared_inter : 1, 1, 1, config,
+                                                   aligned16(sw13_q, sw2_q));
     if (!layer_shape_ok(hidden, inter, n_experts, top_k, tokens, out_dtype) || shared_inter <= 0 ||
         shared_inter % GROUP != 0 || !plan.ok || !shared_plan.ok) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);
@@ -356,8 +397,8 @@ extern "C" void moe_fp8_shared_launcher(void* out, const void* x, const float* l
                                                                       sh.expert_offsets, tokens);
     run_expert_gemms(sh, shared_plan, sw13_q, sw13_s, sw2_q, sw2_s, tokens, hidden, shared_inter, 1, 1, config,
                      stream);
-    launch_combine(out, w.y, plan.tiled ? w.y_scale : nullptr, w.weights, w.pair_pos, sh.y,
-                   shared_plan.tiled ? sh.y_scale : nullptr, tokens, hidden, top_k, out_dtype, stream);
+    launch_combine(out, w.y, plan.y_half ? w.y_scale : nullptr, w.weights, w.pair_pos, sh.y,
+                   shared_plan.y_half ? sh.y_scale : nullptr, tokens, hidden, top_k, out_dtype, stream);
 }
 
 // The layer with a shared expert stored as expert number n_experts behind the routed ones
@@ -373,7 +414,7 @@ extern "C" void moe_fp8_fused_shared_launcher(void* out, const void* x, const fl
                                               int inter, int n_experts, int top_k, int out_dtype,
                                               int config, hipStream_t stream) {
     if (tokens <= 0) return;
-    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts + 1, top_k + 1, config);
+    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts + 1, top_k + 1, config, aligned16(w13_q, w2_q));
     if (!layer_shape_ok(hidden, inter, n_experts, top_k, tokens, out_dtype) || n_experts >= 512 ||
         top_k >= 64 || (long)tokens * (top_k + 1) > 0x7fffffffL / 4 || !plan.ok) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);
@@ -393,7 +434,7 @@ extern "C" void moe_fp8_fused_shared_launcher(void* out, const void* x, const fl
     run_front(w, x, logits, tokens, hidden, n_experts, top_k, CONFIG_SHARED_SLOT, config & CONFIG_UE8M0, stream);
     run_expert_gemms(w, plan, w13_q, w13_s, w2_q, w2_s, tokens, hidden, inter, n_experts + 1, top_k + 1,
                      (config & ~CONFIG_LAST_EXPERT_FIRST) | CONFIG_LAST_EXPERT_FIRST, stream);
-    launch_combine(out, w.y, plan.tiled ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,
+    launch_combine(out, w.y, plan.y_half ? w.y_scale : nullptr, w.weights, w.pair_pos, nullptr, nullptr, tokens, hidden,
                    top_k + 1, out_dtype, stream);
 }
 

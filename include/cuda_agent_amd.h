@@ -385,37 +385,36 @@ size_t moe_fp8_workspace_bytes(int tokens, int hidden, int inter, int n_experts,
  * x_q, x_s, h_q, h_s, y, y_scale (in this order), for checkers that inspect the stages. Writes
  * min(n_offsets, 11) entries and returns the number of fields the layout has (11), so that a caller
  * built against another version of the list can tell.
- * y [tokens*top_k, hidden]: fp32 rows when the layer ran the weight-streaming GEMMs; when it ran the
- * LDS-tiled ones (moe_fp8_uses_tiled_gemms), fp16 rows in the first half of the buffer, to be
- * multiplied by y_scale [tokens*top_k, hidden/256] (one power of two per row and run of 256 columns). */
+ * y [tokens*top_k, hidden]: fp32 rows, or (moe_fp8_uses_tiled_gemms) fp16 rows in the first half of
+ * the buffer, to be multiplied by y_scale [tokens*top_k, hidden/256] (one power of two per row and run of 256 columns). */
 int moe_fp8_workspace_layout(size_t* offsets, int n_offsets, int tokens, int hidden, int inter,
                              int n_experts, int top_k);
 
-/* 1 if moe_fp8_launcher runs these sizes and this config on the LDS-tiled GEMMs, 0 if on the
- * weight-streaming ones, -1 if it rejects them. */
+/* 1 if moe_fp8_launcher stores y for these sizes and this config in the fp16 form of the LDS-tiled
+ * GEMMs for more than 32 pairs per expert, 0 if in fp32 rows, -1 if it rejects them. */
 int moe_fp8_uses_tiled_gemms(int tokens, int hidden, int inter, int n_experts, int top_k, int config);
 
 /* The whole layer: out [tokens, hidden] (bf16 if out_dtype == 0, the operator's output type;
  * fp32 if 1, the same values before the final rounding) from x [tokens, hidden] bf16 and
  * logits [tokens, n_experts] fp32. workspace: moe_fp8_workspace_bytes(...) bytes, 256-byte
  * aligned. hidden and inter multiples of 128. config: 0 picks the GEMM form from the average number
- * of pairs per expert (above 32 and hidden % 256 == 0: LDS-tiled 256x256 GEMMs; otherwise the
- * weight-streaming form); 16 forces the tiled form; 1, 2, 4 (+8) force streaming as for
- * moe_gate_up_launcher. +32 (also understood by moe_quant_bf16_launcher and moe_gate_up_launcher):
+ * of pairs per expert (few: the weight-streaming form; hidden % 256 == 0 and more than 10, or more
+ * than 32 under +512: LDS tiles of 256 weight rows x 62 or, for many, 256 pairs); 16 forces the 256-pair
+ * tiles, 65536 the 62-pair ones; 1, 2, 4 (+8) force streaming as for moe_gate_up_launcher. +32 (also understood by moe_quant_bf16_launcher and moe_gate_up_launcher):
  * every block scale is a power of two (UE8M0). w13_s and w2_s must then hold powers of two; x and
  * the intermediate are quantised with scale = the smallest power of two >= max(amax, 1e-12)/448,
  * and the tiled GEMMs apply the scales inside the MFMA.
  * +256 / +512: how the intermediate h = silu(g) * u is requantised. The e4m3 matrix core sums a
  * 128-block with about 16 significant bits, so about one code of h in a thousand would differ by one
  * step from an fp32 evaluation, and one step on an element near its group's maximum moves single
- * outputs by up to 3 % of their rms. The streaming gate/up GEMM therefore runs on the bf16 matrix core
- * (exact sums, same time: it is bound by the weight stream); +512 puts it on the e4m3 one. The tiled
+ * outputs by up to 3 % of their rms. The streaming and 62-pair gate/up GEMMs therefore run on the bf16 matrix core
+ * (exact sums, same time: it is bound by the weight stream); +512 puts it on the e4m3 one. The 256-pair
  * gate/up GEMM by default stays on the e4m3 matrix core and recomputes, in its epilogue, the elements
  * in the two highest binades of their group's range (at least 128 of 448 code units) that lie within
  * the matrix core's error of a rounding boundary, together with the candidates for the maximum of
  * those groups, as plain dot products: codes of large elements as an fp32 evaluation gives them,
  * small ones (a code step of at most 8/448 of the group's maximum) as the matrix core rounds them.
- * +256: the tiled gate/up GEMM on the bf16 matrix core instead: every code exact, twice the
+ * +256: the 256-pair gate/up GEMM on the bf16 matrix core instead: every code exact, twice the
  * matrix-core time. +512: e4m3 matrix core, no repair. +1024 / +2048 / +3072: the band is half /
  * twice / four times as wide. +4096*s (s = 1..8): repair elements of at least 2^s code units. */
 void moe_fp8_launcher(void* out, const void* x, const float* logits, const void* w13_q,

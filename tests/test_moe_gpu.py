@@ -22,6 +22,7 @@ from moe_checks import code_steps, oracle_down, repaired_below, settle_disputed_
 pytestmark = pytest.mark.gpu
 TOL = 2e-2
 EXACT_REQUANT = 256   # config bit of the layer: the tiled gate/up GEMM on the bf16 matrix core (every code of h exact)
+NARROW_TILES = 65536  # config of the layer: narrow tiles whatever the number of pairs per expert
 APPROX_REQUANT = 512  # config bit of the layer: gate/up on the e4m3 matrix core, codes of h as they come
 
 
@@ -176,6 +177,28 @@ def test_layer_tiled_gemms(capi, dev, shape, requant):
     # matrix core with the repair of the large codes in its epilogue (the default)
     T, H, I, E, k = shape
     check_layer(capi, dev, T=T, H=H, I=I, E=E, k=k, seed=50 + T, config=16, requant=requant)
+
+
+@pytest.mark.parametrize('shape', [(62, 256, 128, 1, 1), (63, 256, 128, 2, 2), (33, 512, 256, 5, 2), (31, 768, 384, 3, 1),
+                                   (125, 512, 384, 2, 2), (300, 256, 256, 4, 2), (3, 1024, 128, 16, 4), (520, 768, 640, 40, 3)])
+def test_layer_narrow_tiles(capi, dev, shape):
+    # 65536 forces the narrow tiles: tiles of 1 and of 62 pairs, experts of 63 and 125 pairs (two and three tiles of
+    # equal size), one and two 32-pair MFMA tiles, 1 to 8 K blocks, y in fp32 (up to 32 pairs per expert) and in fp16
+    T, H, I, E, k = shape
+    check_layer(capi, dev, T=T, H=H, I=I, E=E, k=k, seed=150 + T, config=NARROW_TILES)
+
+
+@pytest.mark.parametrize('pow2', [0, 32])
+def test_layer_narrow_tiles_codes_of_the_streaming_form(capi, dev, pow2):
+    x, logits, w, dts = make_case(dev, 150, 512, 256, 12, 451)
+    if pow2:
+        for i in (3, 5):
+            dts[i] = torch.exp2(torch.round(torch.log2(dts[i])))
+    a, va = run_layer(capi, dts, 2, NARROW_TILES | pow2, torch.float32)
+    b, vb = run_layer(capi, dts, 2, 4 | pow2, torch.float32)
+    # sums of fp32 products in another order: codes differ only where fp32 does not decide them
+    torch.testing.assert_close(va['h_s'], vb['h_s'], rtol=0 if pow2 else 1e-5, atol=0)
+    assert (va['h_q'].view(torch.uint8) != vb['h_q'].view(torch.uint8)).float().mean().item() < 2e-4
 
 
 @pytest.mark.parametrize('seed', range(8))
