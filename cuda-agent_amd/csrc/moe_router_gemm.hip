@@ -215,95 +215,150 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
     }
 }
 
-// The same product for many tokens: a workgroup owns 128 tokens x 64 experts and shares its operand tiles
-// through LDS (per 64 values of k: 128 rows of x and 3 x 64 rows of planes, 128 bytes each = 40 KB, two
-// stages). Every lane fetches 10 chunks of 16 bytes per stage (whole lines: 8 lanes per row), stores them
-// swizzled as above, and after ONE barrier per stage each wavefront (64 tokens x 32 experts) reads its two x
-// tiles and three plane tiles in operand layout. The per-wavefront kernel above asks its CU's L1 for 170
-// bytes per clock at the bf16 MFMA rate; this one for 52.
+// The same product for many tokens: a workgroup of 4 wavefronts owns 128 tokens x 64 experts and shares its operand
+// tiles through LDS (per 64 values of k: 128 rows of x and 3 x 64 rows of planes, 128 bytes each = 40 KB). The per-wavefront
+// kernel above asks its CU's L1 for 170 bytes per clock at the bf16 MFMA rate; this one for 52.
+//
+// One wavefront per SIMD is all there is at 8192 tokens x 256 experts, so everything that takes time is requested
+// early: global -> LDS loads into a ring of three stages, two of them in flight, and the operands of chunk c+1 are read
+// into registers while the 24 MFMAs (768 cycles) of chunk c run. With one stage in flight through registers and the
+// operand reads in front of the MFMAs a chunk took 2600 cycles (137 us for the 8192 x 256 logits
+// of hidden 7168); this takes 83 us, 1.1 PFLOP/s of bf16 products. With K split it also serves fewer tokens: 4096 tokens
+// 86 us on the per-wavefront kernel, 49 here; 1000: 27.7 and 21.9; 200: 15.5 and 13.2, the reduction included.
 constexpr int BIG_TOKENS = 128;
 constexpr int BIG_EXPERTS = 64;
-constexpr int BIG_STAGE = (BIG_TOKENS + 3 * BIG_EXPERTS) * 8;  // 16-byte slots per stage (40 KB)
+constexpr int BIG_STAGE = (BIG_TOKENS + 3 * BIG_EXPERTS) * K_CHUNK * 2;  // bytes (40 KB)
+constexpr int BIG_STAGES = 3;
+constexpr int BIG_LOADS = BIG_STAGE / 1024 / 4;  // load instructions of a wavefront per stage
 
-__global__ __launch_bounds__(256) void moe_router_gemm_split_tiled_kernel(const uint16_t* __restrict__ x,
-                                                                          const uint16_t* __restrict__ planes,
-                                                                          float* __restrict__ out, int tokens,
-                                                                          int hidden, int n_experts) {
-    __shared__ u32x4 s_stage[2][BIG_STAGE];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+typedef const __attribute__((address_space(3))) uint8_t* lds_bytes;
+
+// 64 lanes x 16 bytes, global -> LDS (lds_base + lane*16). asm, so that later LDS reads are not made to wait for it: its
+// completion is awaited once per chunk.
+__device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
+                 : "memory", "m0");
+}
+
+template <int N>
+struct IntConstant {
+    static constexpr int value = N;
+};
+
+// grid: x = 128-token tiles, y = 64-expert tiles, z = K split; out as in moe_router_gemm_kernel
+__global__ __launch_bounds__(256, 1) void moe_router_gemm_split_tiled_kernel(const uint16_t* __restrict__ x,
+                                                                             const uint16_t* __restrict__ planes,
+                                                                             float* __restrict__ out, int tokens,
+                                                                             int hidden, int n_experts,
+                                                                             int chunks_per_split) {
+    __shared__ __attribute__((aligned(16))) uint8_t s_stage[BIG_STAGES * BIG_STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 31;
     const int half = lane >> 5;
     const int t0 = blockIdx.x * BIG_TOKENS;
     const int e0 = blockIdx.y * BIG_EXPERTS;
-    const int n_chunks = hidden / K_CHUNK;
-    const size_t plane = (size_t)n_experts * hidden;
+    const int chunk_begin = blockIdx.z * chunks_per_split;
+    const int n = min(chunks_per_split, hidden / K_CHUNK - chunk_begin);  // (not positive: this split is empty)
 
-    // fill side: slot tid + 256*i of the stage, i < 10; rows 0..127 are x, then 64 rows of each plane
-    const u32x4* src[10];
-    int dst[10];
+    // fill side: instruction wave + 4*i (i < 10) covers 8 rows of the stage, lane -> row lane/8, chunk
+    // (lane%8) ^ ((row >> 1) & 7): i < 4 rows of x, then two instructions per plane. Rows past the end repeat the last.
+    const int ld_row = lane >> 3;
+    const uint32_t ld_chunk = 16u * ((lane & 7) ^ (ld_row >> 1) ^ (4 * (wave & 1)));
+    const uint16_t* base[4];  // x tile, planes
+    base[0] = x + (size_t)t0 * hidden + (size_t)chunk_begin * K_CHUNK;
 #pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        const int r = (tid + 256 * i) >> 3;  // row of the stage
-        const int c = tid & 7;
-        if (r < BIG_TOKENS) {
-            const int t = t0 + r < tokens ? t0 + r : tokens - 1;
-            src[i] = reinterpret_cast<const u32x4*>(x + (size_t)t * hidden) + c;
-        } else {
-            const int p = (r - BIG_TOKENS) / BIG_EXPERTS;
-            const int er = (r - BIG_TOKENS) % BIG_EXPERTS;
-            const int e = e0 + er < n_experts ? e0 + er : n_experts - 1;
-            src[i] = reinterpret_cast<const u32x4*>(planes + p * plane + (size_t)e * hidden) + c;
-        }
-        dst[i] = r * 8 + (c ^ ((r >> 1) & 7));
-    }
-    u32x4 raw[10];
-    auto load_chunk = [&](int c) {
+    for (int p = 0; p < 3; ++p)
+        base[1 + p] = planes + ((size_t)p * n_experts + e0) * hidden + (size_t)chunk_begin * K_CHUNK;
+    uint32_t off[6];  // bytes from the tile's first row: the four instructions of x, the two of any plane
 #pragma unroll
-        for (int i = 0; i < 10; ++i) raw[i] = src[i][(size_t)c * (K_CHUNK * 2 / 16)];
-    };
-    auto store_stage = [&](int st) {
+    for (int i = 0; i < 4; ++i)
+        off[i] = (uint32_t)min((wave + 4 * i) * 8 + ld_row, tokens - 1 - t0) * (uint32_t)hidden * 2u + ld_chunk;
 #pragma unroll
-        for (int i = 0; i < 10; ++i) s_stage[st][dst[i]] = raw[i];
-    };
-    // read side: wavefront (wave & 1) takes tokens [64*(wave&1), +64), (wave >> 1) experts [32*(wave>>1), +32)
-    const int a_row0 = 64 * (wave & 1) + row;
-    const int b_row0 = BIG_TOKENS + 32 * (wave >> 1) + row;
-    auto operand = [&](int st, int r, int s) {
-        return __builtin_bit_cast(bf16x8, s_stage[st][r * 8 + ((4 * half + s) ^ ((r >> 1) & 7))]);
+    for (int i = 0; i < 2; ++i)
+        off[4 + i] = (uint32_t)min((wave + 4 * i) * 8 + ld_row, n_experts - 1 - e0) * (uint32_t)hidden * 2u + ld_chunk;
+    const uint32_t stage_base = (uint32_t)(size_t)((lds_void_ptr)s_stage);
+    auto issue = [&](int c, int i) {
+        const int m = i < 4 ? 0 : 1 + (i - 4) / 2;
+        dma16(base[m] + (size_t)c * K_CHUNK, off[i < 4 ? i : 4 + (i & 1)],
+              stage_base + (c % BIG_STAGES) * BIG_STAGE + (wave + 4 * i) * 1024);
     };
 
+    // read side: wavefront (wave & 1) takes tokens [64*(wave&1), +64), (wave >> 1) experts [32*(wave>>1), +32);
+    // lane (row, half) holds values [32*half, +32) of its row, 8 per MFMA step
+    const int a_row = 64 * (wave & 1) + row;
+    const int b_row = BIG_TOKENS + 32 * (wave >> 1) + row;
+    const int swizzle = (row >> 1) & 7;
+    bf16x8 op[2][5][4];  // [chunk parity][two tiles of x, three planes][step]
+    auto read_operands = [&](int c, bf16x8 (&dst)[5][4]) {
+        const lds_bytes st = (lds_bytes)s_stage + (c % BIG_STAGES) * BIG_STAGE;
+#pragma unroll
+        for (int m = 0; m < 5; ++m)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int r = m < 2 ? a_row + 32 * m : b_row + BIG_EXPERTS * (m - 2);
+                dst[m][s] = *(const __attribute__((address_space(3))) bf16x8*)(st + (r * 8 + ((4 * half + s) ^ swizzle)) * 16);
+            }
+    };
     floatx16 acc[2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
         acc[a] = floatx16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    load_chunk(0);
-    store_stage(0);
-    __syncthreads();
-    for (int c = 0; c < n_chunks; ++c) {
-        const int st = c & 1;
-        if (c + 1 < n_chunks) load_chunk(c + 1);  // in flight under the MFMAs below
-        bf16x8 a_op[2][4];
+
+    // MORE: chunk c+3 exists, and with it c+1 and c+2
+    auto chunk = [&](int c, auto parity_tag, auto more_tag) {
+        constexpr int P = decltype(parity_tag)::value;
+        constexpr bool MORE = decltype(more_tag)::value != 0;
+        // stage c+1 has arrived (that of c+2 may be in flight), and this wavefront holds its operands of chunk c
+        if (MORE || c + 2 < n) __builtin_amdgcn_s_waitcnt(BIG_LOADS | (7 << 4) | (0 << 8));
+        else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // ... in every wavefront: stage c may be filled again
+        asm volatile("" ::: "memory");
+        if (MORE || c + 1 < n) read_operands(c + 1, op[P ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) a_op[a][s] = operand(st, a_row0 + 32 * a, s);
-        // smallest terms first
-#pragma unroll
-        for (int p = 2; p >= 0; --p) {
-            bf16x8 b_op[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) b_op[s] = operand(st, b_row0 + BIG_EXPERTS * p, s);
+        for (int p = 2; p >= 0; --p) {  // smallest terms first
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_op[0][s], b_op[s], acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_op[1][s], b_op[s], acc[1], 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[P][0][s], op[P][2 + p][s], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[P][1][s], op[P][2 + p][s], acc[1], 0, 0, 0);
+                if constexpr (MORE) {
+                    // (a load holds the wavefront until the memory pipeline has taken it: one per two MFMAs)
+                    if ((2 - p) * 4 + s < BIG_LOADS) issue(c + 3, (2 - p) * 4 + s);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
-        if (c + 1 < n_chunks) store_stage(st ^ 1);  // (last read before the barrier that ended the previous pass)
-        __syncthreads();
+    };
+    if (n > 0) {
+#pragma unroll
+        for (int c = 0; c < BIG_STAGES; ++c)
+            if (c < n)
+#pragma unroll
+                for (int i = 0; i < BIG_LOADS; ++i) issue(c, i);
+        if (n > 2) __builtin_amdgcn_s_waitcnt(((2 * BIG_LOADS) & 15) | ((2 * BIG_LOADS) >> 4 << 14) | (7 << 4) | (15 << 8));
+        else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read_operands(0, op[0]);
+        int c = 0;
+        for (; c + 4 < n; c += 2) {
+            chunk(c, IntConstant<0>{}, IntConstant<1>{});
+            chunk(c + 1, IntConstant<1>{}, IntConstant<1>{});
+        }
+        // at most four chunks are left; the first may have one more to request
+        for (; c < n; c += 2) {
+            if (c + 3 < n) chunk(c, IntConstant<0>{}, IntConstant<1>{});
+            else chunk(c, IntConstant<0>{}, IntConstant<0>{});
+            if (c + 1 < n) chunk(c + 1, IntConstant<1>{}, IntConstant<0>{});
+        }
     }
+    float* dst = out + (size_t)blockIdx.z * tokens * n_experts;
     const int e = e0 + 32 * (wave >> 1) + row;
     if (e < n_experts) {
 #pragma unroll
@@ -311,7 +366,7 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_tiled_kernel(const 
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int tt = t0 + 64 * (wave & 1) + 32 * a + 8 * (i / 4) + 4 * half + (i % 4);
-                if (tt < tokens) out[(size_t)tt * n_experts + e] = acc[a][i];
+                if (tt < tokens) dst[(size_t)tt * n_experts + e] = acc[a][i];
             }
     }
 }
@@ -440,21 +495,16 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
         return;
     }
     const int n_chunks = hidden / K_CHUNK;
-    // enough 128 x 64 tiles to fill the chip: the workgroup-tiled kernel (config 1 forces the other one)
-    if (splits == 1 && config != 1 &&
-        (long)((tokens + BIG_TOKENS - 1) / BIG_TOKENS) * ((n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS) >= 192) {
-        const dim3 big_grid((tokens + BIG_TOKENS - 1) / BIG_TOKENS, (n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS);
-        moe_router_gemm_split_tiled_kernel<<<big_grid, 256, 0, stream>>>(
-            static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(planes), logits, tokens, hidden,
-            n_experts);
-        return;
-    }
+    // enough 128 x 64 tiles and splits to fill the chip: the workgroup-tiled kernel (config 2 forces it, 1 the other one)
+    const long big_tiles = (long)((tokens + BIG_TOKENS - 1) / BIG_TOKENS) * ((n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS);
+    const bool tiled = hidden <= (1 << 24) && (config == 2 || (config != 1 && big_tiles * splits >= 192 && tokens >= BIG_TOKENS));
     const int chunks_per_split = (n_chunks + splits - 1) / splits;
     float* out = splits > 1 ? static_cast<float*>(workspace) : logits;
-    const dim3 grid((tokens + 63) / 64, (n_experts + 63) / 64, splits);
-    moe_router_gemm_split_kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(x),
-                                                           static_cast<const uint16_t*>(planes), out, tokens,
-                                                           hidden, n_experts, chunks_per_split);
+    const int tile_tokens = tiled ? BIG_TOKENS : 64;
+    const dim3 grid((tokens + tile_tokens - 1) / tile_tokens, (n_experts + 63) / 64, splits);
+    const auto kernel = tiled ? moe_router_gemm_split_tiled_kernel : moe_router_gemm_split_kernel;
+    kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(planes), out, tokens,
+                                     hidden, n_experts, chunks_per_split);
     if (splits > 1) {
         const size_t count = (size_t)tokens * n_experts;
         moe_router_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
