@@ -193,7 +193,9 @@ def run_logits_split(capi, dev, x, w):
 
 
 @pytest.mark.parametrize('shape', [(64, 7168, 256), (1, 64, 32), (100, 448, 72), (700, 1024, 256), (33, 128, 1),
-                                   (130, 2048, 384), (6200, 448, 250), (12345, 64, 70)])   # the last two: workgroup-tiled kernel
+                                   (130, 2048, 384), (6200, 448, 250), (12345, 64, 70),   # from here: workgroup-tiled kernel
+                                   (24600, 128, 3), (24600, 192, 64), (6145, 256, 256), (6200, 320, 200),  # 1 to 5 chunks
+                                   (385, 7168, 256), (1500, 2048, 130)])                  # K split 32 and 8 ways, ragged splits
 def test_split_weight_logits_match_float64(capi, dev, shape):
     T, H, E = shape
     gen = torch.Generator().manual_seed(T + E + 1)
@@ -244,7 +246,7 @@ def test_router_logits_rejects_bad_arguments(capi, dev):
 
 # ---- RMS norm fused with the activation quantiser -------------------------------------------------
 
-@pytest.mark.parametrize('shape', [(64, 7168), (5, 128), (300, 2048), (1, 8192), (33, 384)])
+@pytest.mark.parametrize('shape', [(64, 7168), (5, 128), (300, 2048), (1, 8192), (33, 384), (513, 7168), (600, 2176), (1030, 128)])
 @pytest.mark.parametrize('config', [0, 32])
 def test_rmsnorm_quant(capi, dev, shape, config):
     R, C = shape
