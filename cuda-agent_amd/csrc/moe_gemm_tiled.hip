@@ -73,64 +73,68 @@ __device__ __forceinline__ double wave_sum(double v) {
 // slot s of the order holds expert slot_expert[s], and tile_start[s] = number of tiles of the slots before s
 // (tile_start[E] = total). Measured on the prefill workload: 2.4 % of the layer's time between the heavily loaded
 // experts evenly spread and all in a row.
-// tile_table: tile_start [n_experts + 1], then slot_expert [n_experts].
-__global__ __launch_bounds__(1024) void moe_tile_start_kernel(const int* __restrict__ expert_offsets,
-                                                              int* __restrict__ tile_table, int n_experts,
-                                                              int tile_pairs) {
-    __shared__ int s_scan[1024];
+// tile_table: tile_start [n_experts + 1], then slot_expert [n_experts]. One workgroup of 1024 lanes.
+__device__ __forceinline__ void number_tiles(const int* __restrict__ expert_offsets, int* __restrict__ tile_table,
+                                             int n_experts, int tile_pairs) {
+    __shared__ int s_wave_total[16];
     __shared__ int s_list[2][1024];  // experts with several tiles, and the others, each in ascending order
-    __shared__ int s_slot_expert[1024];
+    __shared__ int s_tiles[1024];    // tiles of every expert
+    __shared__ int s_loaded;         // number of experts with several tiles
     const int t = threadIdx.x;
-    // inclusive prefix sum of v over the first n_experts lanes
-    auto scan = [&](int v) {
-        if (t < n_experts) s_scan[t] = v;
-        __syncthreads();
-        for (int d = 1; d < n_experts; d <<= 1) {
-            const int add = (t >= d && t < n_experts) ? s_scan[t - d] : 0;
-            __syncthreads();
-            v += add;
-            if (t < n_experts) s_scan[t] = v;
-            __syncthreads();
-        }
-        return v;
-    };
     const int mine = t < n_experts ? (expert_offsets[t + 1] - expert_offsets[t] + tile_pairs - 1) / tile_pairs : 0;
     const bool loaded = mine >= 2;
-    const int loaded_upto = scan(loaded ? 1 : 0);  // experts with several tiles among 0..t
-    const int n_loaded = s_scan[n_experts - 1];
-    if (t < n_experts) s_list[loaded ? 0 : 1][loaded ? loaded_upto - 1 : t - loaded_upto] = t;
+    const int loaded_upto = block_inclusive_scan(loaded ? 1 : 0, s_wave_total);  // experts with several tiles among 0..t
+    if (t < n_experts) {
+        s_list[loaded ? 0 : 1][loaded ? loaded_upto - 1 : t - loaded_upto] = t;
+        s_tiles[t] = mine;
+    }
+    if (t == n_experts - 1) s_loaded = loaded_upto;
     __syncthreads();
+    const int n_loaded = s_loaded;
     // slot s is taken by loaded expert j if s == j * n_experts / n_loaded
     int j = -1;
     if (t < n_experts && n_loaded > 0) {
         const int cand = (int)(((long)t * n_loaded + n_experts - 1) / n_experts);  // smallest j with j*E/n >= t
         if (cand < n_loaded && (int)((long)cand * n_experts / n_loaded) == t) j = cand;
     }
-    const int free_upto = scan(j < 0 ? 1 : 0);  // slots not taken among 0..t
-    if (t < n_experts) s_slot_expert[t] = j >= 0 ? s_list[0][j] : s_list[1][free_upto - 1];
-    __syncthreads();
-    const int tiles_here = t < n_experts ? (expert_offsets[s_slot_expert[t] + 1] - expert_offsets[s_slot_expert[t]] +
-                                            tile_pairs - 1) / tile_pairs
-                                         : 0;
-    const int upto = scan(tiles_here);
+    const int free_upto = block_inclusive_scan(t < n_experts && j < 0 ? 1 : 0, s_wave_total);  // slots not taken among 0..t
+    const int expert = t < n_experts ? (j >= 0 ? s_list[0][j] : s_list[1][free_upto - 1]) : 0;
+    const int tiles_here = t < n_experts ? s_tiles[expert] : 0;
+    const int upto = block_inclusive_scan(tiles_here, s_wave_total);
     if (t < n_experts) {
         tile_table[t] = upto - tiles_here;
-        tile_table[n_experts + 1 + t] = s_slot_expert[t];
+        tile_table[n_experts + 1 + t] = expert;
     }
     if (t == n_experts - 1) tile_table[n_experts] = upto;
 }
 
-// xs_t[kb][pos] = x_s[token of sorted position pos][kb]
-__global__ __launch_bounds__(256) void moe_gather_scales_kernel(const float* __restrict__ x_s,
-                                                                const int* __restrict__ sorted_pairs,
-                                                                float* __restrict__ xs_t, int pairs,
-                                                                int stride, int kb_count, int top_k) {
-    const int pos = blockIdx.x * 256 + threadIdx.x;
-    if (pos >= pairs) return;
-    const int token = sorted_pairs[pos] / top_k;
-    for (int kb = 0; kb < kb_count; ++kb) {
-        xs_t[(size_t)kb * stride + pos] = x_s[(size_t)token * kb_count + kb];
+// Workgroup 0 numbers the tiles; the others write xs_t[kb][pos] = x_s[token of sorted position pos][kb], each for 256
+// positions and 32 K blocks: a lane reads 8 consecutive scales of its token and the lanes of a wavefront write
+// consecutive positions. (As two launches, one lane walking all K blocks of its position, 21 us for 12000 positions.)
+constexpr int GATHER_KB = 32;
+
+__global__ __launch_bounds__(1024) void moe_tiled_prepare_kernel(const int* __restrict__ expert_offsets,
+                                                                 int* __restrict__ tile_table, int n_experts,
+                                                                 int tile_pairs, const float* __restrict__ x_s,
+                                                                 const int* __restrict__ sorted_pairs,
+                                                                 float* __restrict__ xs_t, int pairs, int stride,
+                                                                 int kb_count, int top_k) {
+    if (blockIdx.x == 0) {
+        number_tiles(expert_offsets, tile_table, n_experts, tile_pairs);
+        return;
     }
+    const int kb_tiles = (kb_count + GATHER_KB - 1) / GATHER_KB;
+    const int tile = (int)blockIdx.x - 1;
+    const int pos = tile / kb_tiles * 256 + (threadIdx.x & 255);
+    const int kb0 = tile % kb_tiles * GATHER_KB + (threadIdx.x >> 8) * (GATHER_KB / 4);
+    if (pos >= pairs) return;
+    const float* src = x_s + (size_t)(sorted_pairs[pos] / top_k) * kb_count;
+    float v[GATHER_KB / 4];
+#pragma unroll
+    for (int i = 0; i < GATHER_KB / 4; ++i) v[i] = kb0 + i < kb_count ? src[kb0 + i] : 0.f;
+#pragma unroll
+    for (int i = 0; i < GATHER_KB / 4; ++i)
+        if (kb0 + i < kb_count) xs_t[(size_t)(kb0 + i) * stride + pos] = v[i];
 }
 
 // Phase timing build (-DMOE_PHASE_TIMING): every wavefront of workgroup 0 adds up the core clock
@@ -831,7 +835,7 @@ __global__ __launch_bounds__(512) void moe_tiled_gemm_kernel(
 extern "C" int moe_tiled_tile_pairs() { return TILE_PAIRS; }
 
 // Scratch the tiled path needs beyond the layer's common workspace:
-//   tile_start [2*n_experts+1] ints (moe_tile_start_kernel, for tiles of tile_pairs pairs); xs_t [hidden/128][stride] and
+//   tile_start [2*n_experts+1] ints (moe_tiled_prepare_kernel, for tiles of tile_pairs pairs); xs_t [hidden/128][stride] and
 //   hs_t [inter/128][stride] floats with stride = pairs rounded up to 256, plus 256.
 extern "C" void moe_tiled_prepare_launcher(int* tile_start, float* xs_t, const float* x_s,
                                            const int* sorted_pairs, const int* expert_offsets,
@@ -843,9 +847,10 @@ extern "C" void moe_tiled_prepare_launcher(int* tile_start, float* xs_t, const f
         return;
     }
     const int pairs = tokens * top_k;
-    moe_tile_start_kernel<<<1, 1024, 0, stream>>>(expert_offsets, tile_start, n_experts, tile_pairs);
-    moe_gather_scales_kernel<<<(pairs + 255) / 256, 256, 0, stream>>>(x_s, sorted_pairs, xs_t, pairs,
-                                                                    scale_stride, hidden / GROUP, top_k);
+    const int kb_tiles = (hidden / GROUP + GATHER_KB - 1) / GATHER_KB;
+    moe_tiled_prepare_kernel<<<1 + (pairs + 255) / 256 * kb_tiles, 1024, 0, stream>>>(
+        expert_offsets, tile_start, n_experts, tile_pairs, x_s, sorted_pairs, xs_t, pairs, scale_stride, hidden / GROUP,
+        top_k);
 }
 
 // requant_config: the CONFIG_*_REQUANT, band and significance bits of the layer's config (moe_common.hpp):

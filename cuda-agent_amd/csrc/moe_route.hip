@@ -231,21 +231,15 @@ __global__ __launch_bounds__(256) void moe_hist_kernel(const int* __restrict__ i
     }
 }
 
-// Exclusive prefix sum of s[0..n) in place (n <= 1024, blockDim.x == 1024); s[n] = total.
+// Exclusive prefix sum of s[0..n) in place (n <= 1024, blockDim.x == 1024); s[n] = total. Callers have a barrier between
+// their last write to s and this. (Two barriers; one per doubling step, twice, was 16 of them for 256 experts.)
 __device__ __forceinline__ void block_exclusive_scan(int* s, int n) {
+    __shared__ int s_wave_total[16];
     const int t = threadIdx.x;
     const int mine = t < n ? s[t] : 0;
-    int v = mine;
-    __syncthreads();
-    for (int d = 1; d < n; d <<= 1) {
-        const int add = (t >= d && t < n) ? s[t - d] : 0;
-        __syncthreads();
-        v += add;
-        if (t < n) s[t] = v;
-        __syncthreads();
-    }
-    if (t < n) s[t] = v - mine;
-    if (t == n - 1) s[n] = v;
+    const int upto = block_inclusive_scan(mine, s_wave_total);
+    if (t < n) s[t] = upto - mine;
+    if (t == n - 1) s[n] = upto;
     __syncthreads();
 }
 
@@ -293,17 +287,20 @@ __global__ __launch_bounds__(1024) void moe_scan_kernel(int* __restrict__ chunk_
     if (e == 0) expert_offsets[n_experts] = s_count[n_experts];
 }
 
-// rank of this lane's pair among the pairs of the same 64-pair group with the same expert
-// (`earlier`), and whether a later lane of the group has the same expert
+// rank of this lane's pair among the pairs of the same 64-pair group with the same expert (`earlier`), and whether a
+// later lane of the group has the same expert. e is negative in lanes without a pair (what they get is not used). The
+// lanes of the same expert are those that agree in every bit of its number (below 1024): ten ballots, where comparing
+// with every lane in turn took 64 steps of four instructions.
 __device__ __forceinline__ void group_rank(int e, int lane, int& earlier, bool& later) {
-    earlier = 0;
-    later = false;
-#pragma unroll 8
-    for (int k = 0; k < 64; ++k) {
-        const int ek = __builtin_amdgcn_readlane(e, k);
-        earlier += (ek == e && k < lane) ? 1 : 0;
-        later = later || (ek == e && k > lane);
+    unsigned long long same = __ballot(e >= 0);
+#pragma unroll
+    for (int bit = 0; bit < 10; ++bit) {
+        const bool set = (e >> bit) & 1;
+        const unsigned long long with = __ballot(set);
+        same &= set ? with : ~with;
     }
+    earlier = __popcll(same & ((1ull << lane) - 1ull));
+    later = (same >> lane) > 1ull;
 }
 
 // Stable scatter of one chunk in three parallel phases. The chunk's pairs are taken in groups of
@@ -340,10 +337,16 @@ __global__ __launch_bounds__(1024) void moe_scatter_kernel(const int* __restrict
     __syncthreads();
     for (int e = threadIdx.x; e < n_experts; e += 1024) {
         int running = chunk_base[(size_t)blockIdx.x * n_experts + e];
-        for (int g = 0; g < groups; ++g) {
-            const int v = s_first[g * n_experts + e];
-            s_first[g * n_experts + e] = running;
-            running += v;
+        constexpr int BATCH = 8;  // (the reads of a batch are in flight together)
+        for (int g0 = 0; g0 < groups; g0 += BATCH) {
+            int v[BATCH];
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) v[j] = g0 + j < groups ? s_first[(g0 + j) * n_experts + e] : 0;
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                if (g0 + j < groups) s_first[(g0 + j) * n_experts + e] = running;
+                running += v[j];
+            }
         }
     }
     __syncthreads();

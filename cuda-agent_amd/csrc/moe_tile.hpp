@@ -65,7 +65,7 @@ __device__ __forceinline__ void dma16_once(const void* base, uint32_t lane_byte_
 }
 
 // The tile of a workgroup: row tile `rb` of expert `e`, pair tile number `pt` of the table (see
-// moe_tile_start_kernel), which is tile `in_expert` of that expert's. False if there is none. Consecutive workgroup
+// moe_tiled_prepare_kernel), which is tile `in_expert` of that expert's. False if there is none. Consecutive workgroup
 // ids go round-robin to the 8 XCDs, each with its own L2, so the 32 workgroups that run together on one XCD are given
 // a 4 x 8 block of (row tile, pair tile): they share 4 weight tiles and 8 activation tiles through that L2 instead of
 // pulling 18 different ones.
