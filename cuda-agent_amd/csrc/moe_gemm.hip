@@ -359,26 +359,39 @@ __device__ __forceinline__ void dma16_ptr(const void* lane_ptr, uint32_t lds_bas
                  : "memory", "m0");
 }
 
-template <bool GATE_UP, int NT, bool EXACT = false>
+// H_F32 (NT = 1): h stays in fp32 between the two GEMMs, in `h` [pairs, inter], and the down GEMM quantises it. With one
+// or two tokens the 128 columns that share a scale are too much for a workgroup: 8 experts x 16 of them leave half of the
+// CUs without one, and a CU does not read more than about 45 GB/s (more wavefronts per workgroup change nothing). So a
+// gate/up workgroup takes 64 gate + 64 up rows, and each down workgroup turns the rows of its pairs into codes, in
+// LDS, while its first weights are on their way; those of row block 0 also write them to h_q and h_s. One token: 256
+// experts of 7168 x 2048 77 -> 69 us for the layer, 64 of 4096 x 1536 44 -> 39, 128 of 2048 x 768 31 -> 29.
+constexpr int H_F32_MAX_KB = 16;  // (32 KB of codes)
+
+template <bool GATE_UP, int NT, bool EXACT = false, bool H_F32 = false>
 __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     const uint8_t* __restrict__ w_q, const float* __restrict__ w_s, const uint8_t* __restrict__ a_q,
     const float* __restrict__ a_s, const int* __restrict__ sorted_pairs,
     const int* __restrict__ expert_offsets, uint8_t* __restrict__ h_q, float* __restrict__ h_s,
     float* __restrict__ y, int K, int n_rows, int inter, int top_k, bool pow2,
-    bool last_first, int n_experts) {
-    constexpr int TILES = 4;
-    constexpr int DEPTH = 3;
+    bool last_first, int n_experts, float* __restrict__ h = nullptr) {
+    static_assert(!H_F32 || NT == 1, "one pair tile");
+    constexpr bool SPLIT = GATE_UP && H_F32;   // 64 gate + 64 up rows
+    constexpr bool OWN_CODES = !GATE_UP && H_F32;
+    constexpr int TILES = SPLIT ? 2 : 4;
+    constexpr int DEPTH = SPLIT ? 5 : 3;
     constexpr int TILE_BYTES = 16 * GROUP;                       // 2 KB
-    constexpr int STAGE_BYTES = (TILES + NT) * TILE_BYTES;       // per wavefront
-    constexpr int PER_STAGE = 2 * (TILES + NT);                  // load instructions per stage
+    constexpr int B_TILES = OWN_CODES ? 0 : NT;
+    constexpr int STAGE_BYTES = (TILES + B_TILES) * TILE_BYTES;  // per wavefront
+    constexpr int PER_STAGE = 2 * (TILES + B_TILES);             // load instructions per stage
     constexpr int MAX_KB = 64;
     __shared__ __attribute__((aligned(16))) uint8_t s_ring[4 * DEPTH * STAGE_BYTES];
     __shared__ float s_bscale[MAX_KB][NT * 16];
     __shared__ float s_amax[4][NT * 16];
+    __shared__ __attribute__((aligned(16))) uint8_t s_codes[OWN_CODES ? H_F32_MAX_KB * TILE_BYTES : 16];
 
     const int e = grid_expert(expert_offsets, n_experts, blockIdx.y, gridDim.y, last_first, threadIdx.x & 63);
     if (e < 0) return;
-    const int rb = blockIdx.x;  // block of 256 output rows (GATE_UP: 128 gate + 128 up)
+    const int rb = blockIdx.x;  // block of 256 output rows (GATE_UP: 128 gate + 128 up, or half of that)
     const int begin = expert_offsets[e];
     const int end = expert_offsets[e + 1];
     if (end <= begin) return;
@@ -396,11 +409,13 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     if (GATE_UP) {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
-            const int row = (t >> 1) * inter + rb * GROUP + wave * 32 + (t & 1) * 16;
+            const int row = SPLIT ? t * inter + rb * 64 + wave * 16
+                                  : (t >> 1) * inter + rb * GROUP + wave * 32 + (t & 1) * 16;
             tile_base[t] = w_q + ((size_t)e * n_rows + row) * K;
         }
-        ws_ptr[0] = w_s + ((size_t)e * row_blocks + rb) * KB;
-        ws_ptr[1] = w_s + ((size_t)e * row_blocks + inter / GROUP + rb) * KB;
+        const int block = SPLIT ? rb >> 1 : rb;
+        ws_ptr[0] = w_s + ((size_t)e * row_blocks + block) * KB;
+        ws_ptr[1] = w_s + ((size_t)e * row_blocks + inter / GROUP + block) * KB;
     } else {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
@@ -442,16 +457,57 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
                 b_ld[nt][i] = a_q + (size_t)row * K + 16 * ld_chunk;
             }
         }
-        __syncthreads();  // the previous pass is done with s_bscale / s_amax
-        for (int i = threadIdx.x; i < KB * NT * 16; i += 256) {
-            const int kb = i / (NT * 16);
-            const int c = i - kb * (NT * 16);
-            int p = pass_begin + c;
-            p = p < end ? p : end - 1;
-            const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
-            s_bscale[kb][c] = a_s[(size_t)row * KB + kb];
-        }
-        __syncthreads();
+        // The pair scales (and with H_F32 the down GEMM's codes). With H_F32 they are made while the first blocks are on
+        // their way: what is loaded and stored there is younger than those blocks, so the counted waits of the loop
+        // cover them as they stand. With a workgroup after the other on every CU that order cost 2 %.
+        auto fill_scales = [&]() {
+            __syncthreads();  // the previous pass is done with s_bscale / s_amax
+            if constexpr (OWN_CODES) {
+                // 16 lanes per group of 128 values of a row, 8 values each
+                const int n = min(end - pass_begin, 16) * KB;
+                const int sub = threadIdx.x & 15;
+                for (int i = threadIdx.x >> 4; i < n; i += 16) {
+                    const int c = i / KB, kb = i - c * KB;
+                    const size_t at = (size_t)(pass_begin + c) * K + kb * GROUP + 8 * sub;
+                    float v[8];
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        const floatx4 x = *reinterpret_cast<const floatx4*>(h + at + 4 * r);
+                        v[4 * r] = x.x, v[4 * r + 1] = x.y, v[4 * r + 2] = x.z, v[4 * r + 3] = x.w;
+                    }
+                    float amax = 0.f;
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) amax = fmaxf(amax, fabsf(v[r]));
+#pragma unroll
+                    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+                    const float scale = group_scale(amax, pow2);
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) v[r] = fminf(fmaxf(v[r] / scale, -E4M3_MAX), E4M3_MAX);
+                    int2 code;
+                    code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+                    code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], code.x, true);
+                    code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
+                    code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], code.y, true);
+                    *reinterpret_cast<int2*>(s_codes + kb * TILE_BYTES + (c * 8 + ((sub >> 1) ^ (c & 7))) * 16 + 8 * (sub & 1)) = code;
+                    if (sub == 0) s_bscale[kb][c] = scale;
+                    if (rb == 0) {
+                        *reinterpret_cast<int2*>(h_q + at) = code;
+                        if (sub == 0) h_s[(size_t)(pass_begin + c) * KB + kb] = scale;
+                    }
+                }
+            } else {
+                for (int i = threadIdx.x; i < KB * NT * 16; i += 256) {
+                    const int kb = i / (NT * 16);
+                    const int c = i - kb * (NT * 16);
+                    int p = pass_begin + c;
+                    p = p < end ? p : end - 1;
+                    const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
+                    s_bscale[kb][c] = a_s[(size_t)row * KB + kb];
+                }
+            }
+            __syncthreads();
+        };
+        if constexpr (!H_F32) fill_scales();
         wait_vmcnt<0>();  // nothing of the compiler's is in flight when the counted loads start
 
         auto issue_stage = [&](int kb) {
@@ -463,7 +519,7 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
                              single_pass);
             }
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
+            for (int nt = 0; nt < B_TILES; ++nt) {
                 dma16_ptr(b_ld[nt][0] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES);
                 dma16_ptr(b_ld[nt][1] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES + 1024);
             }
@@ -478,6 +534,7 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
 #pragma unroll
         for (int d = 0; d < DEPTH - 1; ++d)
             if (d < KB) issue_stage(d);
+        if constexpr (H_F32) fill_scales();
 
         for (int kb = 0; kb < KB; ++kb) {
             if (kb + DEPTH - 1 < KB) {
@@ -485,10 +542,15 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
                 wait_vmcnt<(DEPTH - 1) * PER_STAGE>();
             } else if (kb + DEPTH - 2 < KB && DEPTH > 2) {
                 wait_vmcnt<(DEPTH - 2) * PER_STAGE>();
+            } else if (kb + DEPTH - 3 < KB && DEPTH > 3) {
+                wait_vmcnt<(DEPTH > 3 ? DEPTH - 3 : 0) * PER_STAGE>();
             } else {
                 wait_vmcnt<0>();
             }
             const __attribute__((address_space(3))) uint8_t* stage = ring_ptr + (kb % DEPTH) * STAGE_BYTES;
+            const __attribute__((address_space(3))) uint8_t* b_tile =
+                OWN_CODES ? (const __attribute__((address_space(3))) uint8_t*)s_codes + kb * TILE_BYTES
+                          : stage + TILES * TILE_BYTES;
             const float ws0 = ws_ptr[0][kb];
             const float ws1 = ws_ptr[1][kb];
             intx8 a[TILES];
@@ -504,34 +566,41 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
                 for (int t = 0; t < TILES; ++t) ab[t] = to_bf16_block(a[t]);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
-                    const intx4 lo = *(lds_x4)(stage + (TILES + nt) * TILE_BYTES + rd_off);
-                    const intx4 hi = *(lds_x4)(stage + (TILES + nt) * TILE_BYTES + (rd_off ^ 64));
+                    const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
+                    const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
                     const Bf16Block b = to_bf16_block(join(lo, hi));
                     const float bs = s_bscale[kb][nt * 16 + col];
 #pragma unroll
                     for (int t = 0; t < TILES; ++t) {
-                        acc[nt][t] += block_dot_bf16(ab[t], b) * (bs * ((t >> 1) ? ws1 : ws0));
+                        acc[nt][t] += block_dot_bf16(ab[t], b) * (bs * (t >= TILES / 2 ? ws1 : ws0));
                     }
                 }
             } else {
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
-                    const intx4 lo = *(lds_x4)(stage + (TILES + nt) * TILE_BYTES + rd_off);
-                    const intx4 hi = *(lds_x4)(stage + (TILES + nt) * TILE_BYTES + (rd_off ^ 64));
+                    const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
+                    const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
                     const intx8 b = join(lo, hi);
                     const float bs = s_bscale[kb][nt * 16 + col];
 #pragma unroll
                     for (int t = 0; t < TILES; ++t) {
                         const floatx4 part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
                             a[t], b, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-                        acc[nt][t] += part * (bs * ((t >> 1) ? ws1 : ws0));
+                        acc[nt][t] += part * (bs * (t >= TILES / 2 ? ws1 : ws0));
                     }
                 }
             }
             asm volatile("" ::: "memory");  // this stage's LDS reads stay above the next refill
         }
 
-        if constexpr (GATE_UP) {
+        if constexpr (SPLIT) {
+            if (pos[0] < end) {
+                floatx4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = silu(acc[0][0][r]) * acc[0][1][r];
+                *reinterpret_cast<floatx4*>(h + (size_t)pos[0] * inter + rb * 64 + wave * 16 + 4 * g) = v;
+            }
+        } else if constexpr (GATE_UP) {
             gate_up_epilogue<NT>(acc, s_amax, pos, end, h_q, h_s, inter, rb, wave, col, g, pow2);
         } else {
 #pragma unroll
@@ -681,4 +750,33 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
                 top_k, false, last_first, n_experts);
             break;
     }
+}
+
+// Both GEMMs with h in fp32 between them (H_F32 above), for so few workgroups that half of the CUs would have none.
+// Up to 128 gate/up workgroups of 128 columns (32 experts of 4096 x 2048, 2 tokens: exactly these, 58.5 -> 55 us); with more
+// the halves no longer run side by side (9 experts of 7168 x 2048, 144 workgroups: 80 us as they are, 97 in halves).
+// Internal to the library: moe_layer.hip calls it after its own checks, with config 0 or CONFIG_UE8M0 and `scratch` of
+// `scratch_floats` floats. Returns 0, without launching, for sizes it is not made for; h_q, h_s and y are what
+// moe_gate_up_launcher and moe_down_launcher leave there.
+extern "C" int moe_few_pairs_gemms(float* y, void* h_q, float* h_s, float* scratch, size_t scratch_floats, const void* x_q,
+                                   const float* x_s, const void* w13_q, const float* w13_s, const void* w2_q,
+                                   const float* w2_s, const int* sorted_pairs, const int* expert_offsets, int tokens,
+                                   int hidden, int inter, int n_experts, int top_k, int config, hipStream_t stream) {
+    const long pairs = (long)tokens * top_k;
+    const int rows = grid_rows(tokens, top_k, n_experts);
+    if ((long)(inter / GROUP) * rows > 128 || hidden % 256 != 0 || inter % GROUP != 0 || hidden / GROUP > 64 ||
+        inter / GROUP > H_F32_MAX_KB || pairs > 10L * n_experts || (size_t)pairs * inter > scratch_floats ||
+        ((reinterpret_cast<uintptr_t>(h_q) | reinterpret_cast<uintptr_t>(x_q) | reinterpret_cast<uintptr_t>(w13_q) |
+          reinterpret_cast<uintptr_t>(w2_q) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(scratch)) & 15u))
+        return 0;
+    const bool pow2 = (config & CONFIG_UE8M0) != 0;
+    const bool last_first = (config & CONFIG_LAST_EXPERT_FIRST) != 0;
+    auto* hq = static_cast<uint8_t*>(h_q);
+    moe_stream_gemm_lds_kernel<true, 1, true, true><<<dim3(inter / 64, rows), 256, 0, stream>>>(
+        static_cast<const uint8_t*>(w13_q), w13_s, static_cast<const uint8_t*>(x_q), x_s, sorted_pairs, expert_offsets,
+        nullptr, nullptr, nullptr, hidden, 2 * inter, inter, top_k, pow2, last_first, n_experts, scratch);
+    moe_stream_gemm_lds_kernel<false, 1, false, true><<<dim3(hidden / 256, rows), 256, 0, stream>>>(
+        static_cast<const uint8_t*>(w2_q), w2_s, nullptr, nullptr, nullptr, expert_offsets, hq, h_s, y, inter, hidden,
+        inter, top_k, pow2, last_first, n_experts, scratch);
+    return 1;
 }

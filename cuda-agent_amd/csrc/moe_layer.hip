@@ -27,6 +27,10 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
                                   const float* w2_s, const int* expert_offsets, int tokens, int hidden,
                                   int inter, int n_experts, int top_k, int config, hipStream_t stream);
 
+extern "C" int moe_few_pairs_gemms(float* y, void* h_q, float* h_s, float* scratch, size_t scratch_floats, const void* x_q,
+                                   const float* x_s, const void* w13_q, const float* w13_s, const void* w2_q,
+                                   const float* w2_s, const int* sorted_pairs, const int* expert_offsets, int tokens,
+                                   int hidden, int inter, int n_experts, int top_k, int config, hipStream_t stream);
 extern "C" void moe_tiled_prepare_launcher(int* tile_start, float* xs_t, const float* x_s,
                                            const int* sorted_pairs, const int* expert_offsets,
                                            int tokens, int hidden, int n_experts, int top_k,
@@ -285,6 +289,11 @@ void run_expert_gemms(const moe::Workspace& w, const GemmPlan& plan, const void*
                                    w.scale_stride, ue8m0, requant, stream);
         moe_down_tiled_launcher(w.y, w.y_scale, w.h_q, w.hs_t, w2_q, w2_s, w.expert_offsets, w.tile_start, tokens,
                                 hidden, inter, n_experts, top_k, w.scale_stride, ue8m0, stream);
+    } else if (config == 0 && !approx &&
+               moe_few_pairs_gemms(w.y, w.h_q, w.h_s, w.xs_t, (size_t)(hidden / GROUP) * w.scale_stride, w.x_q, w.x_s,
+                                   w13_q, w13_s, w2_q, w2_s, w.sorted_pairs, w.expert_offsets, tokens, hidden, inter,
+                                   n_experts, top_k, ue8m0 | order, stream)) {
+        // (xs_t, which only the tiles use, has held h in fp32)
     } else {
         moe_gate_up_launcher(w.h_q, w.h_s, w.x_q, w.x_s, w13_q, w13_s, w.sorted_pairs, w.expert_offsets,
                              tokens, hidden, inter, n_experts, top_k, config | ue8m0 | order | approx, stream);

@@ -292,6 +292,26 @@ def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
     check_layer(capi, dev, T=T, H=256, I=2048, E=E, k=k, seed=600 + E)
 
 
+@pytest.mark.parametrize('pow2', [0, 32])
+@pytest.mark.parametrize('shape', [(1, 256, 128, 9, 8), (1, 1024, 2048, 8, 2), (3, 512, 256, 16, 1), (20, 768, 128, 2, 1)])
+def test_layer_with_h_in_fp32_between_the_gemms(capi, dev, shape, pow2):
+    # so few workgroups that the down GEMM quantises h itself: every buffer bit for bit that of the form with the
+    # quantiser in the gate/up GEMM (config 1). Scratch that fits exactly, the most K blocks, several tokens, and an
+    # expert with two passes of pairs
+    T, H, I, E, k = shape
+    x, logits, w, dts = make_case(dev, T, H, I, E, 460 + T, torch.tensor([0]) if T == 20 else None)
+    if T == 20:
+        dts[1][:17, 0] = dts[1][:17, 1] + 1.0   # 17 pairs and more on one expert
+    if pow2:
+        for i in (3, 5):
+            dts[i] = torch.exp2(torch.round(torch.log2(dts[i])))
+    a, va = run_layer(capi, dts, k, pow2, torch.float32)
+    b, vb = run_layer(capi, dts, k, 1 | pow2, torch.float32)
+    for name in ('h_q', 'h_s', 'y'):
+        assert torch.equal(va[name].view(torch.uint8), vb[name].view(torch.uint8)), name
+    assert torch.equal(a, b)
+
+
 def test_layer_passes_reference_harness_bound(capi, dev):
     out, ref = check_layer(capi, dev, T=32, H=512, I=2048, E=16, k=8, seed=45)
     torch.testing.assert_close(out, ref.bfloat16(), atol=1e-2, rtol=1e-2)   # outputs are O(0.2)
