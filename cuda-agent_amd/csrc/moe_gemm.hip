@@ -77,19 +77,15 @@ __device__ __forceinline__ floatx4 block_dot_bf16(const Bf16Block& a, const Bf16
 // The expert of grid row `y`. With fewer pairs than experts the grid has one row per pair instead of one per expert,
 // and row y takes the y-th expert that has pairs (-1: there are no more): a workgroup of these kernels needs most of a
 // CU's LDS, so that the empty workgroups of 248 idle experts went through the CUs one at a time before and between
-// the working ones (gate/up of two tokens of the 256-expert layer 106 -> 77 us, of four 171 -> 144). last_first: the last expert is the heaviest (a
-// shared expert that every token uses): its workgroups are dispatched first, so that its several passes do not become
-// the launch's tail.
+// the working ones (gate/up of two tokens of the 256-expert layer 106 -> 77 us, of four 171 -> 144). last_first: the last
+// of these experts comes first (a shared expert behind the routed ones, which every token uses, is the heaviest: its
+// workgroups are dispatched first, so that its several passes do not become the launch's tail). The order decides
+// nothing else: every expert with pairs has its row, also where the last expert has none.
 constexpr int MAX_LISTED_EXPERTS = 512;
 
 __device__ __forceinline__ int grid_expert(const int* __restrict__ expert_offsets, int n_experts, int y, int rows,
                                            bool last_first, int lane) {
-    const bool all = rows >= n_experts;
-    if (last_first) {
-        if (y == 0) return n_experts - 1;
-        --y, --n_experts;
-    }
-    if (all) return y;
+    if (rows >= n_experts) return last_first ? (y == 0 ? n_experts - 1 : y - 1) : y;
     // lane l looks at experts l*per .. l*per + per - 1
     constexpr int MOST = MAX_LISTED_EXPERTS / 64;
     const int per = (n_experts + 63) / 64;
@@ -106,6 +102,9 @@ __device__ __forceinline__ int grid_expert(const int* __restrict__ expert_offset
         const int v = __shfl_up(upto, d);
         if (lane >= d) upto += v;
     }
+    const int listed = __builtin_amdgcn_readlane(upto, 63);
+    if (y >= listed) return -1;
+    if (last_first) y = y == 0 ? listed - 1 : y - 1;
     int left = y - (upto - mine), e = -1;
 #pragma unroll
     for (int i = 0; i < MOST; ++i) {
@@ -114,8 +113,7 @@ __device__ __forceinline__ int grid_expert(const int* __restrict__ expert_offset
             --left;
         }
     }
-    const unsigned long long owner = __ballot(e >= 0);
-    return owner ? __builtin_amdgcn_readlane(e, __builtin_ctzll(owner)) : -1;
+    return __builtin_amdgcn_readlane(e, __builtin_ctzll(__ballot(e >= 0)));
 }
 
 // Epilogue of the streaming gate/up kernels: h = silu(gate) * up, e4m3 with one scale per pair over the

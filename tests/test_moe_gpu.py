@@ -292,6 +292,30 @@ def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
     check_layer(capi, dev, T=T, H=256, I=2048, E=E, k=k, seed=600 + E)
 
 
+@pytest.mark.parametrize('last', ['empty', 'used'])
+@pytest.mark.parametrize('form', [0, 1, 4])
+@pytest.mark.parametrize('shape', [(1, 64, 8), (2, 17, 8), (3, 200, 5), (1, 9, 8), (3, 16, 6)])
+def test_last_expert_first_is_an_order_only(capi, dev, shape, form, last):
+    # config 128: every expert with pairs is computed whether or not the last one, which comes first, has any; pairs far
+    # below, one below and above the number of experts (above: a grid row per expert). Bit for bit config 0, over a
+    # workspace of NaNs
+    T, E, k = shape
+    x, logits, w, dts = make_case(dev, T, 512, 256, E, 700 + E)
+    dts[1][:, -1] = -30.0 if last == 'empty' else 30.0
+    runs = []
+    for order in (0, 128):
+        ws = torch.full((capi.moe_workspace_bytes(T, 512, 256, E, k),), 0xff, dtype=torch.uint8, device=dev)
+        out = torch.empty(T, 512, device=dev)
+        capi.moe_fp8_launch(out, *dts, ws, top_k=k, config=form | order)
+        views = capi.moe_workspace_views(ws, T, 512, 256, E, k)
+        assert (E - 1 in views['ids']) == (last == 'used')
+        runs.append((out, views))
+    (a, va), (b, vb) = runs
+    for name in ('h_q', 'h_s', 'y'):
+        assert torch.equal(va[name].view(torch.uint8), vb[name].view(torch.uint8)), name
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize('pow2', [0, 32])
 @pytest.mark.parametrize('shape', [(1, 256, 128, 9, 8), (1, 1024, 2048, 8, 2), (3, 512, 256, 16, 1), (20, 768, 128, 2, 1)])
 def test_layer_with_h_in_fp32_between_the_gemms(capi, dev, shape, pow2):
