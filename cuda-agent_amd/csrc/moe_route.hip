@@ -163,8 +163,8 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(
     if (lane < share * n_group) {
         const float* mine = s_choice + (lane / share) * group_size;
         for (int i = lane & (share - 1); i < group_size; i += share) {
-            const float c = mine[i];
-            second = fmaxf(second, fminf(first, c));
+            const float c = mine[i];  // (a NaN counts for nothing: the maxima pass it over)
+            second = fmaxf(second, c > first ? first : c);
             first = fmaxf(first, c);
         }
     }

@@ -163,6 +163,26 @@ def test_router_logits_golden_fixture(capi, dev):
         torch.testing.assert_close(got, torch.from_numpy(z[f'{tag}_logits']), rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize('shape', [(64, 8), (128, 8), (256, 8), (512, 8), (64, 32), (60, 3), (512, 64)])
+def test_grouped_routing_passes_nan_over(capi, dev, shape):
+    # a NaN score adds nothing to its group's value, wherever it stands beside the group's largest: every pair of
+    # positions in group 0, which with the NaN left out is worth less than group 1 (two scores of 0.69 against one of 0.88)
+    E, G = shape
+    size = E // G
+    at = torch.tensor([(i, j) for i in range(size) for j in range(size) if i != j])
+    logits = torch.full((len(at), E), -6.0)
+    logits[:, size:size + 2] = 0.8
+    rows = torch.arange(len(at))
+    logits[rows, at[:, 0]] = 2.0
+    want_ids, want_w, _ = moe.route_grouped(logits, None, 2, G, 1)
+    logits[rows, at[:, 1]] = float('nan')
+    ids = torch.empty(len(at), 2, dtype=torch.int32, device=dev)
+    w = torch.empty(len(at), 2, device=dev)
+    capi.moe_route_grouped_launch(ids, w, logits.to(dev), None, G, 1)
+    assert torch.equal(ids.cpu(), want_ids)
+    torch.testing.assert_close(w.cpu(), want_w, rtol=1e-6, atol=1e-7)
+
+
 def test_projection_then_grouped_routing_at_prefill_size(capi, dev):
     # hidden states -> logits -> experts, against the oracle's chain; a token may differ only on a near-tie
     gen = torch.Generator().manual_seed(52)
