@@ -130,6 +130,13 @@ struct SoftmaxState {
     float l;  // running sum of exp2(s - m) over the rows this lane has seen
 };
 
+// Log2-sum-exp of a split whose probabilities sum to l relative to 2^m: -inf for one without rows. A NaN score makes l
+// NaN, and the merge carries it to the output, as the reference's softmax does: whether it shows must not depend on how
+// many splits there are. (v_log_f32 is a base-2 logarithm.)
+__device__ __forceinline__ float split_lse(float m, float l) {
+    return l == 0.f ? -INFINITY : m + __builtin_amdgcn_logf(l);
+}
+
 // The accumulator is kept relative to a per-head reference exponent m, which moves whenever a
 // score exceeds it by more than FRAME_SLACK powers of two. With slack 0 this is the usual strict
 // running maximum: the largest probability of a head is exactly 1, which is what keeps the
@@ -424,12 +431,11 @@ __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
     // run over heads), so it goes through LDS, 128 dv at a time in a region private to the
     // wavefront, to leave as 512-byte row segments.
     const float l_total = st.l + __shfl_xor(st.l, 32);
-    const float inv_l = l_total > 0.f ? 1.f / l_total : 0.f;
+    const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
     const int half = lane >> 5;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
     if (half == 0) {
-        // v_log_f32 is a base-2 logarithm
-        lse_part[part0 + lane] = l_total > 0.f ? st.m + __builtin_amdgcn_logf(l_total) : -INFINITY;
+        lse_part[part0 + lane] = split_lse(st.m, l_total);
     }
     __syncthreads();  // every wavefront is done with the tile buffers
     constexpr int STAGE_STRIDE = 128 + 4;  // floats per staged head row (padded against conflicts)
@@ -1008,7 +1014,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     // log-sum-exp): half the bytes of fp32 for the split kernel to write and the merge to read, and
     // an error of at most 2^-12 of that magnitude.
     const float l_total = st.l + __shfl_xor(st.l, 32);
-    const float inv_l = l_total > 0.f ? 1.f / l_total : 0.f;
+    const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
     constexpr int STAGE_STRIDE = 64 + 4;
     float* stage = reinterpret_cast<float*>(tiles + (wave >> 2) * TILE_CHUNKS) + (wave & 3) * (32 * STAGE_STRIDE);
@@ -1055,7 +1061,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
         __syncthreads();
         if (!live) return;
         if (dh == 0 && half == 0) {
-            lse_part[part0 + lane] = l_total > 0.f ? st.m + __builtin_amdgcn_logf(l_total) : -INFINITY;
+            lse_part[part0 + lane] = split_lse(st.m, l_total);
         }
         float* o_rows = reinterpret_cast<float*>(o_part) + part0 * D_V + 256 * dh + 4 * (lane & 15);
         write_rows(inv_l, [&](int r, int ps, floatx4 v) {
@@ -1074,7 +1080,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     __syncthreads();
     if (!live) return;
     if (dh == 0 && half == 0) {
-        lse_part[part0 + lane] = l_total > 0.f ? st.m + __builtin_amdgcn_logf(l_total) : -INFINITY;
+        lse_part[part0 + lane] = split_lse(st.m, l_total);
     }
     // exponent field of the bound + 1: 2^e > |O| for every element of the head (1 if the head is 0)
     const float bound = fmaxf(s_head_max[wave][lane & 31], s_head_max[wave ^ 1][lane & 31]) * inv_l;
@@ -1138,11 +1144,12 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
     for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     float wsum = 0.f;
     for (int c0 = 0; c0 < n_splits; c0 += 64) {
-        // weight of split c0 + lane (mx = -inf: every split is empty, all weights 0)
+        // weight of split c0 + lane (0 for one without rows, NaN if its log-sum-exp is)
         float w = 0.f, ws = 0.f;
-        if (c0 + lane < n_splits && mx > -INFINITY) {
+        if (c0 + lane < n_splits) {
             const size_t row = base + (size_t)(c0 + lane) * n_heads;
-            w = __builtin_amdgcn_exp2f(lse_part[row] - mx);
+            const float lse = lse_part[row];
+            w = lse == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse - mx);
             ws = w;
             if constexpr (sizeof(PART) == 2) ws = w * scale_part[row];  // (a power of two)
         }
@@ -1153,7 +1160,7 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
             for (int j = 0; j < BATCH; ++j) {
                 const int at = s0 - c0 + NW * j;
                 const float wj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ws), at & 63));
-                if (at < 64 && wj > 0.f) {  // (a split without rows has weight 0 and is not looked at)
+                if (at < 64 && wj != 0.f) {  // (a split without rows has weight 0 and is not looked at)
 #pragma unroll
                     for (int i = 0; i < 8; ++i) o[i] += (float)rows[j][i] * wj;
                 }
@@ -1174,7 +1181,7 @@ __global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __res
             o += floatx8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         }
     }
-    if (wsum > 0.f) o *= 1.f / wsum;
+    if (wsum != 0.f) o *= 1.f / wsum;
     OUT* dst = out + ((size_t)b * n_heads + h) * D_V + lane * 8;
     if constexpr (sizeof(OUT) == 4) {
         reinterpret_cast<floatx4*>(dst)[0] = floatx4{o[0], o[1], o[2], o[3]};

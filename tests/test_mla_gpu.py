@@ -71,6 +71,27 @@ def test_split_counts(capi, dev, heads, splits):
     check(capi, q, kv, idx, splits, oracle_on_gpu(q, kv, idx))
 
 
+@pytest.mark.parametrize('heads', [32, 128])
+@pytest.mark.parametrize('config', [1, 3, 9, 40, 1001, 1003])
+def test_nan_rows_show_whatever_the_splits(capi, dev, heads, config):
+    # a selected row with a NaN makes the request's heads NaN, as in the reference, with one split, with a merge of
+    # every form and on both kernels; other requests, and requests that do not select the row, keep every bit
+    gen = torch.Generator().manual_seed(heads + config)
+    q, kv, idx = (t.to(dev) for t in mla.mla_make_inputs(4, heads, 1500, 1300, generator=gen))
+    idx[3, 1:] = -1                       # one row in all, the splits behind it empty
+    want = run_kernel(capi, q, kv, idx, config, torch.float32)
+    assert torch.isfinite(want).all()
+    bad = kv.clone()
+    bad[1, idx[1, 700]] = float('nan')    # in the middle of the list
+    bad[3, idx[3, 0], 3] = float('nan')   # one value of the only row
+    skipped = torch.ones(1500, dtype=torch.bool, device=dev)
+    skipped[idx[0].long()] = False
+    bad[0, skipped] = float('nan')        # rows that are not selected
+    out = run_kernel(capi, q, bad, idx, config, torch.float32)
+    assert out[1].isnan().all() and out[3].isnan().all()
+    assert torch.equal(out[0], want[0]) and torch.equal(out[2], want[2])
+
+
 @pytest.mark.parametrize('shape', [(3, 32, 700, 300), (5, 64, 900, 129), (1, 64, 2100, 2048)])
 def test_few_heads_over_the_fp8_cache(capi, dev, shape):
     # the kernel that dequantises its tiles against the bf16 decode of the dequantised cache, bit for bit
