@@ -357,6 +357,8 @@ bool sizes_ok(unsigned long long a_bytes, int hidden, int inter) {
     return hidden > 0 && inter > 0 && hidden % ROWS == 0 && inter % GROUP == 0 && a_bytes < (1ull << 32);  // 32-bit offsets
 }
 
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
 }  // namespace
 
 // Pairs of one tile: what moe_tiled_prepare_launcher numbers the tiles for.
@@ -371,6 +373,11 @@ extern "C" void moe_gate_up_narrow_launcher(void* h_q, float* h_s, float* hs_t, 
     if (tokens <= 0) return;
     if (!sizes_ok((unsigned long long)tokens * hidden, hidden, inter)) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);
+        return;
+    }
+    if (!h_q || !h_s || !hs_t || !x_q || !xs_t || !w13_q || !w13_s || !sorted_pairs || !expert_offsets || !tile_start ||
+        !aligned16(h_q) || !aligned16(x_q) || !aligned16(w13_q)) {
+        caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
     const dim3 grid(tiled_grid(inter / GROUP, (int)((long)tokens * top_k / PAIRS) + n_experts));
@@ -388,6 +395,11 @@ extern "C" void moe_down_narrow_launcher(float* y, float* y_scale, const void* h
     if (tokens <= 0) return;
     if (!sizes_ok((unsigned long long)tokens * top_k * inter, hidden, inter)) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);
+        return;
+    }
+    if (!y || !h_q || !hs_t || !w2_q || !w2_s || !expert_offsets || !tile_start || !aligned16(y) || !aligned16(h_q) ||
+        !aligned16(w2_q)) {
+        caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
     const dim3 grid(tiled_grid(hidden / ROWS, (int)((long)tokens * top_k / PAIRS) + n_experts));

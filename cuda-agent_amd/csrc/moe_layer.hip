@@ -220,6 +220,7 @@ struct GemmPlan {
     bool ok;
     Form form;
     bool y_half;  // y leaves as fp16 with power-of-two scales (always from 256-pair tiles, never from the streaming form)
+    bool misaligned;  // narrow tiles, asked for by config, of weights that do not start on 16 bytes
 };
 
 bool aligned16(const void* a, const void* b) {
@@ -247,6 +248,7 @@ GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int
                         pairs <= 128L * n_experts && pairs * (hidden / GROUP) <= 3000L * n_experts;
     if (tiled_ok && (form == CONFIG_NARROW_TILES || (form == 0 && narrow)))
         plan.form = GemmPlan::NARROW;
+    plan.misaligned = plan.form == GemmPlan::NARROW && !aligned;
     plan.ok = tiled_ok || (plan.form == GemmPlan::STREAMING && form != CONFIG_NARROW_TILES);
     return plan;
 }
@@ -339,7 +341,7 @@ extern "C" void moe_fp8_launcher(void* out, const void* x, const float* logits, 
         return;
     }
     if (!out || !x || !logits || !w13_q || !w13_s || !w2_q || !w2_s || !workspace ||
-        (reinterpret_cast<uintptr_t>(workspace) & 255u)) {
+        (reinterpret_cast<uintptr_t>(workspace) & 255u) || plan.misaligned) {
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
@@ -387,7 +389,7 @@ extern "C" void moe_fp8_shared_launcher(void* out, const void* x, const float* l
         return;
     }
     if (!out || !x || !logits || !w13_q || !w13_s || !w2_q || !w2_s || !sw13_q || !sw13_s || !sw2_q ||
-        !sw2_s || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) {
+        !sw2_s || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) || plan.misaligned || shared_plan.misaligned) {
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
@@ -430,7 +432,7 @@ extern "C" void moe_fp8_fused_shared_launcher(void* out, const void* x, const fl
         return;
     }
     if (!out || !x || !logits || !w13_q || !w13_s || !w2_q || !w2_s || !workspace ||
-        (reinterpret_cast<uintptr_t>(workspace) & 255u)) {
+        (reinterpret_cast<uintptr_t>(workspace) & 255u) || plan.misaligned) {
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }

@@ -582,6 +582,30 @@ def test_rejects_bad_arguments(capi, dev):
     with pytest.raises(capi.LaunchRejected, match='unsupported shape'):
         capi.moe_fp8_launch(out, *dts, big, top_k=8)      # top_k > n_experts
 
+    # the narrow tiles take weights that start on 16 bytes only (nothing is launched otherwise)
+    def shifted(t):
+        raw = torch.empty(t.numel() + 16, dtype=torch.uint8, device=dev)
+        raw[8:-8] = t.contiguous().view(torch.uint8).flatten()
+        return raw[8:-8].view(t.shape)
+    for at in (2, 4):
+        odd = [shifted(t) if i == at else t for i, t in enumerate(dts)]
+        with pytest.raises(capi.LaunchRejected, match='bad argument'):
+            capi.moe_fp8_launch(out, *odd, big, top_k=2, config=NARROW_TILES)
+
+
+@pytest.mark.parametrize('shape', [(1, 64, 8), (16, 9, 4), (17, 32, 2)])
+def test_rows_of_x_on_four_bytes(capi, dev, shape):
+    # x on 4 bytes instead of 16: routing, sort and quantiser in one launch (up to 16 tokens) give way to the launches
+    # that make no assumption; every buffer bit for bit
+    T, E, k = shape
+    x, logits, w, dts = make_case(dev, T, 256, 128, E, 800 + T)
+    odd = torch.empty(T * 256 + 2, dtype=torch.bfloat16, device=dev)[2:].view(T, 256).copy_(dts[0])
+    assert odd.data_ptr() % 16 == 4
+    (a, va), (b, vb) = (run_layer(capi, [t, *dts[1:]], k, 0, torch.float32) for t in (dts[0], odd))
+    for name in ('ids', 'weights', 'sorted_pairs', 'pair_pos', 'expert_offsets', 'x_q', 'x_s', 'y'):
+        assert torch.equal(va[name].view(torch.uint8), vb[name].view(torch.uint8)), name
+    assert torch.equal(a, b)
+
 
 BINDING_AT_FULL_SIZE = r"""
 import sys, torch
