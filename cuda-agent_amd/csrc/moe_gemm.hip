@@ -74,47 +74,53 @@ __device__ __forceinline__ floatx4 block_dot_bf16(const Bf16Block& a, const Bf16
     return part;
 }
 
-// The expert of grid row `y`. With fewer pairs than experts the grid has one row per pair instead of one per expert,
-// and row y takes the y-th expert that has pairs (-1: there are no more): a workgroup of these kernels needs most of a
-// CU's LDS, so that the empty workgroups of 248 idle experts went through the CUs one at a time before and between
-// the working ones (gate/up of two tokens of the 256-expert layer 106 -> 77 us, of four 171 -> 144). last_first: the last
-// of these experts comes first (a shared expert behind the routed ones, which every token uses, is the heaviest: its
-// workgroups are dispatched first, so that its several passes do not become the launch's tail). The order decides
-// nothing else: every expert with pairs has its row, also where the last expert has none.
+// With fewer pairs than experts, most experts have none: the workgroups then go by the list of those that have some. (A
+// workgroup of the kernels below needs most of a CU's LDS, so that the empty ones of 248 idle experts went through the
+// CUs one at a time before and between the working ones: gate/up of two tokens of the 256-expert layer 106 -> 77 us.)
+// Lane l holds experts l*per .. l*per + per - 1.
 constexpr int MAX_LISTED_EXPERTS = 512;
+constexpr int CUS = 256;
 
-__device__ __forceinline__ int grid_expert(const int* __restrict__ expert_offsets, int n_experts, int y, int rows,
-                                           bool last_first, int lane) {
-    if (rows >= n_experts) return last_first ? (y == 0 ? n_experts - 1 : y - 1) : y;
-    // lane l looks at experts l*per .. l*per + per - 1
-    constexpr int MOST = MAX_LISTED_EXPERTS / 64;
-    const int per = (n_experts + 63) / 64;
-    const int first = lane * per;
-    int off[MOST + 1];
+struct ExpertList {
+    int first = 0;       // bit i of `mask`: expert first + i has pairs
+    uint32_t mask = 0u;
+    int before = 0;      // experts with pairs in the lanes before
+    int listed = 0;      // in all lanes
+
+    __device__ __forceinline__ void load(const int* __restrict__ expert_offsets, int n_experts, int lane) {
+        constexpr int MOST = MAX_LISTED_EXPERTS / 64;
+        const int per = (n_experts + 63) / 64;
+        first = lane * per;
+        int off[MOST + 1];
 #pragma unroll
-    for (int i = 0; i <= MOST; ++i) off[i] = expert_offsets[first + i < n_experts ? first + i : n_experts];
-    int mine = 0;
+        for (int i = 0; i <= MOST; ++i) off[i] = expert_offsets[first + i < n_experts ? first + i : n_experts];
+        mask = 0u;
 #pragma unroll
-    for (int i = 0; i < MOST; ++i) mine += i < per && off[i + 1] > off[i] ? 1 : 0;
-    int upto = mine;
+        for (int i = 0; i < MOST; ++i) mask |= i < per && off[i + 1] > off[i] ? 1u << i : 0u;
+        const int mine = __popc(mask);
+        int upto = mine;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(upto, d);
-        if (lane >= d) upto += v;
-    }
-    const int listed = __builtin_amdgcn_readlane(upto, 63);
-    if (y >= listed) return -1;
-    if (last_first) y = y == 0 ? listed - 1 : y - 1;
-    int left = y - (upto - mine), e = -1;
-#pragma unroll
-    for (int i = 0; i < MOST; ++i) {
-        if (i < per && off[i + 1] > off[i]) {
-            if (left == 0) e = first + i;
-            --left;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(upto, d);
+            if (lane >= d) upto += v;
         }
+        before = upto - mine;
+        listed = __builtin_amdgcn_readlane(upto, 63);
     }
-    return __builtin_amdgcn_readlane(e, __builtin_ctzll(__ballot(e >= 0)));
-}
+
+    // Expert number y (below `listed`, uniform). last_first: the last of them comes first (a shared expert behind the
+    // routed ones, which every token uses, is the heaviest: it is begun first, so that its several passes do not become
+    // the launch's tail). The order decides nothing else: every expert with pairs has its number, also where the last
+    // expert has none.
+    __device__ __forceinline__ int at(int y, bool last_first) const {
+        if (last_first) y = y == 0 ? listed - 1 : y - 1;
+        const int nth = y - before;
+        uint32_t m = mask;
+        for (int i = 0; i < nth && m != 0u; ++i) m &= m - 1u;
+        const unsigned long long owner = __ballot(nth >= 0 && m != 0u && nth < __popc(mask));
+        return __builtin_amdgcn_readlane(first + __builtin_ctz(m | 0x80000000u), __builtin_ctzll(owner));
+    }
+};
 
 // Epilogue of the streaming gate/up kernels: h = silu(gate) * up, e4m3 with one scale per pair over the
 // workgroup's 128 columns. acc[nt][t]: tiles 0, 1 gate, 2, 3 up; a lane holds rows 4g..4g+3 of each 16-row
@@ -178,8 +184,15 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_kernel(
     constexpr int TILES = GATE_UP ? 4 : 2;
     __shared__ float s_amax[4][NT * 16];
 
-    const int e = grid_expert(expert_offsets, n_experts, blockIdx.y, gridDim.y, last_first, threadIdx.x & 63);
-    if (e < 0) return;
+    // (one grid row per expert, or per pair if there are fewer)
+    const int row = blockIdx.y;
+    int e = last_first ? (row == 0 ? n_experts - 1 : row - 1) : row;
+    if ((int)gridDim.y < n_experts) {
+        ExpertList list;
+        list.load(expert_offsets, n_experts, threadIdx.x & 63);
+        if (row >= list.listed) return;
+        e = list.at(row, last_first);
+    }
     const int rb = blockIdx.x;  // 128-row block of the output dimension
     const int begin = expert_offsets[e];
     const int end = expert_offsets[e + 1];
@@ -339,9 +352,11 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offse
 // The same load with the non-temporal hint, for weights that this launch reads exactly once (an expert whose
 // pairs fit one pass): the stream then does not displace what the caches hold for others and runs 10 % faster
 // (decode layer 1.65 -> 1.48 ms); weights that a later pass reads again keep the plain load (with the hint a
-// 1024-token layer, two passes per expert, was 1.4 % slower).
-__device__ __forceinline__ void dma16_stream(const void* base, uint32_t lane_byte_offset, uint32_t lds_base, bool once) {
-    if (once) {
+// 1024-token layer, two passes per expert, was 1.4 % slower). The choice is made once per stage: a branch per load cost
+// experts of several passes 3 to 9 %.
+template <bool ONCE>
+__device__ __forceinline__ void dma16_stream(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
+    if constexpr (ONCE) {
         asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
                      :
                      : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
@@ -350,6 +365,10 @@ __device__ __forceinline__ void dma16_stream(const void* base, uint32_t lane_byt
         dma16(base, lane_byte_offset, lds_base);
     }
 }
+template <bool B>
+struct Flag {
+    static constexpr bool value = B;
+};
 __device__ __forceinline__ void dma16_ptr(const void* lane_ptr, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
                  :
@@ -365,7 +384,8 @@ __device__ __forceinline__ void dma16_ptr(const void* lane_ptr, uint32_t lds_bas
 // experts of 7168 x 2048 77 -> 69 us for the layer, 64 of 4096 x 1536 44 -> 39, 128 of 2048 x 768 31 -> 29.
 constexpr int H_F32_MAX_KB = 16;  // (32 KB of codes)
 
-template <bool GATE_UP, int NT, bool EXACT = false, bool H_F32 = false>
+// LIST: the workgroups go by the list of experts with pairs.
+template <bool GATE_UP, int NT, bool LIST, bool EXACT = false, bool H_F32 = false>
 __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     const uint8_t* __restrict__ w_q, const float* __restrict__ w_s, const uint8_t* __restrict__ a_q,
     const float* __restrict__ a_s, const int* __restrict__ sorted_pairs,
@@ -387,43 +407,12 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     __shared__ float s_amax[4][NT * 16];
     __shared__ __attribute__((aligned(16))) uint8_t s_codes[OWN_CODES ? H_F32_MAX_KB * TILE_BYTES : 16];
 
-    const int e = grid_expert(expert_offsets, n_experts, blockIdx.y, gridDim.y, last_first, threadIdx.x & 63);
-    if (e < 0) return;
-    const int rb = blockIdx.x;  // block of 256 output rows (GATE_UP: 128 gate + 128 up, or half of that)
-    const int begin = expert_offsets[e];
-    const int end = expert_offsets[e + 1];
-    if (end <= begin) return;
-
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15;
     const int g = lane >> 4;
     const int KB = K / GROUP;
     const int row_blocks = n_rows / GROUP;
-
-    // first weight row of each of this wavefront's tiles, and the scale rows they belong to
-    const uint8_t* tile_base[TILES];
-    const float* ws_ptr[2];
-    if (GATE_UP) {
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-            const int row = SPLIT ? t * inter + rb * 64 + wave * 16
-                                  : (t >> 1) * inter + rb * GROUP + wave * 32 + (t & 1) * 16;
-            tile_base[t] = w_q + ((size_t)e * n_rows + row) * K;
-        }
-        const int block = SPLIT ? rb >> 1 : rb;
-        ws_ptr[0] = w_s + ((size_t)e * row_blocks + block) * KB;
-        ws_ptr[1] = w_s + ((size_t)e * row_blocks + inter / GROUP + block) * KB;
-    } else {
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-            const int row = rb * 256 + wave * 64 + t * 16;
-            tile_base[t] = w_q + ((size_t)e * n_rows + row) * K;
-        }
-        // wavefronts 0,1 sit in the first 128-row block, 2,3 in the second
-        ws_ptr[0] = w_s + ((size_t)e * row_blocks + rb * 2 + (wave >> 1)) * KB;
-        ws_ptr[1] = ws_ptr[0];
-    }
 
     // load side: lane j of instruction i fills slot i*64 + j = (row i*8 + j/8, position j%8),
     // i.e. fetches chunk (j%8) ^ (j/8) of that row
@@ -438,187 +427,265 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
     const __attribute__((address_space(3))) uint8_t* ring_ptr =
         (const __attribute__((address_space(3))) uint8_t*)s_ring + wave * (DEPTH * STAGE_BYTES);
 
-    const bool single_pass = end - begin <= 16 * NT;  // the weights of this workgroup are read once
-    for (int pass_begin = begin; pass_begin < end; pass_begin += 16 * NT) {
-        // activation rows: the one this lane loads (row ld_row / ld_row + 8 of tile nt) and the
-        // one whose results it ends up holding (col)
-        const uint8_t* b_ld[NT][2];
-        int pos[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            pos[nt] = pass_begin + 16 * nt + col;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                int p = pass_begin + 16 * nt + i * 8 + (int)ld_row;
-                p = p < end ? p : end - 1;  // clamped rows are computed, not stored
-                const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
-                b_ld[nt][i] = a_q + (size_t)row * K + 16 * ld_chunk;
-            }
-        }
-        // The pair scales (and with H_F32 the down GEMM's codes). With H_F32 they are made while the first blocks are on
-        // their way: what is loaded and stored there is younger than those blocks, so the counted waits of the loop
-        // cover them as they stand. With a workgroup after the other on every CU that order cost 2 %.
-        auto fill_scales = [&]() {
-            __syncthreads();  // the previous pass is done with s_bscale / s_amax
-            if constexpr (OWN_CODES) {
-                // 16 lanes per group of 128 values of a row, 8 values each
-                const int n = min(end - pass_begin, 16) * KB;
-                const int sub = threadIdx.x & 15;
-                for (int i = threadIdx.x >> 4; i < n; i += 16) {
-                    const int c = i / KB, kb = i - c * KB;
-                    const size_t at = (size_t)(pass_begin + c) * K + kb * GROUP + 8 * sub;
-                    float v[8];
-#pragma unroll
-                    for (int r = 0; r < 2; ++r) {
-                        const floatx4 x = *reinterpret_cast<const floatx4*>(h + at + 4 * r);
-                        v[4 * r] = x.x, v[4 * r + 1] = x.y, v[4 * r + 2] = x.z, v[4 * r + 3] = x.w;
-                    }
-                    float amax = 0.f;
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) amax = fmaxf(amax, fabsf(v[r]));
-#pragma unroll
-                    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-                    const float scale = group_scale(amax, pow2);
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) v[r] = fminf(fmaxf(v[r] / scale, -E4M3_MAX), E4M3_MAX);
-                    int2 code;
-                    code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-                    code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], code.x, true);
-                    code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
-                    code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], code.y, true);
-                    *reinterpret_cast<int2*>(s_codes + kb * TILE_BYTES + (c * 8 + ((sub >> 1) ^ (c & 7))) * 16 + 8 * (sub & 1)) = code;
-                    if (sub == 0) s_bscale[kb][c] = scale;
-                    if (rb == 0) {
-                        *reinterpret_cast<int2*>(h_q + at) = code;
-                        if (sub == 0) h_s[(size_t)(pass_begin + c) * KB + kb] = scale;
-                    }
-                }
-            } else {
-                for (int i = threadIdx.x; i < KB * NT * 16; i += 256) {
-                    const int kb = i / (NT * 16);
-                    const int c = i - kb * (NT * 16);
-                    int p = pass_begin + c;
-                    p = p < end ? p : end - 1;
-                    const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
-                    s_bscale[kb][c] = a_s[(size_t)row * KB + kb];
-                }
-            }
-            __syncthreads();
-        };
-        if constexpr (!H_F32) fill_scales();
-        wait_vmcnt<0>();  // nothing of the compiler's is in flight when the counted loads start
+    // One tile (block rb of 256 output rows; GATE_UP: 128 gate + 128 up, or half of that) of expert e
+    auto compute = [&](int e, int rb) {
+        const int begin = expert_offsets[e];
+        const int end = expert_offsets[e + 1];
+        if (end <= begin) return;
 
-        auto issue_stage = [&](int kb) {
-            const uint32_t stage = ring_base + (kb % DEPTH) * STAGE_BYTES;
+        // first weight row of each of this wavefront's tiles, and the scale rows they belong to
+        const uint8_t* tile_base[TILES];
+        const float* ws_ptr[2];
+        if (GATE_UP) {
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
-                dma16_stream(tile_base[t] + (size_t)kb * GROUP, ld_off, stage + t * TILE_BYTES, single_pass);
-                dma16_stream(tile_base[t] + (size_t)kb * GROUP + (size_t)8 * K, ld_off, stage + t * TILE_BYTES + 1024,
-                             single_pass);
+                const int row = SPLIT ? t * inter + rb * 64 + wave * 16
+                                      : (t >> 1) * inter + rb * GROUP + wave * 32 + (t & 1) * 16;
+                tile_base[t] = w_q + ((size_t)e * n_rows + row) * K;
             }
-#pragma unroll
-            for (int nt = 0; nt < B_TILES; ++nt) {
-                dma16_ptr(b_ld[nt][0] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES);
-                dma16_ptr(b_ld[nt][1] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES + 1024);
-            }
-        };
-
-        floatx4 acc[NT][TILES];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int t = 0; t < TILES; ++t) acc[nt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-#pragma unroll
-        for (int d = 0; d < DEPTH - 1; ++d)
-            if (d < KB) issue_stage(d);
-        if constexpr (H_F32) fill_scales();
-
-        for (int kb = 0; kb < KB; ++kb) {
-            if (kb + DEPTH - 1 < KB) {
-                issue_stage(kb + DEPTH - 1);
-                wait_vmcnt<(DEPTH - 1) * PER_STAGE>();
-            } else if (kb + DEPTH - 2 < KB && DEPTH > 2) {
-                wait_vmcnt<(DEPTH - 2) * PER_STAGE>();
-            } else if (kb + DEPTH - 3 < KB && DEPTH > 3) {
-                wait_vmcnt<(DEPTH > 3 ? DEPTH - 3 : 0) * PER_STAGE>();
-            } else {
-                wait_vmcnt<0>();
-            }
-            const __attribute__((address_space(3))) uint8_t* stage = ring_ptr + (kb % DEPTH) * STAGE_BYTES;
-            const __attribute__((address_space(3))) uint8_t* b_tile =
-                OWN_CODES ? (const __attribute__((address_space(3))) uint8_t*)s_codes + kb * TILE_BYTES
-                          : stage + TILES * TILE_BYTES;
-            const float ws0 = ws_ptr[0][kb];
-            const float ws1 = ws_ptr[1][kb];
-            intx8 a[TILES];
-#pragma unroll
-            for (int t = 0; t < TILES; ++t) {
-                const intx4 lo = *(lds_x4)(stage + t * TILE_BYTES + rd_off);
-                const intx4 hi = *(lds_x4)(stage + t * TILE_BYTES + (rd_off ^ 64));
-                a[t] = join(lo, hi);
-            }
-            if constexpr (EXACT) {
-                Bf16Block ab[TILES];
-#pragma unroll
-                for (int t = 0; t < TILES; ++t) ab[t] = to_bf16_block(a[t]);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
-                    const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
-                    const Bf16Block b = to_bf16_block(join(lo, hi));
-                    const float bs = s_bscale[kb][nt * 16 + col];
-#pragma unroll
-                    for (int t = 0; t < TILES; ++t) {
-                        acc[nt][t] += block_dot_bf16(ab[t], b) * (bs * (t >= TILES / 2 ? ws1 : ws0));
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
-                    const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
-                    const intx8 b = join(lo, hi);
-                    const float bs = s_bscale[kb][nt * 16 + col];
-#pragma unroll
-                    for (int t = 0; t < TILES; ++t) {
-                        const floatx4 part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            a[t], b, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-                        acc[nt][t] += part * (bs * (t >= TILES / 2 ? ws1 : ws0));
-                    }
-                }
-            }
-            asm volatile("" ::: "memory");  // this stage's LDS reads stay above the next refill
-        }
-
-        if constexpr (SPLIT) {
-            if (pos[0] < end) {
-                floatx4 v;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = silu(acc[0][0][r]) * acc[0][1][r];
-                *reinterpret_cast<floatx4*>(h + (size_t)pos[0] * inter + rb * 64 + wave * 16 + 4 * g) = v;
-            }
-        } else if constexpr (GATE_UP) {
-            gate_up_epilogue<NT>(acc, s_amax, pos, end, h_q, h_s, inter, rb, wave, col, g, pow2);
+            const int block = SPLIT ? rb >> 1 : rb;
+            ws_ptr[0] = w_s + ((size_t)e * row_blocks + block) * KB;
+            ws_ptr[1] = w_s + ((size_t)e * row_blocks + inter / GROUP + block) * KB;
         } else {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                if (pos[nt] < end) {
+            for (int t = 0; t < TILES; ++t) {
+                const int row = rb * 256 + wave * 64 + t * 16;
+                tile_base[t] = w_q + ((size_t)e * n_rows + row) * K;
+            }
+            // wavefronts 0,1 sit in the first 128-row block, 2,3 in the second
+            ws_ptr[0] = w_s + ((size_t)e * row_blocks + rb * 2 + (wave >> 1)) * KB;
+            ws_ptr[1] = ws_ptr[0];
+        }
+
+        const bool single_pass = end - begin <= 16 * NT;  // the weights of this workgroup are read once
+        for (int pass_begin = begin; pass_begin < end; pass_begin += 16 * NT) {
+            // activation rows: the one this lane loads (row ld_row / ld_row + 8 of tile nt) and the
+            // one whose results it ends up holding (col)
+            const uint8_t* b_ld[NT][2];
+            int pos[NT];
 #pragma unroll
-                    for (int t = 0; t < TILES; ++t) {
-                        *reinterpret_cast<floatx4*>(y + (size_t)pos[nt] * n_rows + rb * 256 + wave * 64 +
-                                                    t * 16 + 4 * g) = acc[nt][t];
+            for (int nt = 0; nt < NT; ++nt) {
+                pos[nt] = pass_begin + 16 * nt + col;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    int p = pass_begin + 16 * nt + i * 8 + (int)ld_row;
+                    p = p < end ? p : end - 1;  // clamped rows are computed, not stored
+                    const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
+                    b_ld[nt][i] = a_q + (size_t)row * K + 16 * ld_chunk;
+                }
+            }
+            // The pair scales (and with H_F32 the down GEMM's codes). With H_F32 they are made while the first blocks are on
+            // their way: what is loaded and stored there is younger than those blocks, so the counted waits of the loop
+            // cover them as they stand. With a workgroup after the other on every CU that order cost 2 %.
+            auto fill_scales = [&]() {
+                __syncthreads();  // the previous pass is done with s_bscale / s_amax
+                if constexpr (OWN_CODES) {
+                    // 16 lanes per group of 128 values of a row, 8 values each
+                    const int n = min(end - pass_begin, 16) * KB;
+                    const int sub = threadIdx.x & 15;
+                    for (int i = threadIdx.x >> 4; i < n; i += 16) {
+                        const int c = i / KB, kb = i - c * KB;
+                        const size_t at = (size_t)(pass_begin + c) * K + kb * GROUP + 8 * sub;
+                        float v[8];
+#pragma unroll
+                        for (int r = 0; r < 2; ++r) {
+                            const floatx4 x = *reinterpret_cast<const floatx4*>(h + at + 4 * r);
+                            v[4 * r] = x.x, v[4 * r + 1] = x.y, v[4 * r + 2] = x.z, v[4 * r + 3] = x.w;
+                        }
+                        float amax = 0.f;
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) amax = fmaxf(amax, fabsf(v[r]));
+#pragma unroll
+                        for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+                        const float scale = group_scale(amax, pow2);
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) v[r] = fminf(fmaxf(v[r] / scale, -E4M3_MAX), E4M3_MAX);
+                        int2 code;
+                        code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+                        code.x = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], code.x, true);
+                        code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
+                        code.y = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], code.y, true);
+                        *reinterpret_cast<int2*>(s_codes + kb * TILE_BYTES + (c * 8 + ((sub >> 1) ^ (c & 7))) * 16 + 8 * (sub & 1)) = code;
+                        if (sub == 0) s_bscale[kb][c] = scale;
+                        if (rb == 0) {
+                            *reinterpret_cast<int2*>(h_q + at) = code;
+                            if (sub == 0) h_s[(size_t)(pass_begin + c) * KB + kb] = scale;
+                        }
+                    }
+                } else {
+                    for (int i = threadIdx.x; i < KB * NT * 16; i += 256) {
+                        const int kb = i / (NT * 16);
+                        const int c = i - kb * (NT * 16);
+                        int p = pass_begin + c;
+                        p = p < end ? p : end - 1;
+                        const int row = GATE_UP ? sorted_pairs[p] / top_k : p;
+                        s_bscale[kb][c] = a_s[(size_t)row * KB + kb];
+                    }
+                }
+                __syncthreads();
+            };
+            if constexpr (!H_F32) fill_scales();
+            wait_vmcnt<0>();  // nothing of the compiler's is in flight when the counted loads start
+
+            auto issue_weights = [&](int kb, uint32_t stage, auto once) {
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    dma16_stream<decltype(once)::value>(tile_base[t] + (size_t)kb * GROUP, ld_off, stage + t * TILE_BYTES);
+                    dma16_stream<decltype(once)::value>(tile_base[t] + (size_t)kb * GROUP + (size_t)8 * K, ld_off,
+                                                        stage + t * TILE_BYTES + 1024);
+                }
+            };
+            auto issue_stage = [&](int kb) {
+                const uint32_t stage = ring_base + (kb % DEPTH) * STAGE_BYTES;
+                if (single_pass) issue_weights(kb, stage, Flag<true>{});
+                else issue_weights(kb, stage, Flag<false>{});
+#pragma unroll
+                for (int nt = 0; nt < B_TILES; ++nt) {
+                    dma16_ptr(b_ld[nt][0] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES);
+                    dma16_ptr(b_ld[nt][1] + (size_t)kb * GROUP, stage + (TILES + nt) * TILE_BYTES + 1024);
+                }
+            };
+
+            floatx4 acc[NT][TILES];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) acc[nt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+            for (int d = 0; d < DEPTH - 1; ++d)
+                if (d < KB) issue_stage(d);
+            if constexpr (H_F32) fill_scales();
+
+            for (int kb = 0; kb < KB; ++kb) {
+                if (kb + DEPTH - 1 < KB) {
+                    issue_stage(kb + DEPTH - 1);
+                    wait_vmcnt<(DEPTH - 1) * PER_STAGE>();
+                } else if (kb + DEPTH - 2 < KB && DEPTH > 2) {
+                    wait_vmcnt<(DEPTH - 2) * PER_STAGE>();
+                } else if (kb + DEPTH - 3 < KB && DEPTH > 3) {
+                    wait_vmcnt<(DEPTH > 3 ? DEPTH - 3 : 0) * PER_STAGE>();
+                } else {
+                    wait_vmcnt<0>();
+                }
+                const __attribute__((address_space(3))) uint8_t* stage = ring_ptr + (kb % DEPTH) * STAGE_BYTES;
+                const __attribute__((address_space(3))) uint8_t* b_tile =
+                    OWN_CODES ? (const __attribute__((address_space(3))) uint8_t*)s_codes + kb * TILE_BYTES
+                              : stage + TILES * TILE_BYTES;
+                const float ws0 = ws_ptr[0][kb];
+                const float ws1 = ws_ptr[1][kb];
+                intx8 a[TILES];
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    const intx4 lo = *(lds_x4)(stage + t * TILE_BYTES + rd_off);
+                    const intx4 hi = *(lds_x4)(stage + t * TILE_BYTES + (rd_off ^ 64));
+                    a[t] = join(lo, hi);
+                }
+                if constexpr (EXACT) {
+                    Bf16Block ab[TILES];
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t) ab[t] = to_bf16_block(a[t]);
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
+                        const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
+                        const Bf16Block b = to_bf16_block(join(lo, hi));
+                        const float bs = s_bscale[kb][nt * 16 + col];
+#pragma unroll
+                        for (int t = 0; t < TILES; ++t) {
+                            acc[nt][t] += block_dot_bf16(ab[t], b) * (bs * (t >= TILES / 2 ? ws1 : ws0));
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const intx4 lo = *(lds_x4)(b_tile + nt * TILE_BYTES + rd_off);
+                        const intx4 hi = *(lds_x4)(b_tile + nt * TILE_BYTES + (rd_off ^ 64));
+                        const intx8 b = join(lo, hi);
+                        const float bs = s_bscale[kb][nt * 16 + col];
+#pragma unroll
+                        for (int t = 0; t < TILES; ++t) {
+                            const floatx4 part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                                a[t], b, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                            acc[nt][t] += part * (bs * (t >= TILES / 2 ? ws1 : ws0));
+                        }
+                    }
+                }
+                asm volatile("" ::: "memory");  // this stage's LDS reads stay above the next refill
+            }
+
+            if constexpr (SPLIT) {
+                if (pos[0] < end) {
+                    floatx4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = silu(acc[0][0][r]) * acc[0][1][r];
+                    *reinterpret_cast<floatx4*>(h + (size_t)pos[0] * inter + rb * 64 + wave * 16 + 4 * g) = v;
+                }
+            } else if constexpr (GATE_UP) {
+                gate_up_epilogue<NT>(acc, s_amax, pos, end, h_q, h_s, inter, rb, wave, col, g, pow2);
+            } else {
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    if (pos[nt] < end) {
+#pragma unroll
+                        for (int t = 0; t < TILES; ++t) {
+                            *reinterpret_cast<floatx4*>(y + (size_t)pos[nt] * n_rows + rb * 256 + wave * 64 +
+                                                        t * 16 + 4 * g) = acc[nt][t];
+                        }
                     }
                 }
             }
+        }
+    };
+
+    if constexpr (!LIST) {
+        // one grid column per row tile, one grid row per expert
+        const int row = blockIdx.y;
+        compute(last_first ? (row == 0 ? n_experts - 1 : row - 1) : row, blockIdx.x);
+    } else {
+        ExpertList list;
+        list.load(expert_offsets, n_experts, lane);
+        // No more tiles than CUs: one grid row per listed expert. Else one grid row in all, of a workgroup per CU, of which
+        // as few work as still finish in the same number of rounds, so that every round has about equally many: about
+        // 155 CUs take all that the memory delivers, and 272 tiles as 256 and 16 were slower than one workgroup per tile
+        // among those of idle experts, which kept the CUs out of step (256 experts of 7168 x 2048, 3 to 31 tokens: up to
+        // 11 % slower than that; two rounds of 136 and the like: 0 to 15 % faster). What the last round lacks is left
+        // out by the first workgroups, whose first tile is the heaviest under last_first.
+        const bool in_rounds = gridDim.y == 1;
+        const int row_tiles = GATE_UP ? (SPLIT ? inter / 64 : inter / GROUP) : n_rows / 256;
+        int items = 0, rounds = 1, step = 0;
+        if (in_rounds) {
+            items = list.listed * row_tiles;
+            rounds = (items + CUS - 1) / CUS;
+            if (rounds > 1) step = ((items + rounds - 1) / rounds + 7) & ~7;  // (a multiple of the XCDs, at most CUS)
+            if (rounds > 1 && (int)blockIdx.x >= step) return;
+        }
+        for (int r = 0; r < rounds; ++r) {
+            int y = blockIdx.y, rb = blockIdx.x;
+            if (in_rounds) {
+                const int lacks = r * step + step - items;
+                const int item = r * step + (int)blockIdx.x - (lacks > 0 ? lacks : 0);
+                if (item < r * step) return;
+                y = item / row_tiles;
+                rb = item - y * row_tiles;
+            }
+            if (y >= list.listed) return;
+            compute(list.at(y, last_first), rb);
         }
     }
 }
 
-// rows of the grid: see grid_expert
-int grid_rows(int tokens, int top_k, int n_experts) {
-    const long pairs = (long)tokens * top_k;
-    return n_experts <= MAX_LISTED_EXPERTS && pairs < n_experts ? (int)pairs : n_experts;
+// whether the workgroups go by the list of experts with pairs
+bool by_list(int tokens, int top_k, int n_experts) {
+    return n_experts <= MAX_LISTED_EXPERTS && (long)tokens * top_k < n_experts;
+}
+
+// most experts that can have pairs
+int grid_rows(int tokens, int top_k, int n_experts) { return by_list(tokens, top_k, n_experts) ? tokens * top_k : n_experts; }
+
+// grid of the LDS-staged kernel for `row_tiles` tiles per expert (see its end)
+dim3 tile_grid(int row_tiles, int rows, bool listed) {
+    return listed && (long)row_tiles * rows > CUS ? dim3(CUS) : dim3(row_tiles, rows);
 }
 
 bool check_common(int hidden, int inter, int n_experts) {
@@ -651,7 +718,8 @@ extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, con
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
-    const dim3 grid(inter / GROUP, grid_rows(tokens, top_k, n_experts));
+    const int rows = grid_rows(tokens, top_k, n_experts);
+    const bool listed = by_list(tokens, top_k, n_experts);
     auto* hq = static_cast<uint8_t*>(h_q);
     const auto* xq = static_cast<const uint8_t*>(x_q);
     const auto* wq = static_cast<const uint8_t*>(w13_q);
@@ -667,24 +735,36 @@ extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, con
         nt = avg <= 10 ? 1 : avg <= 32 ? 2 : 4;
     }
     const bool lds_path = config < 8 && hidden / GROUP <= 64 && nt < 4;  // config 8+nt: direct-operand loads
-#define MOE_GATE_UP_LAUNCH(KERNEL, NT_, EXACT_)                                                           \
-    KERNEL<true, NT_, EXACT_><<<grid, 256, 0, stream>>>(wq, w13_s, xq, x_s, sorted_pairs, expert_offsets, \
-                                                       hq, h_s, nullptr, hidden, 2 * inter, inter, top_k, \
-                                                       pow2, last_first, n_experts)
-#define MOE_GATE_UP_CASE(NT_)                                                           \
-    if (lds_path && exact) MOE_GATE_UP_LAUNCH(moe_stream_gemm_lds_kernel, NT_, true);   \
-    else if (lds_path) MOE_GATE_UP_LAUNCH(moe_stream_gemm_lds_kernel, NT_, false);      \
-    else if (exact) MOE_GATE_UP_LAUNCH(moe_stream_gemm_kernel, NT_, true);              \
-    else MOE_GATE_UP_LAUNCH(moe_stream_gemm_kernel, NT_, false)
+    const dim3 lds_grid = tile_grid(inter / GROUP, rows, listed);
+#define MOE_GATE_UP_LAUNCH(KERNEL, GRID)                                                                         \
+    KERNEL<<<GRID, 256, 0, stream>>>(wq, w13_s, xq, x_s, sorted_pairs, expert_offsets, hq, h_s, nullptr, hidden, \
+                                     2 * inter, inter, top_k, pow2, last_first, n_experts)
+#define MOE_GATE_UP_DIRECT(NT_, EXACT_) \
+    MOE_GATE_UP_LAUNCH((moe_stream_gemm_kernel<true, NT_, EXACT_>), dim3(inter / GROUP, rows))
+#define MOE_GATE_UP_LDS(NT_, EXACT_)                                                                    \
+    if (listed) MOE_GATE_UP_LAUNCH((moe_stream_gemm_lds_kernel<true, NT_, true, EXACT_>), lds_grid);    \
+    else MOE_GATE_UP_LAUNCH((moe_stream_gemm_lds_kernel<true, NT_, false, EXACT_>), lds_grid)
+#define MOE_GATE_UP_CASE(NT_)                             \
+    if (lds_path && exact) {                              \
+        MOE_GATE_UP_LDS(NT_, true);                       \
+    } else if (lds_path) {                                \
+        MOE_GATE_UP_LDS(NT_, false);                      \
+    } else if (exact) {                                   \
+        MOE_GATE_UP_DIRECT(NT_, true);                    \
+    } else {                                              \
+        MOE_GATE_UP_DIRECT(NT_, false);                   \
+    }
     switch (nt) {
         case 1: MOE_GATE_UP_CASE(1); break;
         case 2: MOE_GATE_UP_CASE(2); break;
         default:
-            if (exact) MOE_GATE_UP_LAUNCH(moe_stream_gemm_kernel, 4, true);
-            else MOE_GATE_UP_LAUNCH(moe_stream_gemm_kernel, 4, false);
+            if (exact) MOE_GATE_UP_DIRECT(4, true);
+            else MOE_GATE_UP_DIRECT(4, false);
             break;
     }
 #undef MOE_GATE_UP_CASE
+#undef MOE_GATE_UP_LDS
+#undef MOE_GATE_UP_DIRECT
 #undef MOE_GATE_UP_LAUNCH
 }
 
@@ -718,13 +798,15 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
         nt = avg <= 10 ? 1 : avg <= 32 ? 2 : 4;
     }
     const bool lds_path = config < 8 && hidden % 256 == 0 && inter / GROUP <= 64;
-    const dim3 grid256(hidden / 256, rows);
+    const bool listed = by_list(tokens, top_k, n_experts);
+    const dim3 grid256 = tile_grid(hidden / 256, rows, listed);
     switch (nt) {
         case 1:
             if (lds_path) {
-                moe_stream_gemm_lds_kernel<false, 1><<<grid256, 256, 0, stream>>>(
+                const auto kernel = listed ? moe_stream_gemm_lds_kernel<false, 1, true> : moe_stream_gemm_lds_kernel<false, 1, false>;
+                kernel<<<grid256, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first, n_experts);
+                    inter, top_k, false, last_first, n_experts, nullptr);
             } else {
                 moe_stream_gemm_kernel<false, 1><<<grid, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
@@ -733,9 +815,10 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
             break;
         case 2:
             if (lds_path) {
-                moe_stream_gemm_lds_kernel<false, 2><<<grid256, 256, 0, stream>>>(
+                const auto kernel = listed ? moe_stream_gemm_lds_kernel<false, 2, true> : moe_stream_gemm_lds_kernel<false, 2, false>;
+                kernel<<<grid256, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
-                    inter, top_k, false, last_first, n_experts);
+                    inter, top_k, false, last_first, n_experts, nullptr);
             } else {
                 moe_stream_gemm_kernel<false, 2><<<grid, 256, 0, stream>>>(
                     wq, w2_s, hq, h_s, nullptr, expert_offsets, nullptr, nullptr, y, inter, hidden,
@@ -762,6 +845,7 @@ extern "C" int moe_few_pairs_gemms(float* y, void* h_q, float* h_s, float* scrat
                                    int hidden, int inter, int n_experts, int top_k, int config, hipStream_t stream) {
     const long pairs = (long)tokens * top_k;
     const int rows = grid_rows(tokens, top_k, n_experts);
+    const bool listed = by_list(tokens, top_k, n_experts);
     if ((long)(inter / GROUP) * rows > 128 || hidden % 256 != 0 || inter % GROUP != 0 || hidden / GROUP > 64 ||
         inter / GROUP > H_F32_MAX_KB || pairs > 10L * n_experts || (size_t)pairs * inter > scratch_floats ||
         ((reinterpret_cast<uintptr_t>(h_q) | reinterpret_cast<uintptr_t>(x_q) | reinterpret_cast<uintptr_t>(w13_q) |
@@ -770,10 +854,12 @@ extern "C" int moe_few_pairs_gemms(float* y, void* h_q, float* h_s, float* scrat
     const bool pow2 = (config & CONFIG_UE8M0) != 0;
     const bool last_first = (config & CONFIG_LAST_EXPERT_FIRST) != 0;
     auto* hq = static_cast<uint8_t*>(h_q);
-    moe_stream_gemm_lds_kernel<true, 1, true, true><<<dim3(inter / 64, rows), 256, 0, stream>>>(
+    const auto gate_up = listed ? moe_stream_gemm_lds_kernel<true, 1, true, true, true> : moe_stream_gemm_lds_kernel<true, 1, false, true, true>;
+    const auto down = listed ? moe_stream_gemm_lds_kernel<false, 1, true, false, true> : moe_stream_gemm_lds_kernel<false, 1, false, false, true>;
+    gate_up<<<tile_grid(inter / 64, rows, listed), 256, 0, stream>>>(
         static_cast<const uint8_t*>(w13_q), w13_s, static_cast<const uint8_t*>(x_q), x_s, sorted_pairs, expert_offsets,
         nullptr, nullptr, nullptr, hidden, 2 * inter, inter, top_k, pow2, last_first, n_experts, scratch);
-    moe_stream_gemm_lds_kernel<false, 1, false, true><<<dim3(hidden / 256, rows), 256, 0, stream>>>(
+    down<<<tile_grid(hidden / 256, rows, listed), 256, 0, stream>>>(
         static_cast<const uint8_t*>(w2_q), w2_s, nullptr, nullptr, nullptr, expert_offsets, hq, h_s, y, inter, hidden,
         inter, top_k, pow2, last_first, n_experts, scratch);
     return 1;

@@ -283,22 +283,25 @@ def test_layer_ragged_expert_load(capi, dev):
     check_layer(capi, dev, T=1, H=128, I=128, E=8, k=8, seed=44)
 
 
-@pytest.mark.parametrize('shape', [(1, 9, 8), (1, 8, 8), (2, 16, 8), (2, 17, 8), (3, 200, 5), (5, 300, 3)])
+@pytest.mark.parametrize('shape', [(1, 9, 8, 256, 2048), (1, 8, 8, 256, 2048), (2, 16, 8, 256, 2048), (2, 17, 8, 256, 2048),
+                                   (3, 200, 5, 256, 2048), (5, 300, 3, 256, 2048),
+                                   (9, 40, 4, 512, 2048), (30, 200, 6, 256, 1024)])
 def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
-    # one grid row per pair instead of per expert: pairs one below, equal to and above the number of experts
-    # (inter 2048: check_layer allows 2e-4 of the codes to be undecided ones, which must be more than one code:
+    # workgroups by the list of experts with pairs: pairs one below, equal to and above the number of experts, and more
+    # gate/up tiles than CUs, which then take them in two and in several rounds
+    # (inter 2048 and 1024: check_layer allows 2e-4 of the codes to be undecided ones, which must be more than one code:
     # 12 to 50 per million are expected)
-    T, E, k = shape
-    check_layer(capi, dev, T=T, H=256, I=2048, E=E, k=k, seed=600 + E)
+    T, E, k, H, I = shape
+    check_layer(capi, dev, T=T, H=H, I=I, E=E, k=k, seed=600 + E)
 
 
 @pytest.mark.parametrize('last', ['empty', 'used'])
 @pytest.mark.parametrize('form', [0, 1, 4])
-@pytest.mark.parametrize('shape', [(1, 64, 8), (2, 17, 8), (3, 200, 5), (1, 9, 8), (3, 16, 6)])
+@pytest.mark.parametrize('shape', [(1, 64, 8), (2, 17, 8), (3, 200, 5), (1, 9, 8), (3, 16, 6), (30, 300, 8)])
 def test_last_expert_first_is_an_order_only(capi, dev, shape, form, last):
     # config 128: every expert with pairs is computed whether or not the last one, which comes first, has any; pairs far
-    # below, one below and above the number of experts (above: a grid row per expert). Bit for bit config 0, over a
-    # workspace of NaNs
+    # below, one below and above the number of experts (above: a grid row per expert); with 300 experts both GEMMs have
+    # more tiles than CUs. Bit for bit config 0, over a workspace of NaNs
     T, E, k = shape
     x, logits, w, dts = make_case(dev, T, 512, 256, E, 700 + E)
     dts[1][:, -1] = -30.0 if last == 'empty' else 30.0
@@ -309,6 +312,7 @@ def test_last_expert_first_is_an_order_only(capi, dev, shape, form, last):
         capi.moe_fp8_launch(out, *dts, ws, top_k=k, config=form | order)
         views = capi.moe_workspace_views(ws, T, 512, 256, E, k)
         assert (E - 1 in views['ids']) == (last == 'used')
+        assert torch.isfinite(out).all()
         runs.append((out, views))
     (a, va), (b, vb) = runs
     for name in ('h_q', 'h_s', 'y'):
