@@ -2,6 +2,7 @@
 // combine). Each stage has its own extern "C" launcher; moe_fp8_launcher chains them.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -57,6 +58,30 @@ constexpr int CONFIG_REQUANT_BITS = CONFIG_EXACT_REQUANT | CONFIG_APPROX_REQUANT
 
 // config value of the layer (with the bits above): the narrow tiles whatever the number of pairs per expert
 constexpr int CONFIG_NARROW_TILES = 1 << 16;
+
+// A number of pairs that no expert is likely to exceed where tokens choose evenly: the mean and sqrt(sure * ln E) standard
+// deviations of the binomial count (one expert, or all experts for every token: the mean itself). One of them does exceed
+// it in about two draws of five with sure = 1, in one of five with sure = 2.
+inline float likely_most_pairs(int tokens, int top_k, int n_experts, float sure) {
+    const float share = top_k < n_experts ? (float)top_k / (float)n_experts : 1.f;
+    const float mean = (float)tokens * (float)top_k / (float)n_experts;
+    return mean + sqrtf(sure * logf((float)n_experts) * mean * (1.f - share));
+}
+
+// Whether the gate/up GEMM in tiles of 128 columns has no more than one workgroup per CU.
+inline bool one_round(int inter, int n_experts) { return (long)(inter / GROUP) * n_experts <= 256; }
+
+// Pairs of one pass of the streaming GEMMs over an expert's weights, in units of 16 (1, 2 or 4). A second pass costs more
+// than an idle half of a pass: 256 experts of 7168 x 2048, 16 pairs each on average, 2.36 ms for the layer with passes of
+// 16, 1.86 with 32; 8: 1.73 and 1.80. Where every workgroup has a CU to itself a pass of 32 takes a fifth longer than one
+// of 16, which two passes of 16 exceed by another fifth: passes of 16 while the odds are that one does (one expert of
+// 7168 x 2048, 16 pairs: 61 us, 74 with passes of 32; 2 experts, 14 pairs each: 68 or, where one of them has 17, 95, and
+// 80; 8 experts, 11 pairs each: 86 or 107, and 93).
+inline int streaming_pass(int tokens, int top_k, int n_experts, int inter) {
+    const long avg = (long)tokens * top_k / n_experts;  // pairs per expert if spread evenly
+    if (avg <= 10 || (one_round(inter, n_experts) && likely_most_pairs(tokens, top_k, n_experts, 1.f) <= 16.f)) return 1;
+    return avg <= 32 ? 2 : 4;
+}
 
 // marks of one element of h
 constexpr uint32_t MARK_NEAR = 1;       // the scaled value may round to either of two codes

@@ -728,12 +728,7 @@ extern "C" void moe_gate_up_launcher(void* h_q, float* h_s, const void* x_q, con
     const bool exact = (config & CONFIG_APPROX_REQUANT) == 0;
     config &= ~(CONFIG_UE8M0 | CONFIG_LAST_EXPERT_FIRST | CONFIG_REQUANT_BITS);
     int nt = config & 7;
-    if (nt != 1 && nt != 2 && nt != 4) {
-        // (a second pass over an expert's weights costs more than an idle half of a pass: 16 pairs per expert on
-        // average 2.36 ms for the layer with passes of 16, 1.86 with 32; 8: 1.73 and 1.80)
-        const long avg = (long)tokens * top_k / n_experts;  // pairs per expert if spread evenly
-        nt = avg <= 10 ? 1 : avg <= 32 ? 2 : 4;
-    }
+    if (nt != 1 && nt != 2 && nt != 4) nt = streaming_pass(tokens, top_k, n_experts, inter);
     const bool lds_path = config < 8 && hidden / GROUP <= 64 && nt < 4;  // config 8+nt: direct-operand loads
     const dim3 lds_grid = tile_grid(inter / GROUP, rows, listed);
 #define MOE_GATE_UP_LAUNCH(KERNEL, GRID)                                                                         \
@@ -793,10 +788,7 @@ extern "C" void moe_down_launcher(float* y, const void* h_q, const float* h_s, c
     // (the down GEMM has no requantisation: nothing depends on the scale convention)
     config &= ~(CONFIG_UE8M0 | CONFIG_LAST_EXPERT_FIRST | CONFIG_REQUANT_BITS);
     int nt = config & 7;
-    if (nt != 1 && nt != 2 && nt != 4) {
-        const long avg = (long)tokens * top_k / n_experts;
-        nt = avg <= 10 ? 1 : avg <= 32 ? 2 : 4;
-    }
+    if (nt != 1 && nt != 2 && nt != 4) nt = streaming_pass(tokens, top_k, n_experts, inter);
     const bool lds_path = config < 8 && hidden % 256 == 0 && inter / GROUP <= 64;
     const bool listed = by_list(tokens, top_k, n_experts);
     const dim3 grid256 = tile_grid(hidden / 256, rows, listed);

@@ -240,12 +240,26 @@ GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int
     plan.form = plan.y_half ? GemmPlan::TILED : GemmPlan::STREAMING;
     // Narrow tiles from 10 pairs per expert (256 experts of 7168 x 2048, 8 pairs: 1.73 ms streaming, 1.77 narrow; 12:
     // 1.84, 1.79; 16: 2.36, 1.82; 31: 2.61, 1.92) to where an expert's second tile, and with it its weights through L2
-    // once more, costs what a 256-pair tile loses while it starts and ends. That is the share of a tile's K blocks:
-    // 7168 x 2048 (56 blocks) 47 pairs 2.34 ms tiled, 2.00 narrow; 53: 2.36, 2.09; 64: 2.41, 2.54; 4096 x 1536 (32)
-    // 94: 0.428, 0.385; 106: 0.436, 0.414; 128: 0.462 both; 2048 x 768 (16) 128: 0.350, 0.318; 192: 0.399, 0.413.
-    // (They have the exact requantisation only.)
-    const bool narrow = !(config & CONFIG_APPROX_REQUANT) && aligned && pairs > 10L * n_experts &&
-                        pairs <= 128L * n_experts && pairs * (hidden / GROUP) <= 3000L * n_experts;
+    // once more, costs what a 256-pair tile loses while it starts and ends. That is the share of a tile's K blocks, of
+    // either GEMM: 7168 x 2048 (56 blocks) 47 pairs 2.34 ms tiled, 2.00 narrow; 53: 2.36, 2.09; 64: 2.41, 2.54; 4096 x
+    // 1536 (32) 94: 0.428, 0.385; 106: 0.436, 0.414; 128: 0.462 both; 2048 x 768 (16) 128: 0.350, 0.318; 192: 0.399, 0.413;
+    // one expert of 7168 x 18432 (144) 33: 0.210, 0.235. (They have the exact requantisation only.)
+    // The figures are for even loads. With a sixteenth of 256 experts of 7168 x 2048 chosen e^2 times as readily, 512 to
+    // 1700 tokens take 1.87 to 2.37 ms in narrow tiles, 2.05 to 2.42 in 256-pair ones, 2.46 to 4.64 streaming; at e^3 times
+    // 1.13 to 2.41, 1.17 to 2.31, 2.03 to 5.39.
+    // With a CU for every workgroup the streaming form in one pass is faster still (one expert of 7168 x 2048, 16 pairs:
+    // 61 us, 84 narrow; 24: 78, 89; 16 experts of 4096 x 1536, 18 pairs: 67, 83), as long as one pass is likely to do: the
+    // second costs half as much again as the narrow tile (8 experts of 7168 x 2048, 24 pairs, 99 and 111; 30: 175 and 127).
+    // (A shared expert, which comes first, has every token.)
+    const bool shared = (config & CONFIG_LAST_EXPERT_FIRST) != 0;
+    auto within = [&](int n, float sure) {
+        return likely_most_pairs(tokens, top_k, n_experts, sure) <= (float)n && !(shared && tokens > n);
+    };
+    const bool one_pass = one_round(inter, n_experts) &&
+                          (within(16, 1.f) || (within(32, 2.f) && hidden / GROUP <= 64 && inter / GROUP <= 64));
+    const bool narrow = !(config & CONFIG_APPROX_REQUANT) && aligned && !one_pass && pairs > 10L * n_experts &&
+                        pairs <= 128L * n_experts && pairs * (hidden / GROUP) <= 3000L * n_experts &&
+                        (pairs <= 32L * n_experts || pairs * (inter / GROUP) <= 3000L * n_experts);
     if (tiled_ok && (form == CONFIG_NARROW_TILES || (form == 0 && narrow)))
         plan.form = GemmPlan::NARROW;
     plan.misaligned = plan.form == GemmPlan::NARROW && !aligned;
@@ -425,7 +439,8 @@ extern "C" void moe_fp8_fused_shared_launcher(void* out, const void* x, const fl
                                               int inter, int n_experts, int top_k, int out_dtype,
                                               int config, hipStream_t stream) {
     if (tokens <= 0) return;
-    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts + 1, top_k + 1, config, aligned16(w13_q, w2_q));
+    const GemmPlan plan = plan_expert_gemms(tokens, hidden, inter, n_experts + 1, top_k + 1,
+                                            config | CONFIG_LAST_EXPERT_FIRST, aligned16(w13_q, w2_q));
     if (!layer_shape_ok(hidden, inter, n_experts, top_k, tokens, out_dtype) || n_experts >= 512 ||
         top_k >= 64 || (long)tokens * (top_k + 1) > 0x7fffffffL / 4 || !plan.ok) {
         caa::set_status(CAA_UNSUPPORTED_SHAPE);

@@ -295,6 +295,15 @@ def test_layer_with_fewer_pairs_than_experts(capi, dev, shape):
     check_layer(capi, dev, T=T, H=H, I=I, E=E, k=k, seed=600 + E)
 
 
+@pytest.mark.parametrize('shape', [(11, 1, 1, 2048), (16, 1, 1, 2048), (17, 1, 1, 2048), (32, 1, 1, 2048), (33, 1, 1, 2048),
+                                   (16, 1, 1, 8320), (17, 1, 1, 8320), (33, 1, 1, 8320), (28, 2, 1, 2048), (30, 4, 2, 2048)])
+def test_layer_of_few_experts(capi, dev, shape):
+    # a CU for every workgroup: streaming in one pass of 16 or 32 pairs while one is likely to do, then narrow tiles; inter
+    # 8320 is more K blocks than the LDS-staged streaming kernel takes and than narrow tiles are used for above 32 pairs
+    T, E, k, I = shape
+    check_layer(capi, dev, T=T, H=256, I=I, E=E, k=k, seed=750 + T, requant='repaired' if (T, I) == (33, 8320) else 'exact')
+
+
 @pytest.mark.parametrize('last', ['empty', 'used'])
 @pytest.mark.parametrize('form', [0, 1, 4])
 @pytest.mark.parametrize('shape', [(1, 64, 8), (2, 17, 8), (3, 200, 5), (1, 9, 8), (3, 16, 6), (30, 300, 8)])
