@@ -1224,14 +1224,27 @@ int max_splits(int batch, int head_groups, int topk, int config) {
 // the merge (5 us and 16 ns per partial of 128 heads; none for a single split). The maximum above puts a few
 // workgroups into a second round whenever the number of requests is not a divisor of 256: with it 24 requests of 2048
 // rows took 57 us, now 37; 48: 86, 58; 96: 136, 103; 150: 198, 164; 200: 211, 180; 4 requests (many partials): 28, 24.
-int pick_splits(int batch, int head_groups, int topk, int config) {
+// The model is that of 128 heads over bf16 rows. For 32 and 64 heads and for e4m3 rows its choice was within 8 % of the
+// best of all counts, 5 % for most (1 to 256 requests, 512 and 2048 rows each): what a workgroup takes there to start, end
+// and fetch a tile is in about the same proportions.
+// few_on_one_wave: on the kernel with one wavefront per 32 heads, 32 or 64 heads take several times as long per tile and
+// leave a quarter of the partials, so that start and merge hardly count: as many splits of equal size as fit the CUs in
+// one round (64 heads, 16 requests of 2048 rows: 59 us with 16 splits, 67 with the model's 13; 24: 90 with 8 to 10, 129 with
+// 11, which is more than one round). For 128 heads on it the model is the better one (24 requests 62 us, with 10 splits 68).
+int pick_splits(int batch, int head_groups, int topk, int config, bool few_on_one_wave) {
     const int most = max_splits(batch, head_groups, topk, config);
     if (config > 0) return most;
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int wgs = batch * head_groups;
+    constexpr int MOST_TILES = MAX_SPLIT_ROWS / TILE_ROWS;  // of a split
+    if (few_on_one_wave) {
+        const int fit = 256 / wgs < 1 ? 1 : 256 / wgs < tiles ? 256 / wgs : tiles;
+        const int per = (tiles + fit - 1) / fit < MOST_TILES ? (tiles + fit - 1) / fit : MOST_TILES;
+        return (tiles + per - 1) / per;
+    }
     int best = most;
     float best_us = 0.f;
-    for (int per = MAX_SPLIT_ROWS / TILE_ROWS < tiles ? MAX_SPLIT_ROWS / TILE_ROWS : tiles; per >= 1; --per) {
+    for (int per = MOST_TILES < tiles ? MOST_TILES : tiles; per >= 1; --per) {
         const int splits = (tiles + per - 1) / per;  // of `per` tiles each
         if (splits > most) break;
         const float us = split_kernel_us(wgs * splits, per) + (splits > 1 ? 5.f + 0.016f * wgs * splits : 0.f);
@@ -1251,7 +1264,8 @@ int head_groups_of(int n_heads) { return n_heads <= 128 ? 1 : n_heads / 128; }
 // config 1000 + n: n splits on the kernel with one wavefront per 32 heads
 extern "C" int sparse_mla_decode_num_splits(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
-    return pick_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config);
+    return pick_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config,
+                       config >= 1000 && n_heads < 128);
 }
 
 // bytes of scratch sparse_mla_decode_launcher needs for these sizes
@@ -1297,7 +1311,7 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
         (unsigned long long)n_kv_rows * (fp8_cache ? FP8_ROW_BYTES : ROW_BYTES) >= 0xffffffffull;
     if (config >= 1000) config -= 1000;
     const int head_groups = head_groups_of(n_heads);
-    const int splits = pick_splits(batch, head_groups, topk, config);
+    const int splits = pick_splits(batch, head_groups, topk, config, one_wave_per_group && n_heads < 128);
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int rows_per_split = ((tiles + splits - 1) / splits) * TILE_ROWS;
     float* o_part = static_cast<float*>(workspace);

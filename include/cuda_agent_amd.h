@@ -162,7 +162,8 @@ void sparse_mla_decode_paged_launcher(void* out, const void* q, const void* kv_p
                                       int d_v, float sm_scale, int out_dtype, int config,
                                       hipStream_t stream);
 
-/* Number of key splits the launcher will use for these sizes and this config. */
+/* Number of key splits the launcher will use for these sizes and this config (with a cache block of 4 GB
+ * or more, what it returns for config + 1000). */
 int sparse_mla_decode_num_splits(int batch, int n_heads, int topk, int config);
 
 /* Bytes of workspace sparse_mla_decode_launcher needs for these sizes and this config. */
