@@ -71,6 +71,16 @@ def test_split_counts(capi, dev, heads, splits):
     check(capi, q, kv, idx, splits, oracle_on_gpu(q, kv, idx))
 
 
+@pytest.mark.parametrize('splits', [8, 9, 13, 1013])
+@pytest.mark.parametrize('batch', [15, 16])
+def test_merge_of_many_heads(capi, dev, batch, splits):
+    # one wavefront per head in the merge where there are 2048 heads and more, several rounds of its 8 rows
+    gen = torch.Generator().manual_seed(batch + splits)
+    q, kv, idx = (t.to(dev) for t in mla.mla_make_inputs(batch, 128, 500, 400, generator=gen))
+    idx[1, 100:390] = -1
+    check(capi, q, kv, idx, splits, oracle_on_gpu(q, kv, idx))
+
+
 @pytest.mark.parametrize('heads', [32, 128])
 @pytest.mark.parametrize('config', [1, 3, 9, 40, 1001, 1003])
 def test_nan_rows_show_whatever_the_splits(capi, dev, heads, config):
