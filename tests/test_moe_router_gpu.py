@@ -42,7 +42,8 @@ def check(capi, dev, logits, bias, k, G, kg, norm=True, scale=1.0):
 
 
 @pytest.mark.parametrize('shape', [(64, 256, 8, 8, 4), (1000, 256, 8, 8, 4), (37, 64, 6, 4, 2), (5, 32, 4, 1, 1),
-                                   (130, 512, 8, 16, 5), (9, 8, 2, 8, 3), (64, 384, 8, 8, 4), (3, 24, 5, 3, 2)])
+                                   (130, 512, 8, 16, 5), (9, 8, 2, 8, 3), (64, 384, 8, 8, 4), (3, 24, 5, 3, 2),
+                                   (50, 128, 8, 8, 4), (21, 65, 6, 5, 2), (40, 64, 8, 2, 1), (30, 60, 4, 30, 9)])   # 1 to 32 lanes a group
 @pytest.mark.parametrize('norm,scale', [(True, 2.5), (False, 1.0)])
 def test_matches_oracle(capi, dev, shape, norm, scale):
     T, E, k, G, kg = shape
