@@ -73,14 +73,55 @@ extern "C" void moe_quant_bf16_launcher(void* q, float* scales, const void* x, i
 
 namespace {
 
+__device__ __forceinline__ void unpack_bf16x8(float (&v)[8], const unsigned (&raw)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = __uint_as_float(raw[j] << 16);
+        v[2 * j + 1] = __uint_as_float(raw[j] & 0xffff0000u);
+    }
+}
+
+// one run of a row: v its values, w their weights, `at` its place in x, group16 the lane's number among the 16 of its group
+__device__ __forceinline__ void normalise_run(float (&v)[8], const float (&w)[8], float rinv, size_t at, int group16,
+                                              __hip_bfloat16* __restrict__ y, uint8_t* __restrict__ q,
+                                              float* __restrict__ scale_at, bool pow2) {
+    typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+    typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+    float amax = 0.f;
+    unsigned packed_y[4];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float n = __bfloat162float(__float2bfloat16(v[j] * rinv));  // the norm's result in bf16
+        const __hip_bfloat16 yb = __float2bfloat16(w[j] * n);            // times the weight, in bf16
+        v[j] = __bfloat162float(yb);
+        amax = fmaxf(amax, fabsf(v[j]));
+        const unsigned bits = (unsigned)(__float_as_uint(v[j]) >> 16);
+        if (j & 1) packed_y[j >> 1] |= bits << 16; else packed_y[j >> 1] = bits;
+    }
+    if (y != nullptr) *reinterpret_cast<uintx4*>(y + at) = uintx4{packed_y[0], packed_y[1], packed_y[2], packed_y[3]};
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    const float scale = group_scale(amax, pow2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);
+    uintx2 packed;
+    int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+    lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
+    int hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
+    hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
+    packed[0] = (unsigned)lo;
+    packed[1] = (unsigned)hi;
+    *reinterpret_cast<uintx2*>(q + at) = packed;
+    if (group16 == 0) *scale_at = scale;
+}
+
 // RMS normalisation of a row followed by the activation quantisation of the result, one workgroup per row (cols <=
 // 8192): y = w * bf16(x * rsqrt(mean(x^2) + eps)) rounded to bf16 (the two roundings of a bf16 norm layer), then per
 // 128-wide group of y the scale and the e4m3 codes of moe_quant_bf16. A lane owns runs of 8 consecutive values (16 lanes
 // per group), 8 * LANES apart; the row is read once and y, the codes and the scales are written once.
 // LANES: 1024 lanes with one run each finish a row soonest, which is what counts while every row has a workgroup's place
-// to itself; with more rows what counts is how many of them are in flight, and a CU holds eight workgroups of
-// 256 lanes against two of 1024. 8192 rows of 7168: 76 -> 60 us (4.9 TB/s, 60 % of them writes), 4096: 36 -> 28; 512: 7.2
-// with 1024 lanes, 8.0 with 256.
+// to itself; with more rows what counts is how many of them are in flight, and a CU holds eight workgroups of 256 lanes
+// against two of 1024. The shorter the row, the sooner lanes without a run outweigh what the others gain.
 // Both forms add the squares in the same order: within a run, over the 64 lanes of 512 consecutive values, then these
 // sums in ascending order.
 template <int LANES>
@@ -91,76 +132,80 @@ __global__ __launch_bounds__(LANES) void moe_rmsnorm_quant_kernel(const __hip_bf
                                                                   float* __restrict__ scales, int cols,
                                                                   float eps, bool pow2) {
     typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-    typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
     constexpr int RUNS = 1024 / LANES;
     __shared__ float s_part[16];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const size_t row = blockIdx.x;
-    uintx4 raw[RUNS], wraw[RUNS];
-#pragma unroll
-    for (int r = 0; r < RUNS; ++r) {
-        const int c0 = (r * LANES + tid) * 8;
-        raw[r] = wraw[r] = uintx4{0, 0, 0, 0};
-        if (c0 < cols) {
-            raw[r] = *reinterpret_cast<const uintx4*>(x + row * cols + c0);
-            wraw[r] = *reinterpret_cast<const uintx4*>(weight + c0);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < RUNS; ++r) {
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float a = __uint_as_float(raw[r][j] << 16), b = __uint_as_float(raw[r][j] & 0xffff0000u);
-            ss = fmaf(a, a, ss);
-            ss = fmaf(b, b, ss);
-        }
+    auto load = [&](unsigned (&raw)[4], const __hip_bfloat16* src) {
+        const uintx4 r = *reinterpret_cast<const uintx4*>(src);
+        raw[0] = r.x, raw[1] = r.y, raw[2] = r.z, raw[3] = r.w;
+    };
+    // the squares of 512 consecutive values, number `part` of the row
+    auto add_squares = [&](float ss, int part) {
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
-        if (lane == 0) s_part[r * (LANES / 64) + wave] = ss;
-    }
-    __syncthreads();
-    float total = 0.f;
+        if (lane == 0) s_part[part] = ss;
+    };
+    auto row_rinv = [&]() {
+        __syncthreads();
+        float total = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) total += s_part[i];
-    const float rinv = 1.f / sqrtf(total / (float)cols + eps);  // correctly rounded, as a CPU evaluation
+        for (int i = 0; i < 16; ++i) total += s_part[i];
+        return 1.f / sqrtf(total / (float)cols + eps);  // correctly rounded, as a CPU evaluation
+    };
+    auto finish = [&](float (&v)[8], const float (&w)[8], float rinv, int c0) {
+        normalise_run(v, w, rinv, row * cols + c0, tid & 15, y, q, scales + row * (cols / GROUP) + c0 / GROUP, pow2);
+    };
+    if constexpr (RUNS == 1) {
+        const int c0 = tid * 8;
+        const bool live = c0 < cols;
+        float v[8], w[8];
+        float ss = 0.f;
+        if (live) {
+            unsigned raw[4], wraw[4];
+            load(raw, x + row * cols + c0);
+            load(wraw, weight + c0);
+            unpack_bf16x8(v, raw);
+            unpack_bf16x8(w, wraw);
 #pragma unroll
-    for (int r = 0; r < RUNS; ++r) {
-        const int c0 = (r * LANES + tid) * 8;
-        if (c0 >= cols) return;
-        float amax = 0.f, v[8];
-        unsigned packed_y[4];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const unsigned xbits = raw[r][j >> 1], wbits = wraw[r][j >> 1];
-            const float xv = __uint_as_float(j & 1 ? xbits & 0xffff0000u : xbits << 16);
-            const float wv = __uint_as_float(j & 1 ? wbits & 0xffff0000u : wbits << 16);
-            const float n = __bfloat162float(__float2bfloat16(xv * rinv));  // the norm's result in bf16
-            const __hip_bfloat16 yb = __float2bfloat16(wv * n);            // times the weight, in bf16
-            v[j] = __bfloat162float(yb);
-            amax = fmaxf(amax, fabsf(v[j]));
-            const unsigned bits = (unsigned)(__float_as_uint(v[j]) >> 16);
-            if (j & 1) packed_y[j >> 1] |= bits << 16; else packed_y[j >> 1] = bits;
+            for (int j = 0; j < 8; ++j) ss = fmaf(v[j], v[j], ss);
         }
-        if (y != nullptr) {
-            *reinterpret_cast<uintx4*>(y + row * cols + c0) = uintx4{packed_y[0], packed_y[1], packed_y[2], packed_y[3]};
+        add_squares(ss, wave);
+        const float rinv = row_rinv();
+        if (live) finish(v, w, rinv, c0);
+    } else {
+        // (four runs stay packed until they are used: 64 registers, which is what eight workgroups on a CU leave)
+        unsigned raw[RUNS][4], wraw[RUNS][4];
+#pragma unroll
+        for (int r = 0; r < RUNS; ++r) {
+            const int c0 = (r * LANES + tid) * 8;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) raw[r][j] = wraw[r][j] = 0u;
+            if (c0 < cols) {
+                load(raw[r], x + row * cols + c0);
+                load(wraw[r], weight + c0);
+            }
         }
 #pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-        const float scale = group_scale(amax, pow2);
+        for (int r = 0; r < RUNS; ++r) {
+            float v[8], ss = 0.f;
+            unpack_bf16x8(v, raw[r]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);
-        uintx2 packed;
-        int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
-        lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo, true);
-        int hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
-        hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
-        packed[0] = (unsigned)lo;
-        packed[1] = (unsigned)hi;
-        *reinterpret_cast<uintx2*>(q + row * cols + c0) = packed;
-        if ((tid & 15) == 0) scales[row * (cols / GROUP) + (c0 / GROUP)] = scale;
+            for (int j = 0; j < 8; ++j) ss = fmaf(v[j], v[j], ss);
+            add_squares(ss, r * (LANES / 64) + wave);
+        }
+        const float rinv = row_rinv();
+#pragma unroll
+        for (int r = 0; r < RUNS; ++r) {
+            const int c0 = (r * LANES + tid) * 8;
+            if (c0 >= cols) return;
+            float v[8], w[8];
+            unpack_bf16x8(v, raw[r]);
+            unpack_bf16x8(w, wraw[r]);
+            finish(v, w, rinv, c0);
+        }
     }
 }
 
@@ -186,7 +231,10 @@ extern "C" void moe_rmsnorm_quant_launcher(void* q, float* scales, void* y, cons
         caa::set_status(CAA_BAD_ARGUMENT);
         return;
     }
-    const bool many = rows > 512;  // 1024-lane workgroups have two places on each of the 256 CUs
+    // us with 1024 lanes and with 256: 7168 columns 1400 rows 13.8 and 14.3, 1700: 16.0, 15.4, 8192: 68.4, 55.9 (4.9 TB/s, 60 %
+    // of them writes); 4096: 1536 rows 9.5 and 10.0, 2000: 11.9, 11.8; 2048: 600 rows 4.6 and 4.8, 1000: 5.6, 5.3; 1024: 513 rows
+    // 3.6 and 3.8, 768: 4.5, 4.1
+    const bool many = rows > (cols > 2048 ? 1600 : cols > 1024 ? 768 : 576);
     const auto kernel = many ? moe_rmsnorm_quant_kernel<256> : moe_rmsnorm_quant_kernel<1024>;
     kernel<<<rows, many ? 256 : 1024, 0, stream>>>(
         static_cast<const __hip_bfloat16*>(x), static_cast<const __hip_bfloat16*>(weight),
