@@ -495,10 +495,20 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
         return;
     }
     const int n_chunks = hidden / K_CHUNK;
-    // enough 128 x 64 tiles and splits to fill the chip: the workgroup-tiled kernel (config 2 forces it, 1 the other one)
-    const long big_tiles = (long)((tokens + BIG_TOKENS - 1) / BIG_TOKENS) * ((n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS);
-    const bool tiled = hidden <= (1 << 24) && (config == 2 || (config != 1 && big_tiles * splits >= 192 && tokens >= BIG_TOKENS));
     const int chunks_per_split = (n_chunks + splits - 1) / splits;
+    // Enough 128 x 64 tiles and splits to fill the chip: the workgroup-tiled kernel (config 2 forces it, 1 the other one).
+    // It has one workgroup on a CU, so that a part of a second round costs a whole one, which few chunks of K do not make up
+    // for, all the less where each has little to share (us, tiled and not; 1500 tokens of 4096 x 64, 384 workgroups of 2
+    // chunks: 17.3, 15.4; 1400 of 1024 x 256, 352 of 2: 15.9, 14.0; one tile of experts, 1200 of 7168 x 64, 320 of 4: 18.7,
+    // 17.9; a third of the rows padding, 160 of 7168 x 384, 384 of 4: 18.1, 17.0; but 300 of 7168 x 256, 384 of 4: 19.2, 20.7).
+    const long token_tiles = (tokens + BIG_TOKENS - 1) / BIG_TOKENS;
+    const long big_wgs = token_tiles * ((n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS) * splits;
+    const bool part_of_second_round = big_wgs > 256 && big_wgs < 512;
+    const bool few_chunks = chunks_per_split <= 2 ||
+                            (chunks_per_split <= 4 && splits >= 16 && big_wgs < 448 &&
+                             (n_experts <= BIG_EXPERTS || 3L * tokens < 2 * BIG_TOKENS * token_tiles));
+    const bool tiled = hidden <= (1 << 24) && (config == 2 || (config != 1 && big_wgs >= 192 && tokens >= BIG_TOKENS &&
+                                                              !(part_of_second_round && few_chunks)));
     float* out = splits > 1 ? static_cast<float*>(workspace) : logits;
     const int tile_tokens = tiled ? BIG_TOKENS : 64;
     const dim3 grid((tokens + tile_tokens - 1) / tile_tokens, (n_experts + 63) / 64, splits);
