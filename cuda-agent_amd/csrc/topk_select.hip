@@ -19,17 +19,21 @@
 //            bin of the k-th largest are sorted out bit by bit. Chosen entries become bits of a bitmap of the row,
 //            whose words are placed in the output by a workgroup-wide scan
 //
-// If the list turns out shorter than k or longer than it may be (rows of few distinct values, a sample that
-// misled), and for rows of up to 8192 entries or k above 3072, the whole row is searched instead: a radix select with
-// digits of 11, 11 and 10 bits, most significant first, which stops as soon as all keys of a digit's bin are wanted.
+// If the sample says that the list would be too long, or it turns out shorter than k or too long (rows of few distinct
+// values, a sample that misled), and for rows of up to 8192 or more than 262144 entries (the bitmaps' size) or k above
+// 3072, the whole row is searched instead: a radix select with digits of 11, 11 and 10 bits, most significant first,
+// which stops as soon as all keys of a digit's bin are wanted or the first digit's bin holds a single key.
 //
 // Rows of up to 65536 scores are held in registers, in words of 64 consecutive entries (a load instruction fetches
 // 256 consecutive bytes; with 16-byte pieces of 64 different lines, as each lane owning consecutive entries asks for,
 // the row came through L1 eight times). Longer rows are read again by each step. The output never depends on timing.
 //
-// Measured (us; one row unless stated, k = 2048; radix select over four 8-bit digits before): n = 16384 10.2 -> 8.1,
-// 32768 19.3 -> 9.4, 64 rows of it 20.2 -> 10.9; 24 rows of 33024 62.9 -> 12.0; n = 65536 115 -> 13.4; 131072
-// 220 -> 20.3. Constant rows, which the whole-row search takes: n = 16384 13.9 -> 16.6, 32768 26 -> 21, 65536 266 -> 32.
+// Measured (us; one row unless stated, k = 2048; radix select over four 8-bit digits before): n = 8192 7.1 -> 6.1,
+// 16384 10.3 -> 7.4, 32768 19.5 -> 9.9, 64 rows of it 20.0 -> 10.3; 65536 115 -> 13.8; 131072 221 -> 20.4. Rows that the
+// whole-row search takes: one value, n = 8192 9.1 -> 5.9, 16384 14.0 -> 11.0, 32768 26 -> 18; two values 8.4 -> 6.6,
+// 12.9 -> 11.5, 24.4 -> 18.9; 95 % masked 9.3 -> 7.0, 14.4 -> 12.9, 27 -> 21. Slower than before: rows that have k
+// entries left unmasked but fewer than the sample's rank asks for, for which the sample is for nothing (95 % of 16384
+// masked, k = 512: 10.8 -> 12.3), and 64 rows of 8192 in some 50 values (7.6 -> 7.9).
 //
 // Entries beyond a request's valid length (lengths[b], optional) are not candidates; if fewer
 // than k candidates exist the remaining outputs are -1, which the attention treats as padding.
@@ -108,6 +112,39 @@ __device__ __forceinline__ Word lowest_set(Word w, int take) {
     return w & (((Word)1 << low) - 1);
 }
 
+// Adds N words of 64 bins to a histogram of COPIES interleaved copies. LDS does additions to one address one after the
+// other, so that where the bin of lane 0 or 32 of the first word is that of more than 16 of its lanes (of a masked row
+// one of the two may hold an entry that is not masked), that bin and one of those left over are added as one number each.
+template <int N, int COPIES>
+__device__ __forceinline__ void count_words(int* hist, const uint32_t (&bin)[N], int lane) {
+    const unsigned long long same0 = __ballot(bin[0] == (uint32_t)__builtin_amdgcn_readlane(bin[0], 0));
+    const unsigned long long same32 = __ballot(bin[0] == (uint32_t)__builtin_amdgcn_readlane(bin[0], 32));
+    bool on[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) on[j] = true;
+    if (__popcll(same0) > 16 || __popcll(same32) > 16) {
+        unsigned long long same = __popcll(same0) > 16 ? same0 : same32;
+        const unsigned long long rest = ~same;
+        for (int probe = 0; probe < 2; ++probe) {
+            const uint32_t b = __builtin_amdgcn_readlane(bin[0], __builtin_ctzll(same));
+            int n = 0;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const bool add = on[j] && bin[j] == b;
+                n += __popcll(__ballot(add));
+                on[j] = on[j] && !add;
+            }
+            if (lane == 0) atomicAdd(&hist[b * COPIES], n);
+            if (n == 64 * N) return;
+            if (rest == 0ull) break;
+            same = rest;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (on[j]) atomicAdd(&hist[bin[j] * COPIES + (lane & (COPIES - 1))], 1);
+}
+
 // P words of 64 entries per wavefront; the row is taken in chunks of CHUNK = 1024 * P entries. RESIDENT: one chunk
 // holds the whole row and stays in registers; else the row is read again by every step.
 template <int P, bool RESIDENT>
@@ -119,8 +156,11 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     constexpr bool FILTER = P >= 16;
     constexpr int HIST_COPIES = FILTER ? 2 : 4;  // of the first digit's histogram
     __shared__ __attribute__((aligned(16))) int s_hist[DIGIT_BINS * HIST_COPIES];  // [bin][copy]
+    // (without the filter there is room to give the later digits histograms of their own, cleared with the first: a
+    // barrier and a clear less for each)
+    __shared__ __attribute__((aligned(16))) int s_hist_later[FILTER ? 4 : 2 * DIGIT_BINS];
     __shared__ int s_wave_sum[2][SELECT_WAVES];
-    __shared__ int s_bin, s_above, s_in_bin, s_count, s_near_count;
+    __shared__ int s_bin, s_above, s_in_bin, s_count, s_near_count, s_differ;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -164,16 +204,15 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         for (int g = 0; g < P; g += GROUP)
             if (64 * g < left) f(g);
     };
-    auto clear_hist = [&](int words) {
-        for (int i = tid; i < words / 4; i += SELECT_THREADS) reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
+    auto clear_hist = [&](int* hist, int words) {
+        for (int i = tid; i < words / 4; i += SELECT_THREADS) reinterpret_cast<int4*>(hist)[i] = make_int4(0, 0, 0, 0);
     };
     // In the histogram of 2^BITS bins x COPIES: the bin in which the rank-th largest key lies (counting from the top
-    // bin down), the keys in bins above it and in it; bin = -1 if there are fewer than `rank` keys.
-    auto find_bin = [&](auto bits_tag, auto copies_tag, int rank, int& bin, int& above_bin, int& in_bin) {
+    // bin down), the keys in bins above it and in it; s_bin as it was if there are fewer than `rank` keys.
+    auto find_bin = [&](const int* hist, auto bits_tag, auto copies_tag, int rank, int& bin, int& above_bin, int& in_bin) {
         constexpr int BINS = 1 << decltype(bits_tag)::value;
         constexpr int COPIES = decltype(copies_tag)::value;
         constexpr int PER = BINS / SELECT_THREADS;  // bins of a lane
-        if (tid == 0) s_bin = -1;
         __syncthreads();  // the counts are complete
         int c[PER];
         int mine = 0;
@@ -181,7 +220,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         for (int j = 0; j < PER; ++j) {
             c[j] = 0;
 #pragma unroll
-            for (int h = 0; h < COPIES; ++h) c[j] += s_hist[(BINS - 1 - (PER * tid + j)) * COPIES + h];
+            for (int h = 0; h < COPIES; ++h) c[j] += hist[(BINS - 1 - (PER * tid + j)) * COPIES + h];
             mine += c[j];
         }
         const int upto = wave_inclusive_sum(mine, lane);
@@ -202,25 +241,39 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     };
     // The want-th largest key (`threshold`) and how many of the keys equal to it are chosen, most significant digit
     // first; if all keys of a digit's bin are wanted the digits below do not matter and the threshold is the bin's
-    // lowest key. count(shift_tag, bits_tag, copies_tag, threshold) adds the keys that share the digits found so far
-    // to the histogram.
-    auto radix_select = [&](auto copies_tag, auto count, uint32_t& threshold, int& need_eq) {
-        threshold = 0u;
-        int remaining = want;
-        auto digit = [&](auto shift_tag, auto bits_tag, auto copies) {
-            clear_hist((1 << decltype(bits_tag)::value) * decltype(copies)::value);
-            __syncthreads();
-            count(shift_tag, bits_tag, copies, threshold);
-            int bin, above, in_bin;
-            find_bin(bits_tag, copies, remaining, bin, above, in_bin);
-            threshold |= (uint32_t)bin << decltype(shift_tag)::value;
+    // lowest key. first(hist) adds all keys to the histogram of the upper 11 bits, later(hist, threshold, shift, above)
+    // those that are threshold from bit `above` up to that of the bits from `shift` up. one_key(threshold): whether all
+    // keys of the first digit's bin are the same, and if so that key; asked where the bin is so full that they may be
+    // (masked entries, rows of a few values): additions to one address are done one after the other, so that two more
+    // digits over 8192 masked entries took 12 us. Not expected, to keep its code out of the others' way: a workgroup
+    // alone on its CU waits for the instructions it fetches, and a few dozen more in line cost 5 % of a short row.
+    auto radix_select = [&](auto copies_tag, auto first, auto later, auto one_key, uint32_t& threshold, int& need_eq) {
+        clear_hist(s_hist, DIGIT_BINS * decltype(copies_tag)::value);
+        if constexpr (!FILTER) clear_hist(s_hist_later, 2 * DIGIT_BINS);
+        if (tid == 0) s_differ = 0;
+        __syncthreads();
+        first(s_hist);
+        int bin, above, in_bin;
+        find_bin(s_hist, IntConstant<11>{}, copies_tag, want, bin, above, in_bin);
+        threshold = (uint32_t)bin << 21;
+        int remaining = want - above;
+        if (__builtin_expect(in_bin != remaining && in_bin >= valid / 4, 0) && one_key(threshold)) {
+            need_eq = remaining;
+            return;
+        }
+#pragma unroll
+        for (int shift = 10; in_bin != remaining && shift >= 0; shift -= 10) {
+            int* hist = FILTER ? s_hist : s_hist_later + (shift == 10 ? 0 : DIGIT_BINS);
+            if constexpr (FILTER) {
+                clear_hist(hist, DIGIT_BINS);
+                __syncthreads();
+            }
+            later(hist, threshold, shift, shift == 10 ? 21 : 10);
+            find_bin(hist, IntConstant<11>{}, IntConstant<1>{}, remaining, bin, above, in_bin);
+            threshold |= (uint32_t)bin << shift;
             remaining -= above;
-            return in_bin == remaining;
-        };
-        bool done = digit(IntConstant<21>{}, IntConstant<11>{}, copies_tag);
-        if (!done) done = digit(IntConstant<10>{}, IntConstant<11>{}, IntConstant<1>{});
-        if (!done) done = digit(IntConstant<0>{}, IntConstant<10>{}, IntConstant<1>{});
-        need_eq = done ? valid : remaining;
+        }
+        need_eq = in_bin == remaining ? valid : remaining;
     };
 
     float val[P];
@@ -232,8 +285,8 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         __shared__ uint32_t s_gt[BITMAP], s_eq[BITMAP];
         if (want <= MAX_FILTER_WANT && want < valid && (RESIDENT || valid <= MAX_FILTER_ROW)) {
             // An eighth of the row, spread evenly: lane l takes word g + l % 8 of every group of words.
-            clear_hist(1 << SAMPLE_BITS);
-            if (tid == 0) s_count = s_near_count = 0;
+            clear_hist(s_hist, 1 << SAMPLE_BITS);
+            if (tid == 0) s_count = s_near_count = 0, s_bin = -1;
             const int words = (valid + 31) / 32;
             for (int i = tid; i < words; i += SELECT_THREADS) s_gt[i] = s_eq[i] = 0u;
             __syncthreads();
@@ -267,9 +320,10 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
             const float expect = 0.125f * (float)want;
             const int rank = (int)(1.5f * expect + 4.f * __builtin_sqrtf(expect)) + 16;
             int bin, above, in_bin;
-            find_bin(IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, rank, bin, above, in_bin);
+            find_bin(s_hist, IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, rank, bin, above, in_bin);
             const uint32_t pivot_key = (uint32_t)bin << (32 - SAMPLE_BITS);
-            if (bin > 0 && pivot_key > 0x007fffffu) {  // (a number: NaN and -inf are below it)
+            // (a number: NaN and -inf are below it; and no list that is sure to be too long, as of rows of few values)
+            if (bin > 0 && pivot_key > 0x007fffffu && 8 * (above + in_bin) <= MAX_CANDIDATES + 1024) {
                 const float pivot = key_score(pivot_key);
                 // (a lane appends its own entries one after the other: what a word costs is VALU time, of which one CU
                 // has 64 lanes a clock)
@@ -337,13 +391,13 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
                     };
                     uint32_t threshold = 0u;
                     int need_eq = valid;
-                    clear_hist(1 << SAMPLE_BITS);
+                    clear_hist(s_hist, 1 << SAMPLE_BITS);
                     __syncthreads();
 #pragma unroll
                     for (int r = 0; r < PER; ++r)
                         if (lkey[r] != 0u) atomicAdd(&s_hist[near_bin(lkey[r])], 1);
                     int tbin, tabove, tin;
-                    find_bin(IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, want, tbin, tabove, tin);
+                    find_bin(s_hist, IntConstant<SAMPLE_BITS>{}, IntConstant<1>{}, want, tbin, tabove, tin);
                     if (tin == want - tabove) {
                         threshold = pivot_key + ((uint32_t)tbin << NEAR_BITS);
                     } else if (tin <= 64 && tbin < (1 << SAMPLE_BITS) - 1) {
@@ -375,14 +429,33 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
                         threshold = (uint32_t)s_bin;
                         need_eq = s_above;
                     } else {
-                        radix_select(IntConstant<1>{}, [&](auto shift_tag, auto bits_tag, auto, uint32_t prefix) {
-                            constexpr int shift = decltype(shift_tag)::value, bits = decltype(bits_tag)::value;
+                        // Rows of few values have many equal keys there. (s_hist has been read: any of the bin's keys.)
 #pragma unroll
-                            for (int r = 0; r < PER; ++r) {
-                                if (lkey[r] != 0u && (shift + bits == 32 || ((lkey[r] ^ prefix) >> ((shift + bits) & 31)) == 0u))
-                                    atomicAdd(&s_hist[(lkey[r] >> shift) & ((1u << bits) - 1u)], 1);
-                            }
-                        }, threshold, need_eq);
+                        for (int r = 0; r < PER; ++r)
+                            if (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin) s_hist[0] = (int)lkey[r];
+                        __syncthreads();
+                        const uint32_t one = (uint32_t)s_hist[0];
+                        bool differs = false;
+#pragma unroll
+                        for (int r = 0; r < PER; ++r)
+                            differs = differs || (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin && lkey[r] != one);
+                        if (__ballot(differs) != 0ull && lane == 0) s_near_count = 1;
+                        __syncthreads();
+                        if (s_near_count == 0) {
+                            threshold = one;
+                            need_eq = want - tabove;
+                        } else {
+                            radix_select(IntConstant<1>{}, [&](int* hist) {
+#pragma unroll
+                                for (int r = 0; r < PER; ++r)
+                                    if (lkey[r] != 0u) atomicAdd(&hist[lkey[r] >> 21], 1);
+                            }, [&](int* hist, uint32_t prefix, int shift, int above) {
+                                const uint32_t mask = (1u << (above - shift)) - 1u;
+#pragma unroll
+                                for (int r = 0; r < PER; ++r)
+                                    if (lkey[r] != 0u && (lkey[r] ^ prefix) >> above == 0u) atomicAdd(&hist[(lkey[r] >> shift) & mask], 1);
+                            }, [](uint32_t&) { return false; }, threshold, need_eq);
+                        }
                     }
 #pragma unroll
                     for (int r = 0; r < PER; ++r) {
@@ -430,37 +503,55 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     uint32_t threshold = 0u;
     int need_eq = valid;
     if (want < valid) {
-        radix_select(IntConstant<HIST_COPIES>{}, [&](auto shift_tag, auto bits_tag, auto copies_tag, uint32_t prefix) {
-            constexpr int shift = decltype(shift_tag)::value, bits = decltype(bits_tag)::value;
-            constexpr int COPIES = decltype(copies_tag)::value;
-            const int copy = lane & (COPIES - 1);
-            auto in_prefix = [&](uint32_t x) { return shift + bits == 32 || ((x ^ prefix) >> ((shift + bits) & 31)) == 0u; };
+        // f(g) for the groups of words of the whole row
+        auto for_row = [&](auto f) {
             for (int c0 = 0; c0 < valid; c0 += CHUNK) {
                 const int left = valid - c0 - span;
                 if constexpr (!RESIDENT) {
                     load_chunk(val, c0 + span, left);
                     make_keys();
                 }
-                for_groups(left, [&](int g) {
-                    // a group of one value (rows that are masked, say) is one addition
-                    uint32_t differ = 0u;
-#pragma unroll
-                    for (int j = g + 1; j < g + GROUP; ++j) differ |= key[j] ^ key[g];
-                    const uint32_t key0 = __builtin_amdgcn_readfirstlane(key[g]);
-                    differ |= key[g] ^ key0;
-                    if (__ballot(differ == 0u) == ~0ull) {
-                        if (lane == 0 && in_prefix(key0))
-                            atomicAdd(&s_hist[((key0 >> shift) & ((1u << bits) - 1u)) * COPIES], 64 * GROUP);
-                        return;
-                    }
-#pragma unroll
-                    for (int j = g; j < g + GROUP; ++j) {
-                        if (in_prefix(key[j]))
-                            atomicAdd(&s_hist[((key[j] >> shift) & ((1u << bits) - 1u)) * COPIES + copy], 1);
-                    }
-                });
+                for_groups(left, f);
                 if (RESIDENT) break;
             }
+        };
+        radix_select(IntConstant<HIST_COPIES>{}, [&](int* hist) {
+            for_row([&](int g) {
+                uint32_t bin[GROUP];
+#pragma unroll
+                for (int j = 0; j < GROUP; ++j) bin[j] = key[g + j] >> 21;
+                count_words<GROUP, HIST_COPIES>(hist, bin, lane);
+            });
+        }, [&](int* hist, uint32_t prefix, int shift, int above) {
+            const uint32_t mask = (1u << (above - shift)) - 1u;  // (fewer than a quarter of the row, or of several keys)
+            for_row([&](int g) {
+#pragma unroll
+                for (int j = g; j < g + GROUP; ++j)
+                    if ((key[j] ^ prefix) >> above == 0u) atomicAdd(&hist[(key[j] >> shift) & mask], 1);
+            });
+        }, [&](uint32_t& prefix) {
+            auto in_bin = [&](uint32_t x) { return (x ^ prefix) >> 21 == 0u; };
+            bool any = false, differs = false;
+            uint32_t mine = 0u;
+            for_row([&](int g) {
+#pragma unroll
+                for (int j = g; j < g + GROUP; ++j) {
+                    any = any || in_bin(key[j]);
+                    mine = in_bin(key[j]) ? key[j] : mine;
+                }
+            });
+            if (any) s_hist[0] = (int)mine;  // (its counts have been read: any key of the bin)
+            __syncthreads();
+            const uint32_t one = (uint32_t)s_hist[0];
+            for_row([&](int g) {
+#pragma unroll
+                for (int j = g; j < g + GROUP; ++j) differs = differs || (in_bin(key[j]) && key[j] != one);
+            });
+            if (__ballot(differs) != 0ull && lane == 0) s_differ = 1;
+            __syncthreads();
+            if (s_differ != 0) return false;
+            prefix = one;
+            return true;
         }, threshold, need_eq);
     }
 
@@ -511,10 +602,13 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         if (take < n_eq) ties = lowest_set(ties, take);
         word |= ties;
         int at = gt_at + (eq_at < need_eq ? eq_at : need_eq);
-        if constexpr (P <= 8) {
-            // few words with many entries each: every lane writes its own entry of each word
+        // Words of many entries are written by all lanes together, one word after the other; where the words outnumber the
+        // entries of the fullest, every lane writes its own word's.
+        const unsigned long long full = __ballot(word != 0ull);
+        if (P <= 8 || __ballot(__popcll(word) > __popcll(full)) != 0ull) {
 #pragma unroll
             for (int j = 0; j < P; ++j) {
+                if (P > 8 && !((full >> j) & 1ull)) continue;
                 const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)word, j);
                 const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(word >> 32), j);
                 const int place = __builtin_amdgcn_readlane(at, j) + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));

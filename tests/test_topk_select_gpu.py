@@ -58,6 +58,13 @@ def _rows(kind, n, gen):
         x = (x * 8).round() / 8
     elif kind == 'wide':         # forty octaves, the threshold far above the sampled pivot or below zero
         x = torch.exp2(x * 10) * torch.where(torch.rand(4, n, generator=gen) < 0.01, 1.0, -1.0)
+    elif kind == 'masked':       # fewer than k entries left above -inf
+        x[torch.rand(4, n, generator=gen) < 0.95] = float('-inf')
+        x[3] = torch.where(x[3] > 0, x[3], torch.full((), float('nan')))
+    elif kind == 'two':          # two values, among them one pair that shares its upper digits
+        x = (x > 0).float()
+        x[2] += 1.0 / 1024 * x[2] + 1.0
+        x[3] = x[3] * 2.0 ** -20 + 1.0
     elif kind == 'special':
         x[0, ::3] = float('nan')
         x[1, torch.rand(n, generator=gen) < 0.95] = float('-inf')
@@ -66,8 +73,8 @@ def _rows(kind, n, gen):
     return x
 
 
-@pytest.mark.parametrize('n', [8192, 8193, 16385, 32768, 32769, 65536, 65537, 98305, 262144, 262145])
-@pytest.mark.parametrize('kind', ['normal', 'clustered', 'distinct', 'wide', 'special'])
+@pytest.mark.parametrize('n', [600, 2500, 4096, 4097, 8192, 8193, 16385, 32768, 32769, 65536, 65537, 98305, 262144, 262145])
+@pytest.mark.parametrize('kind', ['normal', 'clustered', 'distinct', 'wide', 'special', 'masked', 'two'])
 def test_long_rows(capi, dev, n, kind):
     # edges of the row classes (in registers, read again, filtered or not), k at the limits of the candidate list
     gen = torch.Generator().manual_seed(n)
