@@ -188,9 +188,15 @@ def test_layer_narrow_tiles(capi, dev, shape):
     check_layer(capi, dev, T=T, H=H, I=I, E=E, k=k, seed=150 + T, config=NARROW_TILES)
 
 
+@pytest.mark.parametrize('T', [150, 421])
 @pytest.mark.parametrize('pow2', [0, 32])
-def test_layer_narrow_tiles_codes_of_the_streaming_form(capi, dev, pow2):
-    x, logits, w, dts = make_case(dev, 150, 512, 256, 12, 451)
+def test_layer_narrow_tiles_codes_of_the_streaming_form(capi, dev, pow2, T):
+    # T 421: an expert that every token takes (421 pairs, seven tiles) among experts of some 40 pairs and two of none
+    x, logits, w, dts = make_case(dev, T, 512, 256, 12, 451)
+    if T == 421:
+        dts[1][:, 3] += 30.0
+        dts[1][:, 0] -= 30.0
+        dts[1][:, 11] -= 30.0
     if pow2:
         for i in (3, 5):
             dts[i] = torch.exp2(torch.round(torch.log2(dts[i])))
@@ -199,6 +205,15 @@ def test_layer_narrow_tiles_codes_of_the_streaming_form(capi, dev, pow2):
     # sums of fp32 products in another order: codes differ only where fp32 does not decide them
     torch.testing.assert_close(va['h_s'], vb['h_s'], rtol=0 if pow2 else 1e-5, atol=0)
     assert (va['h_q'].view(torch.uint8) != vb['h_q'].view(torch.uint8)).float().mean().item() < 2e-4
+    if T == 421:
+        pairs = va['expert_offsets'].diff().tolist()
+        assert pairs[3] == 421 and pairs[0] == pairs[11] == 0
+        # down projection: y in fp16 with one scale per 256 columns above 32 pairs per expert, as in check_layer
+        # (an undecided code moves single elements of y further than that: the rows of equal codes)
+        same = (va['h_q'].view(torch.uint8) == vb['h_q'].view(torch.uint8)).all(dim=1)
+        assert same.float().mean().item() > 0.9
+        assert moe.rel_rms_error(va['y'][same].cpu(), vb['y'][same].cpu()) <= 3e-3
+        assert moe.rel_rms_error(a.cpu(), b.cpu()) <= TOL
 
 
 @pytest.mark.parametrize('seed', range(8))
