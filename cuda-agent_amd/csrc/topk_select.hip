@@ -429,22 +429,23 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
                         threshold = (uint32_t)s_bin;
                         need_eq = s_above;
                     } else {
-                        // Rows of few values have many equal keys there. (s_hist has been read: any of the bin's keys.)
+                        // Rows of few values have many equal keys there (not in the last bin, with everything beyond it).
+                        bool differs = tbin == (1 << SAMPLE_BITS) - 1;
+                        if (!differs) {
 #pragma unroll
-                        for (int r = 0; r < PER; ++r)
-                            if (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin) s_hist[0] = (int)lkey[r];
-                        __syncthreads();
-                        const uint32_t one = (uint32_t)s_hist[0];
-                        bool differs = false;
-#pragma unroll
-                        for (int r = 0; r < PER; ++r)
-                            differs = differs || (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin && lkey[r] != one);
-                        if (__ballot(differs) != 0ull && lane == 0) s_near_count = 1;
-                        __syncthreads();
-                        if (s_near_count == 0) {
-                            threshold = one;
+                            for (int r = 0; r < PER; ++r)
+                                if (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin) s_hist[0] = (int)lkey[r];
+                            __syncthreads();  // (the counts have been read: any of the bin's keys)
+                            threshold = (uint32_t)s_hist[0];
                             need_eq = want - tabove;
-                        } else {
+#pragma unroll
+                            for (int r = 0; r < PER; ++r)
+                                differs = differs || (lkey[r] != 0u && near_bin(lkey[r]) == (uint32_t)tbin && lkey[r] != threshold);
+                            if (__ballot(differs) != 0ull && lane == 0) s_near_count = 1;
+                            __syncthreads();
+                            differs = s_near_count != 0;
+                        }
+                        if (differs) {
                             radix_select(IntConstant<1>{}, [&](int* hist) {
 #pragma unroll
                                 for (int r = 0; r < PER; ++r)
