@@ -34,14 +34,14 @@ FP8_PEAK_TFLOPS = 5033.0
 METRIC = "GB/s & % HBM peak (GDN/MoE/MLA decode); fp8 TFLOP/s % MFMA peak (MoE prefill)"
 
 # HBM bytes per step (summed over the workload's kernels) from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, scaled
-# by the same counters read on a plain 512 MiB copy kernel (FETCH_SIZE x 1.99986, WRITE_SIZE x 1,
+# by the same counters read on a plain 512 MiB copy kernel (FETCH_SIZE x 1.99987, WRITE_SIZE x 1,
 # both in KiB); the counter summary is profiles/all_workloads_hbm_traffic_pmc.md, whose "HBM bytes" column
 # holds each of these figures (a test checks that). None = not measured.
 # Stamp: taken from the library as built from the sources of this tree; a change to a kernel's data movement needs
 # a new run of the two commands in that file.
-MEASURED_TRAFFIC = {'gdn': 1085858000, 'moe_decode': 10002073000, 'mla': 238270000, 'index_scores': 553927000,
-                    'index_scores_fp8': 289777000, 'moe_prefill': 22426952000, 'mla_fp8_cache': 187610000,
-                    'topk_select': 9216000}
+MEASURED_TRAFFIC = {'gdn': 1085893000, 'moe_decode': 10002073000, 'mla': 238309000, 'index_scores': 553900000,
+                    'index_scores_fp8': 289712000, 'moe_prefill': 22387278000, 'mla_fp8_cache': 187647000,
+                    'topk_select': 9163000}
 # Matrix-pipe occupancy of the dominant kernels from rocprofv3 --pmc (SQ_VALU_MFMA_BUSY_CYCLES over 1024 SIMDs x
 # GRBM_GUI_ACTIVE cycles per XCD, the timed launches of bench.py's own loop; the derived MfmaUtil counter reads
 # 33.3 / 33.7 / 23.5 %) and the clock by GRBM_GUI_ACTIVE / 8 / duration in the same run (SQ_BUSY_CU_CYCLES / 256 /

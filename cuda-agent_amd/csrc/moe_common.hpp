@@ -36,7 +36,8 @@ constexpr int CONFIG_LAST_EXPERT_FIRST = 128;
 //  * The streaming gate/up GEMM (few pairs per expert, bound by the weight stream) converts the codes to bf16
 //    in registers and uses the bf16 matrix core, whose sums are exact to fp32 accuracy: its h agrees with an
 //    fp32 evaluation. CONFIG_APPROX_REQUANT puts it on the e4m3 matrix core.
-//  * The tiled gate/up GEMM (many pairs per expert, bound by the matrix core):
+//  * The gate/up GEMM in narrow tiles (moe_gemm_narrow.hip) does the same, and has no other form.
+//  * The gate/up GEMM in 256-pair tiles (many pairs per expert, bound by the matrix core):
 //      default: e4m3 matrix core, and the epilogue repairs the codes that matter. It marks every element whose
 //        scaled magnitude reaches 2^s code units (s = bits 12-15; 0: default_requant_significance, which is 7 at
 //        the sizes this form is meant for: 128 of 448, i.e. the two highest binades, where one code step is 16 or
@@ -45,7 +46,7 @@ constexpr int CONFIG_LAST_EXPERT_FIRST = 128;
 //        plain dot products; the group's scale then comes from the exact maximum and the marked codes from
 //        the exact values. Smaller elements keep the matrix core's code (a step of at most 8 units there).
 //      CONFIG_EXACT_REQUANT: bf16 matrix core (twice the matrix-core time): every code as an fp32
-//        evaluation gives it, as in the streaming form.
+//        evaluation gives it, as in the two forms above.
 //      CONFIG_APPROX_REQUANT: e4m3 matrix core, codes as they come.
 //    Bits 10-11 scale the width of the band: 0 the default, 1 half, 2 twice, 3 four times as wide.
 constexpr int CONFIG_EXACT_REQUANT = 256;
@@ -212,11 +213,12 @@ struct Workspace {
     float* x_s;           // [T*H/128]
     uint8_t* h_q;         // [T*k*I] e4m3 silu(g)*u, rows in sorted order
     float* h_s;           // [T*k*I/128]
-    float* y;             // [T*k*H] expert outputs, rows in sorted order: fp32 from the streaming down GEMM; from
-                          //         the tiled one fp16 of y / y_scale in the first half of the buffer
-    float* y_scale;       // [T*k][H/256] power of two above the largest |y| of each run of 256 columns (tiled)
-    int* tile_start;      // [2E+1] first 256-pair tile of every slot of the dispatch order, then the slots' experts
-                          //        (tiled path)
+    float* y;             // [T*k*H] expert outputs, rows in sorted order: fp32 from the streaming down GEMM and from
+                          //         narrow tiles of up to 32 pairs per expert; else, from narrow and from 256-pair tiles,
+                          //         fp16 of y / y_scale in the first half of the buffer
+    float* y_scale;       // [T*k][H/256] power of two above the largest |y| of each run of 256 columns (with fp16 y)
+    int* tile_start;      // [2E+1] first tile (256 pairs; narrow: up to 62) of every slot of the dispatch order, then the
+                          //        slots' experts (both tiled forms)
     float* xs_t;          // [H/128][scale_stride] activation scales by sorted position, transposed
     float* hs_t;          // [I/128][scale_stride] the same for h
     int scale_stride;     // pairs rounded up to 256, plus 256 of padding

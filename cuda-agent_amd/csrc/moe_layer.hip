@@ -238,8 +238,8 @@ GemmPlan plan_expert_gemms(int tokens, int hidden, int inter, int n_experts, int
     GemmPlan plan{};
     plan.y_half = form == 16 || ((form == 0 || form == CONFIG_NARROW_TILES) && pairs > 32L * n_experts && tiled_ok);
     plan.form = plan.y_half ? GemmPlan::TILED : GemmPlan::STREAMING;
-    // Narrow tiles from 10 pairs per expert (256 experts of 7168 x 2048, 8 pairs: 1.73 ms streaming, 1.77 narrow; 12:
-    // 1.84, 1.79; 16: 2.36, 1.82; 31: 2.61, 1.92) to where an expert's second tile, and with it its weights through L2
+    // Narrow tiles from 10 pairs per expert (256 experts of 7168 x 2048, 8 pairs: 1.72 ms streaming, 1.75 narrow; 10:
+    // 1.75, 1.77; 12: 1.81, 1.78; 16: 1.83, 1.80; 31: 2.48, 1.90; streaming by the faster of 16 and 32 pairs to a pass) to where an expert's second tile, and with it its weights through L2
     // once more, costs what a 256-pair tile loses while it starts and ends. That is the share of a tile's K blocks, of
     // either GEMM: 7168 x 2048 (56 blocks) 47 pairs 2.34 ms tiled, 2.00 narrow; 53: 2.36, 2.09; 64: 2.41, 2.54; 4096 x
     // 1536 (32) 94: 0.428, 0.385; 106: 0.436, 0.414; 128: 0.462 both; 2048 x 768 (16) 128: 0.350, 0.318; 192: 0.399, 0.413;

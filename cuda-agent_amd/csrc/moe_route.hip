@@ -438,7 +438,7 @@ __global__ __launch_bounds__(1024) void moe_route_sort_small_kernel(
     }
     __syncthreads();
     // Stable rank of every pair inside its expert without walking the earlier pairs: the rank among
-    // the 64 pairs of the wavefront (lane compares), plus the expert's pairs in earlier wavefronts
+    // the 64 pairs of the wavefront (group_rank), plus the expert's pairs in earlier wavefronts
     // (a 16 x experts table, prefix-summed per expert).
     const int p = threadIdx.x;
     const int mine = p < pairs ? s_ids[p] : -1;

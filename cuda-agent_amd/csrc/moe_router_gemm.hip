@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
 // early: global -> LDS loads into a ring of three stages, two of them in flight, and the operands of chunk c+1 are read
 // into registers while the 24 MFMAs (768 cycles) of chunk c run. With one stage in flight through registers and the
 // operand reads in front of the MFMAs a chunk took 2600 cycles (137 us for the 8192 x 256 logits
-// of hidden 7168); this takes 83 us, 1.1 PFLOP/s of bf16 products. With K split it also serves fewer tokens: 4096 tokens
+// of hidden 7168); this takes 83 us, 1.1 PFLOP/s of bf16 products (with the norm's output of that
+// moment still to be written back, as in a layer, 87 to 98). With K split it also serves fewer tokens: 4096 tokens
 // 86 us on the per-wavefront kernel, 49 here; 1000: 27.7 and 21.9; 200: 15.5 and 13.2, the reduction included.
 constexpr int BIG_TOKENS = 128;
 constexpr int BIG_EXPERTS = 64;

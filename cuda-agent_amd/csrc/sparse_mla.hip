@@ -28,9 +28,13 @@
 // the splits and converts to bf16.
 //
 // Two split kernels share this data path. sparse_mla_split_kernel<NW> is the form described
-// above (one wavefront per 32 heads; used for 32 and 64 heads and for caches of 4 GB and more
-// per request). sparse_mla_split8_kernel, further down, is the default: two wavefronts per 32 heads
-// that split Q by d and the accumulator by dv.
+// above (one wavefront per 32 heads; used for caches of 4 GB and more per addressed block and with
+// config >= 1000). sparse_mla_split8_kernel, further down, is the default for 32, 64 and 128 heads: two
+// wavefronts per 32 heads that split Q by d and the accumulator by dv.
+//
+// Error against a float64 evaluation of the same rows, as rms relative to that of the output: 4.7e-4 (64 splits of 32 rows) to 8.6e-4
+// (one split of 300 rows). The probabilities are rounded to bf16 except the largest of a split, which is exactly 1: more
+// splits have more exact ones (24 requests of 2048 rows, 11 splits 6.1e-4, 8 splits 6.5e-4).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -1491,7 +1495,7 @@ extern "C" void sparse_mla_decode_static_launcher(void* out, const void* q, cons
                       sm_scale, out_dtype, config, kva, stream);
 }
 
-// Decode over a cache in the 656-byte e4m3 form with the dequantisation inside the 128-head kernel (see
+// Decode over a cache in the 656-byte e4m3 form with the dequantisation inside the split kernel of 32, 64 and 128 heads (see
 // gather_quarter_fp8 / dequant_quarter). Internal to the library: mla_fp8_cache.hip calls it from
 // sparse_mla_decode_fp8_launcher and its paged form; it is not part of the public header. Returns 1 if the launch was made (or rejected with a status), 0 if
 // this shape has to take the two-step form of sparse_mla_decode_fp8_launcher: config >= 1000, caches of 4 GB and more per addressed block.
