@@ -1,10 +1,14 @@
-// Addressing of a latent cache shared by the sparse-MLA kernels: contiguous per request, one pool of
-// rows, or a pool of pages behind a block table.
+// What the sparse-MLA launchers share: the addressing of a latent cache (contiguous per request, one pool of
+// rows, or a pool of pages behind a block table) and the reading of their config.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
 namespace mla {
+
+// config 2^20 + n: config n, on workgroups of 64 heads. Any other value has no such bit.
+inline bool halves_asked(int config) { return config >> 20 == 1; }
+inline int without_halves(int config) { return halves_asked(config) ? config & 0xfffff : config; }
 
 // Where the rows of a request live. Without a block table a request's rows are
 // kv + (b * batch_rows + key) * row bytes (batch_rows == 0: one pool shared by all requests,

@@ -194,7 +194,7 @@ extern "C" void mla_latent_quant_launcher(void* cache, const void* kv, long rows
 // compact block of dequantised rows and its index list
 extern "C" size_t sparse_mla_decode_fp8_workspace_bytes(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
-    if ((config & 0xfffff) >= 5000) config -= 5000;
+    if (mla::without_halves(config) >= 5000) config -= 5000;
     return align16(sparse_mla_decode_workspace_bytes(batch, n_heads, topk, config)) +
            align16((size_t)batch * topk * ROW_BF16_BYTES) + align16((size_t)batch * topk * sizeof(int));
 }
@@ -221,7 +221,7 @@ void launch_decode_fp8(void* out, const void* q, const void* kv_fp8, const int* 
     }
     // config 5000 + n: the two-step form (gather + dequantise into the workspace, then the bf16 kernels) with
     // config n; otherwise the 8-wavefront kernel dequantises its tiles itself where the shape allows
-    const bool two_step = (config & 0xfffff) >= 5000;
+    const bool two_step = mla::without_halves(config) >= 5000;
     if (two_step) config -= 5000;
     const size_t base_bytes = align16(sparse_mla_decode_workspace_bytes(batch, n_heads, topk, config));
     if (!two_step &&

@@ -1285,9 +1285,6 @@ Pick pick_launch(int batch, int head_groups, int topk, int config, bool few_on_o
 
 namespace {
 
-// config bit: with a number of splits in the lower bits, 64 heads a workgroup
-constexpr int HALVES_SHIFT = 20;
-
 int head_groups_of(int n_heads) { return n_heads <= 128 ? 1 : n_heads / 128; }
 
 }  // namespace
@@ -1295,15 +1292,15 @@ int head_groups_of(int n_heads) { return n_heads <= 128 ? 1 : n_heads / 128; }
 // config 1000 + n: n splits on the kernel with one wavefront per 32 heads
 extern "C" int sparse_mla_decode_num_splits(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
-    config &= (1 << HALVES_SHIFT) - 1;
+    config = mla::without_halves(config);
     return pick_launch(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config,
-                       config >= 1000 && n_heads < 128, config == 0 && n_heads >= 128).splits;
+                       config >= 1000 && n_heads < 128, config <= 0 && n_heads >= 128).splits;
 }
 
 // bytes of scratch sparse_mla_decode_launcher needs for these sizes
 extern "C" size_t sparse_mla_decode_workspace_bytes(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
-    config &= (1 << HALVES_SHIFT) - 1;
+    config = mla::without_halves(config);
     const int splits = max_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config);
     // partial outputs (sized for fp32), log-sum-exp and scale of every (request, split, head)
     return (size_t)batch * splits * n_heads * (D_V + 2) * sizeof(float);
@@ -1339,8 +1336,8 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     }
     // config >= 1000: the kernel with one wavefront per 32 heads (config - 1000 is then the split count)
     // The 8-wavefront kernel addresses a request's cache block with 32-bit byte offsets.
-    const bool halves_asked = config >> HALVES_SHIFT == 1;
-    config &= (1 << HALVES_SHIFT) - 1;
+    const bool halves_asked = mla::halves_asked(config);
+    config = mla::without_halves(config);
     const bool one_wave_per_group =
         config >= 1000 ||
         (unsigned long long)n_kv_rows * (fp8_cache ? FP8_ROW_BYTES : ROW_BYTES) >= 0xffffffffull;
@@ -1542,7 +1539,7 @@ extern "C" int sparse_mla_decode_fp8_fused(void* out, const void* q, const void*
                                            int out_dtype, int config, const int* block_table,
                                            int table_stride, int page_shift, int batch_rows,
                                            hipStream_t stream) {
-    if (n_heads <= 0 || (n_heads % 128 != 0 && n_heads != 32 && n_heads != 64) || (config & ((1 << HALVES_SHIFT) - 1)) >= 1000 || n_kv_rows <= 0 ||
+    if (n_heads <= 0 || (n_heads % 128 != 0 && n_heads != 32 && n_heads != 64) || mla::without_halves(config) >= 1000 || n_kv_rows <= 0 ||
         (unsigned long long)n_kv_rows * FP8_ROW_BYTES >= 0xffffffffull)
         return 0;
     const KvAddressing kva{block_table, table_stride, page_shift, batch_rows};

@@ -84,6 +84,18 @@ def test_rejected_launch_sets_status_without_touching_the_gpu(capi):
     assert lib.cuda_agent_amd_last_status() == 0
 
 
+@pytest.mark.parametrize('batch,heads,topk', [(1, 128, 2048), (24, 128, 2048), (8, 64, 300), (3, 256, 100)])
+def test_sparse_mla_configs_that_name_no_splits(capi, batch, heads, topk):
+    # a negative config chooses as 0 does, and only 2^20 + n carries the bit for workgroups of 64 heads
+    lib = capi.library()
+    sizes = (lib.sparse_mla_decode_num_splits, lib.sparse_mla_decode_workspace_bytes, lib.sparse_mla_decode_fp8_workspace_bytes)
+    for size in sizes:
+        for config in (-1, -5000, -2 ** 31):
+            assert size(batch, heads, topk, config) == size(batch, heads, topk, 0)
+        assert size(batch, heads, topk, (1 << 20) + 3) == size(batch, heads, topk, 3)
+        assert size(batch, heads, topk, (1 << 21) + 3) == size(batch, heads, topk, 4999)     # as many splits as there are tiles
+
+
 @pytest.mark.parametrize('rel', INFRA)
 def test_workspaces_share_identical_infrastructure(rel):
     blobs = {(PKG / 'workspaces' / w / rel).read_bytes() for w in WORKSPACES}
