@@ -72,9 +72,9 @@ class Arg {
 
 int integer(PyObject* object) {
     need(PyLong_CheckExact(object));
-    const long v = PyLong_AsLong(object);
-    if (v == -1 && PyErr_Occurred()) PyErr_Clear();
-    need(v >= INT_MIN && v <= INT_MAX);
+    int overflow;
+    const long v = PyLong_AsLongAndOverflow(object, &overflow);
+    need(overflow == 0 && v >= INT_MIN && v <= INT_MAX);
     return (int)v;
 }
 
