@@ -267,3 +267,18 @@ def test_numbers_beyond_int_are_declined(stub):
     for config in (2 ** 31, -2 ** 31 - 1, 2 ** 63, -2 ** 63 - 1, 2 ** 70):
         assert native.gdn_decode(*args[:7], config, None) == -1
     assert native.gdn_decode(*args[:7], -1, None) == 0
+
+
+def test_the_helpers_serve_calls_without_the_native_checks(stub, monkeypatch, tmp_path):
+    # only the C-ABI library built: every call goes through the checks in Python
+    from cuda_agent_amd import capi
+    _, library = stub
+    monkeypatch.setattr(capi, 'library', lambda: library)
+    monkeypatch.setattr(capi, '_stream', lambda stream=None: 0)
+    monkeypatch.setattr(capi, '_device_contiguous', lambda **tensors: None)
+    monkeypatch.setattr(capi, 'LAUNCH_CHECKS', tmp_path / 'launch_checks.so')
+    monkeypatch.setattr(capi, '_native', capi._LoadedOnFirstUse())
+    for _ in range(2):
+        library.forget()
+        capi.gdn_decode_launch(*ordinary_calls()['gdn_decode_launch'][0])
+        assert library.recorded().startswith(b'gdn_decode_launcher')
