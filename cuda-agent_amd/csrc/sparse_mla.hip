@@ -1224,18 +1224,6 @@ int max_splits(int batch, int head_groups, int topk, int config) {
     return splits;
 }
 
-// The same with 64 heads a workgroup, over e4m3 rows (bf16 rows take 0.3 us less per tile).
-float split_half_kernel_us(int wgs, int tiles) {
-    auto round_us = [&](int n) { return 7.7f + 0.0125f * n + (1.4f + 0.0022f * n) * tiles; };
-    return (wgs / 256) * round_us(256) + (wgs % 256 ? round_us(wgs % 256) : 0.f);
-}
-
-// What a launch takes: `splits`, and whether a workgroup of the 8-wavefront kernel has 64 heads instead of 128.
-struct Pick {
-    int splits;
-    bool halves;
-};
-
 // The splits of a launch: config if it asks for a number, else the one with the least time for the split kernel and
 // the merge (5 us and 16 ns per partial of 128 heads; none for a single split). The maximum above puts a few
 // workgroups into a second round whenever the number of requests is not a divisor of 256: with it 24 requests of 2048
@@ -1247,38 +1235,38 @@ struct Pick {
 // leave a quarter of the partials, so that start and merge hardly count: as many splits of equal size as fit the CUs in
 // one round (64 heads, 16 requests of 2048 rows: 59 us with 16 splits, 67 with the model's 13; 24: 90 with 8 to 10, 129 with
 // 11, which is more than one round). For 128 heads on it the model is the better one (24 requests 62 us, with 10 splits 68).
-// may_halve (128 heads and more on the 8-wavefront kernel): workgroups of 64 heads, twice as many, which take 1.3 to 2 us a
-// tile, have half the Q to fetch and half the partials to store, and let a request have fewer splits; they fetch the rows
-// twice, through one L2. Where the model makes that 5 % less (us, 128 and 64 heads a workgroup, bf16 and e4m3 rows: 1 request
-// of 2048 rows 18.1, 16.7 and 18.5, 17.2; 8 24.6, 22.4 and 24.6, 23.3; 128 of 512 45.7, 37.1 and 47.3, 42.3; with more tiles
-// than that e4m3 rows, which both workgroups then convert, decide: 24 of 2048 37.4, 36.2 but 38.9, 41.9; and both forms of
-// the cache keep the same splits, so that they give the same bits). 32 heads a workgroup were never more than 0.3 us better.
-// A head's result does not depend on it; with fewer splits the error of the fp32 output against float64 is that of fewer splits:
-// 5.59e-4 with 22, 5.86e-4 with 16 (8 requests of 2048 rows); of the bf16 output 1.75e-3, 1.76e-3.
-Pick pick_launch(int batch, int head_groups, int topk, int config, bool few_on_one_wave, bool may_halve) {
+int pick_splits(int batch, int head_groups, int topk, int config, bool few_on_one_wave) {
     const int most = max_splits(batch, head_groups, topk, config);
-    if (config > 0) return {most, false};
+    if (config > 0) return most;
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int wgs = batch * head_groups;
     constexpr int MOST_TILES = MAX_SPLIT_ROWS / TILE_ROWS;  // of a split
     if (few_on_one_wave) {
         const int fit = 256 / wgs < 1 ? 1 : 256 / wgs < tiles ? 256 / wgs : tiles;
         const int per = (tiles + fit - 1) / fit < MOST_TILES ? (tiles + fit - 1) / fit : MOST_TILES;
-        return {(tiles + per - 1) / per, false};
+        return (tiles + per - 1) / per;
     }
-    int best = most, best_half = most;
-    float best_us = 0.f, best_half_us = 0.f;
+    int best = most;
+    float best_us = 0.f;
     for (int per = MOST_TILES < tiles ? MOST_TILES : tiles; per >= 1; --per) {
         const int splits = (tiles + per - 1) / per;  // of `per` tiles each
         if (splits > most) break;
-        const float merge_us = splits > 1 ? 5.f + 0.016f * wgs * splits : 0.f;
-        const float us = split_kernel_us(wgs * splits, per) + merge_us;
+        const float us = split_kernel_us(wgs * splits, per) + (splits > 1 ? 5.f + 0.016f * wgs * splits : 0.f);
         if (best_us == 0.f || us < best_us) best_us = us, best = splits;
-        const float half_us = split_half_kernel_us(2 * wgs * splits, per) + merge_us;
-        if (best_half_us == 0.f || half_us < best_half_us) best_half_us = half_us, best_half = splits;
     }
-    if (may_halve && best_half_us < 0.95f * best_us) return {best_half, true};
-    return {best, false};
+    return best;
+}
+
+// Whether the 8-wavefront kernel takes 128 heads and more in workgroups of 64, twice as many: where these fit the CUs in one
+// round. They take 1.3 to 2 us a tile instead of 2.4 to 3 and have half the Q to fetch, but fetch the rows twice, through one
+// L2. us, 128 and 64 heads a workgroup, bf16 and e4m3 rows: 1 request of 2048 rows 18.0, 16.6 and 18.4, 16.9; 4 24.4, 23.1 and
+// 24.5, 23.2; 16 of 256 17.1, 15.1 and 17.5, 15.2; 128 of 64 15.6, 13.7 and 15.8, 13.7; with 264 workgroups, 6 of 2048, 27.4,
+// 33.4 and 28.2, 34.0; with 300, 150 of 64, 15.8, 24.7 and 16.0, 24.2. 32 heads a workgroup were never more than 0.3 us better.
+// The splits are those of 128 heads either way, and a head's result does not depend on its workgroup: with fewer splits, which
+// would suit the smaller workgroups, the error against float64 is larger (of the fp32 output, 8 requests of 2048 rows: 5.59e-4
+// with 22, 5.86e-4 with 16).
+bool takes_halves(int batch, int head_groups, int splits, int config) {
+    return config <= 0 && 2L * batch * head_groups * splits <= 256;
 }
 
 }  // namespace
@@ -1293,8 +1281,8 @@ int head_groups_of(int n_heads) { return n_heads <= 128 ? 1 : n_heads / 128; }
 extern "C" int sparse_mla_decode_num_splits(int batch, int n_heads, int topk, int config) {
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
     config = mla::without_halves(config);
-    return pick_launch(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config,
-                       config >= 1000 && n_heads < 128, config <= 0 && n_heads >= 128).splits;
+    return pick_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config,
+                       config >= 1000 && n_heads < 128);
 }
 
 // bytes of scratch sparse_mla_decode_launcher needs for these sizes
@@ -1343,9 +1331,7 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
         (unsigned long long)n_kv_rows * (fp8_cache ? FP8_ROW_BYTES : ROW_BYTES) >= 0xffffffffull;
     if (config >= 1000) config -= 1000;
     const int head_groups = head_groups_of(n_heads);
-    const Pick pick = pick_launch(batch, head_groups, topk, config, one_wave_per_group && n_heads < 128,
-                                  !one_wave_per_group && n_heads >= 128);
-    const int splits = pick.splits;
+    const int splits = pick_splits(batch, head_groups, topk, config, one_wave_per_group && n_heads < 128);
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int rows_per_split = ((tiles + splits - 1) / splits) * TILE_ROWS;
     float* o_part = static_cast<float*>(workspace);
@@ -1355,7 +1341,7 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     const __bf16* qb = static_cast<const __bf16*>(q);
     const __bf16* kvb = static_cast<const __bf16*>(kv);
     const dim3 grid(splits, batch, head_groups);
-    const bool halves = n_heads >= 128 && (pick.halves || halves_asked);
+    const bool halves = n_heads >= 128 && (halves_asked || takes_halves(batch, head_groups, splits, config));
     const dim3 grid8(splits, batch, halves ? 2 * head_groups : head_groups);
     const int group_heads = halves ? 64 : n_heads < 128 ? n_heads : 128;
     bool half_parts = false;

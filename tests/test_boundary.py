@@ -96,6 +96,14 @@ def test_sparse_mla_configs_that_name_no_splits(capi, batch, heads, topk):
         assert size(batch, heads, topk, (1 << 21) + 3) == size(batch, heads, topk, 4999)     # as many splits as there are tiles
 
 
+@pytest.mark.parametrize('batch,heads,topk,splits', [
+    (1, 128, 2048, 64), (6, 128, 2048, 22), (8, 128, 2048, 22), (24, 128, 512, 6), (32, 128, 256, 4), (48, 128, 256, 3),
+    (128, 128, 512, 2), (12, 128, 128, 4), (1, 128, 100, 4), (16, 128, 1024, 11), (4, 256, 2048, 22), (256, 128, 2048, 1)])
+def test_sparse_mla_splits_are_those_of_workgroups_of_128_heads(capi, batch, heads, topk, splits):
+    # (the error of the result grows where there are fewer)
+    assert capi.library().sparse_mla_decode_num_splits(batch, heads, topk, 0) == splits
+
+
 @pytest.mark.parametrize('rel', INFRA)
 def test_workspaces_share_identical_infrastructure(rel):
     blobs = {(PKG / 'workspaces' / w / rel).read_bytes() for w in WORKSPACES}

@@ -161,3 +161,6 @@ def test_workgroups_of_64_heads_give_the_same_bits(capi, dev, B, H, topk, splits
         whole = run(capi, dev, q, rows, idx, torch.float32, config=splits)
         assert torch.isfinite(whole).all()
         assert torch.equal(run(capi, dev, q, rows, idx, torch.float32, config=(1 << 20) + splits), whole)
+        # (the launcher's own choice of the workgroups)
+        chosen = capi.library().sparse_mla_decode_num_splits(B, H, topk, 0)
+        assert torch.equal(run(capi, dev, q, rows, idx, torch.float32), run(capi, dev, q, rows, idx, torch.float32, config=chosen))
