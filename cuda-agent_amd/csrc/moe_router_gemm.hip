@@ -61,6 +61,36 @@ __device__ __forceinline__ void load32(float (&dst)[32], const uint16_t* p) {  /
     }
 }
 
+// Sums of chunks [chunk_begin, chunk_end) for 32 tokens x 32 experts on the fp32 matrix cores: lane (row, half) has the
+// `half` 32 values of a chunk of its token's and of its expert's row, from xp and wp on. Register i of a lane: token
+// 8*(i/4) + 4*half + i%4, expert `row`.
+template <typename X>
+__device__ __forceinline__ floatx16 fp32_tile(const X* __restrict__ xp, const float* __restrict__ wp, int chunk_begin,
+                                              int chunk_end) {
+    floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // two register sets: the loads of chunk c+1 are in flight while the MFMAs of chunk c run
+    float a0[32], b0[32], a1[32], b1[32];
+    if (chunk_begin < chunk_end) {
+        load32(a0, xp + (size_t)chunk_begin * K_CHUNK);
+        load32(b0, wp + (size_t)chunk_begin * K_CHUNK);
+    }
+    for (int c = chunk_begin; c < chunk_end; c += 2) {
+        // (past the end the last chunk is read again and not used)
+        const int c1 = c + 1 < chunk_end ? c + 1 : c;
+        load32(a1, xp + (size_t)c1 * K_CHUNK);
+        load32(b1, wp + (size_t)c1 * K_CHUNK);
+#pragma unroll
+        for (int s = 0; s < 32; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b0[s], acc, 0, 0, 0);
+        if (c + 1 >= chunk_end) break;
+        const int c2 = c + 2 < chunk_end ? c + 2 : c + 1;
+        load32(a0, xp + (size_t)c2 * K_CHUNK);
+        load32(b0, wp + (size_t)c2 * K_CHUNK);
+#pragma unroll
+        for (int s = 0; s < 32; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b1[s], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
 // grid: x = 64-token tiles, y = 64-expert tiles, z = K split. out is logits (n_splits == 1) or
 // the partial sums [split][tokens][n_experts].
 template <typename X>
@@ -83,30 +113,7 @@ __global__ __launch_bounds__(256) void moe_router_gemm_kernel(const X* __restric
     int chunk_end = chunk_begin + chunks_per_split;
     const int n_chunks = hidden / K_CHUNK;
     if (chunk_end > n_chunks) chunk_end = n_chunks;
-    const X* xp = x + (size_t)t * hidden + 32 * half;
-    const float* wp = w + (size_t)e * hidden + 32 * half;
-
-    floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // two register sets: the loads of chunk c+1 are in flight while the MFMAs of chunk c run
-    float a0[32], b0[32], a1[32], b1[32];
-    if (chunk_begin < chunk_end) {
-        load32(a0, xp + (size_t)chunk_begin * K_CHUNK);
-        load32(b0, wp + (size_t)chunk_begin * K_CHUNK);
-    }
-    for (int c = chunk_begin; c < chunk_end; c += 2) {
-        // (past the end the last chunk is read again and not used)
-        const int c1 = c + 1 < chunk_end ? c + 1 : c;
-        load32(a1, xp + (size_t)c1 * K_CHUNK);
-        load32(b1, wp + (size_t)c1 * K_CHUNK);
-#pragma unroll
-        for (int s = 0; s < 32; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b0[s], acc, 0, 0, 0);
-        if (c + 1 >= chunk_end) break;
-        const int c2 = c + 2 < chunk_end ? c + 2 : c + 1;
-        load32(a0, xp + (size_t)c2 * K_CHUNK);
-        load32(b0, wp + (size_t)c2 * K_CHUNK);
-#pragma unroll
-        for (int s = 0; s < 32; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b1[s], acc, 0, 0, 0);
-    }
+    const floatx16 acc = fp32_tile(x + (size_t)t * hidden + 32 * half, w + (size_t)e * hidden + 32 * half, chunk_begin, chunk_end);
     // result register i of a lane: token 8*(i/4) + 4*half + i%4 of the tile, expert `row`
     float* dst = out + (size_t)blockIdx.z * tokens * n_experts;
     if (e0 + row < n_experts) {
@@ -397,9 +404,10 @@ struct LongTile {
     static constexpr int LOADS = STAGE / 1024 / 4;  // load instructions of a wavefront per stage (half of them fill one)
 };
 
-// The matrix core takes a bf16 number below 2^-126 for zero: the parts of a weight from 2^-102 on are above it.
-// Magnitudes as doubled bit patterns less one, which puts zero above all others.
-constexpr uint32_t SPLIT_SMALLEST = ((127u - 102u) << 24) - 1u;
+// The last bit of a bf16 number is 2^-133 at the least (the matrix core takes subnormal ones as they are), and that of a
+// weight from 2^-110 on, so that its three parts are the weight. Magnitudes as doubled bit patterns less one, which puts zero
+// above all others.
+constexpr uint32_t SPLIT_SMALLEST = ((127u - 110u) << 24) - 1u;
 
 // 8 consecutive values of fp32 weights as three operands (see moe_router_split_kernel); the smallest magnitude among
 // them goes into `smallest`
@@ -428,6 +436,7 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
                                                                       int chunks_per_split) {
     typedef LongTile T;
     __shared__ __attribute__((aligned(16))) uint8_t s_stage[4 * 32 * 1024 > T::STAGES * T::STAGE ? 4 * 32 * 1024 : T::STAGES * T::STAGE];
+    __shared__ int s_small[BIG_EXPERTS];  // whether an expert has a weight that is not the sum of its parts
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 31;
@@ -473,7 +482,8 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
     typedef const __attribute__((address_space(3))) floatx4* lds_floatx4;
     bf16x8 a[4], b[2][3];
     floatx4 raw[2][2];
-    uint32_t smallest = 0xffffffffu;
+    uint32_t smallest[2] = {0xffffffffu, 0xffffffffu};  // of this lane's experts
+    if (threadIdx.x < BIG_EXPERTS) s_small[threadIdx.x] = 0;
     floatx16 acc[4][2];
 #pragma unroll
     for (int m = 0; m < 4; ++m)
@@ -482,7 +492,7 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
             acc[m][g] = floatx16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // the 12 products of 32 experts, smallest terms first
     auto products = [&](int g) {
-        split_weights(b[g], raw[g], smallest);
+        split_weights(b[g], raw[g], smallest[g]);
 #pragma unroll
         for (int p = 2; p >= 0; --p)
 #pragma unroll
@@ -532,7 +542,12 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
         const floatx16& v = acc[q / 8][q / 4 % 2];
         return floatx4{v[4 * (q & 3)], v[4 * (q & 3) + 1], v[4 * (q & 3) + 2], v[4 * (q & 3) + 3]};
     };
-    const bool plain_sums = __syncthreads_or(smallest < SPLIT_SMALLEST);  // (no weight of a model's is that small)
+    const bool small = __syncthreads_or(min(smallest[0], smallest[1]) < SPLIT_SMALLEST);
+    if (small) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+            if (smallest[g] < SPLIT_SMALLEST) s_small[32 * g + row] = 1;
+    }
     if (parity == 1) {
 #pragma unroll
         for (int q = 0; q < 32; ++q) tile[q * 64] = quad(q);
@@ -548,28 +563,57 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
     __syncthreads();
     float* dst = out + (size_t)blockIdx.z * tokens * n_experts;
     const floatx4* sums = reinterpret_cast<const floatx4*>(s_stage) + lane;
+    // (quads 4*wave + [0, 4): 32 tokens x 32 experts)
+    const int tile_t0 = t0 + 32 * (wave / 2), tile_e0 = e0 + 32 * (wave % 2);
+    const int e = tile_e0 + row;
+    float v[16];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int q = 4 * wave + k;
-        floatx4 v = (sums[q * 64] + sums[2048 + q * 64]) + (sums[4096 + q * 64] + sums[6144 + q * 64]);
-        const int e = e0 + 32 * (q / 4 % 2) + row;
-        const int t = t0 + 32 * (q / 8) + 8 * (q & 3) + 4 * half;
-        if (e < n_experts) {
+        const floatx4 sum = (sums[q * 64] + sums[2048 + q * 64]) + (sums[4096 + q * 64] + sums[6144 + q * 64]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (t + i >= tokens) continue;
-                // An infinite weight leaves infinity - infinity behind, and an infinite x times a part that is zero is
-                // no number either: where the sum is none, it is formed from the values themselves.
-                if (v[i] != v[i] || plain_sums) {
-                    float sum = 0.f;
-#pragma unroll 8
-                    for (int h = chunk_begin * K_CHUNK; h < (chunk_begin + n) * K_CHUNK; ++h)
-                        sum = fmaf(__uint_as_float((uint32_t)x[(size_t)(t + i) * hidden + h] << 16), w[(size_t)e * hidden + h], sum);
-                    v[i] = sum;
+        for (int i = 0; i < 4; ++i) v[4 * k + i] = sum[i];
+    }
+    auto token_of = [&](int i) { return tile_t0 + 8 * (i / 4) + 4 * half + i % 4; };
+    // What the three products don't give is taken from the fp32 matrix cores, as a tile of moe_router_gemm_kernel: the sums of
+    // an expert with too small a weight, and sums that are no number. (An infinite weight leaves infinity - infinity
+    // behind, and an infinite x times a part that is zero is no number either.)
+    // us, 8192 tokens of 7168 x 256, 85 as a rule: with one weight of 2^-120 420, with an infinity in one token 261, with a
+    // NaN in one token 86, in all of them 240 (the fp32 matrix cores for all sums: 400).
+    uint32_t again = 0;  // bit i: v[i]
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        if (e < n_experts && token_of(i) < tokens && v[i] != v[i]) again |= 1u << i;
+    if (__ballot(again != 0) != 0) {
+        // ... but a token whose own values hold a NaN, as those of padding may, keeps it
+        const uint16_t* x_part = x + (size_t)chunk_begin * K_CHUNK + lane * 8;
+        for (int i = 0; i < 16; ++i) {
+            const uint64_t lanes = __ballot(again >> i & 1);
+            for (int h = 0; h < 2; ++h) {
+                if ((uint32_t)(lanes >> (32 * h)) == 0) continue;
+                const uint16_t* at = x_part + (size_t)(tile_t0 + 8 * (i / 4) + 4 * h + i % 4) * hidden;
+                bool nan = false;
+                for (int c = lane * 8; c < n * K_CHUNK; c += 512, at += 512) {
+                    const u32x4 pairs = *reinterpret_cast<const u32x4*>(at);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        nan |= (pairs[j] & 0x7fffu) > 0x7f80u || (pairs[j] & 0x7fff0000u) > 0x7f800000u;
                 }
-                dst[(size_t)(t + i) * n_experts + e] = v[i];
+                if (__ballot(nan) != 0 && half == h) again &= ~(1u << i);
             }
         }
+    }
+    if (small && s_small[e - e0]) again = 0xffff;
+    if (__ballot(again != 0) != 0) {
+        const floatx16 exact = fp32_tile(x + (size_t)min(tile_t0 + row, tokens - 1) * hidden + 32 * half,
+                                         w + (size_t)min(e, n_experts - 1) * hidden + 32 * half, chunk_begin, chunk_begin + n);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = again >> i & 1 ? exact[i] : v[i];
+    }
+    if (e < n_experts) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (token_of(i) < tokens) dst[(size_t)token_of(i) * n_experts + e] = v[i];
     }
 }
 

@@ -293,7 +293,8 @@ void moe_route_launcher(int* ids, float* weights, const float* logits, int token
 /* Router projection in front of the routing (caller-side neighbour, same launcher pattern):
  *   logits [tokens, n_experts] fp32 = x [tokens, hidden] . w [n_experts, hidden]^T
  * x fp32 (x_dtype 0) or bf16 (1), w fp32; every product is exact in fp32 (on the fp32 matrix cores, or with a bf16
- * x of 64 tokens or more on the bf16 ones, w cut into three bf16 numbers on the way), so the result
+ * x of 64 tokens or more on the bf16 ones, w cut into three bf16 numbers on the way; config 1 asks for the former, 3 for
+ * the latter), so the result
  * differs from an fp32 reference only by the order of the additions. hidden a multiple of 64;
  * x, w and workspace 16-byte aligned. For few tokens K is split over workgroups and the partial
  * sums are added in a fixed order from workspace: moe_router_logits_workspace_bytes(...) bytes
@@ -305,7 +306,8 @@ void moe_router_logits_launcher(float* logits, const void* x, const float* w, vo
                                 int x_dtype, int config, hipStream_t stream);
 
 /* The router weight as three bf16 planes [3, n_experts, hidden] whose sum is w exactly (the 24 significand
- * bits of an fp32 number cut 8 + 8 + 8); prepared once per weight for the launcher below. */
+ * bits of an fp32 number cut 8 + 8 + 8; of a weight below 2^-110 the bits below 2^-133, the last of a bf16 number, are
+ * lost); prepared once per weight for the launcher below. */
 void moe_router_split_weight_launcher(void* planes, const float* w, int n_experts, int hidden,
                                       hipStream_t stream);
 

@@ -327,6 +327,52 @@ def test_bf16_parts_of_special_weights(capi, dev):
     assert ((got.double() - x.double() @ w.double().T).abs() <= logits_bound(x, w)).all()
 
 
+def logits_of_config(capi, dev, x, w, config):
+    T, H = x.shape
+    E = w.shape[0]
+    x, w = x.to(dev), w.to(dev)
+    nbytes = capi.moe_router_logits_workspace_bytes(T, H, E)
+    ws = torch.empty(nbytes + 16, dtype=torch.uint8, device=dev)
+    got = torch.full((T * E + 8,), -7.0, device=dev)
+    lib, stream = capi.library(), torch.cuda.current_stream().cuda_stream
+    lib.moe_router_logits_launcher(got.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), nbytes, T, H, E, 1, config, stream)
+    assert lib.cuda_agent_amd_last_status() == 0 and (got[T * E:] == -7.0).all()
+    return got[:T * E].view(T, E).cpu()
+
+
+@pytest.mark.parametrize('shape', [(64, 192, 64), (130, 512, 70), (300, 2112, 256), (4100, 448, 33)])    # one split and several
+def test_bf16_parts_of_numbers_of_every_size(capi, dev, shape):
+    # An expert with a weight too small for three bf16 parts, and sums that infinities turn into a NaN, get the sums of the
+    # fp32 matrix cores; nothing beside them changes. Subnormal values of x count like any others
+    T, H, E = shape
+    gen = torch.Generator().manual_seed(T + H + E)
+    x = torch.randn(T, H, generator=gen).bfloat16()
+    x[3] = (torch.randn(H, generator=gen) * 2.0 ** -128).bfloat16()
+    x[4] = 2.0 ** -133
+    w = torch.randn(E, H, generator=gen) * 2.0 ** 60
+    w[11] = 2.0 ** -110 * (1.0 + 2.0 ** -23)             # (the smallest that is the sum of its parts)
+    plain = logits_of_config(capi, dev, x, w, 3)
+    w0 = w.clone()
+    w0[5] = torch.randn(H, generator=gen) * 2.0 ** -118
+    w0[E - 1, H - 2] = 2.0 ** -149
+    x2, w2 = x.clone(), w0.clone()
+    x2[40, 0], x2[41, H - 1] = float('nan'), float('-inf')
+    w2[7, 9] = float('inf')
+    fp32 = logits_of_config(capi, dev, x2, w2, 1)
+    got = logits_of_config(capi, dev, x2, w2, 3)
+    want = x2.double() @ w2.double().T
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)].double(), want[torch.isinf(want)])
+    assert (~finite).sum() == T + 2 * E - 2
+    small = torch.zeros(T, E, dtype=torch.bool)
+    small[:, [5, E - 1]] = True
+    if capi.library().moe_router_logits_num_splits(T, H, E) == 1:     # (else only the splits that hold such a number)
+        assert torch.equal(got[small & finite], fp32[small & finite])
+    assert torch.equal(got[~small & finite], plain[~small & finite])
+    # (products below 2^-126 are rounded to multiples of 2^-149)
+    assert ((got.double() - want).abs()[finite] <= (logits_bound(torch.nan_to_num(x2, 0, 0, 0), w0) + H * 2.0 ** -149)[finite]).all()
+
+
 def test_router_logits_rejects_bad_arguments(capi, dev):
     logits = torch.zeros(4, 32, device=dev)
     w = torch.zeros(32, 96, device=dev)
