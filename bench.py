@@ -31,6 +31,7 @@ if str(REPO) not in sys.path:
 
 HBM_PEAK_GBS = 8000.0
 FP8_PEAK_TFLOPS = 5033.0
+BF16_PEAK_TFLOPS = 2516.0
 METRIC = "GB/s & % HBM peak (GDN/MoE/MLA decode); fp8 TFLOP/s % MFMA peak (MoE prefill)"
 
 # HBM bytes per step (summed over the workload's kernels) from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, scaled
@@ -292,17 +293,19 @@ def bench_router(torch, capi, dev, steps, warmup, cpu_baseline, prefill):
         res = dict(
             workload="router in front of configs[4]: T=8192 bf16 hidden states x fp32 weight [256, 7168] -> fp32 "
                      "logits, then group-limited biased top-8, seed 20260",
-            value=flops / sec / 1e12, unit="TFLOP/s", ms_per_step=sec * 1e3, dtype="f32",
-            kernel="moe_router_gemm_kernel",
-            roofline=dict(bound="mfma", achieved=flops / sec / 1e12, peak=157.3, unit="TFLOP/s",
-                          frac=flops / sec / 1e12 / 157.3, traffic=None),
+            value=flops / sec / 1e12, unit="TFLOP/s", ms_per_step=sec * 1e3, dtype="f32 as 3 x bf16",
+            kernel="moe_router_gemm_long_kernel",
+            # (executed: three bf16 products for one of fp32)
+            roofline=dict(bound="mfma", achieved=3 * flops / sec / 1e12, peak=BF16_PEAK_TFLOPS, unit="TFLOP/s",
+                          frac=3 * flops / sec / 1e12 / BF16_PEAK_TFLOPS, traffic=None),
             algorithmic_flops=flops)
     else:
         res = dict(
             workload="router in front of configs[2]: T=64 bf16 hidden states x fp32 weight [256, 7168] -> fp32 "
-                     "logits (K split 16 ways + ordered reduce), then group-limited biased top-8, seed 20260",
-            value=nbytes_alg / sec / 1e9, unit="GB/s", ms_per_step=sec * 1e3, dtype="f32",
-            kernel="moe_router_gemm_kernel",
+                     f"logits (K split {capi.library().moe_router_logits_num_splits(T, H, E)} ways + ordered reduce), "
+                     "then group-limited biased top-8, seed 20260",
+            value=nbytes_alg / sec / 1e9, unit="GB/s", ms_per_step=sec * 1e3, dtype="f32 as 3 x bf16",
+            kernel="moe_router_gemm_long_kernel",
             roofline=dict(bound="hbm", achieved=nbytes_alg / sec / 1e9, peak=HBM_PEAK_GBS, unit="GB/s",
                           frac=nbytes_alg / sec / 1e9 / HBM_PEAK_GBS, traffic=None),
             algorithmic_bytes=nbytes_alg)

@@ -4,6 +4,8 @@ import subprocess
 import sys
 from pathlib import Path
 
+import pytest
+
 REPO = Path(__file__).resolve().parent.parent
 
 
@@ -70,3 +72,14 @@ def test_measured_constants_of_bench_are_the_figures_of_the_committed_profiles()
     counters_md = (REPO / 'profiles' / 'moe_prefill_mla_matrix_core_counters_pmc.md').read_text()
     for figure in re.findall(r'mfma_busy(?:_down)?=([0-9.]+)', values['MEASURED_MFMA']):
         assert figure in counters_md, figure
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('prefill', [False, True])
+def test_router_roofline_is_that_of_the_units_it_runs_on(capi, dev, prefill):
+    import torch
+
+    import bench
+    res = bench.bench_router(torch, capi, dev, 10, 3, False, prefill)
+    assert 0 < res['roofline']['frac'] <= 1
+    assert f"K split {capi.library().moe_router_logits_num_splits(64, 7168, 256)} ways" in res['workload'] or prefill

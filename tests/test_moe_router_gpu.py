@@ -271,40 +271,77 @@ def test_split_weight_logits_exact_on_integers_and_routing_chain(capi, dev):
     assert (ids != want_ids).any(dim=1).sum().item() <= 8
 
 
-@pytest.mark.parametrize('shape', [(1, 64, 1), (127, 128, 63), (129, 192, 65), (64, 256, 64), (257, 320, 130), (40, 7168, 8),
-                                   (300, 2112, 256), (8192, 3072, 256)])    # 1 to 5 chunks a split, ragged splits, one split
-def test_long_sums(capi, dev, shape):
-    # the kernel whose wavefronts share K, forced at every size: within the bound of an fp32 summation
-    T, H, E = shape
-    gen = torch.Generator().manual_seed(T + H)
-    x = torch.randn(T, H, generator=gen).bfloat16().to(dev)
-    w = (torch.randn(E, H, generator=gen) * H ** -0.5).to(dev)
+def logits_of_config(capi, dev, x, w, config):
+    """moe_router_logits_launcher on the kernel that `config` names; nothing is written behind the logits"""
+    T, H = x.shape
+    E = w.shape[0]
+    x, w = x.to(dev), w.to(dev)
     nbytes = capi.moe_router_logits_workspace_bytes(T, H, E)
     ws = torch.empty(nbytes + 16, dtype=torch.uint8, device=dev)
-    got = torch.full((T, E), float('nan'), device=dev)
+    got = torch.full((T * E + 8,), -7.0, device=dev)
     lib, stream = capi.library(), torch.cuda.current_stream().cuda_stream
-    lib.moe_router_logits_launcher(got.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), nbytes, T, H, E, 1, 3, stream)
-    assert lib.cuda_agent_amd_last_status() == 0
-    assert ((got.cpu().double() - x.cpu().double() @ w.cpu().double().T).abs() <= logits_bound(x.cpu(), w.cpu())).all()
+    lib.moe_router_logits_launcher(got.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), nbytes, T, H, E, 1, config, stream)
+    assert lib.cuda_agent_amd_last_status() == 0 and (got[T * E:] == -7.0).all()
+    return got[:T * E].view(T, E).cpu()
 
 
-@pytest.mark.parametrize('shape', [(1, 64, 1), (16, 512, 5), (17, 576, 6), (33, 3584, 256), (5, 3648, 64), (64, 7168, 257),
-                                   (130, 2048, 9)])    # 1 to 112 chunks of K for 8 wavefronts of 7 in flight
-def test_few_tokens_in_one_launch(capi, dev, shape):
-    T, H, E = shape
-    gen = torch.Generator().manual_seed(T + H + 1)
-    x = torch.randn(T, H, generator=gen).bfloat16().to(dev)
-    w = (torch.randn(E, H, generator=gen) * H ** -0.5).to(dev)
+def split_logits_of_config(capi, dev, x, w, config):
+    T, H = x.shape
+    E = w.shape[0]
+    x, w = x.to(dev), w.to(dev)
     planes = torch.empty(3, E, H, dtype=torch.bfloat16, device=dev)
     capi.moe_router_split_weight_launch(planes, w)
     nbytes = capi.moe_router_logits_workspace_bytes(T, H, E)
     ws = torch.empty(nbytes + 16, dtype=torch.uint8, device=dev)
     got = torch.full((T * E + 8,), -7.0, device=dev)
     lib, stream = capi.library(), torch.cuda.current_stream().cuda_stream
-    lib.moe_router_logits_split_launcher(got.data_ptr(), x.data_ptr(), planes.data_ptr(), ws.data_ptr(), nbytes, T, H, E, 4, stream)
+    lib.moe_router_logits_split_launcher(got.data_ptr(), x.data_ptr(), planes.data_ptr(), ws.data_ptr(), nbytes, T, H, E, config, stream)
     assert lib.cuda_agent_amd_last_status() == 0 and (got[T * E:] == -7.0).all()
-    error = (got[:T * E].view(T, E).cpu().double() - x.cpu().double() @ w.cpu().double().T).abs()
-    assert (error <= logits_bound(x.cpu(), w.cpu())).all()
+    return got[:T * E].view(T, E).cpu()
+
+
+def check_parts(run, capi, dev, shape, config):
+    """A kernel for weights in three bf16 parts, forced at a size: as close to the exact product as an fp32 evaluation, which it
+    is not without the lowest part; and exact where all sums are, with weights that need all three parts"""
+    T, H, E = shape
+    gen = torch.Generator().manual_seed(T + H + E)
+    x = torch.randn(T, H, generator=gen).bfloat16()
+    w = torch.randn(E, H, generator=gen) * H ** -0.5
+    got, want = run(capi, dev, x, w, config), x.double() @ w.double().T
+    error = (got.double() - want).abs()
+    assert (error <= logits_bound(x, w)).all()
+    # (the oracle's own error as the measure, on at least 64 x 64 sums of this length: it is a maximum over random values)
+    xm, wm = x, w
+    if T < 64 or E < 64:
+        xm, wm = torch.randn(64, H, generator=gen).bfloat16(), torch.randn(64, H, generator=gen) * H ** -0.5
+    ref_err = (moe.router_logits(xm, wm).double() - xm.double() @ wm.double().T).abs().max().item()
+    assert error.max().item() <= 4 * ref_err + 1e-7
+    # integers of 19 bits times -1, 0 and 1, at most 31 of them a token: every sum is below 2^24
+    x = torch.zeros(T, H)
+    at = torch.randint(0, H, (T, 31), generator=gen)
+    x.scatter_(1, at, torch.randint(-1, 2, (T, 31), generator=gen).float())
+    w = torch.randint(-2 ** 19 + 1, 2 ** 19, (E, H), generator=gen).float()
+    assert torch.equal(run(capi, dev, x.bfloat16(), w, config).double(), x.double() @ w.double().T)
+
+
+@pytest.mark.parametrize('shape', [(1, 64, 1), (127, 128, 63), (129, 192, 65), (64, 256, 64), (257, 320, 130), (40, 7168, 8),
+                                   (300, 2112, 256), (8192, 3072, 256)])    # 1 to 5 chunks a split, ragged splits, one split
+def test_long_sums(capi, dev, shape):
+    # the kernel whose wavefronts share K
+    check_parts(logits_of_config, capi, dev, shape, 3)
+
+
+@pytest.mark.parametrize('shape', [(1, 64, 1), (16, 512, 5), (17, 576, 6), (33, 3584, 256), (5, 3648, 64), (64, 7168, 257),
+                                   (130, 2048, 9)])    # 1 to 112 chunks of K for 8 wavefronts of 7 in flight
+def test_few_tokens_in_one_launch(capi, dev, shape):
+    check_parts(split_logits_of_config, capi, dev, shape, 4)
+
+
+@pytest.mark.parametrize('config', [1, 2])     # a wavefront for itself, and tiles of 128 tokens
+@pytest.mark.parametrize('shape', [(1, 64, 32), (100, 448, 72), (33, 128, 1), (96, 512, 64), (300, 2048, 72), (129, 192, 65),
+                                   (2100, 128, 130)])    # one split and several, tokens and experts beyond the last tile
+def test_kernels_of_the_split_weight(capi, dev, shape, config):
+    check_parts(split_logits_of_config, capi, dev, shape, config)
 
 
 def test_bf16_parts_of_special_weights(capi, dev):
@@ -325,19 +362,6 @@ def test_bf16_parts_of_special_weights(capi, dev):
     w = torch.randn(70, 512, generator=gen) * 2.0 ** -130
     got = run_logits(capi, dev, x, w)
     assert ((got.double() - x.double() @ w.double().T).abs() <= logits_bound(x, w)).all()
-
-
-def logits_of_config(capi, dev, x, w, config):
-    T, H = x.shape
-    E = w.shape[0]
-    x, w = x.to(dev), w.to(dev)
-    nbytes = capi.moe_router_logits_workspace_bytes(T, H, E)
-    ws = torch.empty(nbytes + 16, dtype=torch.uint8, device=dev)
-    got = torch.full((T * E + 8,), -7.0, device=dev)
-    lib, stream = capi.library(), torch.cuda.current_stream().cuda_stream
-    lib.moe_router_logits_launcher(got.data_ptr(), x.data_ptr(), w.data_ptr(), ws.data_ptr(), nbytes, T, H, E, 1, config, stream)
-    assert lib.cuda_agent_amd_last_status() == 0 and (got[T * E:] == -7.0).all()
-    return got[:T * E].view(T, E).cpu()
 
 
 @pytest.mark.parametrize('shape', [(64, 192, 64), (130, 512, 70), (300, 2112, 256), (4100, 448, 33)])    # one split and several
