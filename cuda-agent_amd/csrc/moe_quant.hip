@@ -81,7 +81,9 @@ __device__ __forceinline__ void unpack_bf16x8(float (&v)[8], const unsigned (&ra
     }
 }
 
-// one run of a row: v its values, w their weights, `at` its place in x, group16 the lane's number among the 16 of its group
+// one run of a row: v its values, w their weights, `at` its place in x, group16 the lane's number among the 16 of its group.
+// STREAM: the codes carry the non-temporal hint
+template <bool STREAM>
 __device__ __forceinline__ void normalise_run(float (&v)[8], const float (&w)[8], float rinv, size_t at, int group16,
                                               __hip_bfloat16* __restrict__ y, uint8_t* __restrict__ q,
                                               float* __restrict__ scale_at, bool pow2) {
@@ -111,7 +113,8 @@ __device__ __forceinline__ void normalise_run(float (&v)[8], const float (&w)[8]
     hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6], v[7], hi, true);
     packed[0] = (unsigned)lo;
     packed[1] = (unsigned)hi;
-    *reinterpret_cast<uintx2*>(q + at) = packed;
+    if constexpr (STREAM) __builtin_nontemporal_store(packed, reinterpret_cast<uintx2*>(q + at));
+    else *reinterpret_cast<uintx2*>(q + at) = packed;
     if (group16 == 0) *scale_at = scale;
 }
 
@@ -122,7 +125,7 @@ __device__ __forceinline__ void normalise_run(float (&v)[8], const float (&w)[8]
 // LANES: 1024 lanes with one run each finish a row soonest, which is what counts while every row has a workgroup's place
 // to itself; with more rows what counts is how many of them are in flight, and a CU holds six workgroups of 256 lanes
 // against two of 1024. The shorter the row, the sooner lanes without a run outweigh what the others gain.
-// STREAM (256 lanes): x carries the non-temporal hint.
+// STREAM (256 lanes): x and the codes carry the non-temporal hint.
 // Both forms add the squares in the same order: within a run, over the 64 lanes of 512 consecutive values, then these
 // sums in ascending order.
 template <int LANES, bool STREAM>
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(LANES) void moe_rmsnorm_quant_kernel(const __hip_bf
         return 1.f / sqrtf(total / (float)cols + eps);  // correctly rounded, as a CPU evaluation
     };
     auto finish = [&](float (&v)[8], const float (&w)[8], float rinv, int c0) {
-        normalise_run(v, w, rinv, row * cols + c0, tid & 15, y, q, scales + row * (cols / GROUP) + c0 / GROUP, pow2);
+        normalise_run<STREAM>(v, w, rinv, row * cols + c0, tid & 15, y, q, scales + row * (cols / GROUP) + c0 / GROUP, pow2);
     };
     if constexpr (RUNS == 1) {
         const int c0 = tid * 8;
@@ -241,14 +244,16 @@ extern "C" void moe_rmsnorm_quant_launcher(void* q, float* scales, void* y, cons
     // of them writes); 4096: 1536 rows 9.5 and 10.0, 2000: 11.9, 11.8; 2048: 600 rows 4.6 and 4.8, 1000: 5.6, 5.3; 1024: 513 rows
     // 3.6 and 3.8, 768: 4.5, 4.1
     const bool many = rows > (cols > 2048 ? 1600 : cols > 1024 ? 768 : 576);
-    // x past the caches where it, y and the codes don't fit the memory-side one (256 MB) together, so that y and the codes
-    // are there for their readers: us, plainly loaded and so, 8192 rows of 7168 (294 MB) 67.8, 58.8, with the router projection of y
-    // behind it 165.8, 157.6, with a gate/up GEMM over the codes 2427, 2416, with an addition to x 118.5, 114.3; 8192 of 4096
-    // (168 MB) 35.6, 36.4; 98.3, 101.5; 1428, 1419; 65.0, 71.0; 8192 of 2048 (84 MB) 23.7, 25.9; 58.1, 59.0; 731, 725; 39.5, 41.6.
-    // (Codes with that hint cost the GEMM 2 to 3 % at all sizes: 2427, 2501 at the first.)
-    const bool stream_x = many && (size_t)rows * cols * (y ? 5 : 3) > (256u << 20);
-    const auto kernel = stream_x ? moe_rmsnorm_quant_kernel<256, true> : many ? moe_rmsnorm_quant_kernel<256, false>
-                                                                              : moe_rmsnorm_quant_kernel<1024, false>;
+    // x and the codes past the caches where they and y don't fit the memory-side one (256 MB) together, so that y is there for
+    // the router projection. us, through the caches and so: 8192 rows of 7168 (294 MB) alone 67.8, 59.0; with projection and
+    // routing 157.4, 149.7, with a pass over the codes behind these 169.3, 162.0, with an addition to x 210.2, 206.9; norm and
+    // gate/up GEMM of 256 experts of 2048, 8 a token 11748, 11749 (but 2427, 2480 of 8 experts of 128, one a token); 8192 of 4096
+    // (168 MB) 35.6, 36.3; 94.9, 94.7; 107.2, 104.4; 126.5, 124.7; 3000 of 7168 (108 MB) 23.8, 26.1; 79.6, 79.7; 86.2,
+    // 88.2; 100.4, 100.3; 8192 of 2048 (84 MB) 23.7, 25.7; 54.1, 53.8; 60.3, 60.1; 69.8, 71.2.
+    const bool past_caches = many && y && (size_t)rows * cols * 5 > (256u << 20);
+    const auto kernel = past_caches ? moe_rmsnorm_quant_kernel<256, true>
+                        : many        ? moe_rmsnorm_quant_kernel<256, false>
+                                      : moe_rmsnorm_quant_kernel<1024, false>;
     kernel<<<rows, many ? 256 : 1024, 0, stream>>>(
         static_cast<const __hip_bfloat16*>(x), static_cast<const __hip_bfloat16*>(weight),
         static_cast<__hip_bfloat16*>(y), static_cast<uint8_t*>(q), scales, cols, eps, pow2);

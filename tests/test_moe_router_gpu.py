@@ -442,7 +442,7 @@ def test_rmsnorm_quant(capi, dev, shape, config):
 @pytest.mark.parametrize('shape', [(513, 7168), (600, 2176), (1030, 128), (520, 8192), (1601, 7168), (1605, 2176), (1610, 8192),
                                    (769, 2048), (780, 1152), (577, 1024), (7700, 7168)])
 def test_rmsnorm_quant_many_rows(capi, dev, shape):
-    # (the last: x past the caches)
+    # (the last: x and the codes past the caches)
     # Above 576, 768 or 1600 rows, by their length, a workgroup has 256 lanes instead of 1024 but adds the squares in the
     # same order: the result is that of the same rows in launches of at most 300, bit for bit. (Not against the oracle's neighbouring bf16 value as
     # above: a flip of the first rounding is up to 2^-7 of the normalised value and the rounding of its product with the
