@@ -20,7 +20,7 @@
 // ascending split order, so the result does not depend on timing.
 //
 // Split-weight form (moe_router_split_weight_launcher + moe_router_logits_split_launcher): an fp32
-// weight is the exact sum of three bf16 numbers (its 24 significand bits cut into 8 + 8 + 8), and a
+// weight is the exact sum of three bf16 numbers (its 24 significand bits cut into 8 + 8 + 8; from 2^-110 on), and a
 // product of two bf16 numbers is exact in fp32. With the weight stored once as those three planes the
 // projection of a bf16 x runs on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16: 8 times the rate of
 // the fp32 shape, three products per weight) and still differs from an fp32 reference by the order of the
