@@ -334,6 +334,50 @@ __device__ __forceinline__ void wait_all_memory() {
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8));
 }
 
+// Partial outputs lie in the workspace as the accumulators hold them: [request, split, group of 32 heads, dv tile of 32, ...],
+// and within such a tile of 32 heads x 32 dv pieces of 16 bytes, lane after lane. Lane (head lane % 32, half lane / 32) has
+// rows 8*(i/4) + 4*half + i%4 of the tile in register i; a piece is 4 consecutive registers as fp32 or 8 as fp16. So a
+// split stores whole lines straight from its registers, and the merge, which treats all dv alike, reads whole lines. With a
+// transpose through LDS into rows of 512 dv the split kernel took 3.4 to 4.0 us to end, now 1.5 to 2.0 (64 requests of 2048
+// rows 62.8 -> 61.2 us in all, 8 24.4 -> 22.1, 48 of 1024 with 64 heads 29.5 -> 27.5).
+constexpr int PART_TILE = 32 * 32;
+
+// Registers 8j .. 8j+7 of a tile hold rows 16j + 4*half + [0, 4) and 8 rows further: with the upper lanes' first four and the
+// lower lanes' last four exchanged, a lane has the 8 consecutive values 16j + 8*half + [0, 8) of its head.
+__device__ __forceinline__ void consecutive_dv(uint32_t (&first)[4], uint32_t (&second)[4], int words) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i < words) {
+            const auto r = __builtin_amdgcn_permlane32_swap(first[i], second[i], false, false);
+            first[i] = r[0], second[i] = r[1];
+        }
+    }
+}
+
+// Values 16j + 8*half + [0, 8) of a dv tile of this lane's head to `dst` (the head's row from the tile's first value on),
+// from registers 8j .. 8j+7 of the tile.
+template <typename OUT>
+__device__ __forceinline__ void store_dv(OUT* dst, const float (&v)[8], int j, int half) {
+    uint32_t first[4], second[4];
+    if constexpr (sizeof(OUT) == 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) first[i] = __float_as_uint(v[i]), second[i] = __float_as_uint(v[4 + i]);
+        consecutive_dv(first, second, 4);
+        uintx4* to = reinterpret_cast<uintx4*>(dst + 16 * j + 8 * half);
+        to[0] = uintx4{first[0], first[1], first[2], first[3]};
+        to[1] = uintx4{second[0], second[1], second[2], second[3]};
+    } else {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            first[i] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v[2 * i], (__bf16)v[2 * i + 1]});
+            second[i] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v[4 + 2 * i], (__bf16)v[5 + 2 * i]});
+        }
+        consecutive_dv(first, second, 2);
+        *reinterpret_cast<uintx4*>(dst + 16 * j + 8 * half) = uintx4{first[0], first[1], second[0], second[1]};
+    }
+}
+
 // grid: x = split, y = request, z = head group of 32*NW heads
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
@@ -430,40 +474,18 @@ __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
     }
 #undef MLA_STEP
 
-    // Epilogue: normalise and write the partial output [b, split, head, dv] and the
-    // log2-sum-exp. The accumulator is O^T (a lane holds 4 consecutive dv of one head, lanes
-    // run over heads), so it goes through LDS, 128 dv at a time in a region private to the
-    // wavefront, to leave as 512-byte row segments.
+    // Epilogue: normalised partial output and log2-sum-exp
     const float l_total = st.l + __shfl_xor(st.l, 32);
     const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
-    const int half = lane >> 5;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
-    if (half == 0) {
-        lse_part[part0 + lane] = split_lse(st.m, l_total);
-    }
-    __syncthreads();  // every wavefront is done with the tile buffers
-    constexpr int STAGE_STRIDE = 128 + 4;  // floats per staged head row (padded against conflicts)
-    float* stage = reinterpret_cast<float*>(wave < 2 ? tile0 : tile1) + (wave & 1) * (32 * STAGE_STRIDE);
-    float* o_rows = o_part + part0 * D_V;
+    if (lane < 32) lse_part[part0 + lane] = split_lse(st.m, l_total);
+    floatx4* parts = reinterpret_cast<floatx4*>(o_part + part0 * D_V) + lane;
 #pragma unroll
-    for (int ps = 0; ps < 4; ++ps) {
+    for (int t = 0; t < DV_TILES; ++t) {
+        const floatx16 a = acc[t] * inv_l;
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-            const floatx16 a = acc[4 * ps + tt];
-#pragma unroll
-            for (int qd = 0; qd < 4; ++qd) {
-                floatx4 v = {a[4 * qd] * inv_l, a[4 * qd + 1] * inv_l, a[4 * qd + 2] * inv_l,
-                             a[4 * qd + 3] * inv_l};
-                *reinterpret_cast<floatx4*>(stage + (lane & 31) * STAGE_STRIDE + 32 * tt + 8 * qd +
-                                            4 * half) = v;
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < 16; ++it) {
-            const int r = 2 * it + half;
-            const floatx4 v = *reinterpret_cast<const floatx4*>(stage + r * STAGE_STRIDE + 4 * (lane & 31));
-            *reinterpret_cast<floatx4*>(o_rows + (size_t)r * D_V + 128 * ps + 4 * (lane & 31)) = v;
-        }
+        for (int qd = 0; qd < 4; ++qd)
+            parts[(4 * t + qd) * 64] = floatx4{a[4 * qd], a[4 * qd + 1], a[4 * qd + 2], a[4 * qd + 3]};
     }
 }
 
@@ -490,7 +512,7 @@ __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
 // Measured per wavefront and tile (core clock cycles, 16-tile splits): gather issue 2 000 (the
 // memory pipeline accepts one 1 KB load of a wavefront per 150-300 cycles, whatever the
 // addresses), QK^T 950-1 200, softmax + rescale 1 750-1 950, PV 650-900, barriers 500-2 800;
-// the prologue (indices, Q, first tiles) is 10 us and the epilogue (131 KB of fp16 partials) 3 us.
+// the prologue (indices, Q, first tiles) is 3.5 to 6 us and the epilogue (131 KB of fp16 partials) 1.5 to 2 us.
 // ---------------------------------------------------------------------------------------------
 // Phase timing build (-DMLA_PHASE_TIMING): every wavefront of workgroup (0,0,0) adds up the core
 // clock cycles it spends in each phase of the loop and leaves them in g_phase_cycles.
@@ -673,7 +695,6 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     __shared__ floatx4 s_xchg[8][4 * 64];     // partial scores of every wavefront, 4 KB each
     __shared__ int s_idx[MAX_SPLIT_ROWS];
     __shared__ uint32_t s_gather_tab[GATHER_TAB];
-    __shared__ float s_head_max[8][32];  // epilogue: largest |O^T| of every head in a wavefront's half
     __shared__ int s_first_masked_tile;
 
     PHASE_TIMING_BEGIN();
@@ -1012,65 +1033,43 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
         PHASE_MARK(5);  // PV
     }
 
-    // epilogue: normalise; O^T half -> LDS (64 dv at a time, region private to the wavefront)
-    // -> 128-byte row segments of the partial output. The partial is stored as fp16 of
-    // O / 2^e with 2^e the power of two above the head's largest magnitude (kept next to the
-    // log-sum-exp): half the bytes of fp32 for the split kernel to write and the merge to read, and
-    // an error of at most 2^-12 of that magnitude.
+    // epilogue: normalise and store, as fp16 of O / 2^e with 2^e the power of two above the head's largest magnitude in this
+    // wavefront's half of dv (kept next to the log-sum-exp): half the bytes of fp32 for the split kernel to write and
+    // the merge to read, and an error of at most 2^-12 of that magnitude.
+    if (!live) return;
     const float l_total = st.l + __shfl_xor(st.l, 32);
     const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
-    constexpr int STAGE_STRIDE = 64 + 4;
-    float* stage = reinterpret_cast<float*>(tiles + (wave >> 2) * TILE_CHUNKS) + (wave & 3) * (32 * STAGE_STRIDE);
-    typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
-    // O^T half times `scale`, row r of the 32 heads and columns 64*ps + 4*(lane%16) .. +3 of the half to store(r, ps, v)
-    auto write_rows = [&](float scale, auto store) {
-#pragma unroll
-        for (int ps = 0; ps < 4; ++ps) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const floatx16 a = acc[2 * ps + tt];
-#pragma unroll
-                for (int qd = 0; qd < 4; ++qd) {
-                    floatx4 v = {a[4 * qd] * scale, a[4 * qd + 1] * scale, a[4 * qd + 2] * scale, a[4 * qd + 3] * scale};
-                    *reinterpret_cast<floatx4*>(stage + (lane & 31) * STAGE_STRIDE + 32 * tt + 8 * qd + 4 * half) = v;
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                const int r = 4 * it + (lane >> 4);
-                store(r, ps, *reinterpret_cast<const floatx4*>(stage + r * STAGE_STRIDE + 4 * (lane & 15)));
-            }
-        }
-    };
     if (n_splits == 1) {
         // the only split of its request: this is the output (there is no merge)
-        __syncthreads();  // every wavefront is done with the tiles
-        if (!live) return;
-        const size_t o0 = part0 * D_V + 256 * dh + 4 * (lane & 15);
-        if (out_dtype == 0) {
-            write_rows(inv_l, [&](int r, int ps, floatx4 v) {
-                const bf16x4 x = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
-                *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(out) + o0 + (size_t)r * D_V + 64 * ps) = x;
-            });
-        } else {
-            write_rows(inv_l, [&](int r, int ps, floatx4 v) {
-                *reinterpret_cast<floatx4*>(static_cast<float*>(out) + o0 + (size_t)r * D_V + 64 * ps) = v;
-            });
-        }
+        auto store = [&](auto* rows) {
+#pragma unroll
+            for (int tt = 0; tt < HALF_DV_TILES; ++tt)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = acc[tt][8 * j + i] * inv_l;
+                    store_dv(rows + 32 * tt, v, j, half);
+                }
+        };
+        const size_t o0 = (part0 + (lane & 31)) * D_V + 256 * dh;
+        if (out_dtype == 0) store(static_cast<__bf16*>(out) + o0);
+        else store(static_cast<float*>(out) + o0);
         PHASE_TIMING_END(wave, lane);
         return;
     }
+    if (dh == 0 && half == 0) lse_part[part0 + lane] = split_lse(st.m, l_total);
+    const size_t tile0 = part0 * D_V + (size_t)dh * HALF_DV_TILES * PART_TILE;
     if (scale_part == nullptr) {  // fp32 partials (fewer than 128 heads: they are small)
-        __syncthreads();
-        if (!live) return;
-        if (dh == 0 && half == 0) {
-            lse_part[part0 + lane] = split_lse(st.m, l_total);
+        floatx4* parts = reinterpret_cast<floatx4*>(reinterpret_cast<float*>(o_part) + tile0) + lane;
+#pragma unroll
+        for (int tt = 0; tt < HALF_DV_TILES; ++tt) {
+            const floatx16 a = acc[tt] * inv_l;
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd)
+                parts[(4 * tt + qd) * 64] = floatx4{a[4 * qd], a[4 * qd + 1], a[4 * qd + 2], a[4 * qd + 3]};
         }
-        float* o_rows = reinterpret_cast<float*>(o_part) + part0 * D_V + 256 * dh + 4 * (lane & 15);
-        write_rows(inv_l, [&](int r, int ps, floatx4 v) {
-            *reinterpret_cast<floatx4*>(o_rows + (size_t)r * D_V + 64 * ps) = v;
-        });
         PHASE_TIMING_END(wave, lane);
         return;
     }
@@ -1080,121 +1079,174 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[t][i]));
     amax = fmaxf(amax, __shfl_xor(amax, 32));
-    if (half == 0) s_head_max[wave][lane] = amax;
-    __syncthreads();
-    if (!live) return;
-    if (dh == 0 && half == 0) {
-        lse_part[part0 + lane] = split_lse(st.m, l_total);
-    }
-    // exponent field of the bound + 1: 2^e > |O| for every element of the head (1 if the head is 0)
-    const float bound = fmaxf(s_head_max[wave][lane & 31], s_head_max[wave ^ 1][lane & 31]) * inv_l;
+    // exponent field of the bound + 1: 2^e > |O| for every element of the half (1 if it is 0)
+    const float bound = amax * inv_l;
     uint32_t e_bits = ((__float_as_uint(bound) >> 23) & 255u) + 1u;
     e_bits = bound > 0.f ? (e_bits > 253u ? 253u : e_bits) : 127u;
     const float inv_scale = __uint_as_float((254u - e_bits) << 23) * inv_l;
-    if (dh == 0 && half == 0) scale_part[part0 + lane] = __uint_as_float(e_bits << 23);
-    _Float16* o_rows = o_part + part0 * D_V + 256 * dh + 4 * (lane & 15);
-    write_rows(inv_scale, [&](int r, int ps, floatx4 v) {
-        const halfx4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
-        *reinterpret_cast<halfx4*>(o_rows + (size_t)r * D_V + 64 * ps) = h;
-    });
+    if (half == 0) scale_part[2 * part0 - head0 + (size_t)dh * n_heads + lane] = __uint_as_float(e_bits << 23);
+    typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+    halfx8* parts = reinterpret_cast<halfx8*>(o_part + tile0) + lane;
+#pragma unroll
+    for (int tt = 0; tt < HALF_DV_TILES; ++tt)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            halfx8 h;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) h[i] = (_Float16)(acc[tt][8 * j + i] * inv_scale);
+            parts[(2 * tt + j) * 64] = h;
+        }
     PHASE_MARK(10);  // epilogue
     PHASE_TIMING_END(wave, lane);
 }
 
-// out[b, h, :] = sum_s w_s o_part[b, s, h, :],  w_s = exp2(lse_s - max) / sum. NW wavefronts per (b, h), 8 output
-// columns per lane, 4 / NW heads per workgroup (grid x = n_heads * NW / 4, y = request); wavefront i of a head takes
-// the splits i, i + NW, ... of every 64, BATCH of them requested at once, the first before anything else. PART is the
-// type the split kernel stored: float, or fp16 of O / scale with the per-head scale in scale_part.
-// The kernel is a chain of memory latencies: with one request and 64 splits on one wavefront per head, 8 rows at a
-// time and the log-sum-exps one after the other, it took 37 us, three times the split kernel before it; lane s now
-// fetches the log-sum-exp of split s, and above 8 splits four wavefronts share a head (3.9 us).
+// out[b, h, :] = sum_s w_s o_part[b, s, h, :],  w_s = exp2(lse_s - max) / sum. A unit is registers 8j .. 8j+7 of a dv tile of 32
+// heads (16 dv of each, see PART_TILE): there are n_heads of them per request. NW wavefronts per unit, 4 / NW units per
+// workgroup (grid x = n_heads * NW / 4, y = request); wavefront i of a unit takes the splits i, i + NW, ..., BATCH of them
+// requested at once, relative to the largest log-sum-exp it has seen. PART is the type the split kernel stored: float,
+// or fp16 of O / scale with the scale of every head and half of dv in scale_part.
+// The kernel is a chain of memory latencies: with one request and 64 splits on one wavefront, 8 pieces at a
+// time and the log-sum-exps one after the other, it took 37 us, three times the split kernel before it. Above 8 splits four
+// wavefronts share a unit, above 32 eight (us for 64 splits: 3.0, with four 3.8, with sixteen 3.3). The lower lanes fetch the
+// log-sum-exps and scales of the even splits of a batch, the upper ones those of the odd ones: with all of them in all lanes 5.9.
 template <typename OUT, typename PART, int NW, int BATCH>
-__global__ __launch_bounds__(256) void sparse_mla_merge_kernel(const PART* __restrict__ o_part,
-                                                               const float* __restrict__ lse_part,
-                                                               const float* __restrict__ scale_part,
-                                                               OUT* __restrict__ out, int n_heads,
-                                                               int n_splits) {
-    typedef PART partx8 __attribute__((ext_vector_type(8)));
-    typedef float floatx8 __attribute__((ext_vector_type(8)));
+__global__ __launch_bounds__(NW > 4 ? 64 * NW : 256) void sparse_mla_merge_kernel(const PART* __restrict__ o_part,
+                                                                                  const float* __restrict__ lse_part,
+                                                                                  const float* __restrict__ scale_part,
+                                                                                  OUT* __restrict__ out, int n_heads,
+                                                                                  int n_splits) {
+    constexpr bool SCALED = sizeof(PART) == 2;
+    constexpr int WORDS = SCALED ? 4 : 8;
+    constexpr int UNITS = NW > 4 ? 1 : 4 / NW;  // of a workgroup
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int hg = blockIdx.x;
+    int ug = blockIdx.x;
     int b = blockIdx.y;
     // request b on XCD b % 8, where the split kernel wrote its partials (see there)
     if ((gridDim.y & 7) == 0) {
         const int linear = blockIdx.x + gridDim.x * blockIdx.y;
         const int j = linear >> 3;
-        hg = j % (int)gridDim.x;
+        ug = j % (int)gridDim.x;
         b = (linear & 7) + 8 * (j / (int)gridDim.x);
     }
-    const int h = hg * (4 / NW) + wave / NW;
+    const int unit = ug * UNITS + wave / NW;
     const int part = wave % NW;
-    const size_t base = (size_t)b * n_splits * n_heads + h;
-    floatx8 o = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    partx8 rows[BATCH];
-    auto load_rows = [&](int s0) {
+    const int head = (unit >> 5) * 32 + (lane & 31);
+    const int half = lane >> 5;
+    const int tile = (unit >> 1) & 15;
+    const int j8 = unit & 1;
+    const size_t row0 = (size_t)b * n_splits * n_heads;
+    const PART* parts = o_part + (row0 + (unit >> 5) * 32) * D_V + tile * PART_TILE + 512 * j8;
+    const float* lses = lse_part + row0 + head;
+    const float* scales = SCALED ? scale_part + 2 * row0 + (tile >> 3) * n_heads + head : nullptr;
+    // v of the lower and of the upper half of the lanes, in both
+    auto halves = [](float v, float& lower, float& upper) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        lower = __uint_as_float(r[0]), upper = __uint_as_float(r[1]);
+    };
+    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float mx = -INFINITY, wsum = 0.f;
+    for (int s0 = part; s0 < n_splits; s0 += NW * BATCH) {
+        uint32_t rows[BATCH][WORDS];
+        // log-sum-exps and scales of splits 2i + half of the batch
+        float lse[BATCH / 2], scale[BATCH / 2];
+        // (splits past the end repeat the last one; their weight is 0)
+        auto split = [&](int j) { return s0 + NW * j < n_splits ? s0 + NW * j : n_splits - 1; };
+#pragma unroll
+        for (int i = 0; i < BATCH / 2; ++i) {
+            const int s = split(2 * i + half);
+            lse[i] = lses[(size_t)s * n_heads];
+            if constexpr (SCALED) scale[i] = scales[(size_t)s * 2 * n_heads];
+        }
 #pragma unroll
         for (int j = 0; j < BATCH; ++j) {
-            // (splits past the end repeat the last one; their weight is 0)
-            const int s = s0 + NW * j < n_splits ? s0 + NW * j : n_splits - 1;
-            rows[j] = __builtin_nontemporal_load(
-                reinterpret_cast<const partx8*>(o_part + (base + (size_t)s * n_heads) * D_V) + lane);
+            const uintx4* src = reinterpret_cast<const uintx4*>(parts + (size_t)split(j) * n_heads * D_V) + lane;
+#pragma unroll
+            for (int q = 0; q < WORDS / 4; ++q) {
+                const uintx4 r = __builtin_nontemporal_load(src + 64 * q);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rows[j][4 * q + i] = r[i];
+            }
         }
-    };
-    load_rows(part);
-    float mx = -INFINITY;
-    for (int s = lane; s < n_splits; s += 64) mx = fmaxf(mx, lse_part[base + (size_t)s * n_heads]);
+        float top = lse[0];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    float wsum = 0.f;
-    for (int c0 = 0; c0 < n_splits; c0 += 64) {
-        // weight of split c0 + lane (0 for one without rows, NaN if its log-sum-exp is)
-        float w = 0.f, ws = 0.f;
-        if (c0 + lane < n_splits) {
-            const size_t row = base + (size_t)(c0 + lane) * n_heads;
-            const float lse = lse_part[row];
-            w = lse == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse - mx);
-            ws = w;
-            if constexpr (sizeof(PART) == 2) ws = w * scale_part[row];  // (a power of two)
+        for (int i = 1; i < BATCH / 2; ++i) top = fmaxf(top, lse[i]);
+        float lower, upper;
+        halves(top, lower, upper);
+        top = fmaxf(mx, fmaxf(lower, upper));
+        if (s0 != part) {
+            const float alpha = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mx - top);  // (nothing yet, or NaN)
+            wsum *= alpha;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] *= alpha;
         }
-        wsum += w;
-        for (int s0 = c0 + part; s0 < n_splits && s0 < c0 + 64; s0 += NW * BATCH) {
-            if (s0 != part) load_rows(s0);
+        mx = top;
 #pragma unroll
-            for (int j = 0; j < BATCH; ++j) {
-                const int at = s0 - c0 + NW * j;
-                const float wj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ws), at & 63));
-                if (at < 64 && wj != 0.f) {  // (a split without rows has weight 0 and is not looked at)
+        for (int i = 0; i < BATCH / 2; ++i) {
+            // weight of the split (0 for one without rows, NaN if its log-sum-exp is)
+            const float w = s0 + NW * (2 * i + half) >= n_splits || lse[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse[i] - mx);
+            wsum += w;
+            float ws[2];
+            halves(SCALED ? w * scale[i] : w, ws[0], ws[1]);  // (the scale is a power of two)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) o[i] += (float)rows[j][i] * wj;
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t(&row)[WORDS] = rows[2 * i + h];
+                const uint32_t keep = ws[h] == 0.f ? 0u : ~0u;  // (a split of weight 0 is not looked at)
+                if constexpr (SCALED) {
+                    typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const halfx2 v = __builtin_bit_cast(halfx2, row[k] & keep);
+                        o[2 * k] += (float)v[0] * ws[h];
+                        o[2 * k + 1] += (float)v[1] * ws[h];
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) o[k] += __uint_as_float(row[k] & keep) * ws[h];
                 }
             }
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) wsum += __shfl_xor(wsum, off);
+    {
+        float lower, upper;
+        halves(wsum, lower, upper);
+        wsum = lower + upper;
+    }
     if constexpr (NW > 1) {
-        __shared__ floatx4 s_o[4][2][64];
+        __shared__ floatx4 s_o[NW > 4 ? NW : 4][2][64];
+        __shared__ float s_mx[NW > 4 ? NW : 4][64], s_wsum[NW > 4 ? NW : 4][64];
         s_o[wave][0][lane] = floatx4{o[0], o[1], o[2], o[3]};
         s_o[wave][1][lane] = floatx4{o[4], o[5], o[6], o[7]};
+        s_mx[wave][lane] = mx;
+        s_wsum[wave][lane] = wsum;
         __syncthreads();
         if (part != 0) return;
+        float m[NW];
+        float top = mx;
 #pragma unroll
-        for (int i = 1; i < NW; ++i) {
-            const floatx4 lo = s_o[wave + i][0][lane], hi = s_o[wave + i][1][lane];
-            o += floatx8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        for (int w = 1; w < NW; ++w) {
+            m[w] = s_mx[wave + w][lane];
+            top = fmaxf(top, m[w]);
+        }
+        // (a wavefront without splits, or with none but NaN, has 0 or NaN to add)
+        auto factor = [&](float v) { return v == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(v - top); };
+        const float own = factor(mx);
+        wsum *= own;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] *= own;
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            const float f = factor(m[w]);
+            wsum += s_wsum[wave + w][lane] * f;
+            const floatx4 lo = s_o[wave + w][0][lane], hi = s_o[wave + w][1][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] += lo[i] * f, o[4 + i] += hi[i] * f;
         }
     }
-    if (wsum != 0.f) o *= 1.f / wsum;
-    OUT* dst = out + ((size_t)b * n_heads + h) * D_V + lane * 8;
-    if constexpr (sizeof(OUT) == 4) {
-        reinterpret_cast<floatx4*>(dst)[0] = floatx4{o[0], o[1], o[2], o[3]};
-        reinterpret_cast<floatx4*>(dst)[1] = floatx4{o[4], o[5], o[6], o[7]};
-    } else {
-        const bf16x8 r = {(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3],
-                          (__bf16)o[4], (__bf16)o[5], (__bf16)o[6], (__bf16)o[7]};
-        *reinterpret_cast<bf16x8*>(dst) = r;
-    }
+    const float inv = wsum != 0.f ? 1.f / wsum : 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] *= inv;
+    store_dv(out + ((size_t)b * n_heads + head) * D_V + 32 * tile, o, j8, half);
 }
 
 // Microseconds of a launch of `wgs` workgroups of `tiles` tiles each, one workgroup per CU at a time, as measured for
@@ -1290,7 +1342,7 @@ extern "C" size_t sparse_mla_decode_workspace_bytes(int batch, int n_heads, int 
     if (batch <= 0 || n_heads <= 0 || topk <= 0) return 0;
     config = mla::without_halves(config);
     const int splits = max_splits(batch, head_groups_of(n_heads), topk, config >= 1000 ? config - 1000 : config);
-    // partial outputs (sized for fp32), log-sum-exp and scale of every (request, split, head)
+    // partial outputs (sized for fp32) and 2 values more of every (request, split, head)
     return (size_t)batch * splits * n_heads * (D_V + 2) * sizeof(float);
 }
 
@@ -1335,8 +1387,11 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     const int tiles = (topk + TILE_ROWS - 1) / TILE_ROWS;
     const int rows_per_split = ((tiles + splits - 1) / splits) * TILE_ROWS;
     float* o_part = static_cast<float*>(workspace);
-    float* lse_part = o_part + (size_t)batch * splits * n_heads * D_V;
-    float* scale_part = lse_part + (size_t)batch * splits * n_heads;
+    // (behind the partials, which are fp16 on the 8-wavefront kernel from 128 heads on: the log-sum-exps, and two scales each)
+    const bool half_parts = !one_wave_per_group && n_heads >= 128;
+    const size_t part_rows = (size_t)batch * splits * n_heads;
+    float* lse_part = o_part + part_rows * (half_parts ? D_V / 2 : D_V);
+    float* scale_part = half_parts ? lse_part + part_rows : nullptr;
     const float scale_log2 = sm_scale * 1.4426950408889634f;
     const __bf16* qb = static_cast<const __bf16*>(q);
     const __bf16* kvb = static_cast<const __bf16*>(kv);
@@ -1344,7 +1399,6 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     const bool halves = n_heads >= 128 && (halves_asked || takes_halves(batch, head_groups, splits, config));
     const dim3 grid8(splits, batch, halves ? 2 * head_groups : head_groups);
     const int group_heads = halves ? 64 : n_heads < 128 ? n_heads : 128;
-    bool half_parts = false;
     if (one_wave_per_group && n_heads == 32) {
         sparse_mla_split_kernel<1><<<grid, 64, 0, stream>>>(qb, kvb, idx, o_part, lse_part, n_heads,
                                                             n_kv_rows, topk, rows_per_split,
@@ -1358,8 +1412,6 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
                                                              n_kv_rows, topk, rows_per_split,
                                                              scale_log2, kva);
     } else {
-        half_parts = n_heads >= 128;  // this kernel then stores its partials as scaled fp16
-        if (!half_parts) scale_part = nullptr;
         if (fp8_cache) {
             sparse_mla_split8_kernel<true><<<grid8, 512, 0, stream>>>(
                 qb, kvb, idx, reinterpret_cast<_Float16*>(o_part), lse_part, scale_part, n_heads, n_kv_rows,
@@ -1371,18 +1423,19 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
         }
     }
     if (!one_wave_per_group && splits == 1) return;  // (written by the split kernel)
-    // Wavefronts per head, and rows requested at once per lane. Above 8 splits four wavefronts share a head, unless the
-    // heads alone put 8 wavefronts on every CU: 16 requests of 128 heads and 13 splits 34.3 us in all with four, 32.1 with one.
+    // Wavefronts per unit, and pieces requested at once per lane. Above 8 splits four wavefronts share a unit, unless the
+    // units (one per head) alone put 8 wavefronts on every CU: 16 requests of 128 heads and 13 splits 34.3 us in all with four, 32.1 with one.
     const bool heads_fill = (long)batch * n_heads >= 8 * 256;
 #define MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, NW, BATCH)                                      \
-    sparse_mla_merge_kernel<OUT_T, PART_T, NW, BATCH><<<dim3(n_heads * NW / 4, batch), 256, 0, stream>>>( \
+    sparse_mla_merge_kernel<OUT_T, PART_T, NW, BATCH>                                                \
+        <<<dim3(NW > 4 ? n_heads : n_heads * NW / 4, batch), NW > 4 ? 64 * NW : 256, 0, stream>>>(   \
         PARTS, lse_part, SCALES, static_cast<OUT_T*>(out), n_heads, splits)
 #define MLA_MERGE(OUT_T, PART_T, PARTS, SCALES)                                       \
     if (splits <= 2) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 2);              \
     else if (splits <= 4) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 4);         \
     else if (splits <= 8 || (splits <= 32 && heads_fill)) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 1, 8); \
     else if (splits <= 32) MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 4, 8);        \
-    else MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 4, 16);
+    else MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, 8, 8);
     if (half_parts) {
         const _Float16* parts = reinterpret_cast<const _Float16*>(o_part);
         if (out_dtype == 0) {
