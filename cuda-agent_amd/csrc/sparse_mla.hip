@@ -739,6 +739,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     const int head0 = blockIdx.z * group_heads + hg * 32;
     // with 32 or 64 heads the wavefronts of the missing head groups take part in the gather and the barriers only
     const bool live = hg * 32 < group_heads;
+    const int first_group = group_heads == 128 ? 0 : 1;  // the group that fetches tile 0
     const int half = lane >> 5;
 
     const int row_begin = split * rows_per_split;
@@ -762,8 +763,8 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     // (lane -> row 16*(l&1) + lane/4, 16-byte piece lane%4 of line l/2: 16 line requests instead of the 32 that
     // loading the operand layout directly needs); the operand layout is made below through LDS.
     uintx4 qraw[HALF_K_STEPS];
-    {
-        const char* qsrc = reinterpret_cast<const char*>(q + ((size_t)b * n_heads + (live ? head0 : 0)) * D_QK) +
+    if (live) {
+        const char* qsrc = reinterpret_cast<const char*>(q + ((size_t)b * n_heads + head0) * D_QK) +
                            (size_t)(lane >> 2) * ROW_BYTES + 64 * dh + 16 * (lane & 3);
 #pragma unroll
         for (int l = 0; l < HALF_K_STEPS; ++l) {
@@ -800,21 +801,20 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     const char* kv_b = reinterpret_cast<const char*>(kv) + (size_t)b * kva.batch_rows * (FP8 ? FP8_ROW_BYTES : ROW_BYTES);
     PHASE_MARK(7);  // index staging
 
-    // The first two tiles are on their way before Q is fetched: tile 0 by the lead group, tile 1
-    // by the lag group (a cold load instruction takes several hundred cycles to issue, so the
-    // two groups share the work; from tile 2 on the lag group gathers alone).
-    if (group < n_tiles) {
+    // The first two tiles: tile 0 by the lead group, tile 1 by the lag group (a cold load instruction takes several hundred
+    // cycles to issue, so the two groups share the work; from tile 2 on the lag group gathers alone). With 32 or 64
+    // heads the lag group has no Q to fetch and takes both (us: one request of 2048 rows
+    // in workgroups of 64 heads 15.0 -> 14.6, 16 of 32 heads 20.0 -> 18.7).
+#pragma unroll 1
+    for (int t = first_group == 1 ? 0 : group; t <= group && group >= first_group && t < n_tiles; ++t) {
+        const bool pad = t >= first_masked_tile;
         if constexpr (FP8) {
-            gather_quarter_fp8(tiles + group * TILE_CHUNKS, kv_b, s_idx + group * TILE_ROWS, group >= first_masked_tile,
-                               wave & 3, lane);
+            gather_quarter_fp8(tiles + t * TILE_CHUNKS, kv_b, s_idx + t * TILE_ROWS, pad, wave & 3, lane);
         } else {
             uint32_t off[GATHER_INSTR];
-            const bool pad = group >= first_masked_tile;
-            gather_prepare(off, s_idx + group * TILE_ROWS, s_gather_tab, pad, wave & 3, lane);
+            gather_prepare(off, s_idx + t * TILE_ROWS, s_gather_tab, pad, wave & 3, lane);
 #pragma unroll
-            for (int i = 0; i < GATHER_INSTR; ++i) {
-                gather_issue(tiles + group * TILE_CHUNKS, kv_b, off[i], i, pad, wave & 3, lane);
-            }
+            for (int i = 0; i < GATHER_INSTR; ++i) gather_issue(tiles + t * TILE_CHUNKS, kv_b, off[i], i, pad, wave & 3, lane);
         }
     }
     PHASE_MARK(9);  // first gather issue
@@ -824,7 +824,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     // 64 bytes, piece p of row r at slot p ^ ((r >> 2) & 3) so that the 16 rows a read serves per cycle hit
     // 16 different bank groups. No barrier: the LDS operations of a wavefront execute in order.
     bf16x8 qreg[HALF_K_STEPS];
-    {
+    if (live) {
         uintx4* stage = reinterpret_cast<uintx4*>(&s_xchg[wave][0]);
         const int r = lane & 31;
 #pragma unroll
@@ -871,19 +871,20 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
             // tile h/2 must be resident: everything but this wavefront's share of the next tile
             const int t = h >> 1;
             if constexpr (FP8) {
-                // tile 0 was gathered by the lead group: it turns its rows into bf16 here, before the barrier
+                // the group that gathered tile 0 turns its rows into bf16 here, before the barrier
                 // below hands the tile to everyone; every later tile is converted by the lag group inside the
                 // half-step before (see there)
-                if (h == 0 && group == 0) {
-                    wait_all_memory();
+                if (h == 0 && group == first_group) {
+                    if (first_group == 1 && n_tiles > 1) wait_vmcnt<FP8_GATHER_INSTR>();  // (all but those of tile 1)
+                    else wait_all_memory();
                     asm volatile("" ::: "memory");  // the reads below stay behind the wait above
                     dequant_quarter(tiles, s_idx, 0 >= first_masked_tile, wave & 3, lane);
                 }
             } else {
                 const bool plain_wait = t + 1 < n_tiles && t + 1 < first_masked_tile;
-                if (plain_wait) {
-                    wait_vmcnt<GATHER_INSTR>();  // (the lead group has no loads in flight)
-                } else {
+                if (plain_wait && group == 1) {
+                    wait_vmcnt<GATHER_INSTR>();
+                } else {  // (the lead group fetches nothing but tile 0)
                     wait_all_memory();
                 }
             }
