@@ -175,8 +175,17 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     if (want == 0) return;
 
     // Word j of this wavefront in chunk c: entries first + 64*j .. first + 64*j + 63, one per lane, with
-    // first = c*CHUNK + wave*64*P. `left` entries of the wavefront's span exist (uniform); lanes past the end hold NaN.
-    const int span = wave * 64 * P;
+    // first = c*CHUNK + span. `left` entries of the wavefront's span exist (uniform); lanes past the end hold NaN. A row in
+    // registers is dealt out in as many words (whole groups) per wavefront as it needs, not P: of rows that are shorter
+    // than the kernel's CHUNK, by their lengths or because n lies above a power of two, the first wavefronts would have all
+    // (us: 24 rows of 33024 with 8250 to 33024 valid entries 12.1 -> 10.4, in few values 23.2 -> 19.8; one row of 40000 12.3 ->
+    // 10.6; 200 of 10000 10.6 -> 10.3).
+    const int per_wave = RESIDENT ? GROUP * ((valid + SELECT_THREADS * GROUP - 1) / (SELECT_THREADS * GROUP)) : P;
+    const int span = wave * 64 * per_wave;
+    auto left_from = [&](int c0) {
+        const int left = valid - c0 - span;
+        return RESIDENT && left > 64 * per_wave ? 64 * per_wave : left;
+    };
     auto load_chunk = [&](float (&val)[P], int first, int left) {
         const float* src = row + first;
         if (left >= 64 * P) {
@@ -187,7 +196,10 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
             for (int g = 0; g < P; g += GROUP) {
 #pragma unroll
                 for (int j = g; j < g + GROUP; ++j) val[j] = __builtin_nanf("");
-                if (64 * g < left) {
+                if (64 * (g + GROUP) <= left) {
+#pragma unroll
+                    for (int j = g; j < g + GROUP; ++j) val[j] = src[64 * j + lane];
+                } else if (64 * g < left) {
 #pragma unroll
                     for (int j = g; j < g + GROUP; ++j) {
                         const int i = 64 * j + lane;
@@ -277,7 +289,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     };
 
     float val[P];
-    if (RESIDENT) load_chunk(val, span, valid - span);
+    if (RESIDENT) load_chunk(val, span, left_from(0));
 
     if constexpr (FILTER) {
         constexpr int BITMAP = (RESIDENT ? CHUNK : MAX_FILTER_ROW) / 32;
@@ -291,7 +303,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
             for (int i = tid; i < words; i += SELECT_THREADS) s_gt[i] = s_eq[i] = 0u;
             __syncthreads();
             for (int c0 = 0; c0 < valid; c0 += CHUNK) {
-                const int left = valid - c0 - span;
+                const int left = left_from(c0);
                 if constexpr (RESIDENT) {
                     for_groups(left, [&](int g) {
                         float v = val[g];
@@ -353,7 +365,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
                     });
                 };
                 if constexpr (RESIDENT) {
-                    collect(val, span, valid - span);
+                    collect(val, span, left_from(0));
                 } else {
                     float next[P];
                     load_chunk(val, span, valid - span);
@@ -507,7 +519,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         // f(g) for the groups of words of the whole row
         auto for_row = [&](auto f) {
             for (int c0 = 0; c0 < valid; c0 += CHUNK) {
-                const int left = valid - c0 - span;
+                const int left = left_from(c0);
                 if constexpr (!RESIDENT) {
                     load_chunk(val, c0 + span, left);
                     make_keys();
@@ -560,7 +572,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
     // a scan of their counts gives every word its place in the output.
     int gt_before = 0, eq_before = 0;  // in earlier chunks
     for (int c0 = 0; c0 < valid; c0 += CHUNK) {
-        const int left = valid - c0 - span;
+        const int left = left_from(c0);
         if constexpr (!RESIDENT) {
             load_chunk(val, c0 + span, left);
             make_keys();

@@ -84,6 +84,20 @@ def test_long_rows(capi, dev, n, kind):
         assert torch.equal(run_kernel(capi, dev, scores, k, ln), mla.topk_select(scores, k, ln)), (k, ln is not None)
 
 
+@pytest.mark.parametrize('n', [16384, 32768, 65536])
+@pytest.mark.parametrize('kind', ['normal', 'clustered', 'special', 'two'])
+def test_lengths_around_the_words_of_a_wavefront(capi, dev, n, kind):
+    # a row in registers is dealt out in 8 words of 64 entries per wavefront and step: one entry less and more than whole
+    # steps, than what a wavefront takes of them, and than a word
+    gen = torch.Generator().manual_seed(n)
+    lengths = sorted({v for step in (8192, 16384, 24576, 40960, 57344, 65536) for v in (step - 1, step, step + 1)
+                      if v <= n} | {1, 63, 64, 65, 511, 512, 513, 3000, 8192 + 512, 8192 + 513, 8192 + 1025})
+    scores = _rows(kind, n, gen).repeat(-(-len(lengths) // 4), 1)[:len(lengths)]
+    ln = torch.tensor(lengths, dtype=torch.int32)
+    for k in (64, 2048):
+        assert torch.equal(run_kernel(capi, dev, scores, k, ln), mla.topk_select(scores, k, ln)), k
+
+
 def test_selected_indices_feed_the_attention(capi, dev):
     # selection -> sparse-MLA decode; shorter requests leave -1 entries, which the attention skips
     gen = torch.Generator().manual_seed(43)
