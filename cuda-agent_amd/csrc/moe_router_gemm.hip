@@ -704,23 +704,28 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void moe_router_gemm_few_kernel(con
     }
 }
 
-// logits = partial[0] + partial[1] + ... in that order
-__global__ __launch_bounds__(256) void moe_router_reduce_kernel(const float* __restrict__ partial,
-                                                                float* __restrict__ logits,
-                                                                size_t count, int n_splits) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+// logits = partial[0] + partial[1] + ... in that order. A chain of memory latencies: BATCH partial sums are requested at once.
+template <int BATCH>
+__global__ __launch_bounds__(64) void moe_router_reduce_kernel(const float* __restrict__ partial,
+                                                               float* __restrict__ logits,
+                                                               size_t count, int n_splits) {
+    const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     if (i >= count) return;
-    // eight loads at a time are in flight; the additions stay in ascending split order
     float sum = 0.f;
-    for (int s0 = 0; s0 < n_splits; s0 += 8) {
-        float v[8];
+    for (int s0 = 0; s0 < n_splits; s0 += BATCH) {
+        float v[BATCH];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = s0 + j < n_splits ? partial[(size_t)(s0 + j) * count + i] : 0.f;
+        for (int j = 0; j < BATCH; ++j) v[j] = partial[(size_t)(s0 + j < n_splits ? s0 + j : 0) * count + i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+        for (int j = 0; j < BATCH; ++j)
             if (s0 + j < n_splits) sum = (s0 + j == 0) ? v[j] : sum + v[j];
     }
     logits[i] = sum;
+}
+
+void launch_reduce(const void* partial, float* logits, size_t count, int n_splits, hipStream_t stream) {
+    const auto kernel = n_splits <= 2 ? moe_router_reduce_kernel<2> : n_splits <= 8 ? moe_router_reduce_kernel<8> : moe_router_reduce_kernel<32>;
+    kernel<<<(unsigned)((count + 63) / 64), 64, 0, stream>>>(static_cast<const float*>(partial), logits, count, n_splits);
 }
 
 int pick_router_splits(int tokens, int hidden, int n_experts) {
@@ -792,9 +797,7 @@ extern "C" void moe_router_logits_launcher(float* logits, const void* x, const f
             static_cast<const uint16_t*>(x), w, out, tokens, hidden, n_experts, chunks_per_split);
     }
     if (splits > 1) {
-        const size_t count = (size_t)tokens * n_experts;
-        moe_router_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-            static_cast<const float*>(workspace), logits, count, splits);
+        launch_reduce(workspace, logits, (size_t)tokens * n_experts, splits, stream);
     }
 }
 
@@ -869,8 +872,6 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
     kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(planes), out, tokens,
                                      hidden, n_experts, chunks_per_split);
     if (splits > 1) {
-        const size_t count = (size_t)tokens * n_experts;
-        moe_router_reduce_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>(
-            static_cast<const float*>(workspace), logits, count, splits);
+        launch_reduce(workspace, logits, (size_t)tokens * n_experts, splits, stream);
     }
 }
