@@ -143,81 +143,95 @@ __global__ __launch_bounds__(256) void moe_router_split_kernel(const float* __re
     planes[2 * n + i] = (uint16_t)(__float_as_uint(r2) >> 16);
 }
 
-// grid as moe_router_gemm_kernel. A wavefront owns 32 tokens x 32 experts; per 64 values of k it fetches
-// four tiles of 32 rows x 128 bytes (x and the three weight planes), each with 4 load instructions of whole
-// lines (lane l: 16-byte chunk l % 8 of row 8*j + l / 8), and passes them one after the other through its
-// 4 KB LDS buffer (chunk c of row r at slot c ^ ((r >> 1) & 7)) into the operand layout: lane (row, half)
-// holds values [32*half, +32) of its row, 8 per MFMA step. No barrier: the buffer is private and the LDS
-// operations of a wavefront execute in order.
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+typedef const __attribute__((address_space(3))) uint8_t* lds_bytes;
+
+// grid: x = 64-token tiles, y = 32-expert tiles, z = K split; out as in moe_router_gemm_kernel
+// A workgroup owns 64 tokens x 32 experts of one K split; wavefronts 0 and 1 multiply 32 tokens each, all four fetch. What
+// bounds it is the latency of its loads: a split is a few chunks of 64 values of k, and up to FETCHED_CHUNKS of them (64 rows of x and
+// 3 x 32 of the planes, 128 bytes each = 20 KB) are on their way into LDS before the first is waited for. (8 lanes fetch the line of
+// a row, whose chunk p lies in slot p ^ ((row >> 1) & 7); a lane (row, half) of an operand holds values [32*half, +32) of its row, 8
+// per MFMA step.)
+// us, one chunk ahead through registers and 64 experts a workgroup, and this (norm, projection and routing in a row): 64 tokens of 7168 x
+// 256 18.9, 18.3; 200 22.2, 21.9; 128 of 4096 x 256 17.1, 16.9; 1500 of 4096 x 64 28.3, 28.0; the projection alone, 64 tokens 10.3, 9.0.
+constexpr int FETCHED_CHUNKS = 4;
+
 __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16_t* __restrict__ x,
                                                                     const uint16_t* __restrict__ planes,
                                                                     float* __restrict__ out, int tokens,
                                                                     int hidden, int n_experts,
                                                                     int chunks_per_split) {
-    __shared__ u32x4 s_tile[4][32 * 8];
+    constexpr int LOADS = 5;  // load instructions of a wavefront per chunk
+    constexpr int X_BYTES = 64 * K_CHUNK * 2, PLANE_BYTES = 32 * K_CHUNK * 2, CHUNK_BYTES = X_BYTES + 3 * PLANE_BYTES;
+    __shared__ __attribute__((aligned(16))) uint8_t s_chunk[FETCHED_CHUNKS * CHUNK_BYTES];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int row = lane & 31;
     const int half = lane >> 5;
-    const int t0 = blockIdx.x * 64 + (wave & 1) * 32;
-    const int e0 = blockIdx.y * 64 + (wave >> 1) * 32;
-    if (t0 >= tokens || e0 >= n_experts) return;  // (no barrier in this kernel)
-    u32x4* tile = s_tile[wave];
+    const int t0 = blockIdx.x * 64;
+    const int e0 = blockIdx.y * 32;
     const int chunk_begin = blockIdx.z * chunks_per_split;
-    int chunk_end = chunk_begin + chunks_per_split;
-    const int n_chunks = hidden / K_CHUNK;
-    if (chunk_end > n_chunks) chunk_end = n_chunks;
+    const int n = min(chunks_per_split, hidden / K_CHUNK - chunk_begin);  // (not positive: this split is empty)
+
+    // fill side: a wavefront fetches 8 rows of x twice, and 8 of every plane (rows past the end repeat the last)
+    const int ld_row = 8 * wave + (lane >> 3);
+    const size_t ld_piece = (size_t)chunk_begin * K_CHUNK + 8 * ((lane & 7) ^ ((ld_row >> 1) & 7));
+    const uint16_t* src[3] = {x + (size_t)min(t0 + ld_row, tokens - 1) * hidden + ld_piece,
+                              x + (size_t)min(t0 + 32 + ld_row, tokens - 1) * hidden + ld_piece,
+                              planes + (size_t)min(e0 + ld_row, n_experts - 1) * hidden + ld_piece};
     const size_t plane = (size_t)n_experts * hidden;
-
-    // fill side: rows 8*j + lane/8 of the tile, chunk lane%8 (rows beyond the end repeat the last valid one)
-    const u32x4* src[4][4];  // [x, hi, mid, lo][instruction]
+    const uint32_t lds0 = (uint32_t)(size_t)((lds_void_ptr)s_chunk) + wave * 1024;
+    auto fetch = [&](int c) {
+        const uint32_t lds = lds0 + (c % FETCHED_CHUNKS) * CHUNK_BYTES;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = 8 * j + (lane >> 3);
-        const int t = t0 + r < tokens ? t0 + r : tokens - 1;
-        const int e = e0 + r < n_experts ? e0 + r : n_experts - 1;
-        src[0][j] = reinterpret_cast<const u32x4*>(x + (size_t)t * hidden) + (lane & 7);
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-            src[1 + p][j] = reinterpret_cast<const u32x4*>(planes + p * plane + (size_t)e * hidden) + (lane & 7);
-    }
-    u32x4 raw[4][4];
-    auto load_chunk = [&](int c) {
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) raw[m][j] = src[m][j][(size_t)c * (K_CHUNK * 2 / 16)];
-    };
-    // operand of matrix m: through the buffer
-    bf16x8 op[4][4];
-    auto stage = [&](int m) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int r = 8 * j + (lane >> 3);
-            tile[r * 8 + ((lane & 7) ^ ((r >> 1) & 7))] = raw[m][j];
+        for (int i = 0; i < LOADS; ++i) {
+            const uint16_t* from = src[i < 2 ? i : 2] + (i < 2 ? 0 : (i - 2) * plane) + (size_t)c * K_CHUNK;
+            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds + i * 4096) : "memory", "m0");
         }
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            op[m][s] = __builtin_bit_cast(bf16x8, tile[row * 8 + ((4 * half + s) ^ ((row >> 1) & 7))]);
     };
-
     floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (chunk_begin < chunk_end) load_chunk(chunk_begin);
-    for (int c = chunk_begin; c < chunk_end; ++c) {
+    for (int c = 0; c < FETCHED_CHUNKS && c < n; ++c) fetch(c);
+    const bool multiplies = wave < 2 && t0 + 32 * wave < tokens;
+    for (int c = 0; c < n; ++c) {
+        // chunk c has arrived (those behind it may be in flight)
+        static_assert(FETCHED_CHUNKS == 4, "at most three chunks behind");
+        const int behind = min(FETCHED_CHUNKS - 1, n - 1 - c);
+        if (behind == 3) __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (15 << 8));
+        else if (behind == 2) __builtin_amdgcn_s_waitcnt(10 | (7 << 4) | (15 << 8));
+        else if (behind == 1) __builtin_amdgcn_s_waitcnt(5 | (7 << 4) | (15 << 8));
+        else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (multiplies) {
+            const lds_bytes st = (lds_bytes)s_chunk + (c % FETCHED_CHUNKS) * CHUNK_BYTES;
+            auto operand = [&](int r, int s) {
+                return *(const __attribute__((address_space(3))) bf16x8*)(st + (r * 8 + ((4 * half + s) ^ ((row >> 1) & 7))) * 16);
+            };
+            bf16x8 op[4][4];  // x, planes
 #pragma unroll
-        for (int m = 0; m < 4; ++m) stage(m);
-        if (c + 1 < chunk_end) load_chunk(c + 1);  // in flight under the MFMAs below
-        // smallest terms first
+            for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int p = 3; p >= 1; --p)
+                for (int s = 0; s < 4; ++s) op[m][s] = operand(m == 0 ? 32 * wave + row : 64 + 32 * (m - 1) + row, s);
+            // smallest terms first
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[0][s], op[p][s], acc, 0, 0, 0);
+            for (int p = 3; p >= 1; --p)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[0][s], op[p][s], acc, 0, 0, 0);
+        }
+        if (c + FETCHED_CHUNKS < n) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();  // chunk c has been read everywhere
+            asm volatile("" ::: "memory");
+            fetch(c + FETCHED_CHUNKS);
+        }
     }
+    if (!multiplies) return;
     float* dst = out + (size_t)blockIdx.z * tokens * n_experts;
     if (e0 + row < n_experts) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int tt = t0 + 8 * (i / 4) + 4 * half + (i % 4);
+            const int tt = t0 + 32 * wave + 8 * (i / 4) + 4 * half + (i % 4);
             if (tt < tokens) dst[(size_t)tt * n_experts + e0 + row] = acc[i];
         }
     }
@@ -239,9 +253,6 @@ constexpr int BIG_EXPERTS = 64;
 constexpr int BIG_STAGE = (BIG_TOKENS + 3 * BIG_EXPERTS) * K_CHUNK * 2;  // bytes (40 KB)
 constexpr int BIG_STAGES = 3;
 constexpr int BIG_LOADS = BIG_STAGE / 1024 / 4;  // load instructions of a wavefront per stage
-
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
-typedef const __attribute__((address_space(3))) uint8_t* lds_bytes;
 
 // 64 lanes x 16 bytes, global -> LDS (lds_base + lane*16). asm, so that later LDS reads are not made to wait for it: its
 // completion is awaited once per chunk.
@@ -867,7 +878,7 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
                                                               !(part_of_second_round && few_chunks)));
     float* out = splits > 1 ? static_cast<float*>(workspace) : logits;
     const int tile_tokens = tiled ? BIG_TOKENS : 64;
-    const dim3 grid((tokens + tile_tokens - 1) / tile_tokens, (n_experts + 63) / 64, splits);
+    const dim3 grid((tokens + tile_tokens - 1) / tile_tokens, tiled ? (n_experts + 63) / 64 : (n_experts + 31) / 32, splits);
     const auto kernel = tiled ? moe_router_gemm_split_tiled_kernel : moe_router_gemm_split_kernel;
     kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(planes), out, tokens,
                                      hidden, n_experts, chunks_per_split);
