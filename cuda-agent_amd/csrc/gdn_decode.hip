@@ -27,6 +27,7 @@
 #include <hip/hip_bf16.h>
 #include <stdint.h>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 
 namespace {
@@ -153,23 +154,18 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
         kq_part = qv * kv;
     }
     if (tid < DK) {  // waves 0 and 1 (DK == 128): wavefront sum of k_i*q_i
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) kq_part += __shfl_xor(kq_part, off);
+        // (the products of the first step are not rounded)
+        kq_part = lanes::butterfly_sum<16>(fmaf(qv, kv, lanes::other_half(kq_part)));
         if (lane == 0) s_kq[wave] = kq_part;
     }
     if (FUSED && (SPLIT_NORMS ? (tid >= DK && tid < 3 * DK) : tid < DK)) {
         float qq_part = qv * qv, kk_part = kv * kv;  // (one of them is 0 when the work is split)
         if (SPLIT_NORMS) {
-            float part = qq_part + kk_part;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off);
+            const float part = lanes::butterfly_sum<32>(qq_part + kk_part);
             if (lane == 0) (tid < 2 * DK ? s_qq : s_kk)[wave & 1] = part;
         } else {
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-                qq_part += __shfl_xor(qq_part, off);
-                kk_part += __shfl_xor(kk_part, off);
-            }
+            qq_part = lanes::butterfly_sum<16>(fmaf(qv, qv, lanes::other_half(qq_part)));
+            kk_part = lanes::butterfly_sum<16>(fmaf(kv, kv, lanes::other_half(kk_part)));
             if (lane == 0) {
                 s_qq[wave] = qq_part;
                 s_kk[wave] = kk_part;
@@ -211,13 +207,12 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
         c.x += s[m].x * qr;    c.y += s[m].y * qr;    c.z += s[m].z * qr;    c.w += s[m].w * qr;
     }
     // across the rows that share a wavefront (lane bits >= log2(CG))
-#pragma unroll
-    for (int off = 32; off >= CG; off >>= 1) {
-        a.x += __shfl_xor(a.x, off); a.y += __shfl_xor(a.y, off);
-        a.z += __shfl_xor(a.z, off); a.w += __shfl_xor(a.w, off);
-        c.x += __shfl_xor(c.x, off); c.y += __shfl_xor(c.y, off);
-        c.z += __shfl_xor(c.z, off); c.w += __shfl_xor(c.w, off);
-    }
+    auto across = [](float4& v) {
+        v.x = lanes::butterfly_sum<32, CG>(v.x), v.y = lanes::butterfly_sum<32, CG>(v.y);
+        v.z = lanes::butterfly_sum<32, CG>(v.z), v.w = lanes::butterfly_sum<32, CG>(v.w);
+    };
+    across(a);
+    across(c);
     if (lane < CG) {
         s_red[0][wave][lane] = a;
         s_red[1][wave][lane] = c;
@@ -261,9 +256,7 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
 
     if (NORM && r0 == 0) {
         // lanes 0..CG-1 (CG == 32: the lower half of wavefront 0) hold the head's 128 values
-        float ss = ov.x * ov.x + ov.y * ov.y + ov.z * ov.z + ov.w * ov.w;
-#pragma unroll
-        for (int off = CG / 2; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+        const float ss = lanes::butterfly_sum<16>(ov.x * ov.x + ov.y * ov.y + ov.z * ov.z + ov.w * ov.w);
         const float rinv = rsqrtf(ss * (1.f / DV) + norm_eps);
         auto gated = [&](float x, float w, float zz) { return w * (x * rinv) * (zz / (1.f + __expf(-zz))); };
         T* dst = o_norm + (size_t)unit * DV + cg * 4;

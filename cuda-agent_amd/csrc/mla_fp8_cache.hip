@@ -23,6 +23,7 @@
 #include <hip/hip_bf16.h>
 #include <stdint.h>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "mla_addressing.hpp"
 #include "moe_common.hpp"
@@ -76,8 +77,7 @@ __global__ __launch_bounds__(256) void mla_latent_quant_kernel(const __hip_bfloa
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = lanes::butterfly_max<8>(amax);
     const float scale = moe::group_scale(amax, pow2);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -moe::E4M3_MAX), moe::E4M3_MAX);

@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 
 namespace {
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void mla_index_scores_kernel(
 #pragma unroll
                     for (int j = 0; j < 16; ++j) total = fmaf(wf[ht][j / 4][j % 4], fmaxf(scale * acc[j], 0.f), total);
                 }
-                total += __shfl_xor(total, 32);
+                total = lanes::sum_of_halves(total);
             }
             const int t = t0 + row;
             if (half == 0 && t < n_rows) {
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(256) void mla_index_scores_fp8_kernel(
 #pragma unroll
                     for (int j = 0; j < 16; ++j) total = fmaf(wf[ht][j / 4][j % 4], fmaxf(scale * acc[j], 0.f), total);
                 }
-                total += __shfl_xor(total, 32);
+                total = lanes::sum_of_halves(total);
             }
             const int t = t0 + row;
             if (half == 0 && t < n_rows) {

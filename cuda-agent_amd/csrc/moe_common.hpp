@@ -6,6 +6,10 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#ifdef __HIPCC__
+#include "lane_exchange.hpp"
+#endif
+
 namespace moe {
 
 constexpr int GROUP = 128;            // quantisation group along K, and weight block edge
@@ -168,8 +172,7 @@ __device__ __forceinline__ void quantise_group16(const void* __restrict__ x, uin
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = lanes::butterfly_max<8>(amax);
     const float scale = group_scale(amax, pow2);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);

@@ -21,6 +21,7 @@
 // With few pairs per expert (decode) the kernel is a pure weight stream: every weight byte is
 // read once, used by one MFMA per 16 pairs, and the accumulators stay in registers. With many
 // pairs per expert it makes one pass per 16*NT pairs and re-reads the block from L2.
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "moe_common.hpp"
 
@@ -144,7 +145,7 @@ __device__ __forceinline__ void gate_up_epilogue(const floatx4 (&acc)[NT][4], fl
             }
         }
         amax = fmaxf(amax, __shfl_xor(amax, 16));
-        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        amax = lanes::max_of_halves(amax);
         if (g == 0) s_amax[wave][nt * 16 + col] = amax;
     }
     __syncthreads();
@@ -495,8 +496,7 @@ __global__ __launch_bounds__(256) void moe_stream_gemm_lds_kernel(
                         float amax = 0.f;
 #pragma unroll
                         for (int r = 0; r < 8; ++r) amax = fmaxf(amax, fabsf(v[r]));
-#pragma unroll
-                        for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+                        amax = lanes::butterfly_max<8>(amax);
                         const float scale = group_scale(amax, pow2);
 #pragma unroll
                         for (int r = 0; r < 8; ++r) v[r] = fminf(fmaxf(v[r] / scale, -E4M3_MAX), E4M3_MAX);

@@ -24,6 +24,7 @@
 // the bf16 matrix core, as the streaming form does and for its reason: the requantised h agrees with an fp32 evaluation
 // (1500 pairs of 7168 x 2048: 29 of 3.07 million codes are not those of a float64 evaluation, as in the streaming form;
 // 4624 with the 256-pair tiles, which repair the large ones).
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "moe_tile.hpp"
 
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(256, 2) void moe_narrow_gemm_kernel(
                 acc[0][b][i] = silu(acc[0][b][i]) * acc[1][b][i];
                 m = fmaxf(m, fabsf(acc[0][b][i]));
             }
-            m = fmaxf(m, __shfl_xor(m, 32));
+            m = lanes::max_of_halves(m);
             if (half == 0) s_amax[wave * PAIR_COLS + b * 32 + r32] = m;
         }
         __syncthreads();
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void moe_narrow_gemm_kernel(
             for (int a = 0; a < 2; ++a)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(acc[a][b][i]));
-            m = fmaxf(m, __shfl_xor(m, 32));
+            m = lanes::max_of_halves(m);
             if (half == 0) s_max[wave * PAIR_COLS + b * 32 + r32] = m;
         }
         __syncthreads();

@@ -23,6 +23,7 @@
 // for both operand reads. For gate/up the 256 rows are 128 gate rows and the matching 128 up
 // rows, each wavefront holding 32 of either, so SiLU(gate)*up and the e4m3 requantisation of
 // the 128-column group happen in the epilogue without leaving the workgroup.
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "moe_tile.hpp"
 
@@ -629,13 +630,13 @@ __global__ __launch_bounds__(512) void moe_tiled_gemm_kernel(
                 acc[0][b][i] = v;
                 m = fmaxf(m, fabsf(v));
             }
-            m = fmaxf(m, __shfl_xor(m, 32));
+            m = lanes::max_of_halves(m);
             const int at = rg * TILE_PAIRS + th * 128 + b * 32 + r32;
             if (half == 0) s_amax[at] = m;
             if constexpr (FIX) {
-                sumsq += __shfl_xor(sumsq, 32);
-                umax = fmaxf(umax, __shfl_xor(umax, 32));
-                sgmax = fmaxf(sgmax, __shfl_xor(sgmax, 32));
+                sumsq = lanes::sum_of_halves(sumsq);
+                umax = lanes::max_of_halves(umax);
+                sgmax = lanes::max_of_halves(sgmax);
                 if (half == 0) s_sumsq[at] = sumsq, s_umax[at] = umax, s_sgmax[at] = sgmax;
             }
         }
@@ -857,7 +858,7 @@ __global__ __launch_bounds__(512) void moe_tiled_gemm_kernel(
             for (int a = 0; a < 2; ++a)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(acc[a][b][i]));
-            m = fmaxf(m, __shfl_xor(m, 32));
+            m = lanes::max_of_halves(m);
             if (half == 0) s_max[rg * TILE_PAIRS + th * 128 + b * 32 + r32] = m;
         }
         __syncthreads();

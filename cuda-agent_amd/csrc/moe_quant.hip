@@ -6,6 +6,7 @@
 // nearest even but does not saturate (465 -> NaN), hence the clamp.
 #include <hip/hip_bf16.h>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "moe_common.hpp"
 
@@ -24,8 +25,7 @@ __global__ __launch_bounds__(256) void moe_quant_bf16_kernel(const __hip_bfloat1
     const float v0 = __uint_as_float(raw << 16);
     const float v1 = __uint_as_float(raw & 0xffff0000u);
     float amax = fmaxf(fabsf(v0), fabsf(v1));
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = lanes::butterfly_max<32>(amax);
     const float scale = group_scale(amax, pow2);
     const float a = fminf(fmaxf(v0 / scale, -E4M3_MAX), E4M3_MAX);
     const float b = fminf(fmaxf(v1 / scale, -E4M3_MAX), E4M3_MAX);
@@ -101,8 +101,7 @@ __device__ __forceinline__ void normalise_run(float (&v)[8], const float (&w)[8]
         if (j & 1) packed_y[j >> 1] |= bits << 16; else packed_y[j >> 1] = bits;
     }
     if (y != nullptr) *reinterpret_cast<uintx4*>(y + at) = uintx4{packed_y[0], packed_y[1], packed_y[2], packed_y[3]};
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = lanes::butterfly_max<8>(amax);
     const float scale = group_scale(amax, pow2);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);
@@ -148,8 +147,7 @@ __global__ __launch_bounds__(LANES) void moe_rmsnorm_quant_kernel(const __hip_bf
     };
     // the squares of 512 consecutive values, number `part` of the row
     auto add_squares = [&](float ss, int part) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+        ss = lanes::butterfly_sum<32>(ss);
         if (lane == 0) s_part[part] = ss;
     };
     auto row_rinv = [&]() {

@@ -40,6 +40,7 @@
 
 #include <atomic>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 #include "mla_addressing.hpp"
 
@@ -128,23 +129,6 @@ struct TileLoader {
         for (int i = 0; i < PER_WAVE; ++i) issue(tile, s_idx_tile, has_padding, i);
     }
 };
-
-// v of the lower and of the upper half of the wavefront, in both halves (on the vector ALU: a __shfl_xor is a trip through
-// the LDS crossbar)
-__device__ __forceinline__ void both_halves(float v, float& lower, float& upper) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    lower = __uint_as_float(r[0]), upper = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float max_of_halves(float v) {
-    float lower, upper;
-    both_halves(v, lower, upper);
-    return fmaxf(lower, upper);
-}
-__device__ __forceinline__ float sum_of_halves(float v) {
-    float lower, upper;
-    both_halves(v, lower, upper);
-    return lower + upper;
-}
 
 struct SoftmaxState {
     float m;  // reference exponent of the accumulator (log2 domain); same in lanes l and l^32
@@ -263,7 +247,7 @@ __device__ __forceinline__ void process_tile(const uint4* tile, const int* s_idx
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
-    tmax = max_of_halves(tmax);
+    tmax = lanes::max_of_halves(tmax);
 
     // Move the reference exponent only when this tile exceeds it by more than FRAME_SLACK (or
     // when it is still unset). alpha rescales what has been accumulated so far.
@@ -492,7 +476,7 @@ __global__ __launch_bounds__(64 * NW) void sparse_mla_split_kernel(
 #undef MLA_STEP
 
     // Epilogue: normalised partial output and log2-sum-exp
-    const float l_total = sum_of_halves(st.l);
+    const float l_total = lanes::sum_of_halves(st.l);
     const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
     if (lane < 32) lse_part[part0 + lane] = split_lse(st.m, l_total);
@@ -983,7 +967,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
-        tmax = max_of_halves(tmax);
+        tmax = lanes::max_of_halves(tmax);
         const bool move = tmax > st.m + FRAME_SLACK || st.m == -INFINITY;
         const float m_new = move ? tmax : st.m;
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -1055,7 +1039,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     // wavefront's half of dv (kept next to the log-sum-exp): half the bytes of fp32 for the split kernel to write and
     // the merge to read, and an error of at most 2^-12 of that magnitude.
     if (!live) return;
-    const float l_total = sum_of_halves(st.l);
+    const float l_total = lanes::sum_of_halves(st.l);
     const float inv_l = l_total == 0.f ? 0.f : 1.f / l_total;
     const size_t part0 = ((size_t)b * n_splits + split) * n_heads + head0;
     if (n_splits == 1) {
@@ -1096,7 +1080,7 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
     for (int t = 0; t < 8; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[t][i]));
-    amax = max_of_halves(amax);
+    amax = lanes::max_of_halves(amax);
     // exponent field of the bound + 1: 2^e > |O| for every element of the half (1 if it is 0)
     const float bound = amax * inv_l;
     uint32_t e_bits = ((__float_as_uint(bound) >> 23) & 255u) + 1u;
@@ -1184,7 +1168,7 @@ __global__ __launch_bounds__(NW > 4 ? 64 * NW : 256) void sparse_mla_merge_kerne
         float top = lse[0];
 #pragma unroll
         for (int i = 1; i < BATCH / 2; ++i) top = fmaxf(top, lse[i]);
-        top = fmaxf(mx, max_of_halves(top));
+        top = fmaxf(mx, lanes::max_of_halves(top));
         if (s0 != part) {
             const float alpha = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mx - top);  // (nothing yet, or NaN)
             wsum *= alpha;
@@ -1198,7 +1182,7 @@ __global__ __launch_bounds__(NW > 4 ? 64 * NW : 256) void sparse_mla_merge_kerne
             const float w = s0 + NW * (2 * i + half) >= n_splits || lse[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(lse[i] - mx);
             wsum += w;
             float ws[2];
-            both_halves(SCALED ? w * scale[i] : w, ws[0], ws[1]);  // (the scale is a power of two)
+            lanes::both_halves(SCALED ? w * scale[i] : w, ws[0], ws[1]);  // (the scale is a power of two)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t(&row)[WORDS] = rows[2 * i + h];
@@ -1218,7 +1202,7 @@ __global__ __launch_bounds__(NW > 4 ? 64 * NW : 256) void sparse_mla_merge_kerne
             }
         }
     }
-    wsum = sum_of_halves(wsum);
+    wsum = lanes::sum_of_halves(wsum);
     if constexpr (NW > 1) {
         __shared__ floatx4 s_o[NW > 4 ? NW : 4][2][64];
         __shared__ float s_mx[NW > 4 ? NW : 4][64], s_wsum[NW > 4 ? NW : 4][64];
