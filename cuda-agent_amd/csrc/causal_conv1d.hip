@@ -85,10 +85,9 @@ constexpr int channels_per_lane() {
     return CH_GRAIN;
 }
 
-constexpr int REQS = 4;  // requests per lane: their loads are issued together, weights read once
-
-// grid: x = blocks of 256 lanes over channels / CH, y = groups of REQS requests
-template <typename T, int L, int K>
+// grid: x = blocks of 256 lanes over channels / CH, y = groups of REQS requests, whose loads a lane issues together, the
+// weights read once
+template <typename T, int L, int K, int REQS>
 __global__ __launch_bounds__(256) void causal_conv1d_update_kernel(
     T* __restrict__ q_out, T* __restrict__ k_out, T* __restrict__ v_out, T* __restrict__ conv_state,
     const T* __restrict__ x, const T* __restrict__ weight, const T* __restrict__ bias, int batch,
@@ -154,8 +153,13 @@ void launch_lk(void* q_out, void* k_out, void* v_out, void* conv_state, const vo
                const void* weight, const void* bias, int batch, int channels, int key_dim,
                int activation, hipStream_t stream) {
     constexpr int CH = channels_per_lane<T, L>();
-    const dim3 grid((channels / CH + 255) / 256, (batch + REQS - 1) / REQS);
-    causal_conv1d_update_kernel<T, L, K><<<grid, 256, 0, stream>>>(
+    const int blocks = (channels / CH + 255) / 256;
+    // Four requests a lane where these fill the CUs twice over, else one: then the launch is as long as one lane's chain.
+    // us, convolution and step, one and four: 12 requests of 8192 channels 13.1, 13.6; 37 31.0, 31.4; 70 53.4, 53.7; 20 of 2048
+    // in fp32 9.2, 10.2; but 150 (608 workgroups of four) 108.4, 108.1, 250 177.6, 177.0.
+    const bool few = (long)blocks * ((batch + 3) / 4) < 512;
+    const auto kernel = few ? causal_conv1d_update_kernel<T, L, K, 1> : causal_conv1d_update_kernel<T, L, K, 4>;
+    kernel<<<dim3(blocks, few ? batch : (batch + 3) / 4), 256, 0, stream>>>(
         static_cast<T*>(q_out), static_cast<T*>(k_out), static_cast<T*>(v_out),
         static_cast<T*>(conv_state), static_cast<const T*>(x), static_cast<const T*>(weight),
         static_cast<const T*>(bias), batch, channels, key_dim, activation);

@@ -61,6 +61,19 @@ def test_matches_oracle(capi, dev, dtype, L, K, activation):
         assert_out_close(out, want)
 
 
+@pytest.mark.parametrize('batch', [1, 3, 4, 5, 2044, 2045, 2051])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_requests_per_lane(capi, dev, batch, dtype):
+    # one request a lane below 512 workgroups of four, and four
+    gen = torch.Generator().manual_seed(batch)
+    x, state, weight, bias = gdn.conv_make_inputs(batch, 16, 24, 4, 4, dtype, generator=gen)
+    want_state = state.clone()
+    want = gdn.causal_conv1d_update(x, want_state, weight, bias, 'silu')
+    out, new_state = run_kernel(capi, dev, x, state, weight, bias, 16, 'silu')
+    assert torch.equal(new_state, want_state)
+    assert_out_close(out, want)
+
+
 def test_golden_fixture(capi, dev):
     z = np.load(GOLDEN)
     for tag in 'abc':
