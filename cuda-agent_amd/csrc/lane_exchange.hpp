@@ -71,4 +71,21 @@ __device__ __forceinline__ float butterfly_max(float v) {
     return butterfly<FROM, TO>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
+// Inclusive prefix sum over the lanes of a wavefront: running sums inside each row of 16 lanes on DPP row
+// shifts (vector ALU; the __shfl_up form is six dependent trips through the LDS crossbar), then the totals of
+// the rows before a lane's own, read as scalars.
+__device__ __forceinline__ int inclusive_sum(int v, int lane) {
+#define ROW_SHR_ADD(n) v += __builtin_amdgcn_update_dpp(0, v, 0x110 + (n), 0xf, 0xf, false);
+    ROW_SHR_ADD(1)
+    ROW_SHR_ADD(2)
+    ROW_SHR_ADD(4)
+    ROW_SHR_ADD(8)
+#undef ROW_SHR_ADD
+    const int r0 = __builtin_amdgcn_readlane(v, 15);
+    const int r1 = __builtin_amdgcn_readlane(v, 31);
+    const int r2 = __builtin_amdgcn_readlane(v, 47);
+    const int row = lane >> 4;
+    return v + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
+}
+
 }  // namespace lanes

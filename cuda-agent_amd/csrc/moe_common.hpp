@@ -189,11 +189,7 @@ __device__ __forceinline__ void quantise_group16(const void* __restrict__ x, uin
 // Inclusive prefix sum of v over the 1024 lanes of a workgroup; wave_total: 16 ints of LDS.
 __device__ __forceinline__ int block_inclusive_scan(int v, int* wave_total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int add = __shfl_up(v, d);
-        if (lane >= d) v += add;
-    }
+    v = lanes::inclusive_sum(v, lane);
     __syncthreads();  // wave_total may still be read by the scan before
     if (lane == 63) wave_total[wave] = v;
     __syncthreads();

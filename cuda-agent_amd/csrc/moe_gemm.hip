@@ -99,12 +99,7 @@ struct ExpertList {
 #pragma unroll
         for (int i = 0; i < MOST; ++i) mask |= i < per && off[i + 1] > off[i] ? 1u << i : 0u;
         const int mine = __popc(mask);
-        int upto = mine;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int v = __shfl_up(upto, d);
-            if (lane >= d) upto += v;
-        }
+        const int upto = lanes::inclusive_sum(mine, lane);
         before = upto - mine;
         listed = __builtin_amdgcn_readlane(upto, 63);
     }

@@ -40,6 +40,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lane_exchange.hpp"
 #include "launch_status.hpp"
 
 namespace {
@@ -63,23 +64,6 @@ __device__ __forceinline__ uint32_t score_key(float x) {
 // the score with the smallest key that is at least `key` (key above that of -inf)
 __device__ __forceinline__ float key_score(uint32_t key) {
     return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
-}
-
-// Inclusive prefix sum over the lanes of a wavefront: running sums inside each row of 16 lanes on DPP row
-// shifts (vector ALU; the __shfl_up form is six dependent trips through the LDS crossbar), then the totals of
-// the rows before a lane's own, read as scalars.
-__device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
-#define ROW_SHR_ADD(n) v += __builtin_amdgcn_update_dpp(0, v, 0x110 + (n), 0xf, 0xf, false);
-    ROW_SHR_ADD(1)
-    ROW_SHR_ADD(2)
-    ROW_SHR_ADD(4)
-    ROW_SHR_ADD(8)
-#undef ROW_SHR_ADD
-    const int r0 = __builtin_amdgcn_readlane(v, 15);
-    const int r1 = __builtin_amdgcn_readlane(v, 31);
-    const int r2 = __builtin_amdgcn_readlane(v, 47);
-    const int row = lane >> 4;
-    return v + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
 // Sum of the entries of `sums` before entry `wave` (uniform). The 16 entries are scanned by the lanes of a row.
@@ -235,7 +219,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
             for (int h = 0; h < COPIES; ++h) c[j] += hist[(BINS - 1 - (PER * tid + j)) * COPIES + h];
             mine += c[j];
         }
-        const int upto = wave_inclusive_sum(mine, lane);
+        const int upto = lanes::inclusive_sum(mine, lane);
         if (lane == 63) s_wave_sum[0][wave] = upto;
         __syncthreads();
         int above = upto - mine + sum_before(s_wave_sum[0], wave, lane);
@@ -345,7 +329,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
 #pragma unroll
                         for (int j = g; j < g + GROUP; ++j) mine += v[j] >= pivot ? 1 : 0;
                     });
-                    const int upto = wave_inclusive_sum(mine, lane);
+                    const int upto = lanes::inclusive_sum(mine, lane);
                     const int total = __builtin_amdgcn_readlane(upto, 63);
                     if (total == 0) return;
                     int at = 0;
@@ -483,7 +467,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
                     int n_gt = 0, n_eq = 0;
                     for (int w = w0; w < w1; ++w) n_gt += __popc(s_gt[w]), n_eq += __popc(s_eq[w]);
                     // (at most MAX_CANDIDATES of either: one scan of the packed pair)
-                    const int upto = wave_inclusive_sum(n_gt | (n_eq << 16), lane);
+                    const int upto = lanes::inclusive_sum(n_gt | (n_eq << 16), lane);
                     if (lane == 63) s_wave_sum[0][wave] = upto;
                     __syncthreads();
                     const int before = upto - (n_gt | (n_eq << 16)) + sum_before(s_wave_sum[0], wave, lane);
@@ -594,7 +578,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void topk_select_kernel(
         const int in_word = left - 64 * lane;  // entries of the row in this lane's word
         ties &= in_word >= 64 ? ~0ull : in_word <= 0 ? 0ull : (1ull << in_word) - 1ull;
         const int n_gt = __popcll(word), n_eq = __popcll(ties);
-        const int gt_upto = wave_inclusive_sum(n_gt, lane), eq_upto = wave_inclusive_sum(n_eq, lane);
+        const int gt_upto = lanes::inclusive_sum(n_gt, lane), eq_upto = lanes::inclusive_sum(n_eq, lane);
         if (c0 > 0) __syncthreads();  // the sums of the chunk before have been read
         if (lane == 63) {
             s_wave_sum[0][wave] = gt_upto;
