@@ -1,7 +1,7 @@
 // Sums and maxima across lanes on the vector ALU: v_permlane32_swap and v_permlane16_swap between the halves and the rows of 16
 // lanes, DPP rotations inside a row. Every result is that of the butterfly `for (off = FROM; off >= TO; off /= 2) v = op(v,
-// __shfl_xor(v, off))` bit for bit, whose every step is a trip through the LDS crossbar of about 100 cycles (64 tokens
-// through the RMS norm with quantiser, ten such steps in a row: 4.4 -> 4.0 us).
+// __shfl_xor(v, off))` bit for bit, whose every step is a trip through the LDS crossbar of about 100 cycles (us, with those and
+// with these: a GDN layer step of 37 requests 34.2, 31.4; sparse attention of 64 requests over 32768 rows 166, 161).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
