@@ -24,8 +24,8 @@
 // product of two bf16 numbers is exact in fp32. With the weight stored once as those three planes the
 // projection of a bf16 x runs on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16: 8 times the rate of
 // the fp32 shape, three products per weight) and still differs from an fp32 reference by the order of the
-// additions only. At that rate the operand loads are what matters: rows are fetched as whole lines and
-// turned into the operand layout through a small LDS buffer private to the wavefront.
+// additions only. At that rate the operand loads are what matters: rows are fetched as whole lines into LDS, where the
+// wavefronts of a workgroup share them.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -152,10 +152,9 @@ typedef const __attribute__((address_space(3))) uint8_t* lds_bytes;
 // 3 x 32 of the planes, 128 bytes each = 20 KB) are on their way into LDS before the first is waited for. (8 lanes fetch the line of
 // a row, whose chunk p lies in slot p ^ ((row >> 1) & 7); a lane (row, half) of an operand holds values [32*half, +32) of its row, 8
 // per MFMA step.)
-// us, one chunk ahead through registers and 64 experts a workgroup, and this (norm, projection and routing in a row): 64 tokens of 7168 x
-// 256 18.9, 18.3; 200 22.2, 21.9; 128 of 4096 x 256 17.1, 16.9; 1500 of 4096 x 64 28.3, 28.0; the projection alone, 64 tokens 10.3, 9.0.
-constexpr int FETCHED_CHUNKS = 4;
-
+// us of the projection, one chunk ahead through registers and 64 experts a workgroup, and this: 64 tokens of 7168 x 256 11.0, 8.8;
+// 100 11.2, 10.0; 250 of 4096 x 128 10.2, 9.1; 1500 of 4096 x 64 15.3, 13.9; 1400 of 1024 x 256 14.0, 12.7.
+template <int FETCHED_CHUNKS>
 __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16_t* __restrict__ x,
                                                                     const uint16_t* __restrict__ planes,
                                                                     float* __restrict__ out, int tokens,
@@ -194,7 +193,7 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
     const bool multiplies = wave < 2 && t0 + 32 * wave < tokens;
     for (int c = 0; c < n; ++c) {
         // chunk c has arrived (those behind it may be in flight)
-        static_assert(FETCHED_CHUNKS == 4, "at most three chunks behind");
+        static_assert(FETCHED_CHUNKS <= 4, "at most three chunks behind");
         const int behind = min(FETCHED_CHUNKS - 1, n - 1 - c);
         if (behind == 3) __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (15 << 8));
         else if (behind == 2) __builtin_amdgcn_s_waitcnt(10 | (7 << 4) | (15 << 8));
@@ -238,8 +237,8 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
 }
 
 // The same product for many tokens: a workgroup of 4 wavefronts owns 128 tokens x 64 experts and shares its operand
-// tiles through LDS (per 64 values of k: 128 rows of x and 3 x 64 rows of planes, 128 bytes each = 40 KB). The per-wavefront
-// kernel above asks its CU's L1 for 170 bytes per clock at the bf16 MFMA rate; this one for 52.
+// tiles through LDS (per 64 values of k: 128 rows of x and 3 x 64 rows of planes, 128 bytes each = 40 KB). With a
+// tile of 32 x 32 per wavefront a CU's L1 is asked for 170 bytes per clock at the bf16 MFMA rate; here for 52.
 //
 // One wavefront per SIMD is all there is at 8192 tokens x 256 experts, so everything that takes time is requested
 // early: global -> LDS loads into a ring of three stages, two of them in flight, and the operands of chunk c+1 are read
@@ -247,7 +246,7 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
 // operand reads in front of the MFMAs a chunk took 2600 cycles (137 us for the 8192 x 256 logits
 // of hidden 7168); this takes 83 us, 1.1 PFLOP/s of bf16 products (with the norm's output of that
 // moment still to be written back, as in a layer, 87 to 98). With K split it also serves fewer tokens: 4096 tokens
-// 86 us on the per-wavefront kernel, 49 here; 1000: 27.7 and 21.9; 200: 15.5 and 13.2, the reduction included.
+// 85 us on the kernel above, 49 here; 1000: 24.7 and 21.5; 200: 14.6 and 12.5, the reduction included.
 constexpr int BIG_TOKENS = 128;
 constexpr int BIG_EXPERTS = 64;
 constexpr int BIG_STAGE = (BIG_TOKENS + 3 * BIG_EXPERTS) * K_CHUNK * 2;  // bytes (40 KB)
@@ -866,20 +865,27 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
     // Enough 128 x 64 tiles and splits to fill the chip: the workgroup-tiled kernel (config 2 forces it, 1 the other one).
     // It has one workgroup on a CU, so that a part of a second round costs a whole one, which few chunks of K do not make up
     // for, all the less where each has little to share (us, tiled and not; 1500 tokens of 4096 x 64, 384 workgroups of 2
-    // chunks: 17.3, 15.4; 1400 of 1024 x 256, 352 of 2: 15.9, 14.0; one tile of experts, 1200 of 7168 x 64, 320 of 4: 18.7,
-    // 17.9; a third of the rows padding, 160 of 7168 x 384, 384 of 4: 18.1, 17.0; but 300 of 7168 x 256, 384 of 4: 19.2, 20.7).
+    // chunks: 16.7, 13.7; 1400 of 1024 x 256, 352 of 2: 15.3, 12.7; one tile of experts, 1200 of 7168 x 64, 320 of 4: 18.1,
+    // 16.2; a third of the rows padding, 160 of 7168 x 384, 384 of 4: 17.7, 16.7; but 300 of 7168 x 256, 384 of 4: 18.4, 20.1).
     const long token_tiles = (tokens + BIG_TOKENS - 1) / BIG_TOKENS;
     const long big_wgs = token_tiles * ((n_experts + BIG_EXPERTS - 1) / BIG_EXPERTS) * splits;
     const bool part_of_second_round = big_wgs > 256 && big_wgs < 512;
     const bool few_chunks = chunks_per_split <= 2 ||
                             (chunks_per_split <= 4 && splits >= 16 && big_wgs < 448 &&
                              (n_experts <= BIG_EXPERTS || 3L * tokens < 2 * BIG_TOKENS * token_tiles));
-    const bool tiled = hidden <= (1 << 24) && (config == 2 || (config != 1 && big_wgs >= 192 && tokens >= BIG_TOKENS &&
+    const bool wide = n_experts > 32 * 65535;  // (more than a grid has tiles of 32 experts for)
+    const bool tiled = hidden <= (1 << 24) && (config == 2 || wide || (config != 1 && big_wgs >= 192 && tokens >= BIG_TOKENS &&
                                                               !(part_of_second_round && few_chunks)));
     float* out = splits > 1 ? static_cast<float*>(workspace) : logits;
     const int tile_tokens = tiled ? BIG_TOKENS : 64;
     const dim3 grid((tokens + tile_tokens - 1) / tile_tokens, tiled ? (n_experts + 63) / 64 : (n_experts + 31) / 32, splits);
-    const auto kernel = tiled ? moe_router_gemm_split_tiled_kernel : moe_router_gemm_split_kernel;
+    // Four chunks ahead are 80 KB of LDS, two workgroups to a CU; with more workgroups than that two chunks and four workgroups are
+    // faster (us, the projection alone with four and two: 100 tokens of 7168 x 384, 768 workgroups, 13.8, 12.6; 1200 of 7168 x 64
+    // 19.1, 16.2; 160 of 7168 x 384 18.1, 16.6), and two chunks in all need no more.
+    const bool two_ahead = chunks_per_split <= 2 || (long)grid.x * grid.y * grid.z > 512;
+    const auto kernel = tiled       ? moe_router_gemm_split_tiled_kernel
+                        : two_ahead ? moe_router_gemm_split_kernel<2>
+                                    : moe_router_gemm_split_kernel<4>;
     kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(planes), out, tokens,
                                      hidden, n_experts, chunks_per_split);
     if (splits > 1) {

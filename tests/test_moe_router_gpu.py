@@ -339,7 +339,9 @@ def test_few_tokens_in_one_launch(capi, dev, shape):
 
 @pytest.mark.parametrize('config', [1, 2])     # a wavefront for itself, and tiles of 128 tokens
 @pytest.mark.parametrize('shape', [(1, 64, 32), (100, 448, 72), (33, 128, 1), (96, 512, 64), (300, 2048, 72), (129, 192, 65),
-                                   (2100, 128, 130)])    # one split and several, tokens and experts beyond the last tile
+                                   (2100, 128, 130),    # one split and several, tokens and experts beyond the last tile
+                                   # more chunks than are fetched ahead: 512 workgroups (four ahead) and 528 (two)
+                                   (4090, 7168, 30), (4200, 7168, 30)])
 def test_kernels_of_the_split_weight(capi, dev, shape, config):
     check_parts(split_logits_of_config, capi, dev, shape, config)
 
