@@ -22,6 +22,7 @@
 // read once, used by one MFMA per 16 pairs, and the accumulators stay in registers. With many
 // pairs per expert it makes one pass per 16*NT pairs and re-reads the block from L2.
 #include "lane_exchange.hpp"
+#include "lds_load.hpp"
 #include "launch_status.hpp"
 #include "moe_common.hpp"
 
@@ -336,16 +337,7 @@ __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("" ::: "memory");  // LDS reads below must not be moved above the wait
 }
 
-// 64 lanes x 16 bytes: global (base + per-lane byte offset) -> LDS (lds_base + lane*16).
-// An asm statement, so the loads stay outside the compiler's bookkeeping of outstanding memory
-// operations; their completion is awaited explicitly with wait_vmcnt<>().
-__device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
-// The same load with the non-temporal hint, for weights that this launch reads exactly once (an expert whose
+// A load into LDS (awaited with wait_vmcnt<>()), with the non-temporal hint, for weights that this launch reads exactly once (an expert whose
 // pairs fit one pass): the stream then does not displace what the caches hold for others and runs 10 % faster
 // (decode layer 1.65 -> 1.48 ms); weights that a later pass reads again keep the plain load (with the hint a
 // 1024-token layer, two passes per expert, was 1.4 % slower). The choice is made once per stage: a branch per load cost
@@ -353,24 +345,16 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offse
 template <bool ONCE>
 __device__ __forceinline__ void dma16_stream(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
     if constexpr (ONCE) {
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                     :
-                     : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                     : "memory", "m0");
+        lds::dma16_once(base, lane_byte_offset, lds_base);
     } else {
-        dma16(base, lane_byte_offset, lds_base);
+        lds::dma16(base, lane_byte_offset, lds_base);
     }
 }
 template <bool B>
 struct Flag {
     static constexpr bool value = B;
 };
-__device__ __forceinline__ void dma16_ptr(const void* lane_ptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(lane_ptr), "s"(lds_base)
-                 : "memory", "m0");
-}
+using lds::dma16_ptr;
 
 // H_F32 (NT = 1): h stays in fp32 between the two GEMMs, in `h` [pairs, inter], and the down GEMM quantises it. With one
 // or two tokens the 128 columns that share a scale are too much for a workgroup: 8 experts x 16 of them leave half of the

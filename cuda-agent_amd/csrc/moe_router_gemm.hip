@@ -30,6 +30,7 @@
 #include <stdint.h>
 
 #include "launch_status.hpp"
+#include "lds_load.hpp"
 
 namespace {
 
@@ -181,11 +182,11 @@ __global__ __launch_bounds__(256) void moe_router_gemm_split_kernel(const uint16
     const size_t plane = (size_t)n_experts * hidden;
     const uint32_t lds0 = (uint32_t)(size_t)((lds_void_ptr)s_chunk) + wave * 1024;
     auto fetch = [&](int c) {
-        const uint32_t lds = lds0 + (c % FETCHED_CHUNKS) * CHUNK_BYTES;
+        const uint32_t at = lds0 + (c % FETCHED_CHUNKS) * CHUNK_BYTES;
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             const uint16_t* from = src[i < 2 ? i : 2] + (i < 2 ? 0 : (i - 2) * plane) + (size_t)c * K_CHUNK;
-            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds + i * 4096) : "memory", "m0");
+            lds::dma16_ptr(from, at + i * 4096);
         }
     };
     floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -253,14 +254,7 @@ constexpr int BIG_STAGE = (BIG_TOKENS + 3 * BIG_EXPERTS) * K_CHUNK * 2;  // byte
 constexpr int BIG_STAGES = 3;
 constexpr int BIG_LOADS = BIG_STAGE / 1024 / 4;  // load instructions of a wavefront per stage
 
-// 64 lanes x 16 bytes, global -> LDS (lds_base + lane*16). asm, so that later LDS reads are not made to wait for it: its
-// completion is awaited once per chunk.
-__device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
+using lds::dma16;  // (completion is awaited once per chunk)
 
 template <int N>
 struct IntConstant {

@@ -1,6 +1,7 @@
 // Device helpers shared by the MoE GEMMs whose workgroups stage weight rows and pair rows of one expert in LDS
 // (moe_gemm_tiled.hip, moe_gemm_narrow.hip): operand types, global -> LDS loads, and the mapping of workgroups to tiles.
 #pragma once
+#include "lds_load.hpp"
 #include "moe_common.hpp"
 
 namespace moe {
@@ -45,22 +46,8 @@ __device__ __forceinline__ void wait_all_loads() {
     asm volatile("" ::: "memory");
 }
 
-// 64 lanes x 16 bytes, global -> LDS (lds_base + lane*16); asm so that the compiler does not
-// make every later LDS read wait for it: completion is awaited once per block, before the barrier.
-__device__ __forceinline__ void dma16(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
-
-// The same with the non-temporal hint, for bytes that this launch reads once.
-__device__ __forceinline__ void dma16_once(const void* base, uint32_t lane_byte_offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                 :
-                 : "v"(lane_byte_offset), "s"(base), "s"(lds_base)
-                 : "memory", "m0");
-}
+using lds::dma16;  // (completion is awaited once per block, before the barrier)
+using lds::dma16_once;
 
 // The tile of a workgroup: row tile `rb` of expert `e`, pair tile number `pt` of the table (see
 // moe_tiled_prepare_kernel), which is tile `in_expert` of that expert's. False if there is none. Consecutive workgroup

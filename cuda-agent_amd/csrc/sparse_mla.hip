@@ -42,6 +42,7 @@
 
 #include "lane_exchange.hpp"
 #include "launch_status.hpp"
+#include "lds_load.hpp"
 #include "mla_addressing.hpp"
 
 namespace {
@@ -105,17 +106,11 @@ struct TileLoader {
         const int chunk = (pos & ~7) | ((pos ^ row_swizzle(row)) & 7);
         const int key = s_idx_tile[row];
         const char* src = kv_b + (size_t)(key < 0 ? 0 : key) * ROW_BYTES + chunk * 16;
-        // Each lane's 16 bytes land at lds_base + lane*16 (M0 carries the wavefront's base).
-        // Written as an asm statement so that the loads stay outside the compiler's own
-        // bookkeeping of outstanding memory operations: completion is awaited explicitly, per
-        // tile, by wait_vmcnt<>() in the main loop, and LDS reads of one tile do not wait
-        // for the loads of the tiles behind it.
+        // (completion is awaited explicitly, per tile, by wait_vmcnt<>() in the main loop: LDS reads of one tile do not wait
+        // for the loads of the tiles behind it)
         const uint32_t lds_base = (uint32_t)(size_t)((lds_void_ptr)(tile + inst * 64));
         if (!has_padding || key >= 0) {
-            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                         :
-                         : "v"(src), "s"(lds_base)
-                         : "memory", "m0");
+            lds::dma16_ptr(src, lds_base);
         } else {
             // Padding rows are zero-filled rather than fetched: their probabilities are 0, and
             // 0 times whatever a cache row happens to hold (NaN, Inf) would not be.
@@ -576,10 +571,7 @@ __device__ __forceinline__ void gather_issue(uint4* tile, const char* kv_b, uint
     if (!has_padding || off != GATHER_MASKED) {
         const uint32_t lds_base = (uint32_t)(size_t)((lds_void_ptr)dst);
         // (non-temporal: a selected row is read once per launch; 66.6 -> 65.1 us per step)
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                     :
-                     : "v"(off), "s"(kv_b), "s"(lds_base)
-                     : "memory", "m0");
+        lds::dma16_once(kv_b, off, lds_base);
     } else {
         dst[lane] = make_uint4(0u, 0u, 0u, 0u);
     }
@@ -618,10 +610,7 @@ __device__ __forceinline__ void gather_quarter_fp8(uint4* tile, const char* kv_b
 #pragma unroll
     for (int k = 0; k < FP8_GATHER_INSTR; ++k) {
         if (64 * k + 64 <= FP8_STAGE_CHUNKS || lane < FP8_STAGE_CHUNKS - 64 * k) {
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                         :
-                         : "v"(off[k]), "s"(kv_b), "s"(lds_base + 1024u * k)
-                         : "memory", "m0");
+            lds::dma16_once(kv_b, off[k], lds_base + 1024u * k);
         }
     }
 }

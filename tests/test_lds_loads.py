@@ -1,0 +1,59 @@
+"""CPU check of the built kernels: the wait states in front of the loads into LDS that are written as asm (csrc/lds_load.hpp),
+where the compiler puts none."""
+import os
+import re
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+PKG = Path(__file__).resolve().parent.parent / 'cuda-agent_amd'
+LIBRARIES = [PKG / 'lib' / 'libcuda_agent_amd.so', *(PKG / 'workspaces' / w / 'cuda_extension.so' for w in ('moe_fp8', 'sparse_mla'))]
+
+
+def kernel_instructions(library, folder):
+    """The instructions of every gfx950 code object of a library, in order, one list per object."""
+    rocm = os.environ.get('ROCM_PATH') or '/opt/rocm'
+    objdump = shutil.which('llvm-objdump') or f'{rocm}/llvm/bin/llvm-objdump'
+    copy = shutil.copy(library, folder)
+    subprocess.run([objdump, '--offloading', copy], cwd=folder, check=True, capture_output=True)
+    for obj in sorted(folder.glob('*gfx950')):
+        text = subprocess.run([objdump, '-d', '--no-show-raw-insn', obj], check=True, capture_output=True, text=True).stdout
+        yield [line.split('//')[0].strip() for line in text.splitlines() if line.startswith('\t')]
+
+
+def before(code, i, states):
+    """The instructions that can end less than `states` wait states before instruction i, in straight order."""
+    passed = 0
+    while i > 0 and passed < states:
+        i -= 1
+        if re.match(r's_(branch|endpgm|setpc)', code[i]):
+            return
+        nop = re.match(r's_nop (\w+)', code[i])
+        yield code[i]
+        passed += int(nop[1], 0) + 1 if nop else 1
+
+
+def faults(code):
+    """The loads into LDS that come too soon after a write of what they read, and how many there are."""
+    loads = [i for i, text in enumerate(code) if '_load_lds_' in text]
+    return [(code[i], text) for i in loads for text in before(code, i, 1) if re.match(r's_\w+ m0\b', text)], len(loads)
+
+
+def test_scan_finds_what_it_looks_for():
+    load = 'global_load_lds_dwordx4 v2, s[4:5]'
+    assert faults(['s_mov_b32 m0, s7', load]) == ([(load, 's_mov_b32 m0, s7')], 1)
+    assert faults(['s_mov_b32 m0, s7', 's_nop 0', load]) == ([], 1)
+    assert faults(['s_mov_b32 m0, s7', 's_add_u32 s4, s4, s6', load]) == ([], 1)
+
+
+@pytest.mark.parametrize('library', LIBRARIES, ids=lambda p: p.parent.name)
+def test_wait_states_before_loads_into_lds(library, tmp_path):
+    assert library.exists(), 'build first: python __graft_entry__.py'
+    loads = 0
+    for code in kernel_instructions(library, tmp_path):
+        found, n = faults(code)
+        assert not found, found[:5]
+        loads += n
+    assert loads > 100
