@@ -35,10 +35,33 @@ def before(code, i, states):
         passed += int(nop[1], 0) + 1 if nop else 1
 
 
+def scalar_registers(operand):
+    """Numbers of the scalar registers that `s7` or `s[6:7]` names (vcc, exec and anything else: none)."""
+    m = re.fullmatch(r's(\d+)|s\[(\d+):(\d+)\]', operand)
+    if m is None:
+        return set()
+    return {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+
+
+def written_by_vector_instruction(text):
+    """Scalar registers among the results of a vector instruction (the first operand, and the second of a carry out)."""
+    if not text.startswith('v_'):
+        return set()
+    operands = [o.strip() for o in text.split(None, 1)[1].split(',')] if ' ' in text else []
+    results = operands[:2] if re.match(r'v_(add|sub|subrev|addc|subb|subbrev)_co_|v_mad_[iu]64|v_div_scale', text) else operands[:1]
+    return set().union(*map(scalar_registers, results))
+
+
 def faults(code):
-    """The loads into LDS that come too soon after a write of what they read, and how many there are."""
+    """The loads into LDS that come too soon after a write of what they read, and how many there are: 1 wait state behind a
+    scalar write of M0, 5 behind a vector instruction's write of the scalar registers of the address."""
     loads = [i for i, text in enumerate(code) if '_load_lds_' in text]
-    return [(code[i], text) for i in loads for text in before(code, i, 1) if re.match(r's_\w+ m0\b', text)], len(loads)
+    found = []
+    for i in loads:
+        found += [(code[i], text) for text in before(code, i, 1) if re.match(r's_\w+ m0\b', text)]
+        read = set().union(*map(scalar_registers, re.findall(r's\[\d+:\d+\]|\bs\d+', code[i])))
+        found += [(code[i], text) for text in before(code, i, 5) if read & written_by_vector_instruction(text)]
+    return found, len(loads)
 
 
 def test_scan_finds_what_it_looks_for():
@@ -46,6 +69,11 @@ def test_scan_finds_what_it_looks_for():
     assert faults(['s_mov_b32 m0, s7', load]) == ([(load, 's_mov_b32 m0, s7')], 1)
     assert faults(['s_mov_b32 m0, s7', 's_nop 0', load]) == ([], 1)
     assert faults(['s_mov_b32 m0, s7', 's_add_u32 s4, s4, s6', load]) == ([], 1)
+    for write in ('v_readlane_b32 s5, v9, 3', 'v_readfirstlane_b32 s4, v1', 'v_cmp_gt_u32_e64 s[4:5], v1, v2',
+                  'v_add_co_u32 v1, s[4:5], v2, v3'):
+        assert faults([write, 's_mov_b32 m0, s7', 's_nop 2', load]) == ([(load, write)], 1)
+        assert faults([write, 's_mov_b32 m0, s7', 's_nop 3', load]) == ([], 1)
+    assert faults(['v_add_u32_e32 v1, s4, v2', 's_nop 0', load]) == ([], 1)
 
 
 @pytest.mark.parametrize('library', LIBRARIES, ids=lambda p: p.parent.name)
