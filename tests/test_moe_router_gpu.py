@@ -337,13 +337,19 @@ def test_few_tokens_in_one_launch(capi, dev, shape):
     check_parts(split_logits_of_config, capi, dev, shape, 4)
 
 
-@pytest.mark.parametrize('config', [1, 2])     # a wavefront for itself, and tiles of 128 tokens
+@pytest.mark.parametrize('config', [1, 2])     # workgroups of 64 tokens x 32 experts, and of 128 x 64
 @pytest.mark.parametrize('shape', [(1, 64, 32), (100, 448, 72), (33, 128, 1), (96, 512, 64), (300, 2048, 72), (129, 192, 65),
                                    (2100, 128, 130),    # one split and several, tokens and experts beyond the last tile
                                    # more chunks than are fetched ahead: 512 workgroups (four ahead) and 528 (two)
                                    (4090, 7168, 30), (4200, 7168, 30)])
 def test_kernels_of_the_split_weight(capi, dev, shape, config):
     check_parts(split_logits_of_config, capi, dev, shape, config)
+
+
+@pytest.mark.parametrize('config', [0, 1])
+def test_more_experts_than_tiles_of_32_fit_a_grid(capi, dev, config):
+    # ... go to the tiles of 64, also where the other kernel is asked for and for a single token
+    check_parts(split_logits_of_config, capi, dev, (1, 64, 32 * 65535 + 1), config)
 
 
 def test_bf16_parts_of_special_weights(capi, dev):
