@@ -154,7 +154,7 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
         kq_part = qv * kv;
     }
     if (tid < DK) {  // waves 0 and 1 (DK == 128): wavefront sum of k_i*q_i
-        // (the products of the first step are not rounded)
+        // (the lane's own product is not rounded before the first addition, its partner's is; likewise below)
         kq_part = lanes::butterfly_sum<16>(fmaf(qv, kv, lanes::other_half(kq_part)));
         if (lane == 0) s_kq[wave] = kq_part;
     }

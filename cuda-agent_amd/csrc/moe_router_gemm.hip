@@ -744,7 +744,9 @@ int pick_router_splits(int tokens, int hidden, int n_experts) {
     const long tiles = (long)((tokens + 63) / 64) * ((n_experts + 63) / 64);
     const int n_chunks = hidden / K_CHUNK;
     int splits = 1;
-    // aim at about two workgroups per CU; every split keeps at least 2 chunks
+    // Aims at two tiles of 64 x 64 per CU (the split weight's kernel for few workgroups has tiles of 64 x 32, twice as many). Splits
+    // of ceil(n_chunks / splits) chunks, two at least; where the division leaves a remainder the last ones have fewer or none: 112
+    // chunks in 32 splits are 28 of four and 4 that store zeros, which the reduction adds like any others.
     while (tiles * splits < 512 && splits * 2 * 2 <= n_chunks) splits *= 2;
     return splits;
 }

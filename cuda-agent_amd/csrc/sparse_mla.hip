@@ -1097,9 +1097,10 @@ __global__ __launch_bounds__(512) void sparse_mla_split8_kernel(
 }
 
 // out[b, h, :] = sum_s w_s o_part[b, s, h, :],  w_s = exp2(lse_s - max) / sum. A unit is registers 8j .. 8j+7 of a dv tile of 32
-// heads (16 dv of each, see PART_TILE): there are n_heads of them per request. NW wavefronts per unit, 4 / NW units per
-// workgroup (grid x = n_heads * NW / 4, y = request); wavefront i of a unit takes the splits i, i + NW, ..., BATCH of them
-// requested at once, relative to the largest log-sum-exp it has seen. PART is the type the split kernel stored: float,
+// heads (16 dv of each, see PART_TILE): there are n_heads of them per request. NW wavefronts per unit; a workgroup of
+// 4 takes 4 / NW units (grid x = n_heads * NW / 4, y = request), one of NW = 8 a single one (grid x = n_heads).
+// Wavefront i of a unit takes the splits i, i + NW, ..., BATCH of them requested at once, relative to the largest log-sum-exp
+// it has seen. PART is the type the split kernel stored: float,
 // or fp16 of O / scale with the scale of every head and half of dv in scale_part.
 // The kernel is a chain of memory latencies: with one request and 64 splits on one wavefront, 8 pieces at a
 // time and the log-sum-exps one after the other, it took 37 us, three times the split kernel before it. Above 8 splits four
