@@ -626,12 +626,13 @@ __global__ __launch_bounds__(512, 2) void moe_router_gemm_long_kernel(const uint
 // so small a product is the start and end of its launches and the latency of its loads, so there is no second kernel to add
 // partial sums, and a wavefront requests 7 chunks at once (224 KB of loads in flight on a CU). Rows are loaded by consecutive
 // lanes and turned into operands through LDS: with the operand's own 16 rows side by side in a load a CU took one lane a
-// clock, 16 bytes (16 tokens of 7168 x 256: 13.8 us instead of 6.9).
+// clock, 16 bytes (16 tokens of 7168 x 256, the same weight every time: 13.8 us instead of 6.9).
 // Sums: per wavefront, column and token, then over the wavefronts in ascending order, then lo + mid + hi; relative error
 // against float64 1.8e-7 (7168 x 256), as with splits of K.
 //
-// us, with K split over workgroups and so: 16 tokens of 7168 x 256 9.0, 6.9; 64 of 2048 x 128 7.6, 3.6; 64 of 4096 x 256 9.1,
-// 5.9; 128 of 7168 x 64 10.6, 6.9.
+// us, with K split over workgroups and so, six weights in turn: 16 tokens of 7168 x 256 9.1, 8.4; 48 10.0, 9.3; 64 of 2048 x 128
+// 6.1, 4.4; 64 of 4096 x 256 8.6, 7.3; 192 of 7168 x 64 9.6, 8.9. The same weight every time: 7.9, 7.2; 8.8, 8.8; 5.8, 3.8; 7.8,
+// 6.3; 8.7, 7.3.
 constexpr int FEW_TOKENS = 16;
 constexpr int FEW_EXPERTS = 5;
 constexpr int FEW_WAVES = 8;
@@ -854,8 +855,9 @@ extern "C" void moe_router_logits_split_launcher(float* logits, const void* x, c
     }
     // One launch where a round of workgroups does and what they fetch, each its 31 rows, is little enough for the
     // memory-side cache (norm, projection and routing in a row over changing inputs, us, K split and one launch: 48 tokens of
-    // 7168 x 256, 69 MB, 19.0, 18.1; 96 of 7168 x 128, as much, 19.0, 17.2; 64 of 7168 x 256, 92 MB, 19.1, 20.0; 64 of 4096 x
-    // 256, 208 workgroups, 16.7, 14.9; 80 of it, 260, 17.3, 20.0). Config 4 forces it.
+    // 7168 x 256, 69 MB, 18.2, 17.4; 56 of it, 92 MB, 18.5, 20.0; 96 of 7168 x 128, 69 MB, 17.8, 17.1; 112 of it, 81 MB, 18.0, 19.9;
+    // 192 of 7168 x 64, 69 MB, 17.1, 16.3; 208 of it, 75 MB, 17.6, 18.9, but 176, 64 MB, 17.0, 17.8; 64 of 4096 x 256, 208
+    // workgroups, 15.9, 14.5; 80 of it, 260, 17.0, 19.8). Config 4 forces it.
     const dim3 few((tokens + FEW_TOKENS - 1) / FEW_TOKENS, (n_experts + FEW_EXPERTS - 1) / FEW_EXPERTS);
     const long few_wgs = (long)few.x * few.y;
     const long few_bytes = few_wgs * (FEW_TOKENS + 3 * FEW_EXPERTS) * hidden * 2;
