@@ -1235,9 +1235,12 @@ __global__ __launch_bounds__(NW > 4 ? 64 * NW : 256) void sparse_mla_merge_kerne
     store_dv(out + ((size_t)b * n_heads + head) * D_V + 32 * tile, o, j8, half);
 }
 
-// Microseconds of a launch of `wgs` workgroups of `tiles` tiles each, one workgroup per CU at a time, as measured for
-// 128 heads: a workgroup starts and ends in 8 us on an empty chip and 15 on a full one (they compete for memory),
-// and takes 2.35 us per tile up to about 140 busy CUs, then more (memory again, and the clock), 3 on 256.
+// Microseconds of a launch of `wgs` workgroups of `tiles` tiles each, one workgroup per CU at a time, by which split counts are
+// compared; fitted to 128 heads: a workgroup starts and ends in 8 us on an empty chip and 15 on a full one (they compete for
+// memory), and takes 2.35 us per tile up to about 140 busy CUs, then more (memory again, and the clock), 3 on 256. Of long splits it
+// gives the time (us with the merge, modelled and measured: 200 requests of 2048 rows, one split 175, 173; 100 in two 103, 105);
+// start, end and merge of many short ones have become 3 to 10 us shorter than it says (64 in 4 72.5, 62.8; 24 in 8 41.5, 35.5; 8
+// in 22 28.2, 22.8; 1 in 64 18.2, 14.5).
 float split_kernel_us(int wgs, int tiles) {
     auto round_us = [&](int n) {
         const float crowd = n > 140 ? (n - 140) / 116.f : 0.f;
@@ -1264,15 +1267,18 @@ int max_splits(int batch, int head_groups, int topk, int config) {
 
 // The splits of a launch: config if it asks for a number, else the one with the least time for the split kernel and
 // the merge (5 us and 16 ns per partial of 128 heads; none for a single split). The maximum above puts a few
-// workgroups into a second round whenever the number of requests is not a divisor of 256: with it 24 requests of 2048
-// rows took 57 us, now 37; 48: 86, 58; 96: 136, 103; 150: 198, 164; 200: 211, 180; 4 requests (many partials): 28, 24.
-// The model is that of 128 heads over bf16 rows. For 32 and 64 heads and for e4m3 rows its choice was within 8 % of the
-// best of all counts, 5 % for most (1 to 256 requests, 512 and 2048 rows each): what a workgroup takes there to start, end
-// and fetch a tile is in about the same proportions.
+// workgroups into a second round whenever the number of requests is not a divisor of 256 (us, with it and so: 24 requests of
+// 2048 rows 50.5, 35.5; 48 80.7, 53.4; 100 139.1, 105.2; 150 188.3, 164.2; 200 194.8, 173.2; 4, many partials, 25.7, 19.9).
+// Against the best of all counts (1 to 200 requests of 512 and 2048 rows, bf16 and e4m3, 32, 64 and 128 heads: 144 calls) the
+// choice is within 5 % in 123. Of 2048 rows it is 10 % off at most (16 requests 29.0 in 13 splits, 26.5 in 8), of 512 24 % (64
+// requests 34.0 in 4, 27.5 in 2; 100 41.2 in 2, 35.0 in 1; 24 20.8 in 6, 18.0 in 4; 4 14.7 in 16, 13.3 in 8). Nearly all of these would
+// rather have fewer splits, whose error is larger (see takes_halves); with 32 heads 8 and 24 requests of 512 would have more (11.2 in 8,
+// 10.3 in 16; 13.9 in 6, 13.0 in 8).
 // few_on_one_wave: on the kernel with one wavefront per 32 heads, 32 or 64 heads take several times as long per tile and
 // leave a quarter of the partials, so that start and merge hardly count: as many splits of equal size as fit the CUs in
-// one round (64 heads, 16 requests of 2048 rows: 59 us with 16 splits, 67 with the model's 13; 24: 90 with 8 to 10, 129 with
-// 11, which is more than one round). For 128 heads on it the model is the better one (24 requests 62 us, with 10 splits 68).
+// one round (64 heads, 16 requests of 2048 rows: 45.2 us with 16 splits, 48.8 with the model's 13; 24: 64.7 with 8, 64.2 with 10,
+// 93.8 with 11, which is more than one round). For 128 heads on it the model is the better one (24 requests 60.0 us in 8 splits,
+// 62.0 in 10).
 int pick_splits(int batch, int head_groups, int topk, int config, bool few_on_one_wave) {
     const int most = max_splits(batch, head_groups, topk, config);
     if (config > 0) return most;
@@ -1297,9 +1303,9 @@ int pick_splits(int batch, int head_groups, int topk, int config, bool few_on_on
 
 // Whether the 8-wavefront kernel takes 128 heads and more in workgroups of 64, twice as many: where these fit the CUs in one
 // round. They take 1.3 to 2 us a tile instead of 2.4 to 3 and have half the Q to fetch, but fetch the rows twice, through one
-// L2. us, 128 and 64 heads a workgroup, bf16 and e4m3 rows: 1 request of 2048 rows 18.0, 16.6 and 18.4, 16.9; 4 24.4, 23.1 and
-// 24.5, 23.2; 16 of 256 17.1, 15.1 and 17.5, 15.2; 128 of 64 15.6, 13.7 and 15.8, 13.7; with 264 workgroups, 6 of 2048, 27.4,
-// 33.4 and 28.2, 34.0; with 300, 150 of 64, 15.8, 24.7 and 16.0, 24.2. 32 heads a workgroup were never more than 0.3 us better.
+// L2. us, 128 and 64 heads a workgroup, bf16 and e4m3 rows: 1 request of 2048 rows 15.8, 14.5 and 15.8, 14.8; 4 20.4, 19.5 and
+// 21.2, 21.1; 16 of 256 14.5, 12.7 and 14.6, 13.0; 128 of 64 15.8, 13.0 and 16.2, 13.3; with 264 workgroups, 6 of 2048, 23.6,
+// 28.3 and 24.4, 29.9; with 300, 150 of 64, 15.9, 22.8 and 16.4, 24.0. 32 heads a workgroup were never more than 0.3 us better.
 // The splits are those of 128 heads either way, and a head's result does not depend on its workgroup: with fewer splits, which
 // would suit the smaller workgroups, the error against float64 is larger (of the fp32 output, 8 requests of 2048 rows: 5.59e-4
 // with 22, 5.86e-4 with 16).
@@ -1410,7 +1416,9 @@ void launch_sparse_mla(void* out, const void* q, const void* kv, const int* idx,
     }
     if (!one_wave_per_group && splits == 1) return;  // (written by the split kernel)
     // Wavefronts per unit, and pieces requested at once per lane. Above 8 splits four wavefronts share a unit, unless the
-    // units (one per head) alone put 8 wavefronts on every CU: 16 requests of 128 heads and 13 splits 34.3 us in all with four, 32.1 with one.
+    // units (one per head) alone put 8 wavefronts on every CU (us in all with four and with one, 2048 rows: 16 requests of 128 heads,
+    // 13 splits, 28.5, 26.7; 20, 11 splits, 35.6, 34.4; 8, 22 splits, 21.8, 22.0; 10, 16 splits, 26.9 either way; 12, 16 splits, 28.0,
+    // 26.8).
     const bool heads_fill = (long)batch * n_heads >= 8 * 256;
 #define MLA_MERGE_FORM(OUT_T, PART_T, PARTS, SCALES, NW, BATCH)                                      \
     sparse_mla_merge_kernel<OUT_T, PART_T, NW, BATCH>                                                \
