@@ -40,18 +40,18 @@ METRIC = "GB/s & % HBM peak (GDN/MoE/MLA decode); fp8 TFLOP/s % MFMA peak (MoE p
 # holds each of these figures (a test checks that). None = not measured.
 # Stamp: taken from the library as built from the sources of this tree; a change to a kernel's data movement needs
 # a new run of the two commands in that file.
-MEASURED_TRAFFIC = {'gdn': 1085893000, 'moe_decode': 10002073000, 'mla': 238309000, 'index_scores': 553900000,
-                    'index_scores_fp8': 289712000, 'moe_prefill': 22387278000, 'mla_fp8_cache': 187647000,
-                    'topk_select': 9163000}
+MEASURED_TRAFFIC = {'gdn': 1086050000, 'moe_decode': 10002132000, 'mla': 237490000, 'index_scores': 553906000,
+                    'index_scores_fp8': 289713000, 'moe_prefill': 22403266000, 'mla_fp8_cache': 187894000,
+                    'topk_select': 9167000}
 # Matrix-pipe occupancy of the dominant kernels from rocprofv3 --pmc (SQ_VALU_MFMA_BUSY_CYCLES over 1024 SIMDs x
 # GRBM_GUI_ACTIVE cycles per XCD, the timed launches of bench.py's own loop; the derived MfmaUtil counter reads
-# 33.3 / 33.7 / 23.5 %) and the clock by GRBM_GUI_ACTIVE / 8 / duration in the same run (SQ_BUSY_CU_CYCLES / 256 /
+# 32.8 / 32.8 / 24.5 %) and the clock by GRBM_GUI_ACTIVE / 8 / duration in the same run (SQ_BUSY_CU_CYCLES / 256 /
 # duration for the short sparse-MLA kernel); the summary is profiles/moe_prefill_mla_matrix_core_counters_pmc.md.
 # Measured figures of that run, not of this one.
 MEASURED_MFMA = {
-    'moe_prefill': dict(mfma_busy=0.343, clock_ghz=1.97, kernel='moe_tiled_gemm_kernel<true> (gate/up)',
-                        mfma_busy_down=0.345, clock_ghz_down=1.84),
-    'mla': dict(mfma_busy=0.241, clock_ghz=2.05, kernel='sparse_mla_split8_kernel<false>'),
+    'moe_prefill': dict(mfma_busy=0.340, clock_ghz=1.99, kernel='moe_tiled_gemm_kernel<true> (gate/up)',
+                        mfma_busy_down=0.340, clock_ghz_down=1.94),
+    'mla': dict(mfma_busy=0.253, clock_ghz=1.99, kernel='sparse_mla_split8_kernel<false>'),
 }
 
 
