@@ -60,6 +60,18 @@ __device__ __forceinline__ void store_state(float* p, float4 x, bool nt) {
     }
 }
 
+// lanes::butterfly_sum, or the same sum by shuffles through the LDS crossbar
+template <bool SHUFFLED, int FROM, int TO>
+__device__ __forceinline__ float sum_across(float v) {
+    if constexpr (SHUFFLED) {
+#pragma unroll
+        for (int off = FROM; off >= TO; off /= 2) v += __shfl_xor(v, off);
+        return v;
+    } else {
+        return lanes::butterfly_sum<FROM, TO>(v);
+    }
+}
+
 // FUSED: q and k arrive unnormalised and are scaled by rsqrt(sum x^2 + 1e-6) here (the factors are
 // applied to the reductions, not to the 128 values); `g` and `beta` are then the per-request
 // gate inputs a and b, and g = exp(-exp(a_log[h]) * softplus(a + dt_bias[h])), beta = sigmoid(b).
@@ -67,7 +79,9 @@ __device__ __forceinline__ void store_state(float* p, float4 x, bool nt) {
 // NORM (needs COLS == DV, one workgroup per head): the layer's gated RMS normalisation of the read-out
 // is applied before it is stored: out = norm_w * o * rsqrt(mean(o^2) + eps) * silu(z), written in
 // the storage type of q/k/v to o_norm; the fp32 o is not written.
-template <typename T, int COLS, int THREADS, int NT, bool FUSED = false, bool NORM = false>
+//
+// SHUFFLED: the sums over the rows of a wavefront by shuffles. (Same result; see launch_variant.)
+template <typename T, int COLS, int THREADS, int NT, bool FUSED = false, bool NORM = false, bool SHUFFLED = false>
 __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
     float* __restrict__ o, float* __restrict__ state, const T* __restrict__ q,
     const T* __restrict__ k, const T* __restrict__ v, const float* __restrict__ g,
@@ -155,17 +169,17 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
     }
     if (tid < DK) {  // waves 0 and 1 (DK == 128): wavefront sum of k_i*q_i
         // (the lane's own product is not rounded before the first addition, its partner's is; likewise below)
-        kq_part = lanes::butterfly_sum<16>(fmaf(qv, kv, lanes::other_half(kq_part)));
+        kq_part = sum_across<SHUFFLED, 16, 1>(fmaf(qv, kv, lanes::other_half(kq_part)));
         if (lane == 0) s_kq[wave] = kq_part;
     }
     if (FUSED && (SPLIT_NORMS ? (tid >= DK && tid < 3 * DK) : tid < DK)) {
         float qq_part = qv * qv, kk_part = kv * kv;  // (one of them is 0 when the work is split)
         if (SPLIT_NORMS) {
-            const float part = lanes::butterfly_sum<32>(qq_part + kk_part);
+            const float part = sum_across<SHUFFLED, 32, 1>(qq_part + kk_part);
             if (lane == 0) (tid < 2 * DK ? s_qq : s_kk)[wave & 1] = part;
         } else {
-            qq_part = lanes::butterfly_sum<16>(fmaf(qv, qv, lanes::other_half(qq_part)));
-            kk_part = lanes::butterfly_sum<16>(fmaf(kv, kv, lanes::other_half(kk_part)));
+            qq_part = sum_across<SHUFFLED, 16, 1>(fmaf(qv, qv, lanes::other_half(qq_part)));
+            kk_part = sum_across<SHUFFLED, 16, 1>(fmaf(kv, kv, lanes::other_half(kk_part)));
             if (lane == 0) {
                 s_qq[wave] = qq_part;
                 s_kk[wave] = kk_part;
@@ -208,8 +222,8 @@ __global__ __launch_bounds__(THREADS) void gdn_decode_kernel(
     }
     // across the rows that share a wavefront (lane bits >= log2(CG))
     auto across = [](float4& v) {
-        v.x = lanes::butterfly_sum<32, CG>(v.x), v.y = lanes::butterfly_sum<32, CG>(v.y);
-        v.z = lanes::butterfly_sum<32, CG>(v.z), v.w = lanes::butterfly_sum<32, CG>(v.w);
+        v.x = sum_across<SHUFFLED, 32, CG>(v.x), v.y = sum_across<SHUFFLED, 32, CG>(v.y);
+        v.z = sum_across<SHUFFLED, 32, CG>(v.z), v.w = sum_across<SHUFFLED, 32, CG>(v.w);
     };
     across(a);
     across(c);
@@ -273,12 +287,24 @@ void launch_variant(float* o, float* state, const T* q, const T* k, const T* v, 
                     int n_v_heads, int n_qk_heads, hipStream_t stream) {
     const float scale = 0.08838834764831845f;  // 128^-1/2
     const dim3 grid(units * (DV / COLS));
+    // Sums through the LDS crossbar where all workgroups run at once, four to five on a CU (in fp32 three; of the plain step up to
+    // six): they read and write at the rate of the memory then, and those that finish their sums sooner get in the way of the loads of the
+    // others. us on the vector ALU and so, states in the memory-side cache, and not: 272 units in bf16 6.9, 6.8 and 7.3, 7.0; 320 7.2, 7.0
+    // and 7.6, 7.5; pre-step fused 272 7.7, 7.1 and 7.9, 7.5; 320 8.2, 7.5 and 8.4, 8.0; fp32 288 8.1, 7.8 and 9.0, 8.6; fused 240 6.4,
+    // 6.2 and 7.2, 6.9; 320 9.1, 8.5 and 9.6, 9.4; 352 plain 10.3, 9.9 and 10.8, 10.7. Outside: 64 in bf16 3.2, 3.5 and 3.7, 3.8;
+    // fused 3.4, 3.9 and 3.8, 4.2; 176 plain 4.8, 5.0, but 5.6, 5.3; fused 5.0, 5.3 and 5.2, 5.4; 400 10.7, 10.8 and 11.0, 11.1.
+    constexpr bool SMALL = COLS == 32 && NT == 1;  // the tiles of few heads
+    const bool shuffled = SMALL && units > (sizeof(T) == 4 ? 192 : 256) && units <= (a_log ? 320 : 384);
     if (a_log) {
-        gdn_decode_kernel<T, COLS, THREADS, NT, true><<<grid, THREADS, 0, stream>>>(
-            o, state, q, k, v, g, beta, n_v_heads, n_qk_heads, scale, a_log, dt_bias);
+        const auto kernel = shuffled ? gdn_decode_kernel<T, COLS, THREADS, NT, true, false, SMALL>
+                                     : gdn_decode_kernel<T, COLS, THREADS, NT, true>;
+        kernel<<<grid, THREADS, 0, stream>>>(o, state, q, k, v, g, beta, n_v_heads, n_qk_heads, scale, a_log, dt_bias,
+                                             nullptr, nullptr, 0.f, nullptr);
     } else {
-        gdn_decode_kernel<T, COLS, THREADS, NT, false><<<grid, THREADS, 0, stream>>>(
-            o, state, q, k, v, g, beta, n_v_heads, n_qk_heads, scale);
+        const auto kernel = shuffled ? gdn_decode_kernel<T, COLS, THREADS, NT, false, false, SMALL>
+                                     : gdn_decode_kernel<T, COLS, THREADS, NT, false>;
+        kernel<<<grid, THREADS, 0, stream>>>(o, state, q, k, v, g, beta, n_v_heads, n_qk_heads, scale, nullptr, nullptr,
+                                             nullptr, nullptr, 0.f, nullptr);
     }
 }
 

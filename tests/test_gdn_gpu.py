@@ -171,6 +171,22 @@ def test_fused_matches_oracle(capi, dev, shape, config):
     assert gdn.gdn_close(o, want_o) and gdn.gdn_close(s, want_s)
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('batch', [48, 49, 64, 65, 80, 81, 96, 97])
+def test_sums_by_shuffles_are_the_same_sums(capi, dev, batch, dtype):
+    # With 4 heads: the edges of the sizes (193 or 257 to 320 heads of all requests, 384 of the plain step) whose sums go through the LDS
+    # crossbar. A request's result is the oracle's, and that of a call with few requests bit for bit
+    gen = torch.Generator().manual_seed(batch)
+    for make, run, step in ((gdn.gdn_make_inputs, run_kernel, gdn.gdn_decode_step),
+                            (gdn.gdn_make_raw_inputs, run_fused, gdn.gdn_decode_fused_step)):
+        ins = make(batch, 4, 2, qkv_dtype=dtype, generator=gen)
+        o, s = run(capi, dev, ins)
+        want_o, want_s = step(*ins[:-1], ins[-1].clone())
+        assert gdn.gdn_close(o, want_o) and gdn.gdn_close(s, want_s)
+        parts = [run(capi, dev, [t[at:at + 24] if t.shape[0] == batch else t for t in ins]) for at in range(0, batch, 24)]
+        assert torch.equal(o, torch.cat([p[0] for p in parts])) and torch.equal(s, torch.cat([p[1] for p in parts]))
+
+
 def test_fused_golden_fixture(capi, dev):
     z = np.load(FUSED_GOLDEN)
     ins = [torch.from_numpy(z[n]) for n in ('q', 'k', 'v', 'a', 'b', 'a_log', 'dt_bias', 'state')]
