@@ -158,6 +158,8 @@ __device__ __forceinline__ float group_scale(float amax, bool pow2) {
 // Activation quantisation of one 128-wide group by 16 lanes, 8 values (16 bytes in, 8 codes out) each; `sub` is the
 // lane's number among them. The division is IEEE fp32 so that the codes are bit-identical to a CPU evaluation of the
 // same formula; v_cvt_pk_fp8_f32 rounds to nearest even but does not saturate (465 -> NaN), hence the clamp.
+// SHUFFLED: the maximum by shuffles through the LDS crossbar (see moe_quant_bf16_launcher).
+template <bool SHUFFLED = false>
 __device__ __forceinline__ void quantise_group16(const void* __restrict__ x, uint8_t* __restrict__ q,
                                                  float* __restrict__ scales, long group, int sub, bool pow2) {
     typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
@@ -172,7 +174,12 @@ __device__ __forceinline__ void quantise_group16(const void* __restrict__ x, uin
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    amax = lanes::butterfly_max<8>(amax);
+    if constexpr (SHUFFLED) {
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    } else {
+        amax = lanes::butterfly_max<8>(amax);
+    }
     const float scale = group_scale(amax, pow2);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = fminf(fmaxf(v[j] / scale, -E4M3_MAX), E4M3_MAX);

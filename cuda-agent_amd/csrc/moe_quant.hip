@@ -35,12 +35,13 @@ __global__ __launch_bounds__(256) void moe_quant_bf16_kernel(const __hip_bfloat1
 }
 
 // Same result with 16 lanes per group: a lane loads 8 values (16 bytes) and stores 8 codes.
+template <bool SHUFFLED>
 __global__ __launch_bounds__(256) void moe_quant_bf16_vec_kernel(const __hip_bfloat16* __restrict__ x,
                                                                  uint8_t* __restrict__ q,
                                                                  float* __restrict__ scales,
                                                                  long n_groups, bool pow2) {
     const long g = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
-    if (g < n_groups) quantise_group16(x, q, scales, g, threadIdx.x & 15, pow2);
+    if (g < n_groups) quantise_group16<SHUFFLED>(x, q, scales, g, threadIdx.x & 15, pow2);
 }
 
 }  // namespace
@@ -62,7 +63,14 @@ extern "C" void moe_quant_bf16_launcher(void* q, float* scales, const void* x, i
     }
     const long n_groups = (long)rows * (cols / GROUP);
     if (!(reinterpret_cast<uintptr_t>(x) & 15u) && !(reinterpret_cast<uintptr_t>(q) & 7u)) {
-        moe_quant_bf16_vec_kernel<<<dim3((unsigned)((n_groups + 15) / 16)), 256, 0, stream>>>(
+        // The maximum of a group through the LDS crossbar where the workgroups are five to thirty to a CU: wavefronts that wait
+        // for it leave the vector ALU to those that have yet to request their values. us on the vector ALU and so, x in the caches,
+        // and not: 24000 groups 3.5, 3.5 and 4.2, 4.1; 32768 4.0, 3.9 and 4.8, 4.6; 40000 5.1, 4.9 and 5.6, 5.5; 64000 6.9, 6.6 and 7.6,
+        // 7.5; 80000 7.9, 7.5 and 8.7 either way; 112000 9.7, 9.4 and 11.3 either way; but 16000 2.9, 2.9 and 3.5, 3.5; 168000 12.9, 12.8
+        // and 15.2, 15.7.
+        const bool shuffled = n_groups > 16 * 5 * 256 && n_groups <= 16 * 30 * 256;
+        const auto kernel = shuffled ? moe_quant_bf16_vec_kernel<true> : moe_quant_bf16_vec_kernel<false>;
+        kernel<<<dim3((unsigned)((n_groups + 15) / 16)), 256, 0, stream>>>(
             static_cast<const __hip_bfloat16*>(x), static_cast<uint8_t*>(q), scales, n_groups, pow2);
         return;
     }

@@ -126,6 +126,24 @@ def test_activation_quantisation_bit_exact(capi, dev):
     assert torch.equal(q.cpu().view(torch.uint8), want_q.view(torch.uint8))
 
 
+@pytest.mark.parametrize('groups', [20480, 20481, 122879, 122880, 122881])
+def test_quantisation_of_a_group_does_not_depend_on_how_many_there_are(capi, dev, groups):
+    # its maximum goes through the LDS crossbar from 20481 to 122880 groups; NaN and infinities included
+    gen = torch.Generator().manual_seed(groups)
+    x = (torch.randn(groups, 128, generator=gen) * 3).bfloat16()
+    x[-2] = 0
+    q = torch.empty(groups, 128, dtype=torch.uint8, device=dev)
+    s = torch.empty(groups, 1, device=dev)
+    capi.moe_quant_bf16_launch(q, s, x.to(dev))
+    want_q, want_s = moe.quantize_groups(x.float())
+    assert torch.equal(s.cpu(), want_s) and torch.equal(q.cpu(), want_q.view(torch.uint8))
+    x[0, 5], x[1, 127], x[2, 64], x[3] = float('nan'), float('inf'), float('-inf'), float('nan')
+    capi.moe_quant_bf16_launch(q, s, x.to(dev))
+    few_q, few_s = torch.empty(64, 128, dtype=torch.uint8, device=dev), torch.empty(64, 1, device=dev)
+    capi.moe_quant_bf16_launch(few_q, few_s, x[:64].to(dev))
+    assert torch.equal(q[:64], few_q) and torch.equal(s[:64].view(torch.int32), few_s.view(torch.int32))
+
+
 @pytest.mark.parametrize('shape', [(1, 128, 1), (3, 1024, 8), (5, 1152, 9), (2, 2304, 17)])    # batches of eight rows, 1024 columns
 def test_combine_rows_and_columns(capi, dev, shape):
     T, H, k = shape
