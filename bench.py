@@ -41,7 +41,7 @@ METRIC = "GB/s & % HBM peak (GDN/MoE/MLA decode); fp8 TFLOP/s % MFMA peak (MoE p
 # Stamp: taken from the library as built from the sources of this tree; a change to a kernel's data movement needs
 # a new run of the two commands in that file.
 MEASURED_TRAFFIC = {'gdn': 1086050000, 'moe_decode': 10002132000, 'mla': 237490000, 'index_scores': 553906000,
-                    'index_scores_fp8': 289713000, 'moe_prefill': 22403266000, 'mla_fp8_cache': 187894000,
+                    'index_scores_fp8': 289713000, 'moe_prefill': 22403266000, 'mla_fp8_cache': 186829000,
                     'topk_select': 9167000}
 # Matrix-pipe occupancy of the dominant kernels from rocprofv3 --pmc (SQ_VALU_MFMA_BUSY_CYCLES over 1024 SIMDs x
 # GRBM_GUI_ACTIVE cycles per XCD, the timed launches of bench.py's own loop; the derived MfmaUtil counter reads

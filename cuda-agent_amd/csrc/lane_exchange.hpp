@@ -1,7 +1,9 @@
 // Sums and maxima across lanes on the vector ALU: v_permlane32_swap and v_permlane16_swap between the halves and the rows of 16
 // lanes, DPP rotations inside a row. Every result is that of the butterfly `for (off = FROM; off >= TO; off /= 2) v = op(v,
 // __shfl_xor(v, off))` bit for bit, whose every step is a trip through the LDS crossbar of about 100 cycles (us, with those and
-// with these: a GDN layer step of 37 requests 34.2, 31.4; sparse attention of 64 requests over 32768 rows 166, 161).
+// with these: a GDN layer step of 37 requests 34.2, 31.4; sparse attention of 64 requests over 32768 rows 166, 161). They are not the
+// faster ones everywhere: where a chip full of wavefronts is bound by memory, those that finish sooner can be in the way of the
+// others' loads (gdn_decode.hip, moe_quant.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
